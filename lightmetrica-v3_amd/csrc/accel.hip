@@ -554,15 +554,15 @@ constexpr int kPrivDepth = 72;
 // trace_persistent). `next` is this launch's ray counter, zeroed by
 // k_zero_counter on the same stream.
 template <int W, bool ANY, bool COUNT, class Node>
-__global__ __launch_bounds__(kTraceBlock) void k_trace(const Node* __restrict__ nodes,
+__global__ __launch_bounds__(kTraceBlock, 6) void k_trace(const Node* __restrict__ nodes,
                                                         const TriV* __restrict__ tris,
                                                         const lmgpu_ray* __restrict__ rays,
                                                         lmgpu_hit* __restrict__ hits, uint8_t* __restrict__ occl,
-                                                        int64_t n, unsigned long long* __restrict__ next,
+                                                        uint32_t n, unsigned long long* __restrict__ next,
                                                         int32_t* __restrict__ status,
                                                         unsigned long long* __restrict__ counters, int refill) {
-    __shared__ int lds[kLdsDepth][kTraceBlock];
-    auto fetch = [&](int64_t id, f3& o, f3& d, float& tmin, float& tmax) -> int {
+    __shared__ int lds[kLdsDepth + 1][kTraceBlock];
+    auto fetch = [&](uint32_t id, f3& o, f3& d, float& tmin, float& tmax) -> int {
         const float4* rp = reinterpret_cast<const float4*>(rays + id);
         const float4 a = rp[0], c = rp[1];
         o = mk(a.x, a.y, a.z);
@@ -571,7 +571,7 @@ __global__ __launch_bounds__(kTraceBlock) void k_trace(const Node* __restrict__ 
         tmax = c.w;
         return 0;
     };
-    auto emit = [&](int64_t id, const TraceResult& r) {
+    auto emit = [&](uint32_t id, const TraceResult& r) {
         if (ANY) {
             occl[id] = r.prim >= 0 ? 1 : 0;
         } else {
@@ -873,11 +873,15 @@ template <int W, bool ANY, bool COUNT>
 static void launch_trace(const Accel& a, const lmgpu_ray* rays, lmgpu_hit* hits, uint8_t* occl, int64_t n,
                          unsigned long long* next, int32_t* status, unsigned long long* counters, hipStream_t s) {
     using Node = typename TravNode<W>::type;
-    hipLaunchKernelGGL(k_zero_counter, dim3(1), dim3(64), 0, s, next);
-    const int grid = int(std::min<int64_t>(persistent_grid<W, ANY, COUNT, Node>(), (n + kTraceBlock - 1) / kTraceBlock));
-    hipLaunchKernelGGL((k_trace<W, ANY, COUNT, Node>), dim3(grid), dim3(kTraceBlock), 0, s,
-                       static_cast<const Node*>(a.trav_nodes()), a.tris.p, rays, hits, occl, n, next, status, counters,
-                       a.refill);
+    // one launch for all but batches of over 2^30 rays (ray ids are 32 bits on the device)
+    for (int64_t at = 0; at < n; at += kMaxLaunchRays) {
+        const int64_t m = std::min(n - at, kMaxLaunchRays);
+        hipLaunchKernelGGL(k_zero_counter, dim3(1), dim3(64), 0, s, next);
+        const int grid = int(std::min<int64_t>(persistent_grid<W, ANY, COUNT, Node>(), (m + kTraceBlock - 1) / kTraceBlock));
+        hipLaunchKernelGGL((k_trace<W, ANY, COUNT, Node>), dim3(grid), dim3(kTraceBlock), 0, s,
+                           static_cast<const Node*>(a.trav_nodes()), a.tris.p, rays + at, hits ? hits + at : nullptr,
+                           occl ? occl + at : nullptr, uint32_t(m), next, status, counters, a.refill);
+    }
 }
 
 int Accel::trace(const lmgpu_ray* rays, lmgpu_hit* hits, uint8_t* occl, int64_t n, bool any,

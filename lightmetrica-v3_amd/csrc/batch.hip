@@ -206,15 +206,15 @@ __global__ __launch_bounds__(BLOCK) void k_b_regen(const JobDev* __restrict__ jo
 }
 
 template <int W>
-__global__ __launch_bounds__(kBlock) void k_b_extend(const typename TravNode<W>::type* __restrict__ nodes,
+__global__ __launch_bounds__(kBlock, 6) void k_b_extend(const typename TravNode<W>::type* __restrict__ nodes,
                                                      const TriV* __restrict__ tris,
                                                      const JobDev* __restrict__ jobs, PoolDev P, BatchQ q, int in_q,
                                                      unsigned long long* next, int refill, BatchCtl* ctl) {
-    __shared__ int lds[kLds][kBlock];
+    __shared__ int lds[kLds + 1][kBlock];
     const int n = q.counts[in_q];
     if (n == 0) return;   // an idle iteration after the last work item (whole grid)
     const lmgpu_ray* rays = q.ext[in_q];
-    auto fetch = [&](int64_t id, f3& o, f3& d, float& tmin, float& tmax) -> int {
+    auto fetch = [&](uint32_t id, f3& o, f3& d, float& tmin, float& tmax) -> int {
         const float4* rp = reinterpret_cast<const float4*>(rays + id);
         const float4 a = rp[0], b = rp[1];
         o = mk(a.x, a.y, a.z);
@@ -223,7 +223,7 @@ __global__ __launch_bounds__(kBlock) void k_b_extend(const typename TravNode<W>:
         tmax = b.w;
         return jobs[P.job[q.ext_path[in_q][id]]].root;
     };
-    auto emit = [&](int64_t id, const TraceResult& r) {
+    auto emit = [&](uint32_t id, const TraceResult& r) {
         reinterpret_cast<float4*>(q.hit)[id] = make_float4(__int_as_float(r.overflow ? -2 : r.prim), r.t, r.u, r.v);
     };
     trace_persistent<W, false, false, kLds, kPriv, kBlock>(nodes, tris, n, next, lds, fetch, emit, q.counts + 5,
@@ -419,15 +419,15 @@ __global__ void k_b_ggate(int32_t* tcount, int32_t* tready, int32_t* nfin, int n
 }
 
 template <int W, bool GUIDED>
-__global__ __launch_bounds__(kBlock) void k_b_connect(const typename TravNode<W>::type* __restrict__ nodes,
+__global__ __launch_bounds__(kBlock, 6) void k_b_connect(const typename TravNode<W>::type* __restrict__ nodes,
                                                       const TriV* __restrict__ tris,
                                                       const JobDev* __restrict__ jobs, PoolDev P, BatchQ q,
                                                       unsigned long long* next, int refill, BatchCtl* ctl,
                                                       GRec* __restrict__ rec, const int32_t* __restrict__ sh_rec) {
-    __shared__ int lds[kLds][kBlock];
+    __shared__ int lds[kLds + 1][kBlock];
     const int n = q.counts[2];
     if (n == 0) return;   // no shadow rays this iteration (whole grid)
-    auto fetch = [&](int64_t id, f3& o, f3& d, float& tmin, float& tmax) -> int {
+    auto fetch = [&](uint32_t id, f3& o, f3& d, float& tmin, float& tmax) -> int {
         const float4* rp = reinterpret_cast<const float4*>(q.sh + id);
         const float4 a = rp[0], b = rp[1];
         o = mk(a.x, a.y, a.z);
@@ -436,7 +436,7 @@ __global__ __launch_bounds__(kBlock) void k_b_connect(const typename TravNode<W>
         tmax = b.w;
         return jobs[P.job[__float_as_int(q.sh_contrib[id].w)]].root;
     };
-    auto emit = [&](int64_t id, const TraceResult& r) {
+    auto emit = [&](uint32_t id, const TraceResult& r) {
         if (r.prim < 0 && !r.overflow) {
             const float4 c = q.sh_contrib[id];
             const int s = __float_as_int(c.w);

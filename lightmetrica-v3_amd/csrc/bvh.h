@@ -18,7 +18,7 @@
 #include "common.h"
 #include "../../include/lmgpu.h"
 
-// Wave-level step vote of the persistent traversal, in quarters (0 = off):
+// Wave-level step vote of the persistent traversal, in quarters:
 // a wave takes a leaf step when at least LMGPU_LEAF_VOTE_X4 / 4 times as
 // many of its busy lanes sit at a leaf as at an inner node (see
 // trace_persistent). 2 measured best on the 1.32M-triangle mesh (incoherent
@@ -62,7 +62,9 @@ static_assert(sizeof(WNode<4>) == 128, "BVH4 node must be one 128-B line");
 // superset of the nodes of the FP32 tree: hits are unchanged. Child c's
 // lower / upper plane on axis a is byte c % 4 of qlo[a][c / 4] / qhi[a][c / 4];
 // ent[c] is its stack entry (inner node index >= 0, or
-// encode_leaf(first, count) < 0), kQEmpty for an empty slot.
+// encode_leaf(first, count) < 0), kQEmpty, a leaf of no triangles, for an
+// empty slot (whose planes are stored inverted, so that a ray meets it only
+// within the slack of a flat node).
 template <int W>
 struct alignas(W * 16) QNode {
     float ox, oy, oz;
@@ -70,12 +72,13 @@ struct alignas(W * 16) QNode {
     uint32_t qlo[3][W / 4];
     uint32_t qhi[3][W / 4];
     int32_t ent[W];
-    int32_t pad[W == 4 ? 2 : 8];
+    uint32_t es;       // the grid exponents again, unbiased: signed bytes 0, 1, 2
+    float slack;       // 2^-20 * 255 * the largest step: part of the slab test's rounding bound
 };
 using QNode4 = QNode<4>;
 static_assert(sizeof(QNode<4>) == 64, "quantised BVH4 node must be 64 B");
 static_assert(sizeof(QNode<8>) == 128, "quantised BVH8 node must be 128 B");
-constexpr int32_t kQEmpty = INT32_MIN;
+constexpr int32_t kQEmpty = -1;   // encode_leaf(0, 0)
 
 // Node type the traversal of a W-wide BVH reads.
 template <int W>
@@ -106,6 +109,7 @@ LMGPU_HD int leaf_count(int e) { return (-(e + 1)) & 15; }
 
 struct RayPre {
     f3 o, d, inv;
+    f3 bn, bf;       // -o inv lowered / raised by 2^-20 |o inv|: the ray's part of the slab offsets
     float Sx, Sy, Sz;
     int kx, ky, kz;
     float dkz_abs;   // |d[kz]|, relates the watertight det to the MT det
@@ -121,7 +125,16 @@ LMGPU_HD RayPre ray_prepare(f3 o, f3 d) {
     const float dx = fabsf(d.x) < tiny ? copysignf(tiny, d.x) : d.x;
     const float dy = fabsf(d.y) < tiny ? copysignf(tiny, d.y) : d.y;
     const float dz = fabsf(d.z) < tiny ? copysignf(tiny, d.z) : d.z;
+#if defined(__HIP_DEVICE_COMPILE__)
+    // v_rcp_f32 is within 1 ulp, which the slab test's slack covers (child_keys)
+    r.inv = mk(__builtin_amdgcn_rcpf(dx), __builtin_amdgcn_rcpf(dy), __builtin_amdgcn_rcpf(dz));
+#else
     r.inv = mk(1.0f / dx, 1.0f / dy, 1.0f / dz);
+#endif
+    const f3 oi = mk(o.x * r.inv.x, o.y * r.inv.y, o.z * r.inv.z);
+    const f3 e = mk(fabsf(oi.x), fabsf(oi.y), fabsf(oi.z)) * 0x1p-20f;
+    r.bn = -oi - e;
+    r.bf = e - oi;
     const float ax = fabsf(d.x), ay = fabsf(d.y), az = fabsf(d.z);
     int kz = (ax > ay) ? (ax > az ? 0 : 2) : (ay > az ? 1 : 2);
     int kx = kz + 1 == 3 ? 0 : kz + 1;
@@ -138,27 +151,24 @@ LMGPU_HD RayPre ray_prepare(f3 o, f3 d) {
     return r;
 }
 
-// Watertight ray/triangle test. On acceptance (t in [tmin, tmax], closed
-// edges, |det_MT| >= 1e-8 as the reference), writes t and the barycentric
-// weights (u, v) of v1 and v2.
+// Watertight ray/triangle test of a triangle given relative to the ray origin
+// and permuted to (kx, ky, kz): (ax, ay, az), (bx, by, bz), (cx, cy, cz). On
+// acceptance (t in [tmin, tmax], closed edges, |det_MT| >= 1e-8 as the
+// reference), writes t and the barycentric weights (u, v) of v1 and v2.
 // Watertightness needs each edge function to be the exact negative of the
 // same edge's function in the neighbouring triangle (a*b - c*d against
 // c*d - a*b). Both products must therefore be rounded before the
 // subtraction: fusing one of them into an FMA would break the antisymmetry
 // and let a ray through a shared edge miss both triangles, so contraction is
 // switched off for the three edge functions.
-LMGPU_HD bool tri_intersect(const RayPre& r, float4 p0, float4 p1, float4 p2, float tmin, float tmax, float& t,
-                            float& u, float& v) {
-    const f3 A = mk(p0.x - r.o.x, p0.y - r.o.y, p0.z - r.o.z);
-    const f3 B = mk(p1.x - r.o.x, p1.y - r.o.y, p1.z - r.o.z);
-    const f3 C = mk(p2.x - r.o.x, p2.y - r.o.y, p2.z - r.o.z);
-    const float Akz = comp(A, r.kz), Bkz = comp(B, r.kz), Ckz = comp(C, r.kz);
-    const float Ax = fmaf(-r.Sx, Akz, comp(A, r.kx));
-    const float Ay = fmaf(-r.Sy, Akz, comp(A, r.ky));
-    const float Bx = fmaf(-r.Sx, Bkz, comp(B, r.kx));
-    const float By = fmaf(-r.Sy, Bkz, comp(B, r.ky));
-    const float Cx = fmaf(-r.Sx, Ckz, comp(C, r.kx));
-    const float Cy = fmaf(-r.Sy, Ckz, comp(C, r.ky));
+LMGPU_HD bool tri_test(const RayPre& r, float ax, float ay, float Akz, float bx, float by, float Bkz, float cx,
+                       float cy, float Ckz, float tmin, float tmax, float& t, float& u, float& v) {
+    const float Ax = fmaf(-r.Sx, Akz, ax);
+    const float Ay = fmaf(-r.Sy, Akz, ay);
+    const float Bx = fmaf(-r.Sx, Bkz, bx);
+    const float By = fmaf(-r.Sy, Bkz, by);
+    const float Cx = fmaf(-r.Sx, Ckz, cx);
+    const float Cy = fmaf(-r.Sy, Ckz, cy);
     float U, V, Wt;
     {
 #pragma clang fp contract(off)
@@ -187,6 +197,16 @@ LMGPU_HD bool tri_intersect(const RayPre& r, float4 p0, float4 p1, float4 p2, fl
     u = V * rcp;
     v = Wt * rcp;
     return true;
+}
+
+// The same test on the triangle's world-space vertices.
+LMGPU_HD bool tri_intersect(const RayPre& r, float4 p0, float4 p1, float4 p2, float tmin, float tmax, float& t,
+                            float& u, float& v) {
+    const f3 A = mk(p0.x - r.o.x, p0.y - r.o.y, p0.z - r.o.z);
+    const f3 B = mk(p1.x - r.o.x, p1.y - r.o.y, p1.z - r.o.z);
+    const f3 C = mk(p2.x - r.o.x, p2.y - r.o.y, p2.z - r.o.z);
+    return tri_test(r, comp(A, r.kx), comp(A, r.ky), comp(A, r.kz), comp(B, r.kx), comp(B, r.ky), comp(B, r.kz),
+                    comp(C, r.kx), comp(C, r.ky), comp(C, r.kz), tmin, tmax, t, u, v);
 }
 
 // Slab test of one child box; conservative against FP32 rounding by scaling
@@ -231,21 +251,22 @@ LMGPU_HD float qplane(uint32_t q, int c, float step, float origin) {
 // and no decoded plane: the planes are the exact reals ox + q * step. Each
 // axis picks its near and far plane by the sign of inv_x, so one fma gives
 // the entry and one the exit distance (no per-axis min / max). Bounds, with
-// u = 2^-24: bx is within 2u |bx| of (ox - o_x) * inv_x; the exact plane
-// ox + q step lies within u (|ox| + 255 step) of the FP32 plane the builder
-// rounded outward (quantise_node); the fma and inv_x round relatively, which
-// the 1 + 2 gamma(3) factor on the exit distance covers (box_near). The entry
-// offset is lowered and the exit offset raised by
-//   Ex = 16u (|bx| + |inv_x| |ox| + 255 |ax|),
-// which exceeds the absolute terms with their own rounding, so every child
-// box the FP32 test of the decoded planes would hit is hit here too.
+// u = 2^-24 and P = |ox| + 255 step: the exact plane lies within u P of the
+// FP32 plane the builder rounded outward (quantise_node); inv_x is within 2u
+// (v_rcp_f32), -o inv, the two fmas that form bx and the plane's fma round
+// relatively, each within u |inv| (P + |o|). The entry offset is lowered and
+// the exit offset raised by
+//   16u |inv| (P + |o|),
+// more than twice their sum, so every child box the exact planes' test would
+// hit is hit here too, with no further factor on the exit distance. The step's
+// part is one number per node (slack), |o|'s comes with the ray (bn, bf).
 template <int W>
 LMGPU_HD void child_keys(const QNode<W>& nd, const RayPre& r, float tmin, float tmax, float (&key)[W],
                          int (&ent)[W]) {
-    constexpr float kSlack = 0x1p-20f;   // 16u
     const float org[3] = {nd.ox, nd.oy, nd.oz};
-    const float o[3] = {r.o.x, r.o.y, r.o.z};
     const float inv[3] = {r.inv.x, r.inv.y, r.inv.z};
+    const float bn0[3] = {r.bn.x, r.bn.y, r.bn.z};
+    const float bf0[3] = {r.bf.x, r.bf.y, r.bf.z};
     float a[3], bn[3], bf[3];
     uint32_t wn[3][W / 4], wf[3][W / 4];
     // both plane words of every axis as loaded (whole 16-B loads of the node);
@@ -264,12 +285,10 @@ LMGPU_HD void child_keys(const QNode<W>& nd, const RayPre& r, float tmin, float 
         }
 #pragma unroll
     for (int k = 0; k < 3; k++) {
-        const float step = __builtin_bit_cast(float, ((nd.e >> (8 * k)) & 0xffu) << 23);
-        a[k] = step * inv[k];
-        const float b = (org[k] - o[k]) * inv[k];
-        const float E = (fabsf(b) + fmaf(fabsf(org[k]), fabsf(inv[k]), 255.f * fabsf(a[k]))) * kSlack;
-        bn[k] = b - E;
-        bf[k] = b + E;
+        a[k] = ldexpf(inv[k], int32_t(nd.es << (24 - 8 * k)) >> 24);
+        const float e = fmaf(fabsf(org[k]), 0x1p-20f, nd.slack);
+        bn[k] = fmaf(-fabsf(inv[k]), e, fmaf(org[k], inv[k], bn0[k]));
+        bf[k] = fmaf(fabsf(inv[k]), e, fmaf(org[k], inv[k], bf0[k]));
         const bool pos = inv[k] >= 0.f;
 #pragma unroll
         for (int w = 0; w < W / 4; w++) {
@@ -288,10 +307,8 @@ LMGPU_HD void child_keys(const QNode<W>& nd, const RayPre& r, float tmin, float 
         }
         const float n = fmaxf(fmaxf(tn[0], tn[1]), fmaxf(tn[2], tmin));
         const float f = fminf(fminf(tf[0], tf[1]), fminf(tf[2], tmax));
-        const int e = nd.ent[c];
-        const bool hit = n <= f * 1.00000036f && e != kQEmpty;
-        key[c] = hit ? n : __builtin_inff();
-        ent[c] = e;
+        key[c] = n <= f ? n : __builtin_inff();
+        ent[c] = nd.ent[c];
     }
 }
 
@@ -305,7 +322,8 @@ LMGPU_HD QNode<W> quantise_node(const WNode<W>& n) {
     const float* lo[3] = {n.lox, n.loy, n.loz};
     const float* hi[3] = {n.hix, n.hiy, n.hiz};
     float org[3];
-    uint32_t ebits = 0;
+    uint32_t ebits = 0, esigned = 0;
+    float step_max = 0.f;
     for (int a = 0; a < 3; a++) {
         float mn = __builtin_inff(), mx = -__builtin_inff();
         for (int c = 0; c < W; c++)
@@ -328,10 +346,12 @@ LMGPU_HD QNode<W> quantise_node(const WNode<W>& n) {
         }
         while (e < 127 && std::fma(255.f, std::ldexp(1.f, e), mn) < mx) e++;
         ebits |= uint32_t(e + 127) << (8 * a);
+        esigned |= uint32_t(e & 0xff) << (8 * a);
+        step_max = std::max(step_max, std::ldexp(1.f, e));
         uint32_t ql[W / 4] = {}, qh[W / 4] = {};
         const float step = std::ldexp(1.f, e);
         for (int c = 0; c < W; c++) {
-            int l = 0, h = 0;
+            int l = 255, h = 0;   // an empty slot: no ray lies above plane 255 and below plane 0
             if (n.count[c] >= 0) {
                 // division by the power-of-two step is an exact scaling
                 l = int(std::floor(std::ldexp(double(lo[a][c]) - double(mn), -e)));
@@ -353,61 +373,27 @@ LMGPU_HD QNode<W> quantise_node(const WNode<W>& n) {
     q.oy = org[1];
     q.oz = org[2];
     q.e = ebits;
+    q.es = esigned;
+    q.slack = (255.f * 0x1p-20f) * step_max;
     for (int c = 0; c < W; c++)
         q.ent[c] = n.count[c] < 0 ? kQEmpty : (n.count[c] == 0 ? n.child[c] : encode_leaf(n.child[c], n.count[c]));
-    for (int k = 0; k < int(sizeof(q.pad) / sizeof(q.pad[0])); k++) q.pad[k] = 0;
     return q;
 }
 
-// Per-lane traversal stack: the first LDS_DEPTH entries live in LDS,
-// [entry][lane] so a wave's accesses hit distinct banks, the rest in
-// private memory (only reached by deep, rare traversals). The private
-// entries are a separate array owned by the caller, so that the stack
-// pointer itself stays in a register (an aggregate holding the array would
-// be placed in scratch memory whole, stack pointer included).
-template <int LDS_DEPTH, int PRIV_DEPTH, int BLOCK>
-struct Stack {
-    int (*lds)[BLOCK];
-    int* priv;
-    int sp;
-    int lane;
-    static constexpr int capacity = LDS_DEPTH + PRIV_DEPTH;
-    __device__ __forceinline__ bool push(int e) {
-        if (sp < LDS_DEPTH) {
-            lds[sp][lane] = e;
-        } else {
-            if (sp >= capacity) return false;
-            priv[sp - LDS_DEPTH] = e;
-        }
-        sp++;
-        return true;
-    }
-    __device__ __forceinline__ int pop() {
-        --sp;
-        // an LDS read on every pop (a clamped slot when the entry is
-        // private), so the common case stays a ds_read and is not merged
-        // with the private read into one generic-address load
-        int v = lds[sp < LDS_DEPTH ? sp : 0][lane];
-        asm volatile("" : "+v"(v));
-        if (sp >= LDS_DEPTH) v = priv[sp - LDS_DEPTH];
-        return v;
-    }
-};
-
 struct TraceResult {
-    int prim;
-    float t, u, v;
-    int best;   // index of the hit triangle in traversal order (-1 if none)
+    int prim;        // original triangle index, -1 for a miss
+    float t, u, v;   // of the hit; t of a miss is the ray's tmax
     bool overflow;
-    int node_visits, tri_tests;
 };
 
 // Hit record of the accepted triangle re-evaluated once in FP64 with the
 // reference's Moller-Trumbore formula (accel_sahbvh.cpp:58-75), whose Hit
 // carries FP64 t and uv. The hit decision itself stays the FP32 watertight
 // test; this only removes the FP32 conditioning error of t at grazing
-// incidence (error ~ eps * edge / (t * cos)).
-__device__ __forceinline__ void refine_hit(const TriV& tv, f3 o, f3 d, float& t, float& u, float& v) {
+// incidence (error ~ eps * edge / (t * cos)). A triangle whose FP64
+// determinant vanishes keeps the FP32 values.
+__device__ __forceinline__ void refine_hit(const TriV& tv, const RayPre& r, float tmin, float& t, float& u, float& v) {
+    const f3 o = r.o, d = r.d;
     const double p1x = tv.v0.x, p1y = tv.v0.y, p1z = tv.v0.z;
     const double e1x = double(tv.v1.x) - p1x, e1y = double(tv.v1.y) - p1y, e1z = double(tv.v1.z) - p1z;
     const double e2x = double(tv.v2.x) - p1x, e2y = double(tv.v2.y) - p1y, e2z = double(tv.v2.z) - p1z;
@@ -416,53 +402,68 @@ __device__ __forceinline__ void refine_hit(const TriV& tv, f3 o, f3 d, float& t,
     const double tx = double(o.x) - p1x, ty = double(o.y) - p1y, tz = double(o.z) - p1z;
     const double qx = ty * e1z - tz * e1y, qy = tz * e1x - tx * e1z, qz = tx * e1y - ty * e1x;
     const double det = e1x * px + e1y * py + e1z * pz;
-    if (det == 0.0) return;
+    if (det == 0.0) {
+        (void)tri_intersect(r, tv.v0, tv.v1, tv.v2, tmin, __builtin_inff(), t, u, v);
+        return;
+    }
     const double inv = 1.0 / det;
     t = float((e2x * qx + e2y * qy + e2z * qz) * inv);
     u = float((tx * px + ty * py + tz * pz) * inv);
     v = float((dx * qx + dy * qy + dz * qz) * inv);
 }
 
-// Sorting network helper: orders (k, e) pairs by k ascending.
-__device__ __forceinline__ void cswap(float& ka, int& ea, float& kb, int& eb) {
-    const bool s = kb < ka;
-    const float tk = s ? kb : ka;
-    const int te = s ? eb : ea;
-    kb = s ? ka : kb;
-    eb = s ? ea : eb;
-    ka = tk;
-    ea = te;
+// A child's sort item: its slab key in the high word, its stack entry in the
+// low word of a double. Keys are finite non-NaN floats or +inf, whose bits as
+// the high word never form an FP64 NaN or infinity (exponent at most 0x7f8),
+// and for non-negative keys the doubles order as the keys do. So one compare
+// and exchange of a (key, entry) pair is a v_min_f64 and a v_max_f64 (full
+// rate) instead of a compare and four selects. Inline asm because the
+// builtins first quiet signalling NaNs, which the items never are.
+__device__ __forceinline__ double sort_item(float key, int ent) { return __hiloint2double(__float_as_int(key), ent); }
+__device__ __forceinline__ float item_key(double x) { return __int_as_float(__double2hiint(x)); }
+__device__ __forceinline__ int item_ent(double x) { return __double2loint(x); }
+__device__ __forceinline__ void cswap(double& a, double& b) {
+    double lo, hi;
+    asm("v_min_f64 %0, %1, %2" : "=v"(lo) : "v"(a), "v"(b));
+    asm("v_max_f64 %0, %1, %2" : "=v"(hi) : "v"(a), "v"(b));
+    a = lo;
+    b = hi;
 }
 
 template <int W>
-__device__ __forceinline__ void sort_children(float (&k)[W], int (&e)[W]) {
+__device__ __forceinline__ void sort_children(double (&x)[W]) {
     if constexpr (W == 2) {
-        cswap(k[0], e[0], k[1], e[1]);
+        cswap(x[0], x[1]);
     } else if constexpr (W == 4) {
-        cswap(k[0], e[0], k[1], e[1]);
-        cswap(k[2], e[2], k[3], e[3]);
-        cswap(k[0], e[0], k[2], e[2]);
-        cswap(k[1], e[1], k[3], e[3]);
-        cswap(k[1], e[1], k[2], e[2]);
+        cswap(x[0], x[1]);
+        cswap(x[2], x[3]);
+        cswap(x[0], x[2]);
+        cswap(x[1], x[3]);
+        cswap(x[1], x[2]);
     } else {
         // Batcher odd-even merge sort network for 8 inputs (19 comparators).
-        cswap(k[0], e[0], k[1], e[1]); cswap(k[2], e[2], k[3], e[3]);
-        cswap(k[4], e[4], k[5], e[5]); cswap(k[6], e[6], k[7], e[7]);
-        cswap(k[0], e[0], k[2], e[2]); cswap(k[1], e[1], k[3], e[3]);
-        cswap(k[4], e[4], k[6], e[6]); cswap(k[5], e[5], k[7], e[7]);
-        cswap(k[1], e[1], k[2], e[2]); cswap(k[5], e[5], k[6], e[6]);
-        cswap(k[0], e[0], k[4], e[4]); cswap(k[1], e[1], k[5], e[5]);
-        cswap(k[2], e[2], k[6], e[6]); cswap(k[3], e[3], k[7], e[7]);
-        cswap(k[2], e[2], k[4], e[4]); cswap(k[3], e[3], k[5], e[5]);
-        cswap(k[1], e[1], k[2], e[2]); cswap(k[3], e[3], k[4], e[4]);
-        cswap(k[5], e[5], k[6], e[6]);
+        cswap(x[0], x[1]); cswap(x[2], x[3]); cswap(x[4], x[5]); cswap(x[6], x[7]);
+        cswap(x[0], x[2]); cswap(x[1], x[3]); cswap(x[4], x[6]); cswap(x[5], x[7]);
+        cswap(x[1], x[2]); cswap(x[5], x[6]);
+        cswap(x[0], x[4]); cswap(x[1], x[5]); cswap(x[2], x[6]); cswap(x[3], x[7]);
+        cswap(x[2], x[4]); cswap(x[3], x[5]);
+        cswap(x[1], x[2]); cswap(x[3], x[4]); cswap(x[5], x[6]);
     }
 }
 
+// Stack entry of a lane with nothing left to visit: the bottom of every
+// stack, so that popping an empty stack needs no test.
+constexpr int32_t kDone = INT32_MAX;
+// Ray id of a lane without a ray; ray ids stay below 2^31 (n of a launch).
+constexpr uint32_t kNoRay = UINT32_MAX;
+// Most rays of one launch of the persistent traversal.
+constexpr int64_t kMaxLaunchRays = int64_t(1) << 30;
+
 // Persistent traversal: every lane owns one ray at a time; when at least
-// `refill` lanes of a wave are idle (or the whole wave is), the idle lanes
-// take new rays from the wave's pool, which the wave refills by chunks of
-// chunk_rays (default LMGPU_RAY_CHUNK) from one global counter with one atomic (Aila & Laine,
+// `refill` lanes of a wave have finished (or the whole wave has), the
+// finished lanes hand over their results together and take new rays from the
+// wave's pool, which the wave refills by chunks of chunk_rays (default
+// LMGPU_RAY_CHUNK) from one global counter with one atomic (Aila & Laine,
 // HPG 2009, "persistent threads"), so lanes do not sit idle behind a wave's
 // slowest ray and the counter sees few atomics. refill = 64 keeps whole
 // waves of consecutive rays together (best for coherent rays), smaller
@@ -474,131 +475,209 @@ __device__ __forceinline__ void sort_children(float (&k)[W], int (&e)[W]) {
 // `id` and returns the node its traversal starts from (0, or a root inside a
 // multi-BVH arena);
 // `emit(id, res)` consumes its result.
+//
+// The loop is bound by the instructions it issues (26 of 64 lanes active),
+// so a node step has no branch in the common case: lds[0][lane] holds kDone
+// and entry i of the lane's stack lds[1 + i][lane]; each child is written at
+// the top of the stack and the stack grows by one only if the child was hit,
+// so what lies above the top is garbage that the next push overwrites; and
+// the entry to pop is read before the test, behind the node's own load. The
+// first LDS_DEPTH entries live there, at [entry][lane] (bank-conflict free),
+// the rest in private memory: a wave with a lane that could pass LDS_DEPTH in
+// this step takes a separate, branchy path. Results are emitted
+// only when lanes are refilled: done as each ray ends, the FP64
+// re-evaluation ran in most iterations for a lane or two.
+// Measured together with the slab test's shared offsets, the pair sort and
+// the branch-free push, on the 1.32M-triangle mesh: 2.07M primary rays 723 ->
+// 539 us, 2M incoherent rays 952 -> 907 (bound by the 16-B accesses of its
+// divergent node loads: the address unit is busy 75% of the time), 500K
+// any-hit rays on the 8-wide tree 515 -> 448, a 16-spp 1080p path-traced frame
+// 74.4 -> 63.4 ms.
 template <int W, bool ANY, bool COUNT, int LDS_DEPTH, int PRIV_DEPTH, int BLOCK, class Node, class Fetch, class Emit>
 __device__ __forceinline__ void trace_persistent(const Node* __restrict__ nodes, const TriV* __restrict__ tris,
-                                                 int64_t n, unsigned long long* next, int (*lds)[BLOCK],
+                                                 uint32_t n, unsigned long long* next, int (*lds)[BLOCK],
                                                  Fetch fetch, Emit emit, int32_t* status,
                                                  unsigned long long* counters, int refill,
-                                                 int chunk_rays = LMGPU_RAY_CHUNK) {
+                                                 uint32_t chunk_rays = LMGPU_RAY_CHUNK) {
+    static_assert(LDS_DEPTH >= W, "one node's children must fit the LDS part of an empty stack");
     const int lane = threadIdx.x & 63;
+    const int tid = threadIdx.x;
     int priv[PRIV_DEPTH];
-    Stack<LDS_DEPTH, PRIV_DEPTH, BLOCK> st;
-    st.lds = lds;
-    st.priv = priv;
-    st.sp = 0;
-    st.lane = threadIdx.x;
     RayPre r{};
-    TraceResult res{};
-    int64_t rid = -1;       // ray of this lane, -1 idle
-    bool exhausted = false;
+    f3 ok = mk(0.f, 0.f, 0.f);   // ray origin permuted to (kx, ky, kz)
+    uint32_t kk = 0;             // 1 << kx, 1 << ky, 1 << kz in bits 0-2, 3-5, 6-8
+    uint32_t rid = kNoRay;       // ray of this lane whose result is still to be emitted
+    float tmin = 0.f, tfar = 0.f;
+    int best = -1;               // hit triangle in traversal order
+    bool overflow = false;
+    int cur = kDone;             // node (>= 0), leaf (< 0) or kDone
+    int sp = 0;                  // stack entries
+    lds[0][tid] = kDone;
     // wave-uniform: ray ids taken from `next` and not yet handed to a lane
-    int64_t pool_next = 0, pool_end = 0;
-    float tmin = 0.f;
-    int cur = 0;
+    uint32_t pool_next = 0, pool_end = 0;
+    bool exhausted = false;
     unsigned long long nv = 0, nt = 0;
+    // component kx (shift 0), ky (3) or kz (6) of v: tests of single bits
+    // stay two selects, where a test of the number itself becomes branches
+    auto pick = [&](int shift, float x, float y, float z) {
+        return kk & (1u << shift) ? x : (kk & (2u << shift) ? y : z);
+    };
+    // the ray with what the loop does not hold in registers of its own
+    auto with_axes = [&]() {
+        RayPre q = r;
+        q.dkz_abs = fabsf(pick(6, r.d.x, r.d.y, r.d.z));
+        return q;
+    };
+    // pop for a wave with stacks past LDS_DEPTH
+    auto pop_deep = [&]() -> int {
+        int v = lds[min(sp, LDS_DEPTH)][tid];
+        asm volatile("" : "+v"(v));   // keep the ds_read apart from the private read
+        if (sp > LDS_DEPTH) v = priv[sp - 1 - LDS_DEPTH];
+        if (sp > 0) sp--;
+        return v;
+    };
     while (true) {
-        const bool idle = rid < 0 && !exhausted;
-        const unsigned long long idle_mask = __ballot(idle);
-        const unsigned long long busy_mask = __ballot(rid >= 0);
-        const int nidle = __popcll(idle_mask);
-        if (nidle >= refill || (busy_mask == 0 && nidle > 0)) {
-            // idle lanes take, in lane order, the rest of the wave's pool and
-            // then the start of a new chunk of LMGPU_RAY_CHUNK ids
-            const int64_t avail = pool_end - pool_next;
-            int64_t chunk = 0;
-            if (avail < nidle) {
-                const int leader = __ffsll(idle_mask) - 1;
-                unsigned long long b = 0;
-                if (lane == leader) b = atomicAdd(next, (unsigned long long)chunk_rays);
-                b = (unsigned long long)__shfl((long long)b, leader);
-                // wave-uniform from here on: scalar registers for the pool
-                chunk = int64_t((uint64_t(uint32_t(__builtin_amdgcn_readfirstlane(uint32_t(b >> 32)))) << 32) |
-                                uint32_t(__builtin_amdgcn_readfirstlane(uint32_t(b))));
+        const unsigned long long busy = __ballot(cur != kDone);
+        if (busy == 0 || (!exhausted && 64 - __popcll(busy) >= refill)) {
+            // hand over the results of the lanes that finished
+            if (rid != kNoRay && cur == kDone) {
+                TraceResult res;
+                res.prim = -1;
+                res.t = tfar;
+                res.u = res.v = 0.f;
+                res.overflow = overflow;
+                if (overflow) atomicOr(status, 1);
+                if (best >= 0) {
+                    const TriV tv = tris[best];
+                    res.prim = __float_as_int(tv.v0.w);
+                    if (!ANY) {
+                        RayPre q = with_axes();
+                        q.kx = kk & 1u ? 0 : (kk & 2u ? 1 : 2);
+                        q.ky = kk & 8u ? 0 : (kk & 16u ? 1 : 2);
+                        q.kz = kk & 64u ? 0 : (kk & 128u ? 1 : 2);
+                        // the inverse of the permutation that made ok
+                        q.o = mk(kk & 1u ? ok.x : (kk & 8u ? ok.y : ok.z), kk & 2u ? ok.x : (kk & 16u ? ok.y : ok.z),
+                                 kk & 4u ? ok.x : (kk & 32u ? ok.y : ok.z));
+                        refine_hit(tv, q, tmin, res.t, res.u, res.v);
+                    }
+                }
+                emit(rid, res);
+                rid = kNoRay;
             }
-            if (idle) {
-                const int rank = __popcll(idle_mask & ((1ull << lane) - 1ull));
-                const int64_t id = rank < avail ? pool_next + rank : chunk + (rank - avail);
-                if (id < n) {
-                    rid = id;
-                    f3 o, d;
-                    float tmax;
-                    cur = fetch(id, o, d, tmin, tmax);
-                    r = ray_prepare(o, d);
-                    res.prim = -1;
-                    res.t = tmax;
-                    res.u = res.v = 0.f;
-                    res.best = -1;
-                    res.overflow = false;
-                    st.sp = 0;
+            if (!exhausted) {
+                // idle lanes take, in lane order, the rest of the wave's pool
+                // and then the start of a new chunk
+                const bool idle = cur == kDone;
+                const unsigned long long idle_mask = ~busy;
+                const uint32_t nidle = __popcll(idle_mask);
+                const uint32_t avail = pool_end - pool_next;
+                uint32_t chunk = 0;
+                if (avail < nidle) {
+                    uint32_t b = 0;
+                    if (lane == 0) b = uint32_t(atomicAdd(next, (unsigned long long)chunk_rays));
+                    // wave-uniform from here on: scalar registers for the pool
+                    chunk = __builtin_amdgcn_readfirstlane(b);
+                }
+                if (idle) {
+                    const uint32_t rank = __popcll(idle_mask & ((1ull << lane) - 1ull));
+                    const uint32_t id = rank < avail ? pool_next + rank : chunk + (rank - avail);
+                    if (id < n) {
+                        rid = id;
+                        f3 o, d;
+                        cur = fetch(id, o, d, tmin, tfar);
+                        r = ray_prepare(o, d);
+                        ok = mk(comp(o, r.kx), comp(o, r.ky), comp(o, r.kz));
+                        kk = (1u << r.kx) | (8u << r.ky) | (64u << r.kz);
+                        best = -1;
+                        overflow = false;
+                        sp = 0;
+                    }
+                }
+                if (avail < nidle) {
+                    pool_next = chunk + (nidle - avail);
+                    pool_end = chunk + chunk_rays;
                 } else {
-                    exhausted = true;
+                    pool_next += nidle;
+                }
+                exhausted = pool_next >= n;   // the counter only grows: no id below n is left
+            }
+            if (__ballot(cur != kDone) == 0) break;
+        }
+        // One kind of step per iteration for the whole wave, so inner-node
+        // and leaf code do not both run, each for a part of the lanes: leaves
+        // when enough lanes sit at a leaf, else inner nodes; the other lanes
+        // wait one iteration.
+        const unsigned long long leaf_mask = __ballot(cur < 0);
+        const int nleaf = __popcll(leaf_mask);
+        const int nnode = __popcll(__ballot(cur != kDone)) - nleaf;
+        if (4 * nleaf >= LMGPU_LEAF_VOTE_X4 * nnode) {
+            if (cur < 0) {
+                const int first = leaf_first(cur), cnt = leaf_count(cur);
+                const RayPre q = with_axes();
+                bool hit = false;
+                for (int k = 0; k < cnt; k++) {
+                    if (COUNT) nt++;
+                    const TriV tv = tris[first + k];
+                    float t, u, v;
+                    const float4 a = tv.v0, b = tv.v1, c = tv.v2;
+                    if (tri_test(q, pick(0, a.x, a.y, a.z) - ok.x, pick(3, a.x, a.y, a.z) - ok.y,
+                                 pick(6, a.x, a.y, a.z) - ok.z, pick(0, b.x, b.y, b.z) - ok.x,
+                                 pick(3, b.x, b.y, b.z) - ok.y, pick(6, b.x, b.y, b.z) - ok.z,
+                                 pick(0, c.x, c.y, c.z) - ok.x, pick(3, c.x, c.y, c.z) - ok.y,
+                                 pick(6, c.x, c.y, c.z) - ok.z, tmin, tfar, t, u, v)) {
+                        tfar = t;
+                        best = first + k;
+                        hit = true;
+                        if (ANY) break;
+                    }
+                }
+                if (ANY && hit) cur = kDone;
+                else if (__ballot(sp > LDS_DEPTH) != 0) cur = pop_deep();
+                else {
+                    cur = lds[sp][tid];
+                    sp = max(sp - 1, 0);
                 }
             }
-            if (avail < nidle) {
-                pool_next = chunk + (nidle - avail);
-                pool_end = chunk + chunk_rays;
-            } else {
-                pool_next += nidle;
-            }
-        }
-        if (__ballot(rid >= 0) == 0) break;
-        if (rid < 0) continue;
-#if LMGPU_LEAF_VOTE_X4 > 0
-        {
-            // one kind of step per iteration for the whole wave, so inner-node
-            // and leaf code do not both run, each for a part of the lanes:
-            // leaves when enough lanes sit at a leaf, else inner nodes; the
-            // other lanes wait one iteration
-            const int nleaf = __popcll(__ballot(cur < 0));
-            const int nnode = __popcll(__ballot(cur >= 0));
-            const bool leaf_step = 4 * nleaf >= LMGPU_LEAF_VOTE_X4 * nnode;
-            if (leaf_step != (cur < 0)) continue;
-        }
-#endif
-        bool finished = false;
-        if (cur >= 0) {
+        } else if (uint32_t(cur) < uint32_t(kDone)) {
             if (COUNT) nv++;
+            const Node& nd = nodes[cur];
+            const int top = lds[min(sp, LDS_DEPTH)][tid];
             float key[W];
             int ent[W];
-            child_keys<W>(nodes[cur], r, tmin, res.t, key, ent);
-            sort_children<W>(key, ent);
-            bool ok = true;
+            child_keys<W>(nd, r, tmin, tfar, key, ent);
+            double x[W];
 #pragma unroll
-            for (int c = W - 1; c >= 1; c--)
-                if (key[c] != __builtin_inff()) ok = ok && st.push(ent[c]);
-            if (!ok) {
-                res.overflow = true;
-                finished = true;
-            } else if (key[0] != __builtin_inff()) {
-                cur = ent[0];
-            } else if (st.sp == 0) {
-                finished = true;
+            for (int c = 0; c < W; c++) x[c] = sort_item(key[c], ent[c]);
+            sort_children<W>(x);
+            const float kInfF = __builtin_inff();
+            if (__ballot(sp + W - 1 > LDS_DEPTH) == 0) {
+#pragma unroll
+                for (int c = W - 1; c >= 1; c--) {
+                    lds[sp + 1][tid] = item_ent(x[c]);
+                    sp += item_key(x[c]) != kInfF ? 1 : 0;
+                }
+                const bool any_child = item_key(x[0]) != kInfF;
+                cur = any_child ? item_ent(x[0]) : top;
+                sp = any_child ? sp : max(sp - 1, 0);
             } else {
-                cur = st.pop();
-            }
-        } else {
-            const int first = leaf_first(cur), cnt = leaf_count(cur);
-            for (int k = 0; k < cnt; k++) {
-                const TriV tv = tris[first + k];
-                if (COUNT) nt++;
-                float t, u, v;
-                if (tri_intersect(r, tv.v0, tv.v1, tv.v2, tmin, res.t, t, u, v)) {
-                    res.t = t;
-                    res.u = u;
-                    res.v = v;
-                    res.prim = __float_as_int(tv.v0.w);
-                    res.best = first + k;
-                    if (ANY) break;
+                bool full = false;
+#pragma unroll
+                for (int c = W - 1; c >= 1; c--)
+                    if (item_key(x[c]) != kInfF) {
+                        if (sp < LDS_DEPTH) lds[sp + 1][tid] = item_ent(x[c]);
+                        else if (sp < LDS_DEPTH + PRIV_DEPTH) priv[sp - LDS_DEPTH] = item_ent(x[c]);
+                        else full = true;
+                        if (!full) sp++;
+                    }
+                if (full) {
+                    overflow = true;
+                    cur = kDone;
+                } else if (item_key(x[0]) != kInfF) {
+                    cur = item_ent(x[0]);
+                } else {
+                    cur = pop_deep();
                 }
             }
-            if ((ANY && res.prim >= 0) || st.sp == 0) finished = true;
-            else cur = st.pop();
-        }
-        if (finished) {
-            if (res.overflow) atomicOr(status, 1);
-            if (!ANY && res.best >= 0) refine_hit(tris[res.best], r.o, r.d, res.t, res.u, res.v);
-            emit(rid, res);
-            rid = -1;
         }
     }
     if (COUNT) {

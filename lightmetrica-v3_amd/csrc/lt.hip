@@ -317,12 +317,12 @@ __global__ __launch_bounds__(kBlock) void k_lt_shade(SceneDev sc, PathState ps, 
 }
 
 template <int W>
-__global__ __launch_bounds__(kBlock) void k_lt_connect(SceneDev sc, Queues q, unsigned long long* next, int refill,
+__global__ __launch_bounds__(kBlock, 6) void k_lt_connect(SceneDev sc, Queues q, unsigned long long* next, int refill,
                                                        double* __restrict__ film, int chunk_rays) {
-    __shared__ int lds[kLds][kBlock];
+    __shared__ int lds[kLds + 1][kBlock];
     const int n = q.counts[2];
     if (n == 0) return;   // no connections (whole grid)
-    auto fetch = [&](int64_t id, f3& o, f3& d, float& tmin, float& tmax) -> int {
+    auto fetch = [&](uint32_t id, f3& o, f3& d, float& tmin, float& tmax) -> int {
         const float4* rp = reinterpret_cast<const float4*>(q.sh + id);
         const float4 a = rp[0], b = rp[1];
         o = mk(a.x, a.y, a.z);
@@ -331,7 +331,7 @@ __global__ __launch_bounds__(kBlock) void k_lt_connect(SceneDev sc, Queues q, un
         tmax = b.w;
         return 0;
     };
-    auto emit = [&](int64_t id, const TraceResult& r) {
+    auto emit = [&](uint32_t id, const TraceResult& r) {
         if (r.prim < 0 && !r.overflow) {
             const float4 c = q.sh_contrib[id];
             double* f = film + 3 * int64_t(__float_as_int(c.w));

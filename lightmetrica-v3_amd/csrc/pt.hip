@@ -154,13 +154,13 @@ __global__ void k_reset_counts(int32_t* counts, int out_q) {
 // baseline (the NEE of a vertex is not part of its sampled direction's
 // incident radiance).
 template <int W>
-__global__ __launch_bounds__(kBlock) void k_connect(SceneDev sc, PathState ps, Queues q, unsigned long long* next,
+__global__ __launch_bounds__(kBlock, 6) void k_connect(SceneDev sc, PathState ps, Queues q, unsigned long long* next,
                                                    int refill, GRec* __restrict__ rec, const int32_t* __restrict__ sh_rec,
                                                    double* __restrict__ splat) {
-    __shared__ int lds[kLds][kBlock];
+    __shared__ int lds[kLds + 1][kBlock];
     const int n = q.counts[2];
     if (n == 0) return;   // no shadow rays (whole grid)
-    auto fetch = [&](int64_t id, f3& o, f3& d, float& tmin, float& tmax) -> int {
+    auto fetch = [&](uint32_t id, f3& o, f3& d, float& tmin, float& tmax) -> int {
         const float4* rp = reinterpret_cast<const float4*>(q.sh + id);
         const float4 a = rp[0], b = rp[1];
         o = mk(a.x, a.y, a.z);
@@ -169,7 +169,7 @@ __global__ __launch_bounds__(kBlock) void k_connect(SceneDev sc, PathState ps, Q
         tmax = b.w;
         return 0;
     };
-    auto emit = [&](int64_t id, const TraceResult& r) {
+    auto emit = [&](uint32_t id, const TraceResult& r) {
         if (r.prim < 0 && !r.overflow) {
             const float4 c = q.sh_contrib[id];
             const int p = __float_as_int(c.w);
@@ -320,22 +320,22 @@ struct RaycastConsts {
 };
 
 template <int W>
-__global__ __launch_bounds__(kBlock) void k_raycast(SceneDev sc, unsigned long long* next, int refill, RaycastConsts rc,
+__global__ __launch_bounds__(kBlock, 6) void k_raycast(SceneDev sc, unsigned long long* next, int refill, RaycastConsts rc,
                                                     double* __restrict__ film, int32_t* status) {
-    __shared__ int lds[kLds][kBlock];
+    __shared__ int lds[kLds + 1][kBlock];
     const int n = sc.w * sc.h;
-    auto dir_of = [&](int64_t id) {
+    auto dir_of = [&](uint32_t id) {
         const int x = int(id % sc.w), y = int(id / sc.w);
         return primary_dir(sc.cam, (x + .5f) / sc.w, (y + .5f) / sc.h);
     };
-    auto fetch = [&](int64_t id, f3& o, f3& d, float& tmin, float& tmax) -> int {
+    auto fetch = [&](uint32_t id, f3& o, f3& d, float& tmin, float& tmax) -> int {
         o = sc.cam.pos;
         d = dir_of(id);
         tmin = kEps;
         tmax = kInf;
         return 0;
     };
-    auto emit = [&](int64_t id, const TraceResult& r) {
+    auto emit = [&](uint32_t id, const TraceResult& r) {
         f3 C = rc.bg;
         if (r.prim >= 0) {
             const ShadeTri st = sc.stri[r.prim];

@@ -522,13 +522,13 @@ __device__ __forceinline__ void shade_vertex(const SceneDev& sc, const PTConsts&
 // written as (prim or -1 / -2 on stack overflow, t, u, v); shared by the
 // path and light tracers.
 template <int W>
-__global__ __launch_bounds__(kBlock) void k_extend(SceneDev sc, Queues q, int in_q, unsigned long long* next, int refill,
+__global__ __launch_bounds__(kBlock, 6) void k_extend(SceneDev sc, Queues q, int in_q, unsigned long long* next, int refill,
                                                   int chunk_rays) {
-    __shared__ int lds[kLds][kBlock];
+    __shared__ int lds[kLds + 1][kBlock];
     const int n = q.counts[in_q];
     if (n == 0) return;   // an empty queue (whole grid)
     const lmgpu_ray* rays = q.ext[in_q];
-    auto fetch = [&](int64_t id, f3& o, f3& d, float& tmin, float& tmax) -> int {
+    auto fetch = [&](uint32_t id, f3& o, f3& d, float& tmin, float& tmax) -> int {
         const float4* rp = reinterpret_cast<const float4*>(rays + id);
         const float4 a = rp[0], b = rp[1];
         o = mk(a.x, a.y, a.z);
@@ -537,7 +537,7 @@ __global__ __launch_bounds__(kBlock) void k_extend(SceneDev sc, Queues q, int in
         tmax = b.w;
         return 0;
     };
-    auto emit = [&](int64_t id, const TraceResult& r) {
+    auto emit = [&](uint32_t id, const TraceResult& r) {
         reinterpret_cast<float4*>(q.hit)[id] = make_float4(__int_as_float(r.overflow ? -2 : r.prim), r.t, r.u, r.v);
     };
     trace_persistent<W, false, false, kLds, kPriv, kBlock>(nodes_of<W>(sc), sc.tris, n, next, lds, fetch, emit,
