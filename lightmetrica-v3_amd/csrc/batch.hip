@@ -48,6 +48,8 @@ __device__ __forceinline__ uint64_t job_seed(const JobDev& J) { return (uint64_t
 // Most grid-stride iterations of k_b_regen per block (the host sizes the grid
 // so that a block covers at most this many BLOCK-slot strides of the pool).
 constexpr int kRegenMaxIter = 32;
+// Block size of the regenerate and shade kernels of a single scene's render.
+constexpr int kSingleBlock = 128;
 // Entries of k_b_regen's per-block table of finished-sample counts per job.
 constexpr int kRegenJobSlots = 64;
 
@@ -58,17 +60,24 @@ constexpr int kRegenJobSlots = 64;
 // (per stride and wave, in LDS), one atomic on work_next then reserves the
 // block's items and one on the queue count its queue entries; finished
 // samples are counted per job in an LDS table and added to the job's and
-// the run's counters at the end of the block.
-template <int BLOCK>
+// the run's counters at the end of the block. SINGLE: the run has one job
+// (kernels of a single scene's render read its fields as scalars, with no
+// job index per path), whose work items are its samples' pixels in order.
+// The kernel also clears the counters of the iteration it opens: the ray
+// counters `next` and the counts of the other extension queue and the shadow
+// queue, which nothing reads until the traversal and shading that follow.
+template <int BLOCK, bool SINGLE>
 __global__ __launch_bounds__(BLOCK) void k_b_regen(const JobDev* __restrict__ jobs, const WorkSeg* __restrict__ segs,
                                                    int nsegs, int64_t total, PoolDev P, BatchQ q, int in_q, int cap,
-                                                   BatchCtl* ctl, unsigned long long* job_done,
-                                                   unsigned long long* job_time, double* film_sum, double* film_sq) {
+                                                   BatchCtl* ctl, unsigned long long* next,
+                                                   unsigned long long* job_done, unsigned long long* job_time,
+                                                   double* film_sum, double* film_sq) {
     constexpr int kWaves = BLOCK / 64;
     __shared__ int s_want[kRegenMaxIter][kWaves];   // slots taking work, then their exclusive prefix
     __shared__ unsigned long long s_base;           // first work item of the block
     __shared__ int s_qbase;                         // first queue entry of the block
     __shared__ int s_emit;                          // queue entries of the block
+    __shared__ int s_sample, s_pixel;               // SINGLE: sample and pixel of the first work item
     __shared__ int s_key[kRegenJobSlots];
     __shared__ unsigned int s_cnt[kRegenJobSlots];
     __shared__ unsigned int s_fin;
@@ -78,6 +87,12 @@ __global__ __launch_bounds__(BLOCK) void k_b_regen(const JobDev* __restrict__ jo
     // (the host enqueues iterations up to a bound without watching). One
     // thread reads the counter, so the whole block takes the same branch
     // (other blocks of this launch may lower it meanwhile).
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        next[0] = 0ull;
+        next[1] = 0ull;
+        q.counts[in_q ^ 1] = 0;
+        q.counts[2] = 0;
+    }
     if (threadIdx.x == 0)
         s_idle = __hip_atomic_load(&ctl->remaining, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0;
     __syncthreads();
@@ -87,17 +102,18 @@ __global__ __launch_bounds__(BLOCK) void k_b_regen(const JobDev* __restrict__ jo
     const int n_iter = (cap + stride - 1) / stride;   // <= kRegenMaxIter (host)
     const int lane = __lane_id();
     const int wave = threadIdx.x >> 6;
-    for (int k = threadIdx.x; k < kRegenJobSlots; k += BLOCK) {
-        s_key[k] = -1;
-        s_cnt[k] = 0u;
-    }
+    if (!SINGLE)
+        for (int k = threadIdx.x; k < kRegenJobSlots; k += BLOCK) {
+            s_key[k] = -1;
+            s_cnt[k] = 0u;
+        }
     if (threadIdx.x == 0) s_fin = 0u;
     // sweep 1: slots that take work (free now or freed below)
     for (int it = 0; it < n_iter; it++) {
         const int s = it * stride + blockIdx.x * BLOCK + threadIdx.x;
         bool want = false;
         if (s < cap) {
-            const int32_t st = P.state[s];
+            const int32_t st = P.state[s] & kStateMask;
             want = st == kFinishing || st == kFree;
         }
         const unsigned long long m = __ballot(want);
@@ -123,6 +139,11 @@ __global__ __launch_bounds__(BLOCK) void k_b_regen(const JobDev* __restrict__ jo
         s_base = base;
         s_emit = emit;
         s_qbase = qb;
+        if (SINGLE) {
+            const unsigned long long np = (unsigned long long)jobs[0].npix;
+            s_sample = segs[0].sample + int(base / np);
+            s_pixel = int(base % np);
+        }
     }
     __syncthreads();
     const unsigned long long base = s_base;
@@ -132,9 +153,9 @@ __global__ __launch_bounds__(BLOCK) void k_b_regen(const JobDev* __restrict__ jo
         const int s = it * stride + blockIdx.x * BLOCK + threadIdx.x;
         bool want = false;
         if (s < cap) {
-            int32_t st = P.state[s];
+            int32_t st = P.state[s] & kStateMask;
             if (st == kFinishing) {
-                const int fj = P.job[s];
+                const int fj = SINGLE ? 0 : P.job[s];
                 const JobDev& J = jobs[fj];
                 const float4 L = P.L[s];
                 const int64_t f = J.film_off + 3 * int64_t(P.pixel[s]);
@@ -149,13 +170,15 @@ __global__ __launch_bounds__(BLOCK) void k_b_regen(const JobDev* __restrict__ jo
                 // count the finished sample in the block's job table, or
                 // straight into the job's counter when its entry is taken
                 atomicAdd(&s_fin, 1u);
-                const int h = fj & (kRegenJobSlots - 1);
-                const int prev = atomicCAS(&s_key[h], -1, fj);
-                if (prev == -1 || prev == fj) {
-                    atomicAdd(&s_cnt[h], 1u);
-                } else {
-                    const unsigned long long need = (unsigned long long)J.npix * (unsigned long long)J.spp;
-                    if (atomicAdd(job_done + fj, 1ull) + 1ull == need) job_time[fj] = wall_clock64();
+                if (!SINGLE) {
+                    const int h = fj & (kRegenJobSlots - 1);
+                    const int prev = atomicCAS(&s_key[h], -1, fj);
+                    if (prev == -1 || prev == fj) {
+                        atomicAdd(&s_cnt[h], 1u);
+                    } else {
+                        const unsigned long long need = (unsigned long long)J.npix * (unsigned long long)J.spp;
+                        if (atomicAdd(job_done + fj, 1ull) + 1ull == need) job_time[fj] = wall_clock64();
+                    }
                 }
                 st = kFree;
                 P.state[s] = kFree;
@@ -166,27 +189,38 @@ __global__ __launch_bounds__(BLOCK) void k_b_regen(const JobDev* __restrict__ jo
         if (want) {
             const int r = s_want[it][wave] + __popcll(mask & ((1ull << lane) - 1ull));   // rank in the block
             if (r < emit_n) {
-                const unsigned long long w = base + (unsigned long long)r;
-                // segment of item w: the last one starting at or before w
-                int lo = 0, hi = nsegs - 1;
-                while (lo < hi) {
-                    const int mid = (lo + hi + 1) >> 1;
-                    if (segs[mid].start <= int64_t(w)) lo = mid;
-                    else hi = mid - 1;
+                int job = 0, sample, pix;
+                if (SINGLE) {
+                    const uint32_t np = uint32_t(jobs[0].npix);
+                    const uint32_t at = uint32_t(s_pixel) + uint32_t(r);   // < 2^28 + kRegenMaxIter * BLOCK
+                    sample = s_sample + int(at / np);
+                    pix = int(at % np);
+                } else {
+                    const unsigned long long w = base + (unsigned long long)r;
+                    // segment of item w: the last one starting at or before w
+                    int lo = 0, hi = nsegs - 1;
+                    while (lo < hi) {
+                        const int mid = (lo + hi + 1) >> 1;
+                        if (segs[mid].start <= int64_t(w)) lo = mid;
+                        else hi = mid - 1;
+                    }
+                    const WorkSeg seg = segs[lo];
+                    job = seg.job;
+                    sample = seg.sample;
+                    pix = int(int64_t(w) - seg.start);
+                    P.job[s] = job;
                 }
-                const WorkSeg seg = segs[lo];
-                const JobDev& J = jobs[seg.job];
-                const int sample = seg.sample, pix = int(int64_t(w) - seg.start);
-                P.job[s] = seg.job;
+                const JobDev& J = jobs[job];
                 P.pixel[s] = pix;
-                P.sample[s] = sample;
                 P.state[s] = kActive;
-                P.thr[s] = make_float4(1.f, 1.f, 1.f, 0.f);
-                P.L[s] = make_float4(0.f, 0.f, 0.f, 0.f);
-                P.prev[s] = make_float4(0.f, 0.f, 0.f, 0.f);
-                P.info[s] = make_int4(1, 0, 2, 0);   // camera vertex: degenerate, not NEE-samplable
-                q.ext[in_q][qbase + r] = camera_ray(J.sc, pix, uint32_t(sample), job_seed(J));
-                q.ext_path[in_q][qbase + r] = s;
+                P.L[s] = make_float4(0.f, 0.f, 0.f, __int_as_float(sample));
+                // camera vertex: degenerate, not NEE-samplable
+                lmgpu_ray ray = camera_ray(J.sc, pix, uint32_t(sample), job_seed(J));
+                ray.tmin = __int_as_float(s);
+                ray.tmax = 0.f;
+                q.ext[in_q][qbase + r] = ray;
+                q.thr[in_q][qbase + r] = make_float4(1.f, 1.f, 1.f, __int_as_float(pack_info(1, 2)));
+                q.prev[in_q][qbase + r] = make_float4(0.f, 0.f, 0.f, __int_as_float(pix));
             }
         }
     }
@@ -194,7 +228,7 @@ __global__ __launch_bounds__(BLOCK) void k_b_regen(const JobDev* __restrict__ jo
     __syncthreads();
     if (threadIdx.x == 0 && s_fin > 0u)
         atomicAdd(&ctl->remaining, (unsigned long long)(-(long long)s_fin));
-    for (int k = threadIdx.x; k < kRegenJobSlots; k += BLOCK) {
+    for (int k = threadIdx.x; k < (SINGLE ? 0 : kRegenJobSlots); k += BLOCK) {
         const int j = s_key[k];
         if (j >= 0 && s_cnt[k] > 0u) {
             const JobDev& J = jobs[j];
@@ -205,7 +239,7 @@ __global__ __launch_bounds__(BLOCK) void k_b_regen(const JobDev* __restrict__ jo
     }
 }
 
-template <int W>
+template <int W, bool SINGLE>
 __global__ __launch_bounds__(kBlock, 6) void k_b_extend(const typename TravNode<W>::type* __restrict__ nodes,
                                                      const TriV* __restrict__ tris,
                                                      const JobDev* __restrict__ jobs, PoolDev P, BatchQ q, int in_q,
@@ -219,9 +253,9 @@ __global__ __launch_bounds__(kBlock, 6) void k_b_extend(const typename TravNode<
         const float4 a = rp[0], b = rp[1];
         o = mk(a.x, a.y, a.z);
         d = mk(b.x, b.y, b.z);
-        tmin = a.w;
-        tmax = b.w;
-        return jobs[P.job[q.ext_path[in_q][id]]].root;
+        tmin = kEps;   // every camera and bounce ray; the entry holds its slot and pdf in their place
+        tmax = kInf;
+        return SINGLE ? jobs[0].root : jobs[P.job[__float_as_int(a.w)]].root;
     };
     auto emit = [&](uint32_t id, const TraceResult& r) {
         reinterpret_cast<float4*>(q.hit)[id] = make_float4(__int_as_float(r.overflow ? -2 : r.prim), r.t, r.u, r.v);
@@ -231,7 +265,11 @@ __global__ __launch_bounds__(kBlock, 6) void k_b_extend(const typename TravNode<
     if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&ctl->ext_rays, (unsigned long long)n);
 }
 
-template <int BLOCK, bool GUIDED>
+// One vertex of every path of extension queue in_q (shade_vertex). A path's
+// state travels in its queue entry, as arrays over the queue that a wave reads
+// and writes whole lines of: by slot, as the radiance still is, a wave's
+// entries are spread over two to three times as many lines.
+template <int BLOCK, bool GUIDED, bool SINGLE>
 __global__ __launch_bounds__(BLOCK) void k_b_shade(const JobDev* __restrict__ jobs, PoolDev P, BatchQ q, int in_q,
                                                    GuideDev gd, int cap) {
     const int n = q.counts[in_q];
@@ -241,16 +279,21 @@ __global__ __launch_bounds__(BLOCK) void k_b_shade(const JobDev* __restrict__ jo
     for (int it = 0; it < n_iter; it++) {
         const int i = it * stride + blockIdx.x * BLOCK + threadIdx.x;
         VertexOut out;
-        int s = 0;
+        int s = 0, pixel = 0;
+        PathRegs R{};
         if (i < n) {
-            s = q.ext_path[in_q][i];
-            const JobDev& J = jobs[P.job[s]];
             const float4* rp = reinterpret_cast<const float4*>(q.ext[in_q] + i);
             const float4 ra = rp[0], rb = rp[1];
             const float4 h = reinterpret_cast<const float4*>(q.hit)[i];
+            const float4 thr4 = q.thr[in_q][i], prev4 = q.prev[in_q][i];
+            s = __float_as_int(ra.w);
+            const float4 L4 = P.L[s];
+            const JobDev& J = jobs[SINGLE ? 0 : P.job[s]];
             if (__float_as_int(h.x) == -2) atomicOr(q.counts + 5, 1);
-            const float4 thr4 = P.thr[s], L4 = P.L[s];
-            PathRegs R{mk(thr4.x, thr4.y, thr4.z), mk(L4.x, L4.y, L4.z), P.prev[s], P.info[s]};
+            pixel = __float_as_int(prev4.w);
+            const int nv = info_verts(__float_as_int(thr4.w));
+            R = PathRegs{mk(thr4.x, thr4.y, thr4.z), mk(L4.x, L4.y, L4.z), make_float4(prev4.x, prev4.y, prev4.z, rb.w),
+                         make_int4(nv, 0, info_flags(__float_as_int(thr4.w)), 0)};
             PTConsts c;
             c.max_verts = J.max_verts;
             c.mode = J.mode;
@@ -259,24 +302,21 @@ __global__ __launch_bounds__(BLOCK) void k_b_shade(const JobDev* __restrict__ jo
             c.seed_hi = J.seed_hi;
             // guided: the records of slot s sit at (vertex - 1) * cap + s
             c.npix = GUIDED ? cap : J.npix;
-            shade_vertex<GUIDED>(J.sc, c, uint32_t(P.pixel[s]), uint32_t(P.sample[s]), job_seed(J), s,
+            shade_vertex<GUIDED>(J.sc, c, uint32_t(pixel), uint32_t(__float_as_int(L4.w)), job_seed(J), s,
                                  mk(ra.x, ra.y, ra.z), mk(rb.x, rb.y, rb.z), h, R, gd,
                                  GUIDED ? gd.mix + int64_t(i) * kOut : nullptr, out);
-            if (out.ext) {
-                P.prev[s] = R.prev;
-                P.info[s] = R.info;
-                P.thr[s] = make_float4(R.thr.x, R.thr.y, R.thr.z, 0.f);
-            } else {
-                // the path ends here; its NEE of this vertex lands in connect
-                P.state[s] = kFinishing;
-            }
-            P.L[s] = make_float4(R.L.x, R.L.y, R.L.z, 0.f);
+            // a path that ends here: its NEE of this vertex lands in connect
+            if (!out.ext) P.state[s] = kFinishing | (nv << kStateShift);
+            P.L[s] = make_float4(R.L.x, R.L.y, R.L.z, L4.w);
         }
         int se, ss;
         block_append2<BLOCK>(q.counts + out_q, q.counts + 2, out.ext, out.sh, se, ss);
         if (out.ext) {
+            out.ext_ray.tmin = __int_as_float(s);
+            out.ext_ray.tmax = R.prev.w;
             q.ext[out_q][se] = out.ext_ray;
-            q.ext_path[out_q][se] = s;
+            q.thr[out_q][se] = make_float4(R.thr.x, R.thr.y, R.thr.z, __int_as_float(pack_info(R.info.x, R.info.z)));
+            q.prev[out_q][se] = make_float4(R.prev.x, R.prev.y, R.prev.z, __int_as_float(pixel));
         }
         if (out.sh) {
             q.sh[ss] = out.sh_ray;
@@ -325,11 +365,12 @@ __global__ __launch_bounds__(256) void k_b_gcollect(PoolDev P, int cap, GRec* __
         const int j = it * stride + blockIdx.x * 256 + threadIdx.x;
         const uint32_t run = (uint32_t(j >> 6) * kScramble) & uint32_t((cap >> 6) - 1);
         const int s = int(run << 6) + lane;
-        const bool fin = j < cap && P.state[s] == kFinishing;
+        const int32_t st = j < cap ? P.state[s] : kFree;
+        const bool fin = (st & kStateMask) == kFinishing;
         const float4 Lf = fin ? P.L[s] : make_float4(0.f, 0.f, 0.f, 0.f);
-        // a vertex that sampled a direction left the path's vertex count at
-        // its own count + 1, so only records d < count - 1 can have been written
-        const int dmax = fin ? min(rec_depth, P.info[s].x - 1) : 0;
+        // the state holds the vertex count at the vertex that ended the path,
+        // which wrote no record: only records d < count - 1 can have been written
+        const int dmax = fin ? min(rec_depth, (st >> kStateShift) - 1) : 0;
         int cnt = 0;
         if (fin) {
             for (int d = 0; d < dmax; d++) {
@@ -418,7 +459,7 @@ __global__ void k_b_ggate(int32_t* tcount, int32_t* tready, int32_t* nfin, int n
     }
 }
 
-template <int W, bool GUIDED>
+template <int W, bool GUIDED, bool SINGLE>
 __global__ __launch_bounds__(kBlock, 6) void k_b_connect(const typename TravNode<W>::type* __restrict__ nodes,
                                                       const TriV* __restrict__ tris,
                                                       const JobDev* __restrict__ jobs, PoolDev P, BatchQ q,
@@ -434,7 +475,7 @@ __global__ __launch_bounds__(kBlock, 6) void k_b_connect(const typename TravNode
         d = mk(b.x, b.y, b.z);
         tmin = a.w;
         tmax = b.w;
-        return jobs[P.job[__float_as_int(q.sh_contrib[id].w)]].root;
+        return SINGLE ? jobs[0].root : jobs[P.job[__float_as_int(q.sh_contrib[id].w)]].root;
     };
     auto emit = [&](uint32_t id, const TraceResult& r) {
         if (r.prim < 0 && !r.overflow) {
@@ -505,17 +546,6 @@ __global__ void k_b_fill_u64(unsigned long long* p, int64_t n) {
 __global__ void k_b_fill_f64(double* p, int64_t n) {
     const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i < n) p[i] = 0.0;
-}
-
-__global__ void k_b_zero2(unsigned long long* next) {
-    if (threadIdx.x < 2) next[threadIdx.x] = 0ull;
-}
-
-__global__ void k_b_reset(int32_t* counts, int out_q) {
-    if (threadIdx.x == 0) {
-        counts[out_q] = 0;
-        counts[2] = 0;
-    }
 }
 
 inline unsigned nblk(int64_t n, int b) { return unsigned((n + b - 1) / b); }
@@ -708,10 +738,10 @@ int Batch::build_arena(int width, int leaf, hipStream_t s) {
 int Wavefront::ensure_pool(int c) {
     if (cap == c) return LMGPU_OK;
     cap = 0;
-    LMGPU_TRY(pjob.alloc(c)); LMGPU_TRY(ppix.alloc(c)); LMGPU_TRY(psample.alloc(c)); LMGPU_TRY(pstate.alloc(c));
-    LMGPU_TRY(pthr.alloc(c)); LMGPU_TRY(pL.alloc(c)); LMGPU_TRY(pprev.alloc(c)); LMGPU_TRY(pinfo.alloc(c));
+    LMGPU_TRY(pjob.alloc(c)); LMGPU_TRY(ppix.alloc(c)); LMGPU_TRY(pstate.alloc(c)); LMGPU_TRY(pL.alloc(c));
     LMGPU_TRY(ext0.alloc(c)); LMGPU_TRY(ext1.alloc(c)); LMGPU_TRY(sh.alloc(c));
-    LMGPU_TRY(path0.alloc(c)); LMGPU_TRY(path1.alloc(c)); LMGPU_TRY(hit.alloc(c)); LMGPU_TRY(shc.alloc(c));
+    LMGPU_TRY(thr0.alloc(c)); LMGPU_TRY(thr1.alloc(c)); LMGPU_TRY(prev0.alloc(c)); LMGPU_TRY(prev1.alloc(c));
+    LMGPU_TRY(hit.alloc(c)); LMGPU_TRY(shc.alloc(c));
     if (!counts.p) LMGPU_TRY(counts.alloc(16));
     if (!ctl.p) LMGPU_TRY(ctl.alloc(1));
     if (!next.p) LMGPU_TRY(next.alloc(2));
@@ -751,13 +781,14 @@ int Wavefront::ensure_guided(int rec_depth, int64_t train_cap) {
     return LMGPU_OK;
 }
 
-int Wavefront::run(const void* trav_nodes, const TriV* tris, int width, int block, int64_t total, int max_verts,
+int Wavefront::run(const void* trav_nodes, const TriV* tris, int width, int block, bool single, int64_t total, int max_verts,
                    double* film_sum, double* fsq, double* elapsed, int64_t* iters, hipStream_t s,
                    const RegenGuide* G) {
     const int nsegs = int(dsegs.n);
-    PoolDev P{pjob.p, ppix.p, psample.p, pstate.p, pthr.p, pL.p, pprev.p, pinfo.p};
-    BatchQ q{{ext0.p, ext1.p}, {path0.p, path1.p}, hit.p, sh.p, shc.p, counts.p};
+    PoolDev P{pjob.p, ppix.p, pstate.p, pL.p};
+    BatchQ q{{ext0.p, ext1.p}, {thr0.p, thr1.p}, {prev0.p, prev1.p}, hit.p, sh.p, shc.p, counts.p};
     const int refill = 32;
+    if (single) block = kSingleBlock;
     GuideDev gd{};
     const bool train = G && G->steps > 0 && G->rec_depth > 0;
     const int tcap = G ? G->batch * G->steps : 0;
@@ -785,63 +816,44 @@ int Wavefront::run(const void* trav_nodes, const TriV* tris, int width, int bloc
         // at most kRegenMaxIter strides of the pool per block
         const unsigned rg = unsigned(std::max<int64_t>(std::max<int64_t>(1, std::min<int64_t>(nblk(cap, block), 4096)),
                                                        nblk(cap, block * kRegenMaxIter)));
-        if (block == 128)
-            hipLaunchKernelGGL(k_b_regen<128>, dim3(rg), dim3(128), 0, cs, djobs.p, dsegs.p, nsegs, total, P, q, in_q, cap,
-                               ctl.p, job_done.p, job_time.p, film_sum, fsq);
-        else
-            hipLaunchKernelGGL(k_b_regen<256>, dim3(rg), dim3(256), 0, cs, djobs.p, dsegs.p, nsegs, total, P, q, in_q, cap,
-                               ctl.p, job_done.p, job_time.p, film_sum, fsq);
-        hipLaunchKernelGGL(k_b_zero2, dim3(1), dim3(64), 0, cs, next.p);
-        if (width == 2)
-            hipLaunchKernelGGL(k_b_extend<2>, dim3(occupancy_grid(k_b_extend<2>, kBlock)), dim3(kBlock), 0, cs,
-                               static_cast<const TravNode<2>::type*>(trav_nodes), tris, djobs.p, P, q, in_q, next.p, refill, ctl.p);
-        else if (width == 4)
-            hipLaunchKernelGGL(k_b_extend<4>, dim3(occupancy_grid(k_b_extend<4>, kBlock)), dim3(kBlock), 0, cs,
-                               static_cast<const TravNode<4>::type*>(trav_nodes), tris, djobs.p, P, q, in_q, next.p, refill, ctl.p);
-        else
-            hipLaunchKernelGGL(k_b_extend<8>, dim3(occupancy_grid(k_b_extend<8>, kBlock)), dim3(kBlock), 0, cs,
-                               static_cast<const TravNode<8>::type*>(trav_nodes), tris, djobs.p, P, q, in_q, next.p, refill, ctl.p);
-        hipLaunchKernelGGL(k_b_reset, dim3(1), dim3(64), 0, cs, counts.p, in_q ^ 1);
-        if (G)
-            hipLaunchKernelGGL(k_pt_guide_infer<BatchQ>, dim3(unsigned(std::max(1, std::min(cap / 128, 512)))), dim3(256),
-                               0, cs, G->sc, q, in_q, G->g->Wbf.p, G->g->P.p, G->box, gmix.p);
+        auto regen = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(rg), dim3(unsigned(block)), 0, cs, djobs.p, dsegs.p, nsegs, total, P, q, in_q,
+                               cap, ctl.p, next.p, job_done.p, job_time.p, film_sum, fsq);
+        };
+        auto extend = [&](auto kernel, auto* nd) {
+            hipLaunchKernelGGL(kernel, dim3(occupancy_grid(kernel, kBlock)), dim3(kBlock), 0, cs, nd, tris, djobs.p, P, q,
+                               in_q, next.p, refill, ctl.p);
+        };
         const unsigned sg = unsigned(std::max<int64_t>(1, std::min<int64_t>(nblk(cap, block), 2048 * 256 / block)));
-        if (G) {
-            if (block == 128)
-                hipLaunchKernelGGL((k_b_shade<128, true>), dim3(sg), dim3(128), 0, cs, djobs.p, P, q, in_q, gd, cap);
-            else
-                hipLaunchKernelGGL((k_b_shade<256, true>), dim3(sg), dim3(256), 0, cs, djobs.p, P, q, in_q, gd, cap);
-        } else {
-            if (block == 128)
-                hipLaunchKernelGGL((k_b_shade<128, false>), dim3(sg), dim3(128), 0, cs, djobs.p, P, q, in_q, gd, cap);
-            else
-                hipLaunchKernelGGL((k_b_shade<256, false>), dim3(sg), dim3(256), 0, cs, djobs.p, P, q, in_q, gd, cap);
-        }
-        if (width == 2) {
-            const auto* nd = static_cast<const TravNode<2>::type*>(trav_nodes);
+        auto shade = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(sg), dim3(unsigned(block)), 0, cs, djobs.p, P, q, in_q, gd, cap);
+        };
+        auto connect = [&](auto kernel, auto* nd) {
+            hipLaunchKernelGGL(kernel, dim3(occupancy_grid(kernel, kBlock)), dim3(kBlock), 0, cs, nd, tris, djobs.p, P, q,
+                               next.p + 1, refill, ctl.p, gd.rec, gd.sh_rec);
+        };
+        auto iterate = [&](auto w) {
+            constexpr int W = decltype(w)::value;
+            const auto* nd = static_cast<const typename TravNode<W>::type*>(trav_nodes);
+            if (single) regen(k_b_regen<kSingleBlock, true>);
+            else if (block == 128) regen(k_b_regen<128, false>);
+            else regen(k_b_regen<256, false>);
+            if (single) extend(k_b_extend<W, true>, nd);
+            else extend(k_b_extend<W, false>, nd);
             if (G)
-                hipLaunchKernelGGL((k_b_connect<2, true>), dim3(occupancy_grid(k_b_connect<2, true>, kBlock)), dim3(kBlock), 0,
-                                   cs, nd, tris, djobs.p, P, q, next.p + 1, refill, ctl.p, gd.rec, gd.sh_rec);
-            else
-                hipLaunchKernelGGL((k_b_connect<2, false>), dim3(occupancy_grid(k_b_connect<2, false>, kBlock)), dim3(kBlock),
-                                   0, cs, nd, tris, djobs.p, P, q, next.p + 1, refill, ctl.p, gd.rec, gd.sh_rec);
-        } else if (width == 4) {
-            const auto* nd = static_cast<const TravNode<4>::type*>(trav_nodes);
-            if (G)
-                hipLaunchKernelGGL((k_b_connect<4, true>), dim3(occupancy_grid(k_b_connect<4, true>, kBlock)), dim3(kBlock), 0,
-                                   cs, nd, tris, djobs.p, P, q, next.p + 1, refill, ctl.p, gd.rec, gd.sh_rec);
-            else
-                hipLaunchKernelGGL((k_b_connect<4, false>), dim3(occupancy_grid(k_b_connect<4, false>, kBlock)), dim3(kBlock),
-                                   0, cs, nd, tris, djobs.p, P, q, next.p + 1, refill, ctl.p, gd.rec, gd.sh_rec);
-        } else {
-            const auto* nd = static_cast<const TravNode<8>::type*>(trav_nodes);
-            if (G)
-                hipLaunchKernelGGL((k_b_connect<8, true>), dim3(occupancy_grid(k_b_connect<8, true>, kBlock)), dim3(kBlock), 0,
-                                   cs, nd, tris, djobs.p, P, q, next.p + 1, refill, ctl.p, gd.rec, gd.sh_rec);
-            else
-                hipLaunchKernelGGL((k_b_connect<8, false>), dim3(occupancy_grid(k_b_connect<8, false>, kBlock)), dim3(kBlock),
-                                   0, cs, nd, tris, djobs.p, P, q, next.p + 1, refill, ctl.p, gd.rec, gd.sh_rec);
-        }
+                hipLaunchKernelGGL(k_pt_guide_infer<BatchQ>, dim3(unsigned(std::max(1, std::min(cap / 128, 512)))),
+                                   dim3(256), 0, cs, G->sc, q, in_q, G->g->Wbf.p, G->g->P.p, G->box, gmix.p);
+            if (G) shade(k_b_shade<kSingleBlock, true, true>);
+            else if (single) shade(k_b_shade<kSingleBlock, false, true>);
+            else if (block == 128) shade(k_b_shade<128, false, false>);
+            else shade(k_b_shade<256, false, false>);
+            if (G) connect(k_b_connect<W, true, true>, nd);
+            else if (single) connect(k_b_connect<W, false, true>, nd);
+            else connect(k_b_connect<W, false, false>, nd);
+        };
+        if (width == 2) iterate(std::integral_constant<int, 2>{});
+        else if (width == 4) iterate(std::integral_constant<int, 4>{});
+        else iterate(std::integral_constant<int, 8>{});
     };
     return loop(iteration, total, max_verts, elapsed, iters, s);
 }
@@ -990,7 +1002,7 @@ int Batch::run_once(int width, int block, int spp_cap, bool keep_results, bool w
     LMGPU_TRY(wf.set_work(jobdev, segs, s));
     hipLaunchKernelGGL(k_b_fill_f64, dim3(nblk(film_n, 256)), dim3(256), 0, s, film.p, film_n);
     if (with_sumsq) hipLaunchKernelGGL(k_b_fill_f64, dim3(nblk(film_n, 256)), dim3(256), 0, s, film_sq.p, film_n);
-    LMGPU_TRY(wf.run(trav_nodes(), tris.p, width, block, total, max_v, film.p, with_sumsq ? film_sq.p : nullptr,
+    LMGPU_TRY(wf.run(trav_nodes(), tris.p, width, block, false, total, max_v, film.p, with_sumsq ? film_sq.p : nullptr,
                      elapsed, iters, s));
     if (keep_results) {
         // job latency = device clock at the job's last sample - clock at the start
@@ -1030,8 +1042,8 @@ int Scene::render_regen(const PTConsts& c, int spp, int sample_offset, double* s
     J.seed_hi = c.seed_hi;
     J.film_off = 0;
     const int64_t total = int64_t(c.npix) * spp;
-    std::vector<WorkSeg> segs(static_cast<size_t>(spp));
-    for (int k = 0; k < spp; k++) segs[size_t(k)] = WorkSeg{int64_t(k) * c.npix, 0, sample_offset + k};
+    // one job: items are its samples' pixels in order from the first sample
+    const std::vector<WorkSeg> segs{WorkSeg{0, 0, sample_offset}};
     // pool: LMGPU_REGEN_SLOTS_PER_PIXEL paths per pixel (the slots of a
     // sample's short paths take the next sample's pixels)
     const int cap = gp ? Wavefront::pool_size(total, c.npix, LMGPU_REGEN_GUIDED_SLOTS_PER_PIXEL,
@@ -1061,7 +1073,7 @@ int Scene::render_regen(const PTConsts& c, int spp, int sample_offset, double* s
                      : accel.width == 8 ? static_cast<const void*>(dev.nodes8) : static_cast<const void*>(dev.nodes2);
     double sec = 0;
     int64_t iters = 0;
-    LMGPU_TRY(wf->run(tn, accel.tris.p, accel.width, 128, total, c.max_verts, sum, sumsq, &sec, &iters, s,
+    LMGPU_TRY(wf->run(tn, accel.tris.p, accel.width, kSingleBlock, true, total, c.max_verts, sum, sumsq, &sec, &iters, s,
                       gp ? &G : nullptr));
     BatchCtl hc;
     LMGPU_HIP(hipMemcpy(&hc, wf->ctl.p, sizeof(hc), hipMemcpyDeviceToHost));
@@ -1195,8 +1207,14 @@ int lmgpu_batch_run(lmgpu_batch* bh, const lmgpu_batch_opts* opts, lmgpu_batch_s
                 int64_t it;
                 return b.run_once(w, bl, 1, false, o.film_sumsq != 0, o.queue_order, sec, &it, s);
             };
-            const int widths[3] = {4, 8, 2}, caps[3] = {1 << 22, 1 << 21, 1 << 23}, blocks[2] = {256, 128};
-            int bw = width ? width : 4, bc = capv ? capv : (1 << 22), bb = block ? block : 256;
+            const int widths[3] = {4, 8, 2}, blocks[2] = {256, 128};
+            // a pool of more slots than the run has samples holds no more paths
+            int64_t all = 0;
+            for (const auto& J : b.jobs) all += int64_t(J.desc.w) * J.desc.h * J.spp;
+            std::vector<int> caps;
+            for (int c : {1 << 22, 1 << 21, 1 << 23})
+                if (c == (1 << 21) || c / 2 < all) caps.push_back(c);
+            int bw = width ? width : 4, bc = capv ? capv : caps[0], bb = block ? block : 256;
             double best = 1e30, sec;
             if (!width)
                 for (int w : widths) {

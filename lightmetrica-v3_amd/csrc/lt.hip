@@ -372,8 +372,13 @@ template <int W>
 void lt_regen_iteration(Scene& S, Wavefront& wf, const LTConsts& c, int64_t total, int npix, uint32_t pass0,
                         double* film, int in_q, hipStream_t s) {
     const int cap = wf.cap;
-    Queues q{{wf.ext0.p, wf.ext1.p}, wf.hit.p, {wf.path0.p, wf.path1.p}, wf.sh.p, wf.shc.p, wf.counts.p};
-    PathState ps{wf.pthr.p, wf.pL.p, wf.pprev.p, wf.pinfo.p};
+    // the path tracer's per-entry state arrays hold the light paths' slots,
+    // vertex counts and passes
+    int32_t* paths[2] = {reinterpret_cast<int32_t*>(wf.prev0.p), reinterpret_cast<int32_t*>(wf.prev1.p)};
+    int4* info = reinterpret_cast<int4*>(wf.thr1.p);
+    int32_t* ppass = reinterpret_cast<int32_t*>(wf.pL.p);
+    Queues q{{wf.ext0.p, wf.ext1.p}, wf.hit.p, {paths[0], paths[1]}, wf.sh.p, wf.shc.p, wf.counts.p};
+    PathState ps{wf.thr0.p, nullptr, nullptr, info};
     constexpr int kRegenBlock = 128;
     // at most 32 strides of the pool per regenerate block
     const unsigned rg = unsigned(std::max<int64_t>(std::min<int64_t>((cap + kRegenBlock - 1) / kRegenBlock, 4096),
@@ -381,11 +386,11 @@ void lt_regen_iteration(Scene& S, Wavefront& wf, const LTConsts& c, int64_t tota
     const int sg = std::max(1, std::min((cap + kBlock - 1) / kBlock, 2048));
     const int refill = 32;
     hipLaunchKernelGGL(k_lt_regen<kRegenBlock>, dim3(rg), dim3(kRegenBlock), 0, s, S.dev, c, total, npix, pass0,
-                       wf.ppix.p, wf.psample.p, wf.pstate.p, wf.pthr.p, wf.pinfo.p, q, in_q, cap, wf.ctl.p);
+                       wf.ppix.p, ppass, wf.pstate.p, wf.thr0.p, info, q, in_q, cap, wf.ctl.p);
     hipLaunchKernelGGL(k_lt_begin, dim3(1), dim3(64), 0, s, wf.next.p, wf.counts.p, in_q ^ 1);
     hipLaunchKernelGGL(k_extend<W>, dim3(extend_grid<W>()), dim3(kBlock), 0, s, S.dev, q, in_q, wf.next.p, refill,
                        LMGPU_REGEN_RAY_CHUNK);
-    hipLaunchKernelGGL(k_lt_shade, dim3(sg), dim3(kBlock), 0, s, S.dev, ps, q, c, in_q, wf.ppix.p, wf.psample.p,
+    hipLaunchKernelGGL(k_lt_shade, dim3(sg), dim3(kBlock), 0, s, S.dev, ps, q, c, in_q, wf.ppix.p, ppass,
                        wf.pstate.p);
     hipLaunchKernelGGL(k_lt_connect<W>, dim3(lt_connect_grid<W>()), dim3(kBlock), 0, s, S.dev, q, wf.next.p + 1, refill,
                        film, LMGPU_REGEN_RAY_CHUNK);

@@ -57,17 +57,30 @@ struct WorkSeg {
     int32_t job, sample;
 };
 
+// Slot states, in the low bits; a finishing path's slot holds the vertex
+// count at which it ended above them.
 constexpr int32_t kFree = 0, kActive = 1, kFinishing = 2;
+constexpr int kStateShift = 8;
+constexpr int32_t kStateMask = (1 << kStateShift) - 1;
 
+// Path slots: what outlives one iteration of a path. L.w holds the sample
+// index's bits.
 struct PoolDev {
-    int32_t *job, *pixel, *sample, *state;
-    float4 *thr, *L, *prev;
-    int4* info;
+    int32_t *job, *pixel, *state;
+    float4* L;
 };
 
+// Vertex count and flags (PathRegs::info.x, .z) of a path in one word.
+LMGPU_HD int32_t pack_info(int nv, int flags) { return nv | (flags << 8); }
+LMGPU_HD int info_verts(int32_t w) { return w & 0xff; }
+LMGPU_HD int info_flags(int32_t w) { return w >> 8; }
+
+// Extension queues: entry i of a queue is a path's next ray with its state,
+// written by the vertex that sampled it and read once by the next.
 struct BatchQ {
-    lmgpu_ray* ext[2];
-    int32_t* ext_path[2];
+    lmgpu_ray* ext[2];    // tmin holds the slot's bits, tmax the pdf of the direction (projected SA)
+    float4* thr[2];       // throughput, w = pack_info bits
+    float4* prev[2];      // shading normal of the previous vertex, w = pixel bits
     lmgpu_hit* hit;
     lmgpu_ray* sh;
     float4* sh_contrib;   // xyz contribution, w = path slot bits
@@ -101,11 +114,9 @@ struct RegenGuide {
 // and by lmgpu_pt_render's regenerating path.
 struct Wavefront {
     int cap = 0;
-    DevBuf<int32_t> pjob, ppix, psample, pstate;
-    DevBuf<float4> pthr, pL, pprev;
-    DevBuf<int4> pinfo;
+    DevBuf<int32_t> pjob, ppix, pstate, counts;
+    DevBuf<float4> pL, thr0, thr1, prev0, prev1;
     DevBuf<lmgpu_ray> ext0, ext1, sh;
-    DevBuf<int32_t> path0, path1, counts;
     DevBuf<lmgpu_hit> hit;
     DevBuf<float4> shc;
     DevBuf<BatchCtl> ctl;
@@ -137,7 +148,9 @@ struct Wavefront {
     // With a guide, the directions at diffuse and glossy vertices come from
     // the one-sample mixture of guide and BSDF, and the guide trains online
     // on the records of finished paths.
-    int run(const void* trav_nodes, const TriV* tris, int width, int block, int64_t total, int max_verts,
+    // single: one job, whose work segment 0 starts at its first sample
+    // (kernels specialised for it, at their own block size).
+    int run(const void* trav_nodes, const TriV* tris, int width, int block, bool single, int64_t total, int max_verts,
             double* film_sum, double* film_sq, double* elapsed, int64_t* iters, hipStream_t s,
             const RegenGuide* guide = nullptr);
     // The loop itself: frees the pool, sets the run's counters for `total`
