@@ -877,7 +877,8 @@ static void launch_trace(const Accel& a, const lmgpu_ray* rays, lmgpu_hit* hits,
     for (int64_t at = 0; at < n; at += kMaxLaunchRays) {
         const int64_t m = std::min(n - at, kMaxLaunchRays);
         hipLaunchKernelGGL(k_zero_counter, dim3(1), dim3(64), 0, s, next);
-        const int grid = int(std::min<int64_t>(persistent_grid<W, ANY, COUNT, Node>(), (m + kTraceBlock - 1) / kTraceBlock));
+        // a block per 64 rays: few rays spread over the CUs one wave each
+        const int grid = int(std::min<int64_t>(persistent_grid<W, ANY, COUNT, Node>(), (m + 63) / 64));
         hipLaunchKernelGGL((k_trace<W, ANY, COUNT, Node>), dim3(grid), dim3(kTraceBlock), 0, s,
                            static_cast<const Node*>(a.trav_nodes()), a.tris.p, rays + at, hits ? hits + at : nullptr,
                            occl ? occl + at : nullptr, uint32_t(m), next, status, counters, a.refill);

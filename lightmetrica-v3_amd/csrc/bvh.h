@@ -462,7 +462,7 @@ constexpr int64_t kMaxLaunchRays = int64_t(1) << 30;
 // Persistent traversal: every lane owns one ray at a time; when at least
 // `refill` lanes of a wave have finished (or the whole wave has), the
 // finished lanes hand over their results together and take new rays from the
-// wave's pool, which the wave refills by chunks of chunk_rays (default
+// wave's pool: a share of its own, then chunks of chunk_rays (default
 // LMGPU_RAY_CHUNK) from one global counter with one atomic (Aila & Laine,
 // HPG 2009, "persistent threads"), so lanes do not sit idle behind a wave's
 // slowest ray and the counter sees few atomics. refill = 64 keeps whole
@@ -513,9 +513,25 @@ __device__ __forceinline__ void trace_persistent(const Node* __restrict__ nodes,
     int cur = kDone;             // node (>= 0), leaf (< 0) or kDone
     int sp = 0;                  // stack entries
     lds[0][tid] = kDone;
-    // wave-uniform: ray ids taken from `next` and not yet handed to a lane
-    uint32_t pool_next = 0, pool_end = 0;
-    bool exhausted = false;
+    // Wave-uniform: ray ids of the wave not yet handed to a lane, and whether
+    // ids are left beyond them. Every wave starts with a share of its own, half
+    // of an even split in whole waves of rays (at least one), and `next` hands
+    // out what lies past all shares: atomics on one address from all XCDs take
+    // 12 ns each, so one per wave before any ray started took 74 us of every
+    // launch (at 1080p and below, path tracing of small scenes lost a third of
+    // its time to it: 16 spp of the room at 256x256 6.40 -> 4.48 ms, one 360p
+    // preview pass 2.70 -> 1.74). Shares go to the waves of a block in a row, whose
+    // rays then meet in its L1; with fewer shares than waves they go to the
+    // blocks in turn, over all CUs.
+    const uint32_t nblk = gridDim.x, nwaves = nblk * (BLOCK / 64);
+    const uint32_t share = max(64u, n / nwaves / 2u & ~63u);
+    const uint32_t in_blk = threadIdx.x >> 6;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(n < nwaves * 64u ? in_blk * nblk + blockIdx.x
+                                                                         : blockIdx.x * (BLOCK / 64) + in_blk);
+    const uint32_t shared_from = nwaves * share;   // < n + 64 nwaves
+    uint32_t pool_next = min(n, wave * share), pool_end = min(n, wave * share + share);
+    bool more = shared_from < n;                   // ids beyond the pool may be left
+    bool exhausted = pool_next == pool_end && !more;
     unsigned long long nv = 0, nt = 0;
     // component kx (shift 0), ky (3) or kz (6) of v: tests of single bits
     // stay two selects, where a test of the number itself becomes branches
@@ -566,22 +582,24 @@ __device__ __forceinline__ void trace_persistent(const Node* __restrict__ nodes,
             }
             if (!exhausted) {
                 // idle lanes take, in lane order, the rest of the wave's pool
-                // and then the start of a new chunk
+                // and then the start of a new chunk (chunk_end - chunk rays)
                 const bool idle = cur == kDone;
                 const unsigned long long idle_mask = ~busy;
                 const uint32_t nidle = __popcll(idle_mask);
                 const uint32_t avail = pool_end - pool_next;
-                uint32_t chunk = 0;
-                if (avail < nidle) {
+                uint32_t chunk = n, chunk_end = n;
+                if (avail < nidle && more) {
                     uint32_t b = 0;
                     if (lane == 0) b = uint32_t(atomicAdd(next, (unsigned long long)chunk_rays));
                     // wave-uniform from here on: scalar registers for the pool
-                    chunk = __builtin_amdgcn_readfirstlane(b);
+                    chunk = min(n, shared_from + __builtin_amdgcn_readfirstlane(b));
+                    chunk_end = min(n, chunk + chunk_rays);
+                    more = chunk_end < n;
                 }
                 if (idle) {
                     const uint32_t rank = __popcll(idle_mask & ((1ull << lane) - 1ull));
                     const uint32_t id = rank < avail ? pool_next + rank : chunk + (rank - avail);
-                    if (id < n) {
+                    if (rank < avail || id < chunk_end) {
                         rid = id;
                         f3 o, d;
                         cur = fetch(id, o, d, tmin, tfar);
@@ -594,12 +612,12 @@ __device__ __forceinline__ void trace_persistent(const Node* __restrict__ nodes,
                     }
                 }
                 if (avail < nidle) {
-                    pool_next = chunk + (nidle - avail);
-                    pool_end = chunk + chunk_rays;
+                    pool_next = min(chunk + (nidle - avail), chunk_end);
+                    pool_end = chunk_end;
                 } else {
                     pool_next += nidle;
                 }
-                exhausted = pool_next >= n;   // the counter only grows: no id below n is left
+                exhausted = pool_next == pool_end && !more;
             }
             if (__ballot(cur != kDone) == 0) break;
         }
