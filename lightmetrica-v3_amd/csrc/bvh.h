@@ -73,7 +73,6 @@ struct alignas(W * 16) QNode {
     uint32_t qhi[3][W / 4];
     int32_t ent[W];
     uint32_t es;       // the grid exponents again, unbiased: signed bytes 0, 1, 2
-    float slack;       // 2^-20 * 255 * the largest step: part of the slab test's rounding bound
 };
 using QNode4 = QNode<4>;
 static_assert(sizeof(QNode<4>) == 64, "quantised BVH4 node must be 64 B");
@@ -109,7 +108,6 @@ LMGPU_HD int leaf_count(int e) { return (-(e + 1)) & 15; }
 
 struct RayPre {
     f3 o, d, inv;
-    f3 bn, bf;       // -o inv lowered / raised by 2^-20 |o inv|: the ray's part of the slab offsets
     float Sx, Sy, Sz;
     int kx, ky, kz;
     float dkz_abs;   // |d[kz]|, relates the watertight det to the MT det
@@ -125,16 +123,7 @@ LMGPU_HD RayPre ray_prepare(f3 o, f3 d) {
     const float dx = fabsf(d.x) < tiny ? copysignf(tiny, d.x) : d.x;
     const float dy = fabsf(d.y) < tiny ? copysignf(tiny, d.y) : d.y;
     const float dz = fabsf(d.z) < tiny ? copysignf(tiny, d.z) : d.z;
-#if defined(__HIP_DEVICE_COMPILE__)
-    // v_rcp_f32 is within 1 ulp, which the slab test's slack covers (child_keys)
-    r.inv = mk(__builtin_amdgcn_rcpf(dx), __builtin_amdgcn_rcpf(dy), __builtin_amdgcn_rcpf(dz));
-#else
     r.inv = mk(1.0f / dx, 1.0f / dy, 1.0f / dz);
-#endif
-    const f3 oi = mk(o.x * r.inv.x, o.y * r.inv.y, o.z * r.inv.z);
-    const f3 e = mk(fabsf(oi.x), fabsf(oi.y), fabsf(oi.z)) * 0x1p-20f;
-    r.bn = -oi - e;
-    r.bf = e - oi;
     const float ax = fabsf(d.x), ay = fabsf(d.y), az = fabsf(d.z);
     int kz = (ax > ay) ? (ax > az ? 0 : 2) : (ay > az ? 1 : 2);
     int kx = kz + 1 == 3 ? 0 : kz + 1;
@@ -251,22 +240,23 @@ LMGPU_HD float qplane(uint32_t q, int c, float step, float origin) {
 // and no decoded plane: the planes are the exact reals ox + q * step. Each
 // axis picks its near and far plane by the sign of inv_x, so one fma gives
 // the entry and one the exit distance (no per-axis min / max). Bounds, with
-// u = 2^-24 and P = |ox| + 255 step: the exact plane lies within u P of the
-// FP32 plane the builder rounded outward (quantise_node); inv_x is within 2u
-// (v_rcp_f32), -o inv, the two fmas that form bx and the plane's fma round
-// relatively, each within u |inv| (P + |o|). The entry offset is lowered and
-// the exit offset raised by
-//   16u |inv| (P + |o|),
-// more than twice their sum, so every child box the exact planes' test would
-// hit is hit here too, with no further factor on the exit distance. The step's
-// part is one number per node (slack), |o|'s comes with the ray (bn, bf).
+// u = 2^-24: bx is within 2u |bx| of (ox - o_x) * inv_x; the exact plane
+// ox + q step lies within u (|ox| + 255 step) of the FP32 plane the builder
+// rounded outward (quantise_node); the fma and inv_x round relatively, which
+// the 1 + 2 gamma(3) factor on the exit distance covers (box_near). The entry
+// offset is lowered and the exit offset raised by
+//   Ex = 16u (|bx| + |inv_x| |ox| + 255 |ax|),
+// which exceeds the absolute terms with their own rounding, so every child
+// box the FP32 test of the decoded planes would hit is hit here too.
+// The keys order the traversal, and where coplanar triangles tie in t (a box
+// standing on a floor) the one visited last is the hit: the keys' rounding
+// is part of the result, and a cheaper bound for Ex is not a free choice.
 template <int W>
 LMGPU_HD void child_keys(const QNode<W>& nd, const RayPre& r, float tmin, float tmax, float (&key)[W],
                          int (&ent)[W]) {
     const float org[3] = {nd.ox, nd.oy, nd.oz};
     const float inv[3] = {r.inv.x, r.inv.y, r.inv.z};
-    const float bn0[3] = {r.bn.x, r.bn.y, r.bn.z};
-    const float bf0[3] = {r.bf.x, r.bf.y, r.bf.z};
+    const float o[3] = {r.o.x, r.o.y, r.o.z};
     float a[3], bn[3], bf[3];
     uint32_t wn[3][W / 4], wf[3][W / 4];
     // both plane words of every axis as loaded (whole 16-B loads of the node);
@@ -286,9 +276,10 @@ LMGPU_HD void child_keys(const QNode<W>& nd, const RayPre& r, float tmin, float 
 #pragma unroll
     for (int k = 0; k < 3; k++) {
         a[k] = ldexpf(inv[k], int32_t(nd.es << (24 - 8 * k)) >> 24);
-        const float e = fmaf(fabsf(org[k]), 0x1p-20f, nd.slack);
-        bn[k] = fmaf(-fabsf(inv[k]), e, fmaf(org[k], inv[k], bn0[k]));
-        bf[k] = fmaf(fabsf(inv[k]), e, fmaf(org[k], inv[k], bf0[k]));
+        const float b = (org[k] - o[k]) * inv[k];
+        const float x = fabsf(b) + fmaf(fabsf(org[k]), fabsf(inv[k]), 255.f * fabsf(a[k]));
+        bn[k] = fmaf(x, -0x1p-20f, b);   // Ex = 2^-20 x
+        bf[k] = fmaf(x, 0x1p-20f, b);
         const bool pos = inv[k] >= 0.f;
 #pragma unroll
         for (int w = 0; w < W / 4; w++) {
@@ -307,7 +298,7 @@ LMGPU_HD void child_keys(const QNode<W>& nd, const RayPre& r, float tmin, float 
         }
         const float n = fmaxf(fmaxf(tn[0], tn[1]), fmaxf(tn[2], tmin));
         const float f = fminf(fminf(tf[0], tf[1]), fminf(tf[2], tmax));
-        key[c] = n <= f ? n : __builtin_inff();
+        key[c] = n <= f * 1.00000036f ? n : __builtin_inff();
         ent[c] = nd.ent[c];
     }
 }
@@ -323,7 +314,6 @@ LMGPU_HD QNode<W> quantise_node(const WNode<W>& n) {
     const float* hi[3] = {n.hix, n.hiy, n.hiz};
     float org[3];
     uint32_t ebits = 0, esigned = 0;
-    float step_max = 0.f;
     for (int a = 0; a < 3; a++) {
         float mn = __builtin_inff(), mx = -__builtin_inff();
         for (int c = 0; c < W; c++)
@@ -347,7 +337,6 @@ LMGPU_HD QNode<W> quantise_node(const WNode<W>& n) {
         while (e < 127 && std::fma(255.f, std::ldexp(1.f, e), mn) < mx) e++;
         ebits |= uint32_t(e + 127) << (8 * a);
         esigned |= uint32_t(e & 0xff) << (8 * a);
-        step_max = std::max(step_max, std::ldexp(1.f, e));
         uint32_t ql[W / 4] = {}, qh[W / 4] = {};
         const float step = std::ldexp(1.f, e);
         for (int c = 0; c < W; c++) {
@@ -374,7 +363,6 @@ LMGPU_HD QNode<W> quantise_node(const WNode<W>& n) {
     q.oz = org[2];
     q.e = ebits;
     q.es = esigned;
-    q.slack = (255.f * 0x1p-20f) * step_max;
     for (int c = 0; c < W; c++)
         q.ent[c] = n.count[c] < 0 ? kQEmpty : (n.count[c] == 0 ? n.child[c] : encode_leaf(n.child[c], n.count[c]));
     return q;
@@ -412,42 +400,35 @@ __device__ __forceinline__ void refine_hit(const TriV& tv, const RayPre& r, floa
     v = float((dx * qx + dy * qy + dz * qz) * inv);
 }
 
-// A child's sort item: its slab key in the high word, its stack entry in the
-// low word of a double. Keys are finite non-NaN floats or +inf, whose bits as
-// the high word never form an FP64 NaN or infinity (exponent at most 0x7f8),
-// and for non-negative keys the doubles order as the keys do. So one compare
-// and exchange of a (key, entry) pair is a v_min_f64 and a v_max_f64 (full
-// rate) instead of a compare and four selects. Inline asm because the
-// builtins first quiet signalling NaNs, which the items never are.
-__device__ __forceinline__ double sort_item(float key, int ent) { return __hiloint2double(__float_as_int(key), ent); }
-__device__ __forceinline__ float item_key(double x) { return __int_as_float(__double2hiint(x)); }
-__device__ __forceinline__ int item_ent(double x) { return __double2loint(x); }
-__device__ __forceinline__ void cswap(double& a, double& b) {
-    double lo, hi;
-    asm("v_min_f64 %0, %1, %2" : "=v"(lo) : "v"(a), "v"(b));
-    asm("v_max_f64 %0, %1, %2" : "=v"(hi) : "v"(a), "v"(b));
-    a = lo;
-    b = hi;
+// Orders the (key, entry) pairs of a node's children by key. Equal keys (a ray
+// starting inside several boxes, boxes that share a plane) stay in place at
+// each compare: their order decides which of coplanar triangles is hit, so
+// the network's own order on ties is part of the result.
+__device__ __forceinline__ void cswap(float& ka, int& ea, float& kb, int& eb) {
+    const bool s = kb < ka;
+    const float tk = s ? kb : ka;
+    const int te = s ? eb : ea;
+    kb = s ? ka : kb;
+    eb = s ? ea : eb;
+    ka = tk;
+    ea = te;
 }
 
 template <int W>
-__device__ __forceinline__ void sort_children(double (&x)[W]) {
+__device__ __forceinline__ void sort_children(float (&k)[W], int (&e)[W]) {
+    auto cs = [&](int a, int b) { cswap(k[a], e[a], k[b], e[b]); };
     if constexpr (W == 2) {
-        cswap(x[0], x[1]);
+        cs(0, 1);
     } else if constexpr (W == 4) {
-        cswap(x[0], x[1]);
-        cswap(x[2], x[3]);
-        cswap(x[0], x[2]);
-        cswap(x[1], x[3]);
-        cswap(x[1], x[2]);
+        cs(0, 1); cs(2, 3); cs(0, 2); cs(1, 3); cs(1, 2);
     } else {
         // Batcher odd-even merge sort network for 8 inputs (19 comparators).
-        cswap(x[0], x[1]); cswap(x[2], x[3]); cswap(x[4], x[5]); cswap(x[6], x[7]);
-        cswap(x[0], x[2]); cswap(x[1], x[3]); cswap(x[4], x[6]); cswap(x[5], x[7]);
-        cswap(x[1], x[2]); cswap(x[5], x[6]);
-        cswap(x[0], x[4]); cswap(x[1], x[5]); cswap(x[2], x[6]); cswap(x[3], x[7]);
-        cswap(x[2], x[4]); cswap(x[3], x[5]);
-        cswap(x[1], x[2]); cswap(x[3], x[4]); cswap(x[5], x[6]);
+        cs(0, 1); cs(2, 3); cs(4, 5); cs(6, 7);
+        cs(0, 2); cs(1, 3); cs(4, 6); cs(5, 7);
+        cs(1, 2); cs(5, 6);
+        cs(0, 4); cs(1, 5); cs(2, 6); cs(3, 7);
+        cs(2, 4); cs(3, 5);
+        cs(1, 2); cs(3, 4); cs(5, 6);
     }
 }
 
@@ -481,18 +462,16 @@ constexpr int64_t kMaxLaunchRays = int64_t(1) << 30;
 // and entry i of the lane's stack lds[1 + i][lane]; each child is written at
 // the top of the stack and the stack grows by one only if the child was hit,
 // so what lies above the top is garbage that the next push overwrites; and
-// the entry to pop is read before the test, behind the node's own load. The
+// the entry to pop is read before the test, with the node's own load. The
 // first LDS_DEPTH entries live there, at [entry][lane] (bank-conflict free),
 // the rest in private memory: a wave with a lane that could pass LDS_DEPTH in
 // this step takes a separate, branchy path. Results are emitted
 // only when lanes are refilled: done as each ray ends, the FP64
 // re-evaluation ran in most iterations for a lane or two.
-// Measured together with the slab test's shared offsets, the pair sort and
-// the branch-free push, on the 1.32M-triangle mesh: 2.07M primary rays 723 ->
-// 539 us, 2M incoherent rays 952 -> 907 (bound by the 16-B accesses of its
-// divergent node loads: the address unit is busy 75% of the time), 500K
-// any-hit rays on the 8-wide tree 515 -> 448, a 16-spp 1080p path-traced frame
-// 74.4 -> 63.4 ms.
+// Measured on the 1.32M-triangle mesh together with the waves' own shares
+// (below): 2.07M primary rays 723 -> 492 us, 2M incoherent rays 952 -> 890
+// (bound by the 16-B accesses of its divergent node loads: the address unit is
+// busy 75% of the time), 500K any-hit rays on the 8-wide tree 515 -> 382.
 template <int W, bool ANY, bool COUNT, int LDS_DEPTH, int PRIV_DEPTH, int BLOCK, class Node, class Fetch, class Emit>
 __device__ __forceinline__ void trace_persistent(const Node* __restrict__ nodes, const TriV* __restrict__ tris,
                                                  uint32_t n, unsigned long long* next, int (*lds)[BLOCK],
@@ -518,8 +497,7 @@ __device__ __forceinline__ void trace_persistent(const Node* __restrict__ nodes,
     // of an even split in whole waves of rays (at least one), and `next` hands
     // out what lies past all shares: atomics on one address from all XCDs take
     // 12 ns each, so one per wave before any ray started took 74 us of every
-    // launch (at 1080p and below, path tracing of small scenes lost a third of
-    // its time to it: 16 spp of the room at 256x256 6.40 -> 4.48 ms, one 360p
+    // launch (16 spp of a small room at 256x256 6.40 -> 4.48 ms, one 360p
     // preview pass 2.70 -> 1.74). Shares go to the waves of a block in a row, whose
     // rays then meet in its L1; with fewer shares than waves they go to the
     // blocks in turn, over all CUs.
@@ -571,9 +549,6 @@ __device__ __forceinline__ void trace_persistent(const Node* __restrict__ nodes,
                         q.kx = kk & 1u ? 0 : (kk & 2u ? 1 : 2);
                         q.ky = kk & 8u ? 0 : (kk & 16u ? 1 : 2);
                         q.kz = kk & 64u ? 0 : (kk & 128u ? 1 : 2);
-                        // the inverse of the permutation that made ok
-                        q.o = mk(kk & 1u ? ok.x : (kk & 8u ? ok.y : ok.z), kk & 2u ? ok.x : (kk & 16u ? ok.y : ok.z),
-                                 kk & 4u ? ok.x : (kk & 32u ? ok.y : ok.z));
                         refine_hit(tv, q, tmin, res.t, res.u, res.v);
                     }
                 }
@@ -663,35 +638,32 @@ __device__ __forceinline__ void trace_persistent(const Node* __restrict__ nodes,
             float key[W];
             int ent[W];
             child_keys<W>(nd, r, tmin, tfar, key, ent);
-            double x[W];
-#pragma unroll
-            for (int c = 0; c < W; c++) x[c] = sort_item(key[c], ent[c]);
-            sort_children<W>(x);
+            sort_children<W>(key, ent);
             const float kInfF = __builtin_inff();
             if (__ballot(sp + W - 1 > LDS_DEPTH) == 0) {
 #pragma unroll
                 for (int c = W - 1; c >= 1; c--) {
-                    lds[sp + 1][tid] = item_ent(x[c]);
-                    sp += item_key(x[c]) != kInfF ? 1 : 0;
+                    lds[sp + 1][tid] = ent[c];
+                    sp += key[c] != kInfF ? 1 : 0;
                 }
-                const bool any_child = item_key(x[0]) != kInfF;
-                cur = any_child ? item_ent(x[0]) : top;
+                const bool any_child = key[0] != kInfF;
+                cur = any_child ? ent[0] : top;
                 sp = any_child ? sp : max(sp - 1, 0);
             } else {
                 bool full = false;
 #pragma unroll
                 for (int c = W - 1; c >= 1; c--)
-                    if (item_key(x[c]) != kInfF) {
-                        if (sp < LDS_DEPTH) lds[sp + 1][tid] = item_ent(x[c]);
-                        else if (sp < LDS_DEPTH + PRIV_DEPTH) priv[sp - LDS_DEPTH] = item_ent(x[c]);
+                    if (key[c] != kInfF) {
+                        if (sp < LDS_DEPTH) lds[sp + 1][tid] = ent[c];
+                        else if (sp < LDS_DEPTH + PRIV_DEPTH) priv[sp - LDS_DEPTH] = ent[c];
                         else full = true;
                         if (!full) sp++;
                     }
                 if (full) {
                     overflow = true;
                     cur = kDone;
-                } else if (item_key(x[0]) != kInfF) {
-                    cur = item_ent(x[0]);
+                } else if (key[0] != kInfF) {
+                    cur = ent[0];
                 } else {
                     cur = pop_deep();
                 }
