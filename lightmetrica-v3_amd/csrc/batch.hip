@@ -45,11 +45,10 @@ namespace {
 
 __device__ __forceinline__ uint64_t job_seed(const JobDev& J) { return (uint64_t(J.seed_hi) << 32) | J.seed_lo; }
 
-// Most grid-stride iterations of k_b_regen per block (the host sizes the grid
-// so that a block covers at most this many BLOCK-slot strides of the pool).
-constexpr int kRegenMaxIter = 32;
-// Block size of the regenerate and shade kernels of a single scene's render.
-constexpr int kSingleBlock = 128;
+// Block size of the regenerate and shade kernels of a single scene's render (16
+// spp at 1080p: 128 48.7 ms, 256 44.9, 512 45.9, as an append is one atomic a
+// block).
+constexpr int kSingleBlock = 256;
 // Entries of k_b_regen's per-block table of finished-sample counts per job.
 constexpr int kRegenJobSlots = 64;
 
@@ -73,7 +72,7 @@ __global__ __launch_bounds__(BLOCK) void k_b_regen(const JobDev* __restrict__ jo
                                                    unsigned long long* job_done, unsigned long long* job_time,
                                                    double* film_sum, double* film_sq) {
     constexpr int kWaves = BLOCK / 64;
-    __shared__ int s_want[kRegenMaxIter][kWaves];   // slots taking work, then their exclusive prefix
+    __shared__ int s_want[kRegenStrides][kWaves];   // slots taking work, then their exclusive prefix
     __shared__ unsigned long long s_base;           // first work item of the block
     __shared__ int s_qbase;                         // first queue entry of the block
     __shared__ int s_emit;                          // queue entries of the block
@@ -90,8 +89,8 @@ __global__ __launch_bounds__(BLOCK) void k_b_regen(const JobDev* __restrict__ jo
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         next[0] = 0ull;
         next[1] = 0ull;
-        q.counts[in_q ^ 1] = 0;
-        q.counts[2] = 0;
+        q.counts[ext_count(in_q ^ 1)] = 0;
+        q.counts[shadow_count(in_q ^ 1)] = 0;
     }
     if (threadIdx.x == 0)
         s_idle = __hip_atomic_load(&ctl->remaining, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0;
@@ -99,7 +98,7 @@ __global__ __launch_bounds__(BLOCK) void k_b_regen(const JobDev* __restrict__ jo
     if (s_idle) return;
     if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&ctl->iterations, 1ull);
     const int stride = gridDim.x * BLOCK;
-    const int n_iter = (cap + stride - 1) / stride;   // <= kRegenMaxIter (host)
+    const int n_iter = (cap + stride - 1) / stride;   // <= kRegenStrides (host)
     const int lane = __lane_id();
     const int wave = threadIdx.x >> 6;
     if (!SINGLE)
@@ -131,10 +130,12 @@ __global__ __launch_bounds__(BLOCK) void k_b_regen(const JobDev* __restrict__ jo
         unsigned long long base = 0;
         int emit = 0, qb = 0;
         if (acc > 0) {
-            base = atomicAdd(&ctl->work_next, (unsigned long long)acc);
+            // no atomic (12 ns each, on one address) once the queue is empty
+            base = __hip_atomic_load(&ctl->work_next, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (base < (unsigned long long)total) base = atomicAdd(&ctl->work_next, (unsigned long long)acc);
             if (base < (unsigned long long)total)
                 emit = int(min((unsigned long long)acc, (unsigned long long)total - base));
-            if (emit > 0) qb = atomicAdd(q.counts + in_q, emit);
+            if (emit > 0) qb = atomicAdd(q.counts + ext_count(in_q), emit);
         }
         s_base = base;
         s_emit = emit;
@@ -192,7 +193,7 @@ __global__ __launch_bounds__(BLOCK) void k_b_regen(const JobDev* __restrict__ jo
                 int job = 0, sample, pix;
                 if (SINGLE) {
                     const uint32_t np = uint32_t(jobs[0].npix);
-                    const uint32_t at = uint32_t(s_pixel) + uint32_t(r);   // < 2^28 + kRegenMaxIter * BLOCK
+                    const uint32_t at = uint32_t(s_pixel) + uint32_t(r);   // < 2^28 + kRegenStrides * BLOCK
                     sample = s_sample + int(at / np);
                     pix = int(at % np);
                 } else {
@@ -245,7 +246,7 @@ __global__ __launch_bounds__(kBlock, 6) void k_b_extend(const typename TravNode<
                                                      const JobDev* __restrict__ jobs, PoolDev P, BatchQ q, int in_q,
                                                      unsigned long long* next, int refill, BatchCtl* ctl) {
     __shared__ int lds[kLds + 1][kBlock];
-    const int n = q.counts[in_q];
+    const int n = q.counts[ext_count(in_q)];
     if (n == 0) return;   // an idle iteration after the last work item (whole grid)
     const lmgpu_ray* rays = q.ext[in_q];
     auto fetch = [&](uint32_t id, f3& o, f3& d, float& tmin, float& tmax) -> int {
@@ -272,7 +273,7 @@ __global__ __launch_bounds__(kBlock, 6) void k_b_extend(const typename TravNode<
 template <int BLOCK, bool GUIDED, bool SINGLE>
 __global__ __launch_bounds__(BLOCK) void k_b_shade(const JobDev* __restrict__ jobs, PoolDev P, BatchQ q, int in_q,
                                                    GuideDev gd, int cap) {
-    const int n = q.counts[in_q];
+    const int n = q.counts[ext_count(in_q)];
     const int out_q = in_q ^ 1;
     const int stride = gridDim.x * BLOCK;
     const int n_iter = (n + stride - 1) / stride;
@@ -310,7 +311,7 @@ __global__ __launch_bounds__(BLOCK) void k_b_shade(const JobDev* __restrict__ jo
             P.L[s] = make_float4(R.L.x, R.L.y, R.L.z, L4.w);
         }
         int se, ss;
-        block_append2<BLOCK>(q.counts + out_q, q.counts + 2, out.ext, out.sh, se, ss);
+        block_append2<BLOCK>(q.counts + ext_count(out_q), out.ext, out.sh, se, ss);
         if (out.ext) {
             out.ext_ray.tmin = __int_as_float(s);
             out.ext_ray.tmax = R.prev.w;
@@ -462,11 +463,11 @@ __global__ void k_b_ggate(int32_t* tcount, int32_t* tready, int32_t* nfin, int n
 template <int W, bool GUIDED, bool SINGLE>
 __global__ __launch_bounds__(kBlock, 6) void k_b_connect(const typename TravNode<W>::type* __restrict__ nodes,
                                                       const TriV* __restrict__ tris,
-                                                      const JobDev* __restrict__ jobs, PoolDev P, BatchQ q,
+                                                      const JobDev* __restrict__ jobs, PoolDev P, BatchQ q, int out_q,
                                                       unsigned long long* next, int refill, BatchCtl* ctl,
                                                       GRec* __restrict__ rec, const int32_t* __restrict__ sh_rec) {
     __shared__ int lds[kLds + 1][kBlock];
-    const int n = q.counts[2];
+    const int n = q.counts[shadow_count(out_q)];
     if (n == 0) return;   // no shadow rays this iteration (whole grid)
     auto fetch = [&](uint32_t id, f3& o, f3& d, float& tmin, float& tmax) -> int {
         const float4* rp = reinterpret_cast<const float4*>(q.sh + id);
@@ -549,6 +550,7 @@ __global__ void k_b_fill_f64(double* p, int64_t n) {
 }
 
 inline unsigned nblk(int64_t n, int b) { return unsigned((n + b - 1) / b); }
+
 
 // Graph replays (two iterations each) the host enqueues between looks at the
 // device's progress.
@@ -813,9 +815,7 @@ int Wavefront::run(const void* trav_nodes, const TriV* tris, int width, int bloc
                 (void)G->g->enqueue_train(gtrain.p + int64_t(t) * G->batch * kRecordFloats, G->batch, G->batch,
                                           gcnt.p + 1, int64_t(t) * G->batch, G->lr, nullptr, cs, G->wclamp);
         }
-        // at most kRegenMaxIter strides of the pool per block
-        const unsigned rg = unsigned(std::max<int64_t>(std::max<int64_t>(1, std::min<int64_t>(nblk(cap, block), 4096)),
-                                                       nblk(cap, block * kRegenMaxIter)));
+        const unsigned rg = regen_grid(cap, block);
         auto regen = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, dim3(rg), dim3(unsigned(block)), 0, cs, djobs.p, dsegs.p, nsegs, total, P, q, in_q,
                                cap, ctl.p, next.p, job_done.p, job_time.p, film_sum, fsq);
@@ -830,7 +830,7 @@ int Wavefront::run(const void* trav_nodes, const TriV* tris, int width, int bloc
         };
         auto connect = [&](auto kernel, auto* nd) {
             hipLaunchKernelGGL(kernel, dim3(occupancy_grid(kernel, kBlock)), dim3(kBlock), 0, cs, nd, tris, djobs.p, P, q,
-                               next.p + 1, refill, ctl.p, gd.rec, gd.sh_rec);
+                               in_q ^ 1, next.p + 1, refill, ctl.p, gd.rec, gd.sh_rec);
         };
         auto iterate = [&](auto w) {
             constexpr int W = decltype(w)::value;

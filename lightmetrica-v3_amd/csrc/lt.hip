@@ -107,7 +107,7 @@ __global__ __launch_bounds__(BLOCK) void k_lt_regen(SceneDev sc, LTConsts c, int
                                                     int4* __restrict__ pinfo, Queues q, int in_q, int cap,
                                                     BatchCtl* ctl) {
     constexpr int kWaves = BLOCK / 64;
-    constexpr int kMaxIter = 32;
+    constexpr int kMaxIter = kRegenStrides;
     __shared__ int s_want[kMaxIter][kWaves];
     __shared__ unsigned long long s_base;
     __shared__ int s_qbase, s_emit, s_idle;
@@ -144,9 +144,10 @@ __global__ __launch_bounds__(BLOCK) void k_lt_regen(SceneDev sc, LTConsts c, int
         unsigned long long base = 0;
         int emit = 0, qb = 0;
         if (acc > 0) {
-            base = atomicAdd(&ctl->work_next, (unsigned long long)acc);
+            base = __hip_atomic_load(&ctl->work_next, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (base < (unsigned long long)total) base = atomicAdd(&ctl->work_next, (unsigned long long)acc);
             if (base < (unsigned long long)total) emit = int(min((unsigned long long)acc, (unsigned long long)total - base));
-            if (emit > 0) qb = atomicAdd(q.counts + in_q, emit);
+            if (emit > 0) qb = atomicAdd(q.counts + ext_count(in_q), emit);
         }
         s_base = base;
         s_emit = emit;
@@ -199,7 +200,7 @@ __global__ __launch_bounds__(BLOCK) void k_lt_regen(SceneDev sc, LTConsts c, int
 __global__ __launch_bounds__(kBlock) void k_lt_shade(SceneDev sc, PathState ps, Queues q, LTConsts c, int in_q,
                                                     const int32_t* __restrict__ ppid,
                                                     const int32_t* __restrict__ ppass, int32_t* __restrict__ pstate) {
-    const int n = q.counts[in_q];
+    const int n = q.counts[ext_count(in_q)];
     const int out_q = in_q ^ 1;
     const uint64_t seed = lt_seed(c);
     const int stride = gridDim.x * kBlock;
@@ -304,7 +305,7 @@ __global__ __launch_bounds__(kBlock) void k_lt_shade(SceneDev sc, PathState ps, 
         }
         if (i < n && !emit_ext) pstate[p] = kFinishing;
         int se, ss;
-        block_append2<kBlock>(q.counts + out_q, q.counts + 2, emit_ext, emit_sh, se, ss);
+        block_append2<kBlock>(q.counts + ext_count(out_q), emit_ext, emit_sh, se, ss);
         if (emit_ext) {
             q.ext[out_q][se] = ext_ray;
             q.ext_path[out_q][se] = p;
@@ -317,10 +318,10 @@ __global__ __launch_bounds__(kBlock) void k_lt_shade(SceneDev sc, PathState ps, 
 }
 
 template <int W>
-__global__ __launch_bounds__(kBlock, 6) void k_lt_connect(SceneDev sc, Queues q, unsigned long long* next, int refill,
+__global__ __launch_bounds__(kBlock, 6) void k_lt_connect(SceneDev sc, Queues q, int out_q, unsigned long long* next, int refill,
                                                        double* __restrict__ film, int chunk_rays) {
     __shared__ int lds[kLds + 1][kBlock];
-    const int n = q.counts[2];
+    const int n = q.counts[shadow_count(out_q)];
     if (n == 0) return;   // no connections (whole grid)
     auto fetch = [&](uint32_t id, f3& o, f3& d, float& tmin, float& tmax) -> int {
         const float4* rp = reinterpret_cast<const float4*>(q.sh + id);
@@ -349,8 +350,8 @@ __global__ __launch_bounds__(kBlock, 6) void k_lt_connect(SceneDev sc, Queues q,
 __global__ void k_lt_begin(unsigned long long* next, int32_t* counts, int out_q) {
     if (threadIdx.x < 2) next[threadIdx.x] = 0ull;
     if (threadIdx.x == 0) {
-        counts[out_q] = 0;
-        counts[2] = 0;
+        counts[ext_count(out_q)] = 0;
+        counts[shadow_count(out_q)] = 0;
     }
 }
 
@@ -380,9 +381,7 @@ void lt_regen_iteration(Scene& S, Wavefront& wf, const LTConsts& c, int64_t tota
     Queues q{{wf.ext0.p, wf.ext1.p}, wf.hit.p, {paths[0], paths[1]}, wf.sh.p, wf.shc.p, wf.counts.p};
     PathState ps{wf.thr0.p, nullptr, nullptr, info};
     constexpr int kRegenBlock = 128;
-    // at most 32 strides of the pool per regenerate block
-    const unsigned rg = unsigned(std::max<int64_t>(std::min<int64_t>((cap + kRegenBlock - 1) / kRegenBlock, 4096),
-                                                   (cap + kRegenBlock * 32 - 1) / (kRegenBlock * 32)));
+    const unsigned rg = regen_grid(cap, kRegenBlock);
     const int sg = std::max(1, std::min((cap + kBlock - 1) / kBlock, 2048));
     const int refill = 32;
     hipLaunchKernelGGL(k_lt_regen<kRegenBlock>, dim3(rg), dim3(kRegenBlock), 0, s, S.dev, c, total, npix, pass0,
@@ -392,7 +391,7 @@ void lt_regen_iteration(Scene& S, Wavefront& wf, const LTConsts& c, int64_t tota
                        LMGPU_REGEN_RAY_CHUNK);
     hipLaunchKernelGGL(k_lt_shade, dim3(sg), dim3(kBlock), 0, s, S.dev, ps, q, c, in_q, wf.ppix.p, ppass,
                        wf.pstate.p);
-    hipLaunchKernelGGL(k_lt_connect<W>, dim3(lt_connect_grid<W>()), dim3(kBlock), 0, s, S.dev, q, wf.next.p + 1, refill,
+    hipLaunchKernelGGL(k_lt_connect<W>, dim3(lt_connect_grid<W>()), dim3(kBlock), 0, s, S.dev, q, in_q ^ 1, wf.next.p + 1, refill,
                        film, LMGPU_REGEN_RAY_CHUNK);
 }
 
@@ -472,40 +471,77 @@ __device__ __forceinline__ float env_pdf_ray(const SceneDev& sc, const BDConsts&
 __global__ __launch_bounds__(kBlock) void k_bd_lgen(SceneDev sc, PathState ps, Queues q, BDConsts c,
                                                     LVert* __restrict__ lv, int32_t* __restrict__ lcount) {
     const int i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= c.npaths) return;
-    const uint64_t seed = bd_seed(c);
-    const rand4 r0 = rng(uint32_t(i), c.pass, 0u, 0u, seed);
-    const rand4 r1 = rng(uint32_t(i), c.pass, 0u, 1u, seed);
-    const int li = min(max(int(r0.u[0] * sc.num_lights), 0), sc.num_lights - 1);
-    if (i == 0) {
-        q.counts[0] = c.npaths;
-        atomicAdd(reinterpret_cast<unsigned long long*>(q.counts + 8), (unsigned long long)c.npaths);
-    }
-    if (li >= sc.num_area_lights) {
-        const f3 d = sample_uniform_sphere(r1.u[0], r1.u[1]);
-        const float rr = sqrtf(fmaxf(0.f, r0.u[2])) * c.sph_r;
-        float sn, cs;
-        sincosf(2.f * kPi * r0.u[3], &sn, &cs);
+    bool emit_sh = false;
+    lmgpu_ray sr;
+    float4 sh_c;
+    auto start = [&]() {
+        const uint64_t seed = bd_seed(c);
+        const rand4 r0 = rng(uint32_t(i), c.pass, 0u, 0u, seed);
+        const rand4 r1 = rng(uint32_t(i), c.pass, 0u, 1u, seed);
+        const int li = min(max(int(r0.u[0] * sc.num_lights), 0), sc.num_lights - 1);
+        if (i == 0) {
+            q.counts[ext_count(0)] = c.npaths;
+            atomicAdd(reinterpret_cast<unsigned long long*>(q.counts + 8), (unsigned long long)c.npaths);
+        }
+        if (li >= sc.num_area_lights) {
+            const f3 d = sample_uniform_sphere(r1.u[0], r1.u[1]);
+            const float rr = sqrtf(fmaxf(0.f, r0.u[2])) * c.sph_r;
+            float sn, cs;
+            sincosf(2.f * kPi * r0.u[3], &sn, &cs);
+            f3 u, v;
+            onb(d, u, v);
+            const f3 org = c.sph_c - d * c.sph_r + u * (rr * cs) + v * (rr * sn);
+            const float pray = env_pdf_ray(sc, c);
+            LVert y;
+            y.a = make_float4(org.x, org.y, org.z, __int_as_float(-1 - li));
+            y.b = make_float4(d.x, d.y, d.z, __int_as_float(-1));
+            y.c = make_float4(d.x, d.y, d.z, 0.f);
+            y.d = make_float4(0.f, 0.f, 0.f, 0.f);
+            y.e = make_float4(1.f, 1.f, 1.f, __int_as_float(kFlagSpec));   // never connected
+            y.f = make_float4(1.f, 0.f, 0.f, 0.f);
+            lv[int64_t(i) * c.lstride] = y;
+            lcount[i] = 1;
+            // weight toward y_1: Le / p_ray (bidir.h:254-256)
+            const f3 w = sc.env_Le * (1.f / pray);
+            ps.thr[i] = make_float4(w.x, w.y, w.z, 1.f);          // pL(y_0) = 1
+            ps.L[i] = make_float4(org.x, org.y, org.z, pray);     // pL(y_1) = p_ray G(y_0, y_1)
+            ps.prev[i] = make_float4(1.f, 1.f, 0.f, 0.f);         // cos 1 at infinity, T(0) = 1
+            // strategy s = 1 is not samplable: y_1 sees its predecessor as specular
+            ps.info[i] = make_int4(1, kFlagSpec | kFlagInfPrev, 0, 0);
+            lmgpu_ray ray;
+            ray.org[0] = org.x; ray.org[1] = org.y; ray.org[2] = org.z;
+            ray.tmin = kEps;
+            ray.dir[0] = d.x; ray.dir[1] = d.y; ray.dir[2] = d.z;
+            ray.tmax = kInf;
+            q.ext[0][i] = ray;
+            q.ext_path[0][i] = i;
+            return;
+        }
+        const DevLight dl = sc.lights[li];
+        f3 org, nL;
+        sample_light_point(sc, li, r0.u[1], r0.u[2], r0.u[3], org, nL);
         f3 u, v;
-        onb(d, u, v);
-        const f3 org = c.sph_c - d * c.sph_r + u * (rr * cs) + v * (rr * sn);
-        const float pray = env_pdf_ray(sc, c);
+        onb(nL, u, v);
+        const f3 dl_ = sample_cosine_weighted(r1.u[0], r1.u[1]);
+        const f3 d = u * dl_.x + v * dl_.y + nL * dl_.z;
+        // pL(y_0) = p_sel / area (path::pdf_position of the light endpoint)
+        const float pL0 = dl.Ke_invA.w / float(sc.num_lights);
+        const float a0 = 1.f / pL0;
         LVert y;
         y.a = make_float4(org.x, org.y, org.z, __int_as_float(-1 - li));
-        y.b = make_float4(d.x, d.y, d.z, __int_as_float(-1));
-        y.c = make_float4(d.x, d.y, d.z, 0.f);
+        y.b = make_float4(nL.x, nL.y, nL.z, __int_as_float(-1));
+        y.c = make_float4(nL.x, nL.y, nL.z, 0.f);
         y.d = make_float4(0.f, 0.f, 0.f, 0.f);
-        y.e = make_float4(1.f, 1.f, 1.f, __int_as_float(kFlagSpec));   // never connected
-        y.f = make_float4(1.f, 0.f, 0.f, 0.f);
+        y.e = make_float4(a0, a0, a0, __int_as_float(0));
+        y.f = make_float4(pL0, 0.f, 0.f, 0.f);
         lv[int64_t(i) * c.lstride] = y;
         lcount[i] = 1;
-        // weight toward y_1: Le / p_ray (bidir.h:254-256)
-        const f3 w = sc.env_Le * (1.f / pray);
-        ps.thr[i] = make_float4(w.x, w.y, w.z, 1.f);          // pL(y_0) = 1
-        ps.L[i] = make_float4(org.x, org.y, org.z, pray);     // pL(y_1) = p_ray G(y_0, y_1)
-        ps.prev[i] = make_float4(1.f, 1.f, 0.f, 0.f);         // cos 1 at infinity, T(0) = 1
-        // strategy s = 1 is not samplable: y_1 sees its predecessor as specular
-        ps.info[i] = make_int4(1, kFlagSpec | kFlagInfPrev, 0, 0);
+        // weight toward y_1: alpha_0 Le / pdf_dir, pdf_dir = 1 / pi (projected solid angle)
+        const f3 w = mk(dl.Ke_invA.x, dl.Ke_invA.y, dl.Ke_invA.z) * (a0 * kPi);
+        ps.thr[i] = make_float4(w.x, w.y, w.z, pL0);
+        ps.L[i] = make_float4(org.x, org.y, org.z, 1.f / kPi);
+        ps.prev[i] = make_float4(fabsf(dot(nL, d)), 1.f, 0.f, 0.f);   // |cos| at y_0, T(0) = 1
+        ps.info[i] = make_int4(1, 0, 0, 0);                          // index of the next vertex, flags
         lmgpu_ray ray;
         ray.org[0] = org.x; ray.org[1] = org.y; ray.org[2] = org.z;
         ray.tmin = kEps;
@@ -513,63 +549,35 @@ __global__ __launch_bounds__(kBlock) void k_bd_lgen(SceneDev sc, PathState ps, Q
         ray.tmax = kInf;
         q.ext[0][i] = ray;
         q.ext_path[0][i] = i;
-        return;
-    }
-    const DevLight dl = sc.lights[li];
-    f3 org, nL;
-    sample_light_point(sc, li, r0.u[1], r0.u[2], r0.u[3], org, nL);
-    f3 u, v;
-    onb(nL, u, v);
-    const f3 dl_ = sample_cosine_weighted(r1.u[0], r1.u[1]);
-    const f3 d = u * dl_.x + v * dl_.y + nL * dl_.z;
-    // pL(y_0) = p_sel / area (path::pdf_position of the light endpoint)
-    const float pL0 = dl.Ke_invA.w / float(sc.num_lights);
-    const float a0 = 1.f / pL0;
-    LVert y;
-    y.a = make_float4(org.x, org.y, org.z, __int_as_float(-1 - li));
-    y.b = make_float4(nL.x, nL.y, nL.z, __int_as_float(-1));
-    y.c = make_float4(nL.x, nL.y, nL.z, 0.f);
-    y.d = make_float4(0.f, 0.f, 0.f, 0.f);
-    y.e = make_float4(a0, a0, a0, __int_as_float(0));
-    y.f = make_float4(pL0, 0.f, 0.f, 0.f);
-    lv[int64_t(i) * c.lstride] = y;
-    lcount[i] = 1;
-    // weight toward y_1: alpha_0 Le / pdf_dir, pdf_dir = 1 / pi (projected solid angle)
-    const f3 w = mk(dl.Ke_invA.x, dl.Ke_invA.y, dl.Ke_invA.z) * (a0 * kPi);
-    ps.thr[i] = make_float4(w.x, w.y, w.z, pL0);
-    ps.L[i] = make_float4(org.x, org.y, org.z, 1.f / kPi);
-    ps.prev[i] = make_float4(fabsf(dot(nL, d)), 1.f, 0.f, 0.f);   // |cos| at y_0, T(0) = 1
-    ps.info[i] = make_int4(1, 0, 0, 0);                          // index of the next vertex, flags
-    lmgpu_ray ray;
-    ray.org[0] = org.x; ray.org[1] = org.y; ray.org[2] = org.z;
-    ray.tmin = kEps;
-    ray.dir[0] = d.x; ray.dir[1] = d.y; ray.dir[2] = d.z;
-    ray.tmax = kInf;
-    q.ext[0][i] = ray;
-    q.ext_path[0][i] = i;
-    // strategy (s, t) = (1, 1): y_0 seen by the pinhole; the only other
-    // strategy of this two-vertex path is the eye ray hitting the light (s = 0)
-    const Camera& cam = sc.cam;
-    const f3 dc = org - cam.pos;
-    const float dc2 = dot(dc, dc);
-    const float dist = sqrtf(dc2);
-    const f3 woc = dc / dist;
-    float rx, ry;
-    if (c.min_verts <= 2 && cam_raster(cam, woc, rx, ry) && dot(-woc, nL) > 0.f) {
-        const float G = fabsf(dot(nL, woc)) / dc2;
-        const float J = cam_J(cam, woc);
-        const float q0 = J * G / pL0;
-        const f3 Cw = mk(dl.Ke_invA.x, dl.Ke_invA.y, dl.Ke_invA.z) * (a0 * G * J / (1.f + q0 * q0));
-        const int px = min(max(int(rx * float(sc.w)), 0), sc.w - 1);
-        const int py = min(max(int(ry * float(sc.h)), 0), sc.h - 1);
-        const int ss = atomicAdd(q.counts + 2, 1);
-        lmgpu_ray sr;
-        sr.org[0] = org.x; sr.org[1] = org.y; sr.org[2] = org.z;
-        sr.tmin = kEps;
-        sr.dir[0] = -woc.x; sr.dir[1] = -woc.y; sr.dir[2] = -woc.z;
-        sr.tmax = dist * (1.f - kEps);
+        // strategy (s, t) = (1, 1): y_0 seen by the pinhole; the only other
+        // strategy of this two-vertex path is the eye ray hitting the light (s = 0)
+        const Camera& cam = sc.cam;
+        const f3 dc = org - cam.pos;
+        const float dc2 = dot(dc, dc);
+        const float dist = sqrtf(dc2);
+        const f3 woc = dc / dist;
+        float rx, ry;
+        if (c.min_verts <= 2 && cam_raster(cam, woc, rx, ry) && dot(-woc, nL) > 0.f) {
+            const float G = fabsf(dot(nL, woc)) / dc2;
+            const float J = cam_J(cam, woc);
+            const float q0 = J * G / pL0;
+            const f3 Cw = mk(dl.Ke_invA.x, dl.Ke_invA.y, dl.Ke_invA.z) * (a0 * G * J / (1.f + q0 * q0));
+            const int px = min(max(int(rx * float(sc.w)), 0), sc.w - 1);
+            const int py = min(max(int(ry * float(sc.h)), 0), sc.h - 1);
+            emit_sh = true;
+            sr.org[0] = org.x; sr.org[1] = org.y; sr.org[2] = org.z;
+            sr.tmin = kEps;
+            sr.dir[0] = -woc.x; sr.dir[1] = -woc.y; sr.dir[2] = -woc.z;
+            sr.tmax = dist * (1.f - kEps);
+            sh_c = make_float4(Cw.x, Cw.y, Cw.z, __int_as_float(py * sc.w + px));
+        }
+    };
+    if (i < c.npaths) start();
+    // every thread of the block takes part in the append
+    const int ss = block_append1<kBlock>(q.counts + shadow_count(1), emit_sh);
+    if (emit_sh) {
         q.sh[ss] = sr;
-        q.sh_contrib[ss] = make_float4(Cw.x, Cw.y, Cw.z, __int_as_float(py * sc.w + px));
+        q.sh_contrib[ss] = sh_c;
     }
 }
 
@@ -577,7 +585,7 @@ __global__ __launch_bounds__(kBlock) void k_bd_lgen(SceneDev sc, PathState ps, Q
 // (strategy t = 1) and sample the next direction (path::sample_direction, LE).
 __global__ __launch_bounds__(kBlock) void k_bd_lshade(SceneDev sc, PathState ps, Queues q, BDConsts c, int in_q,
                                                       LVert* __restrict__ lv, int32_t* __restrict__ lcount) {
-    const int n = q.counts[in_q];
+    const int n = q.counts[ext_count(in_q)];
     const int out_q = in_q ^ 1;
     const uint64_t seed = bd_seed(c);
     const int stride = gridDim.x * kBlock;
@@ -696,7 +704,7 @@ __global__ __launch_bounds__(kBlock) void k_bd_lshade(SceneDev sc, PathState ps,
             }
         }
         int se, ss;
-        block_append2<kBlock>(q.counts + out_q, q.counts + 2, emit_ext, emit_sh, se, ss);
+        block_append2<kBlock>(q.counts + ext_count(out_q), emit_ext, emit_sh, se, ss);
         if (emit_ext) {
             q.ext[out_q][se] = ext_ray;
             q.ext_path[out_q][se] = p;
@@ -729,7 +737,7 @@ __global__ __launch_bounds__(kBlock) void k_bd_egen(SceneDev sc, PathState ps, Q
     ray.tmax = kInf;
     q.ext[0][i] = ray;
     q.ext_path[0][i] = i;
-    if (i == 0) q.counts[0] = c.npaths;
+    if (i == 0) q.counts[ext_count(0)] = c.npaths;
 }
 
 // An eye subpath vertex z_{t-1} (t >= 2): the emitter strategy (s = 0),
@@ -738,7 +746,7 @@ __global__ __launch_bounds__(kBlock) void k_bd_egen(SceneDev sc, PathState ps, Q
 __global__ __launch_bounds__(kBlock) void k_bd_eshade(SceneDev sc, PathState ps, Queues q, BDConsts c, int in_q,
                                                       const LVert* __restrict__ lv, const int32_t* __restrict__ lcount,
                                                       double* __restrict__ film) {
-    const int n = q.counts[in_q];
+    const int n = q.counts[ext_count(in_q)];
     const int out_q = in_q ^ 1;
     const uint64_t seed = bd_seed(c);
     const int stride = gridDim.x * kBlock;
@@ -856,7 +864,7 @@ __global__ __launch_bounds__(kBlock) void k_bd_eshade(SceneDev sc, PathState ps,
                 }
             }
         }
-        const int se = block_append1<kBlock>(q.counts + out_q, emit_ext);
+        const int se = block_append1<kBlock>(q.counts + ext_count(out_q), emit_ext);
         if (emit_ext) {
             q.ext[out_q][se] = ext_ray;
             q.ext_path[out_q][se] = p;
@@ -925,7 +933,7 @@ __global__ __launch_bounds__(kBlock) void k_bd_eshade(SceneDev sc, PathState ps,
                     }
                 }
             }
-            const int ss = block_append1<kBlock>(q.counts + 2, emit_sh);
+            const int ss = block_append1<kBlock>(q.counts + shadow_count(out_q), emit_sh);
             if (emit_sh) {
                 q.sh[ss] = sh_ray;
                 q.sh_contrib[ss] = sh_c;
@@ -944,14 +952,14 @@ void bd_pass(Scene& S, const BDConsts& c, double* film, int refill, LVert* lv, h
     const int cg = lt_connect_grid<W>();
     hipLaunchKernelGGL(k_lt_begin, dim3(1), dim3(64), 0, s, S.next.p, S.counts.p, 1);
     hipLaunchKernelGGL(k_bd_lgen, dim3(gb), dim3(kBlock), 0, s, S.dev, ps, q, c, lv, S.blcount.p);
-    hipLaunchKernelGGL(k_lt_connect<W>, dim3(cg), dim3(kBlock), 0, s, S.dev, q, S.next.p + 1, refill, film,
+    hipLaunchKernelGGL(k_lt_connect<W>, dim3(cg), dim3(kBlock), 0, s, S.dev, q, 1, S.next.p + 1, refill, film,
                            LMGPU_RAY_CHUNK);
     for (int b = 0; b < c.max_verts - 2; b++) {   // y_1 .. y_{max_verts - 2}
         const int in_q = b & 1;
         hipLaunchKernelGGL(k_lt_begin, dim3(1), dim3(64), 0, s, S.next.p, S.counts.p, in_q ^ 1);
         hipLaunchKernelGGL(k_extend<W>, dim3(tg), dim3(kBlock), 0, s, S.dev, q, in_q, S.next.p, refill, LMGPU_RAY_CHUNK);
         hipLaunchKernelGGL(k_bd_lshade, dim3(sg), dim3(kBlock), 0, s, S.dev, ps, q, c, in_q, lv, S.blcount.p);
-        hipLaunchKernelGGL(k_lt_connect<W>, dim3(cg), dim3(kBlock), 0, s, S.dev, q, S.next.p + 1, refill, film,
+        hipLaunchKernelGGL(k_lt_connect<W>, dim3(cg), dim3(kBlock), 0, s, S.dev, q, in_q ^ 1, S.next.p + 1, refill, film,
                            LMGPU_RAY_CHUNK);
     }
     hipLaunchKernelGGL(k_bd_egen, dim3(gb), dim3(kBlock), 0, s, S.dev, ps, q, c);
@@ -960,7 +968,7 @@ void bd_pass(Scene& S, const BDConsts& c, double* film, int refill, LVert* lv, h
         hipLaunchKernelGGL(k_lt_begin, dim3(1), dim3(64), 0, s, S.next.p, S.counts.p, in_q ^ 1);
         hipLaunchKernelGGL(k_extend<W>, dim3(tg), dim3(kBlock), 0, s, S.dev, q, in_q, S.next.p, refill, LMGPU_RAY_CHUNK);
         hipLaunchKernelGGL(k_bd_eshade, dim3(sg), dim3(kBlock), 0, s, S.dev, ps, q, c, in_q, lv, S.blcount.p, film);
-        hipLaunchKernelGGL(k_lt_connect<W>, dim3(cg), dim3(kBlock), 0, s, S.dev, q, S.next.p + 1, refill, film,
+        hipLaunchKernelGGL(k_lt_connect<W>, dim3(cg), dim3(kBlock), 0, s, S.dev, q, in_q ^ 1, S.next.p + 1, refill, film,
                            LMGPU_RAY_CHUNK);
     }
 }

@@ -45,7 +45,7 @@ template <bool IMAGE>
 __global__ __launch_bounds__(kBlock) void k_generate(SceneDev sc, PathState ps, Queues q, PTConsts c) {
     const int p = blockIdx.x * kBlock + threadIdx.x;
     if (p >= c.npix) return;
-    const uint32_t sample = uint32_t(q.counts[3]);
+    const uint32_t sample = uint32_t(q.counts[4]);
     const uint64_t seed = (uint64_t(c.seed_hi) << 32) | c.seed_lo;
     const lmgpu_ray ray = camera_ray(sc, p, sample, seed, IMAGE);
     ps.thr[p] = make_float4(1.f, 1.f, 1.f, 0.f);
@@ -63,7 +63,7 @@ __global__ __launch_bounds__(kBlock) void k_generate(SceneDev sc, PathState ps, 
     q.ext[0][p] = ray;
     q.ext_path[0][p] = p;
     if (p == 0) {
-        q.counts[0] = c.npix;
+        q.counts[ext_count(0)] = c.npix;
         atomicAdd(reinterpret_cast<unsigned long long*>(q.counts + 8), (unsigned long long)c.npix);
     }
 }
@@ -80,7 +80,7 @@ __global__ __launch_bounds__(kBlock) void k_camera_nee(SceneDev sc, Queues q, PT
     lmgpu_ray ray;
     float4 C;
     if (p < c.npix) {
-        const uint32_t sample = uint32_t(q.counts[3]);
+        const uint32_t sample = uint32_t(q.counts[4]);
         const uint64_t seed = (uint64_t(c.seed_hi) << 32) | c.seed_lo;
         const rand4 r1 = rng(uint32_t(p), sample, 0u, 1u, seed);
         const int li = min(max(int(r1.u[0] * sc.num_lights), 0), sc.num_lights - 1);
@@ -134,7 +134,7 @@ __global__ __launch_bounds__(kBlock) void k_camera_nee(SceneDev sc, Queues q, PT
             }
         }
     }
-    const int ss = wave_append(q.counts + 2, emit);
+    const int ss = wave_append(q.counts + shadow_count(0), emit);
     if (emit) {
         q.sh[ss] = ray;
         q.sh_contrib[ss] = C;
@@ -143,8 +143,8 @@ __global__ __launch_bounds__(kBlock) void k_camera_nee(SceneDev sc, Queues q, PT
 
 __global__ void k_reset_counts(int32_t* counts, int out_q) {
     if (threadIdx.x == 0) {
-        counts[out_q] = 0;
-        counts[2] = 0;
+        counts[ext_count(out_q)] = 0;
+        counts[shadow_count(out_q)] = 0;
     }
 }
 
@@ -155,10 +155,10 @@ __global__ void k_reset_counts(int32_t* counts, int out_q) {
 // incident radiance).
 template <int W>
 __global__ __launch_bounds__(kBlock, 6) void k_connect(SceneDev sc, PathState ps, Queues q, unsigned long long* next,
-                                                   int refill, GRec* __restrict__ rec, const int32_t* __restrict__ sh_rec,
-                                                   double* __restrict__ splat) {
+                                                   int out_q, int refill, GRec* __restrict__ rec,
+                                                   const int32_t* __restrict__ sh_rec, double* __restrict__ splat) {
     __shared__ int lds[kLds + 1][kBlock];
-    const int n = q.counts[2];
+    const int n = q.counts[shadow_count(out_q)];
     if (n == 0) return;   // no shadow rays (whole grid)
     auto fetch = [&](uint32_t id, f3& o, f3& d, float& tmin, float& tmax) -> int {
         const float4* rp = reinterpret_cast<const float4*>(q.sh + id);
@@ -213,9 +213,9 @@ __global__ void k_bounce_begin(unsigned long long* next) {
 // entry), appending the next extension rays and the shadow rays.
 template <bool GUIDED>
 __global__ __launch_bounds__(kBlock) void k_shade(SceneDev sc, PathState ps, Queues q, PTConsts c, int in_q, GuideDev gd) {
-    const int n = q.counts[in_q];
+    const int n = q.counts[ext_count(in_q)];
     const int out_q = in_q ^ 1;
-    const uint32_t sample = uint32_t(q.counts[3]);
+    const uint32_t sample = uint32_t(q.counts[4]);
     const uint64_t seed = (uint64_t(c.seed_hi) << 32) | c.seed_lo;
     const int stride = gridDim.x * kBlock;
     // every thread of the grid runs the same number of iterations: the
@@ -243,7 +243,7 @@ __global__ __launch_bounds__(kBlock) void k_shade(SceneDev sc, PathState ps, Que
             ps.L[p] = make_float4(P.L.x, P.L.y, P.L.z, 0.f);
         }
         int se, ss;
-        block_append2<kBlock>(q.counts + out_q, q.counts + 2, out.ext, out.sh, se, ss);
+        block_append2<kBlock>(q.counts + ext_count(out_q), out.ext, out.sh, se, ss);
         if (out.ext) {
             q.ext[out_q][se] = out.ext_ray;
             q.ext_path[out_q][se] = p;
@@ -383,7 +383,7 @@ __global__ __launch_bounds__(kBlock) void k_accumulate(SceneDev sc, PathState ps
     const float4 L = ps.L[p];
     if (c.image) {
         if (L.x == 0.f && L.y == 0.f && L.z == 0.f) return;
-        const rand4 r = rng(uint32_t(p), uint32_t(q.counts[3]), 0u, 0u, (uint64_t(c.seed_hi) << 32) | c.seed_lo);
+        const rand4 r = rng(uint32_t(p), uint32_t(q.counts[4]), 0u, 0u, (uint64_t(c.seed_hi) << 32) | c.seed_lo);
         double* f = sum + 3 * int64_t(raster_pixel(sc.w, sc.h, r.u[2], r.u[3]));
         atomicAdd(f + 0, double(L.x));
         atomicAdd(f + 1, double(L.y));
@@ -401,12 +401,12 @@ __global__ __launch_bounds__(kBlock) void k_accumulate(SceneDev sc, PathState ps
 }
 
 __global__ void k_next_sample(int32_t* counts) {
-    if (threadIdx.x == 0) counts[3] += 1;
+    if (threadIdx.x == 0) counts[4] += 1;
 }
 
 __global__ void k_set_sample(int32_t* counts, int s) {
     if (threadIdx.x == 0) {
-        counts[3] = s;
+        counts[4] = s;
         counts[5] = 0;
     }
 }
@@ -716,18 +716,18 @@ int Scene::enqueue_pass(const PTConsts& c, double* sum, double* sumsq, const Gui
     const int tg = accel.width == 4 ? pt_trace_grid<4>() : (accel.width == 8 ? pt_trace_grid<8>() : pt_trace_grid<2>());
     if (c.image && c.mode != LMGPU_SAMPLING_NAIVE) {
         // the camera vertex's light samples, traced before the first bounce
-        hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(64), 0, s, counts.p + 2, 1);
+        hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(64), 0, s, counts.p + shadow_count(0), 1);
         hipLaunchKernelGGL(k_camera_nee, dim3(gb), dim3(kBlock), 0, s, dev, q, c);
         hipLaunchKernelGGL(k_bounce_begin, dim3(1), dim3(64), 0, s, next.p);
         unsigned long long* nx = next.p + 1;
         if (accel.width == 4)
-            hipLaunchKernelGGL(k_connect<4>, dim3(tg), dim3(kBlock), 0, s, dev, ps, q, nx, refill_primary, nullptr,
+            hipLaunchKernelGGL(k_connect<4>, dim3(tg), dim3(kBlock), 0, s, dev, ps, q, nx, 0, refill_primary, nullptr,
                                nullptr, sum);
         else if (accel.width == 8)
-            hipLaunchKernelGGL(k_connect<8>, dim3(tg), dim3(kBlock), 0, s, dev, ps, q, nx, refill_primary, nullptr,
+            hipLaunchKernelGGL(k_connect<8>, dim3(tg), dim3(kBlock), 0, s, dev, ps, q, nx, 0, refill_primary, nullptr,
                                nullptr, sum);
         else
-            hipLaunchKernelGGL(k_connect<2>, dim3(tg), dim3(kBlock), 0, s, dev, ps, q, nx, refill_primary, nullptr,
+            hipLaunchKernelGGL(k_connect<2>, dim3(tg), dim3(kBlock), 0, s, dev, ps, q, nx, 0, refill_primary, nullptr,
                                nullptr, sum);
     }
     for (int b = 0; b < c.max_verts - 1; b++) {
@@ -747,10 +747,10 @@ int Scene::enqueue_pass(const PTConsts& c, double* sum, double* sumsq, const Gui
         if (c.mode != LMGPU_SAMPLING_NAIVE) {
             unsigned long long* nx = next.p + 1;
             if (accel.width == 4)
-                hipLaunchKernelGGL(k_connect<4>, dim3(tg), dim3(kBlock), 0, s, dev, ps, q, nx, pm, crec, cshrec, sum);
+                hipLaunchKernelGGL(k_connect<4>, dim3(tg), dim3(kBlock), 0, s, dev, ps, q, nx, in_q ^ 1, pm, crec, cshrec, sum);
             else if (accel.width == 8)
-                hipLaunchKernelGGL(k_connect<8>, dim3(tg), dim3(kBlock), 0, s, dev, ps, q, nx, pm, crec, cshrec, sum);
-            else hipLaunchKernelGGL(k_connect<2>, dim3(tg), dim3(kBlock), 0, s, dev, ps, q, nx, pm, crec, cshrec, sum);
+                hipLaunchKernelGGL(k_connect<8>, dim3(tg), dim3(kBlock), 0, s, dev, ps, q, nx, in_q ^ 1, pm, crec, cshrec, sum);
+            else hipLaunchKernelGGL(k_connect<2>, dim3(tg), dim3(kBlock), 0, s, dev, ps, q, nx, in_q ^ 1, pm, crec, cshrec, sum);
         }
     }
     hipLaunchKernelGGL(k_accumulate, dim3(gb), dim3(kBlock), 0, s, dev, ps, q, c, sum, sumsq);

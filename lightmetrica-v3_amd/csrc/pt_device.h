@@ -65,8 +65,14 @@ struct Queues {
     int32_t* ext_path[2];
     lmgpu_ray* sh;
     float4* sh_contrib;   // xyz contribution, w = path index bits
-    int32_t* counts;      // [0],[1] extension queues, [2] shadow queue, [3] sample index, [4..] stats
+    int32_t* counts;      // see ext_count, shadow_count; [4] sample index, [5] stack overflow flag, [8..] stats
 };
+
+// Indices of the queue counts: extension queue k and the shadow queue filled
+// by the vertices that filled it, side by side so that one 64-bit atomic
+// reserves entries of both (block_append2).
+LMGPU_HD int ext_count(int k) { return 2 * k; }
+LMGPU_HD int shadow_count(int k) { return 2 * k + 1; }
 
 struct PTConsts {
     int max_verts;
@@ -153,12 +159,15 @@ __device__ __forceinline__ int wave_append(int32_t* counter, bool want) {
     return want ? base + __popcll(lower) : -1;
 }
 
-// Appends to two queues for the whole block: one atomic per block and queue
-// on the queue counts (which every block of the launch shares) instead of
-// one per wave. i0 / i1 are the entries of the lanes whose flag is set.
-// Every thread of the block calls it, the same number of times.
+// Appends to an extension queue and its shadow queue for the whole block with
+// one 64-bit atomic on their pair of counts. Every block of the launch updates
+// that one address and an update takes 12 ns, so a wave's or a block's own
+// two atomics bounded the shading kernels (16.8M vertices in blocks of 128:
+// 3.0 ms, at a quarter of the vector rate). i0 / i1 are the entries of the
+// lanes whose flag is set. Every thread of the block calls it, the same number
+// of times.
 template <int BLOCK>
-__device__ __forceinline__ void block_append2(int32_t* c0, int32_t* c1, bool f0, bool f1, int& i0, int& i1) {
+__device__ __forceinline__ void block_append2(int32_t* pair, bool f0, bool f1, int& i0, int& i1) {
     constexpr int kW = BLOCK / 64;
     __shared__ int cnt[2][kW];
     __shared__ int base[2];
@@ -170,16 +179,18 @@ __device__ __forceinline__ void block_append2(int32_t* c0, int32_t* c1, bool f0,
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-        int a = 0, b = 0;
+        uint32_t a = 0, b = 0;
         for (int w = 0; w < kW; w++) {
-            const int x = cnt[0][w], y = cnt[1][w];
+            const uint32_t x = cnt[0][w], y = cnt[1][w];
             cnt[0][w] = a;
             cnt[1][w] = b;
             a += x;
             b += y;
         }
-        base[0] = a ? atomicAdd(c0, a) : 0;
-        base[1] = b ? atomicAdd(c1, b) : 0;
+        const unsigned long long both = (unsigned long long)b << 32 | a;
+        const unsigned long long at = both ? atomicAdd(reinterpret_cast<unsigned long long*>(pair), both) : 0ull;
+        base[0] = int(uint32_t(at));
+        base[1] = int(uint32_t(at >> 32));
     }
     __syncthreads();
     const unsigned long long lt = (1ull << lane) - 1ull;
@@ -525,7 +536,7 @@ template <int W>
 __global__ __launch_bounds__(kBlock, 6) void k_extend(SceneDev sc, Queues q, int in_q, unsigned long long* next, int refill,
                                                   int chunk_rays) {
     __shared__ int lds[kLds + 1][kBlock];
-    const int n = q.counts[in_q];
+    const int n = q.counts[ext_count(in_q)];
     if (n == 0) return;   // an empty queue (whole grid)
     const lmgpu_ray* rays = q.ext[in_q];
     auto fetch = [&](uint32_t id, f3& o, f3& d, float& tmin, float& tmax) -> int {
@@ -573,7 +584,7 @@ __global__ __launch_bounds__(256) void k_pt_guide_infer(SceneDev sc, Q q, int in
     uint16_t* lx = reinterpret_cast<uint16_t*>(lds + kWeightLds + wave * kWaveLds);
     uint16_t* lh = lx + 32 * kPitchX;
     float* ly = reinterpret_cast<float*>(lx);
-    const int n = q.counts[in_q];
+    const int n = q.counts[ext_count(in_q)];
     // two lanes per row: lanes r and r + 32 share row r of the wave's 32-row
     // tile and each encode and decode half of it
     const int r = lane & 31, half = lane >> 5;
