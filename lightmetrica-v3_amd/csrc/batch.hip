@@ -12,8 +12,8 @@
 //     its last sample records the device clock (job latency);
 //   * an iteration is regenerate -> extend (persistent closest hit) -> shade
 //     (shade_vertex, the transport of renderer::pt) -> connect (persistent
-//     any hit); two iterations (both queue parities) are captured once as a
-//     hipGraph and replayed until every work item has been accumulated.
+//     any hit); pairs of iterations (both queue parities) are enqueued one
+//     ahead of the device until every work item has been accumulated.
 // A job renders exactly what lmgpu_pt_render renders for the same scene,
 // seed and BVH: same Philox streams, same per-vertex code.
 //
@@ -552,10 +552,6 @@ __global__ void k_b_fill_f64(double* p, int64_t n) {
 inline unsigned nblk(int64_t n, int b) { return unsigned((n + b - 1) / b); }
 
 
-// Graph replays (two iterations each) the host enqueues between looks at the
-// device's progress.
-constexpr int64_t kChunkReplays = 16;
-
 template <class K>
 int occupancy_grid(K kernel, int block) {
     int dev = 0, cus = 0, occ = 0;
@@ -759,9 +755,8 @@ int Wavefront::set_work(const std::vector<JobDev>& jobs, const std::vector<WorkS
         LMGPU_TRY(job_done.alloc(nj));
         LMGPU_TRY(job_time.alloc(nj));
     }
-    LMGPU_HIP(hipStreamSynchronize(s));
-    LMGPU_HIP(hipMemcpy(djobs.p, jobs.data(), sizeof(JobDev) * nj, hipMemcpyHostToDevice));
-    LMGPU_HIP(hipMemcpy(dsegs.p, segs.data(), sizeof(WorkSeg) * segs.size(), hipMemcpyHostToDevice));
+    LMGPU_HIP(hipMemcpyAsync(djobs.p, jobs.data(), sizeof(JobDev) * nj, hipMemcpyHostToDevice, s));
+    LMGPU_HIP(hipMemcpyAsync(dsegs.p, segs.data(), sizeof(WorkSeg) * segs.size(), hipMemcpyHostToDevice, s));
     hipLaunchKernelGGL(k_b_fill_u64, dim3(nblk(nj, 256)), dim3(256), 0, s, job_done.p, int64_t(nj));
     hipLaunchKernelGGL(k_b_fill_u64, dim3(nblk(nj, 256)), dim3(256), 0, s, job_time.p, int64_t(nj));
     LMGPU_HIP(hipGetLastError());
@@ -803,6 +798,7 @@ int Wavefront::run(const void* trav_nodes, const TriV* tris, int width, int bloc
         hipLaunchKernelGGL(k_b_fill_i32, dim3(1), dim3(64), 0, s, gcnt.p, int64_t(3), 0);
         hipLaunchKernelGGL(k_b_fill_u64, dim3(1), dim3(64), 0, s, grecorded.p, int64_t(1));
     }
+    int extend_grid = 0, connect_grid = 0;   // resident grids, looked up once per run
     auto iteration = [&](hipStream_t cs, int in_q) {
         if (train) {
             // online training: the records of the paths that finished in the
@@ -821,16 +817,18 @@ int Wavefront::run(const void* trav_nodes, const TriV* tris, int width, int bloc
                                cap, ctl.p, next.p, job_done.p, job_time.p, film_sum, fsq);
         };
         auto extend = [&](auto kernel, auto* nd) {
-            hipLaunchKernelGGL(kernel, dim3(occupancy_grid(kernel, kBlock)), dim3(kBlock), 0, cs, nd, tris, djobs.p, P, q,
-                               in_q, next.p, refill, ctl.p);
+            if (!extend_grid) extend_grid = occupancy_grid(kernel, kBlock);
+            hipLaunchKernelGGL(kernel, dim3(extend_grid), dim3(kBlock), 0, cs, nd, tris, djobs.p, P, q, in_q, next.p, refill,
+                               ctl.p);
         };
         const unsigned sg = unsigned(std::max<int64_t>(1, std::min<int64_t>(nblk(cap, block), 2048 * 256 / block)));
         auto shade = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, dim3(sg), dim3(unsigned(block)), 0, cs, djobs.p, P, q, in_q, gd, cap);
         };
         auto connect = [&](auto kernel, auto* nd) {
-            hipLaunchKernelGGL(kernel, dim3(occupancy_grid(kernel, kBlock)), dim3(kBlock), 0, cs, nd, tris, djobs.p, P, q,
-                               in_q ^ 1, next.p + 1, refill, ctl.p, gd.rec, gd.sh_rec);
+            if (!connect_grid) connect_grid = occupancy_grid(kernel, kBlock);
+            hipLaunchKernelGGL(kernel, dim3(connect_grid), dim3(kBlock), 0, cs, nd, tris, djobs.p, P, q, in_q ^ 1, next.p + 1,
+                               refill, ctl.p, gd.rec, gd.sh_rec);
         };
         auto iterate = [&](auto w) {
             constexpr int W = decltype(w)::value;
@@ -855,103 +853,104 @@ int Wavefront::run(const void* trav_nodes, const TriV* tris, int width, int bloc
         else if (width == 4) iterate(std::integral_constant<int, 4>{});
         else iterate(std::integral_constant<int, 8>{});
     };
-    return loop(iteration, total, max_verts, elapsed, iters, s);
+    return loop(iteration, total, max_verts, train, elapsed, iters, s);
 }
 
-int Wavefront::loop(const std::function<void(hipStream_t, int)>& iteration, int64_t total, int max_verts,
+int Wavefront::loop(const std::function<void(hipStream_t, int)>& iteration, int64_t total, int max_verts, bool graph,
                     double* elapsed, int64_t* iters, hipStream_t s) {
     hipLaunchKernelGGL(k_b_fill_i32, dim3(nblk(cap, 256)), dim3(256), 0, s, pstate.p, int64_t(cap), kFree);
     hipLaunchKernelGGL(k_b_init, dim3(1), dim3(64), 0, s, ctl.p, total, counts.p);
-    // two iterations (queue parities 0 and 1) captured as one graph
-    hipStream_t cs;
-    LMGPU_HIP(hipStreamCreateWithFlags(&cs, hipStreamNonBlocking));
-    hipGraph_t g;
-    LMGPU_HIP(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
-    iteration(cs, 0);
-    iteration(cs, 1);
-    hipError_t e = hipStreamEndCapture(cs, &g);
-    if (e != hipSuccess) {
+    // A pair of iterations (queue parities 0 and 1) is launched as it is, or,
+    // when an iteration has many short kernels (guide training), from a
+    // hipGraph: capturing and instantiating one takes the host 200 us, which
+    // four to five launches an iteration do not need.
+    hipError_t e;
+    hipGraphExec_t ge = nullptr;
+    if (graph) {
+        hipStream_t cs;
+        LMGPU_HIP(hipStreamCreateWithFlags(&cs, hipStreamNonBlocking));
+        hipGraph_t g;
+        LMGPU_HIP(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
+        iteration(cs, 0);
+        iteration(cs, 1);
+        e = hipStreamEndCapture(cs, &g);
+        if (e != hipSuccess) {
+            (void)hipStreamDestroy(cs);
+            return fail(LMGPU_ERR_DEVICE, std::string("batch graph capture: ") + hipGetErrorString(e));
+        }
+        e = hipGraphInstantiate(&ge, g, nullptr, nullptr, 0);
+        (void)hipGraphDestroy(g);
         (void)hipStreamDestroy(cs);
-        return fail(LMGPU_ERR_DEVICE, std::string("batch graph capture: ") + hipGetErrorString(e));
+        if (e != hipSuccess)
+            return fail(LMGPU_ERR_DEVICE, std::string("batch graph instantiate: ") + hipGetErrorString(e));
     }
-    hipGraphExec_t ge;
-    e = hipGraphInstantiate(&ge, g, nullptr, nullptr, 0);
-    (void)hipGraphDestroy(g);
-    (void)hipStreamDestroy(cs);
-    if (e != hipSuccess) return fail(LMGPU_ERR_DEVICE, std::string("batch graph instantiate: ") + hipGetErrorString(e));
     // every work item needs at most max_verts + 1 iterations in its slot
     const int max_v = std::max(2, max_verts);
     const int64_t iter_cap = (total / cap + 2) * (max_v + 2) + 64;
-    hipEvent_t e0, e1;
-    LMGPU_HIP(hipEventCreate(&e0));
-    LMGPU_HIP(hipEventCreate(&e1));
-    LMGPU_HIP(hipEventRecord(e0, s));
+    int rc = ensure_host();
+    if (rc == LMGPU_OK && (e = hipEventRecord(ev[0], s)) != hipSuccess)
+        rc = fail(LMGPU_ERR_DEVICE, std::string("batch start: ") + hipGetErrorString(e));
     hipLaunchKernelGGL(k_b_clock, dim3(1), dim3(64), 0, s, ctl.p);
-    // The host never stalls the device: replays go out in chunks and the host
-    // stays one chunk ahead. After each chunk the stream copies the control
-    // block into pinned memory and records an event; before deciding on the
-    // next chunk the host blocks on the event of the chunk before (no
-    // stream synchronization, no spinning) and stops once that copy shows no
-    // work left. Replays already queued when the work runs out find the
-    // remaining-work counter at 0 and return at entry (k_b_regen). The
-    // iteration bound turns a stall into an error.
-    int rc = LMGPU_OK;
-    if (!ctl_mirror) {
-        LMGPU_HIP(hipHostMalloc(reinterpret_cast<void**>(&ctl_mirror), 2 * sizeof(BatchCtl), hipHostMallocDefault));
-    }
-    hipEvent_t chunk_ev[2];
-    LMGPU_HIP(hipEventCreateWithFlags(&chunk_ev[0], hipEventBlockingSync | hipEventDisableTiming));
-    LMGPU_HIP(hipEventCreateWithFlags(&chunk_ev[1], hipEventBlockingSync | hipEventDisableTiming));
-    const int64_t max_replays = (iter_cap + 1) / 2;
-    int64_t enqueued = 0;
-    for (int64_t k = 0; enqueued < max_replays; k++) {
-        const int64_t nrep = std::min<int64_t>(kChunkReplays, max_replays - enqueued);
-        for (int64_t r = 0; r < nrep && rc == LMGPU_OK; r++)
-            if ((e = hipGraphLaunch(ge, s)) != hipSuccess)
-                rc = fail(LMGPU_ERR_DEVICE, std::string("batch graph launch: ") + hipGetErrorString(e));
-        if (rc != LMGPU_OK) break;
-        enqueued += nrep;
-        if ((e = hipMemcpyAsync(ctl_mirror + (k & 1), ctl.p, sizeof(BatchCtl), hipMemcpyDeviceToHost, s)) !=
-                hipSuccess ||
-            (e = hipEventRecord(chunk_ev[k & 1], s)) != hipSuccess) {
-            rc = fail(LMGPU_ERR_DEVICE, std::string("batch progress copy: ") + hipGetErrorString(e));
-            break;
+    // The host never stalls the device: pairs go out one ahead of it. After
+    // each pair the stream copies the control block and the queue counts into
+    // pinned memory and records an event; before deciding on the next pair the
+    // host blocks on the event of the pair before (no stream synchronization,
+    // no spinning) and stops once that copy shows no work left. A pair queued
+    // when the work runs out finds the remaining-work counter at 0 and returns
+    // at entry (k_b_regen), 5 us a kernel: pairs of 16 looked at less often cost
+    // a small render up to 0.7 ms. The iteration bound turns a stall into an error.
+    const int64_t max_pairs = (iter_cap + 1) / 2;
+    int64_t k = 0;
+    for (; rc == LMGPU_OK && k < max_pairs; k++) {
+        if (graph) {
+            e = hipGraphLaunch(ge, s);
+        } else {
+            iteration(s, 0);
+            iteration(s, 1);
+            e = hipGetLastError();
         }
-        if (k >= 1) {
-            if ((e = hipEventSynchronize(chunk_ev[(k - 1) & 1])) != hipSuccess) {
-                rc = fail(LMGPU_ERR_DEVICE, std::string("batch progress: ") + hipGetErrorString(e));
-                break;
-            }
-            if (ctl_mirror[(k - 1) & 1].remaining == 0) break;
+        HostMirror* m = mirror + (k & 1);
+        if (e == hipSuccess) e = hipMemcpyAsync(&m->ctl, ctl.p, sizeof(BatchCtl), hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess) e = hipMemcpyAsync(m->counts, counts.p, sizeof(m->counts), hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess) e = hipEventRecord(pair_ev[k & 1], s);
+        if (e == hipSuccess && k >= 1) {
+            e = hipEventSynchronize(pair_ev[(k - 1) & 1]);
+            if (e == hipSuccess && mirror[(k - 1) & 1].ctl.remaining == 0) break;
         }
+        if (e != hipSuccess) rc = fail(LMGPU_ERR_DEVICE, std::string("batch loop: ") + hipGetErrorString(e));
     }
-    BatchCtl hc{};
-    if (rc == LMGPU_OK) {
-        if ((e = hipMemcpyAsync(&hc, ctl.p, sizeof(hc), hipMemcpyDeviceToHost, s)) != hipSuccess ||
-            (e = hipStreamSynchronize(s)) != hipSuccess)
-            rc = fail(LMGPU_ERR_DEVICE, std::string("batch run: ") + hipGetErrorString(e));
-        else if (hc.remaining != 0)
-            rc = fail(LMGPU_ERR_FAILED_TO_RENDER, "batch did not finish within its iteration bound");
-    } else {
-        (void)hipStreamSynchronize(s);
-    }
-    (void)hipEventDestroy(chunk_ev[0]);
-    (void)hipEventDestroy(chunk_ev[1]);
-    const int64_t it = int64_t(hc.iterations);
-    (void)hipEventRecord(e1, s);
-    (void)hipEventSynchronize(e1);
+    // the end of the last pair: all counters are final in its copy
     float ms = 0.f;
-    (void)hipEventElapsedTime(&ms, e0, e1);
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
-    (void)hipGraphExecDestroy(ge);
+    if (rc == LMGPU_OK && ((e = hipEventRecord(ev[1], s)) != hipSuccess || (e = hipStreamSynchronize(s)) != hipSuccess))
+        rc = fail(LMGPU_ERR_DEVICE, std::string("batch run: ") + hipGetErrorString(e));
+    else if (rc != LMGPU_OK) (void)hipStreamSynchronize(s);
+    if (ge) (void)hipGraphExecDestroy(ge);
     if (rc != LMGPU_OK) return rc;
-    int32_t cnt[16];
-    LMGPU_HIP(hipMemcpy(cnt, counts.p, sizeof(cnt), hipMemcpyDeviceToHost));
-    if (cnt[5]) return fail(LMGPU_ERR_STACK_OVERFLOW, "BVH traversal stack capacity exceeded during rendering");
+    (void)hipEventElapsedTime(&ms, ev[0], ev[1]);
+    last = mirror[(std::min(k, max_pairs - 1)) & 1];
+    if (last.ctl.remaining != 0) return fail(LMGPU_ERR_FAILED_TO_RENDER, "batch did not finish within its iteration bound");
+    if (last.counts[5]) return fail(LMGPU_ERR_STACK_OVERFLOW, "BVH traversal stack capacity exceeded during rendering");
     *elapsed = ms * 1e-3;
-    *iters = it;
+    *iters = int64_t(last.ctl.iterations);
     return LMGPU_OK;
+}
+
+int Wavefront::ensure_host() {
+    if (mirror) return LMGPU_OK;
+    for (hipEvent_t& x : ev)
+        if (!x) LMGPU_HIP(hipEventCreate(&x));
+    for (hipEvent_t& x : pair_ev)
+        if (!x) LMGPU_HIP(hipEventCreateWithFlags(&x, hipEventBlockingSync | hipEventDisableTiming));
+    LMGPU_HIP(hipHostMalloc(reinterpret_cast<void**>(&mirror), 2 * sizeof(HostMirror), hipHostMallocDefault));
+    return LMGPU_OK;
+}
+
+Wavefront::~Wavefront() {
+    if (mirror) (void)hipHostFree(mirror);
+    for (hipEvent_t x : ev)
+        if (x) (void)hipEventDestroy(x);
+    for (hipEvent_t x : pair_ev)
+        if (x) (void)hipEventDestroy(x);
 }
 
 // Renders every job once with the current arena and pool: at most spp_cap
@@ -1007,9 +1006,8 @@ int Batch::run_once(int width, int block, int spp_cap, bool keep_results, bool w
     if (keep_results) {
         // job latency = device clock at the job's last sample - clock at the start
         std::vector<unsigned long long> t(nj);
-        BatchCtl hc;
+        const BatchCtl& hc = wf.last.ctl;
         LMGPU_HIP(hipMemcpy(t.data(), wf.job_time.p, sizeof(unsigned long long) * nj, hipMemcpyDeviceToHost));
-        LMGPU_HIP(hipMemcpy(&hc, wf.ctl.p, sizeof(hc), hipMemcpyDeviceToHost));
         int dev = 0, khz = 0;
         LMGPU_HIP(hipGetDevice(&dev));
         LMGPU_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev));
@@ -1068,17 +1066,16 @@ int Scene::render_regen(const PTConsts& c, int spp, int sample_offset, double* s
         if (G.steps > 0) LMGPU_TRY(gp->g->ensure_train(G.batch));
         LMGPU_TRY(wf->ensure_guided(G.rec_depth, int64_t(G.batch) * G.steps));
     }
-    LMGPU_TRY(wf->set_work(std::vector<JobDev>{J}, segs, s));
+    const std::vector<JobDev> jobs{J};
+    LMGPU_TRY(wf->set_work(jobs, segs, s));
     const void* tn = accel.width == 4 ? static_cast<const void*>(dev.nodes4)
                      : accel.width == 8 ? static_cast<const void*>(dev.nodes8) : static_cast<const void*>(dev.nodes2);
     double sec = 0;
     int64_t iters = 0;
     LMGPU_TRY(wf->run(tn, accel.tris.p, accel.width, kSingleBlock, true, total, c.max_verts, sum, sumsq, &sec, &iters, s,
                       gp ? &G : nullptr));
-    BatchCtl hc;
-    LMGPU_HIP(hipMemcpy(&hc, wf->ctl.p, sizeof(hc), hipMemcpyDeviceToHost));
-    *ext_rays = int64_t(hc.ext_rays);
-    *shadow_rays = int64_t(hc.shadow_rays);
+    *ext_rays = int64_t(wf->last.ctl.ext_rays);
+    *shadow_rays = int64_t(wf->last.ctl.shadow_rays);
     if (guide_records) {
         unsigned long long r = 0;
         if (gp) LMGPU_HIP(hipMemcpy(&r, wf->grecorded.p, sizeof(r), hipMemcpyDeviceToHost));
@@ -1250,8 +1247,7 @@ int lmgpu_batch_run(lmgpu_batch* bh, const lmgpu_batch_opts* opts, lmgpu_batch_s
     LMGPU_TRY(b.run_once(width, block, 0, true, o.film_sumsq != 0, o.queue_order, &sec, &iters, s));
     if (stats) {
         std::memset(stats, 0, sizeof(*stats));
-        lmgpu::BatchCtl hc;
-        LMGPU_HIP(hipMemcpy(&hc, b.wf.ctl.p, sizeof(hc), hipMemcpyDeviceToHost));
+        const lmgpu::BatchCtl& hc = b.wf.last.ctl;
         int64_t samples = 0;
         for (const auto& J : b.jobs) samples += int64_t(J.desc.w) * J.desc.h * J.spp;
         stats->jobs = int64_t(b.jobs.size());

@@ -1023,11 +1023,9 @@ int Scene::lt_render(const lmgpu_lt_params* p, double* film_in, bool on_device, 
         };
         double sec = 0;
         int64_t iters = 0;
-        LMGPU_TRY(wf->loop(iteration, total, p->max_verts, &sec, &iters, s));
-        int32_t cnt[16];
-        LMGPU_HIP(hipMemcpy(cnt, wf->counts.p, sizeof(cnt), hipMemcpyDeviceToHost));
+        LMGPU_TRY(wf->loop(iteration, total, p->max_verts, false, &sec, &iters, s));
         int64_t v[3];
-        std::memcpy(v, cnt + 8, sizeof(v));
+        std::memcpy(v, wf->last.counts + 8, sizeof(v));
         ext += v[1];
         shd += v[2];
         return LMGPU_OK;

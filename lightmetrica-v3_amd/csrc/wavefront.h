@@ -2,8 +2,7 @@
 // renderers (batch.hip: the batch and fixed-spp path tracing; lt.hip:
 // light tracing): a fixed pool of path slots whose free slots take the next
 // work items, an iteration of regenerate -> extend -> shade -> connect
-// kernels, two iterations captured as one hipGraph and replayed until every
-// item is done.
+// kernels, enqueued in pairs until every item is done.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -136,7 +135,15 @@ struct Wavefront {
     DevBuf<lmgpu_hit> hit;
     DevBuf<float4> shc;
     DevBuf<BatchCtl> ctl;
-    BatchCtl* ctl_mirror = nullptr;   // pinned host copies of ctl, one per chunk parity
+    // pinned host copies of the control block and the queue counts, one per
+    // parity of the pairs of iterations, with the pairs' events
+    struct HostMirror {
+        BatchCtl ctl;
+        int32_t counts[16];
+    };
+    HostMirror* mirror = nullptr;
+    HostMirror last{};                // the copy that ended the last run
+    hipEvent_t pair_ev[2] = {nullptr, nullptr}, ev[2] = {nullptr, nullptr};
     DevBuf<unsigned long long> next;
     // per-run tables: jobs, work segments, per-job completion counters and clocks
     DevBuf<JobDev> djobs;
@@ -151,13 +158,16 @@ struct Wavefront {
     DevBuf<float> gmix, gtrain;
     DevBuf<int32_t> gshrec, gcnt;
     DevBuf<unsigned long long> grecorded;
-    ~Wavefront() {
-        if (ctl_mirror) (void)hipHostFree(ctl_mirror);
-    }
+    Wavefront() = default;
+    Wavefront(const Wavefront&) = delete;
+    Wavefront& operator=(const Wavefront&) = delete;
+    ~Wavefront();
+    int ensure_host();
     int ensure_pool(int cap);
     // Guided buffers for the current pool (records zeroed when allocated).
     int ensure_guided(int rec_depth, int64_t train_cap);
-    // Uploads the jobs and the work segments (queue order) of one run.
+    // Uploads the jobs and the work segments (queue order) of one run, on s; the
+    // vectors live until the run has ended.
     int set_work(const std::vector<JobDev>& jobs, const std::vector<WorkSeg>& segs, hipStream_t s);
     // Renders every work item of the tables set last into film_sum / film_sq
     // (FP64 atomics; film_sq may be null) and waits for the end.
@@ -170,11 +180,12 @@ struct Wavefront {
             double* film_sum, double* film_sq, double* elapsed, int64_t* iters, hipStream_t s,
             const RegenGuide* guide = nullptr);
     // The loop itself: frees the pool, sets the run's counters for `total`
-    // items, captures iteration(stream, 0) and iteration(stream, 1) (the
-    // kernels of one iteration on queue parity 0 / 1) as one graph and
-    // replays it until every item is done; max_verts bounds the iterations.
-    int loop(const std::function<void(hipStream_t, int)>& iteration, int64_t total, int max_verts, double* elapsed,
-             int64_t* iters, hipStream_t s);
+    // items and enqueues pairs of iteration(stream, 0) and iteration(stream, 1)
+    // (the kernels of one iteration on queue parity 0 / 1), captured as one
+    // graph if `graph`, until every item is done; max_verts bounds the
+    // iterations. `last` holds the final counters.
+    int loop(const std::function<void(hipStream_t, int)>& iteration, int64_t total, int max_verts, bool graph,
+             double* elapsed, int64_t* iters, hipStream_t s);
     // Slot count for `total` items over `npix` pixels: per_pixel slots per
     // pixel, a power of two in [4096, max_slots].
     static int pool_size(int64_t total, int npix, int per_pixel = LMGPU_REGEN_SLOTS_PER_PIXEL,
