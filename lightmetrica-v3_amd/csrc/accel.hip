@@ -31,12 +31,6 @@
 #include "bvh.h"
 #include "lmgpu_internal.h"
 
-// Rays a wave of the ray-cast kernel takes per atomic on the ray counter
-// (128: coherent config-1 rays +10% over 64, incoherent level).
-#ifndef LMGPU_TRACE_RAY_CHUNK
-#define LMGPU_TRACE_RAY_CHUNK 128
-#endif
-
 namespace lmgpu {
 
 // Build defaults: leaves of at most 2 triangles, and a triangle test costing
@@ -580,7 +574,7 @@ __global__ __launch_bounds__(kTraceBlock, 6) void k_trace(const Node* __restrict
         }
     };
     trace_persistent<W, ANY, COUNT, kLdsDepth, kPrivDepth, kTraceBlock>(nodes, tris, n, next, lds, fetch, emit,
-                                                                         status, counters, refill, LMGPU_TRACE_RAY_CHUNK);
+                                                                         status, counters, refill);
 }
 
 // Quantised copy of a built W-wide node array (bvh.h, quantise_node).
@@ -596,7 +590,7 @@ __global__ void k_zero_i32_1(int32_t* c) {
 }
 
 __global__ void k_zero_counter(unsigned long long* c) {
-    if (threadIdx.x == 0) *c = 0ull;
+    if (threadIdx.x < kRayCounters) c[threadIdx.x * kRayCounterStride] = 0ull;
 }
 
 // ---------------------------------------------------------------------------
@@ -876,9 +870,12 @@ static void launch_trace(const Accel& a, const lmgpu_ray* rays, lmgpu_hit* hits,
     // one launch for all but batches of over 2^30 rays (ray ids are 32 bits on the device)
     for (int64_t at = 0; at < n; at += kMaxLaunchRays) {
         const int64_t m = std::min(n - at, kMaxLaunchRays);
-        hipLaunchKernelGGL(k_zero_counter, dim3(1), dim3(64), 0, s, next);
         // a block per 64 rays: few rays spread over the CUs one wave each
         const int grid = int(std::min<int64_t>(persistent_grid<W, ANY, COUNT, Node>(), (m + 63) / 64));
+        // few rays are all in the waves' own shares: no counter is read
+        const uint32_t nwaves = uint32_t(grid) * (kTraceBlock / 64);
+        if (int64_t(nwaves) * ray_share(uint32_t(m), nwaves) < m)
+            hipLaunchKernelGGL(k_zero_counter, dim3(1), dim3(64), 0, s, next);
         hipLaunchKernelGGL((k_trace<W, ANY, COUNT, Node>), dim3(grid), dim3(kTraceBlock), 0, s,
                            static_cast<const Node*>(a.trav_nodes()), a.tris.p, rays + at, hits ? hits + at : nullptr,
                            occl ? occl + at : nullptr, uint32_t(m), next, status, counters, a.refill);

@@ -83,17 +83,18 @@ __global__ __launch_bounds__(BLOCK) void k_b_regen(const JobDev* __restrict__ jo
     __shared__ int s_idle;
     // Every item accumulated: no slot is finishing and nothing is left to
     // hand out, so this and the rest of the iteration's kernels are no-ops
-    // (the host enqueues iterations up to a bound without watching). One
+    // (the host enqueues iterations ahead of the device). One
     // thread reads the counter, so the whole block takes the same branch
-    // (other blocks of this launch may lower it meanwhile).
+    // (other blocks of this launch may lower it meanwhile). It and work_next
+    // are read through the cache, as the kernels before left them: an atomic
+    // load of a line that other blocks update waits its turn like an update.
+    if (blockIdx.x == 0 && threadIdx.x < 2 * kRayCounters) next[threadIdx.x * kRayCounterStride] = 0ull;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
-        next[0] = 0ull;
-        next[1] = 0ull;
         q.counts[ext_count(in_q ^ 1)] = 0;
         q.counts[shadow_count(in_q ^ 1)] = 0;
     }
     if (threadIdx.x == 0)
-        s_idle = __hip_atomic_load(&ctl->remaining, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0;
+        s_idle = ctl->remaining == 0;
     __syncthreads();
     if (s_idle) return;
     if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&ctl->iterations, 1ull);
@@ -130,8 +131,8 @@ __global__ __launch_bounds__(BLOCK) void k_b_regen(const JobDev* __restrict__ jo
         unsigned long long base = 0;
         int emit = 0, qb = 0;
         if (acc > 0) {
-            // no atomic (12 ns each, on one address) once the queue is empty
-            base = __hip_atomic_load(&ctl->work_next, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            // no atomic once the queue was empty before this launch
+            base = ctl->work_next;
             if (base < (unsigned long long)total) base = atomicAdd(&ctl->work_next, (unsigned long long)acc);
             if (base < (unsigned long long)total)
                 emit = int(min((unsigned long long)acc, (unsigned long long)total - base));
@@ -262,7 +263,7 @@ __global__ __launch_bounds__(kBlock, 6) void k_b_extend(const typename TravNode<
         reinterpret_cast<float4*>(q.hit)[id] = make_float4(__int_as_float(r.overflow ? -2 : r.prim), r.t, r.u, r.v);
     };
     trace_persistent<W, false, false, kLds, kPriv, kBlock>(nodes, tris, n, next, lds, fetch, emit, q.counts + 5,
-                                                           nullptr, refill, LMGPU_REGEN_RAY_CHUNK);
+                                                           nullptr, refill);
     if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&ctl->ext_rays, (unsigned long long)n);
 }
 
@@ -501,7 +502,7 @@ __global__ __launch_bounds__(kBlock, 6) void k_b_connect(const typename TravNode
         }
     };
     trace_persistent<W, true, false, kLds, kPriv, kBlock>(nodes, tris, n, next, lds, fetch, emit, q.counts + 5, nullptr,
-                                                          refill, LMGPU_REGEN_RAY_CHUNK);
+                                                          refill);
     if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&ctl->shadow_rays, (unsigned long long)n);
 }
 
@@ -742,7 +743,7 @@ int Wavefront::ensure_pool(int c) {
     LMGPU_TRY(hit.alloc(c)); LMGPU_TRY(shc.alloc(c));
     if (!counts.p) LMGPU_TRY(counts.alloc(16));
     if (!ctl.p) LMGPU_TRY(ctl.alloc(1));
-    if (!next.p) LMGPU_TRY(next.alloc(2));
+    if (!next.p) LMGPU_TRY(next.alloc(2 * kRayCounterWords));
     cap = c;
     return LMGPU_OK;
 }
@@ -827,7 +828,7 @@ int Wavefront::run(const void* trav_nodes, const TriV* tris, int width, int bloc
         };
         auto connect = [&](auto kernel, auto* nd) {
             if (!connect_grid) connect_grid = occupancy_grid(kernel, kBlock);
-            hipLaunchKernelGGL(kernel, dim3(connect_grid), dim3(kBlock), 0, cs, nd, tris, djobs.p, P, q, in_q ^ 1, next.p + 1,
+            hipLaunchKernelGGL(kernel, dim3(connect_grid), dim3(kBlock), 0, cs, nd, tris, djobs.p, P, q, in_q ^ 1, next.p + kRayCounterWords,
                                refill, ctl.p, gd.rec, gd.sh_rec);
         };
         auto iterate = [&](auto w) {

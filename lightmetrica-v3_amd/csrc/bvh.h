@@ -36,9 +36,10 @@
 #define LMGPU_QNODE 1
 #endif
 
-// Rays a wave takes from the global ray counter with one atomic (at least
-// 64, so one chunk always covers the idle lanes of a refill); the wave hands
-// them to its idle lanes over several refills.
+// Rays a wave takes from a ray counter with one atomic (at least 64, so one
+// chunk always covers the idle lanes of a refill); the wave hands them to its
+// idle lanes over several refills. 64, 128, 256: 463, 481, 553 us for 2.07M
+// primary rays, 44.0, 44.3, 44.8 ms for a 1080p path-traced frame.
 #ifndef LMGPU_RAY_CHUNK
 #define LMGPU_RAY_CHUNK 64
 #endif
@@ -439,14 +440,27 @@ constexpr int32_t kDone = INT32_MAX;
 constexpr uint32_t kNoRay = UINT32_MAX;
 // Most rays of one launch of the persistent traversal.
 constexpr int64_t kMaxLaunchRays = int64_t(1) << 30;
+// Ray counters of one launch, in cache lines of their own; zeroed before it.
+constexpr uint32_t kRayCounters = 8;
+constexpr uint32_t kRayCounterStride = 16;   // in 64-bit words
+constexpr uint32_t kRayCounterWords = kRayCounters * kRayCounterStride;
+// Rays a wave starts with: its whole part of an even split in whole waves of
+// rays when that is at most 256 rays (room at 256x256, 85 rays a wave: 2.03 ms
+// with half of it, 1.48 with all; 2M rays of uneven cost, 325 a wave: 889 us
+// with half, 1030 with all), else half of it, at most 256 rays (2730 a wave at
+// 1080p: half 45.9 ms a frame, 256 rays 44.0); the ray counters hand out the rest.
+__device__ __host__ inline uint32_t ray_share(uint32_t n, uint32_t nwaves) {
+    const uint32_t per = (n + nwaves - 1) / nwaves;
+    return per <= 256u ? (per + 63u) & ~63u : (per < 512u ? per / 2u : 256u) & ~63u;
+}
 
 // Persistent traversal: every lane owns one ray at a time; when at least
 // `refill` lanes of a wave have finished (or the whole wave has), the
 // finished lanes hand over their results together and take new rays from the
-// wave's pool: a share of its own, then chunks of chunk_rays (default
-// LMGPU_RAY_CHUNK) from one global counter with one atomic (Aila & Laine,
-// HPG 2009, "persistent threads"), so lanes do not sit idle behind a wave's
-// slowest ray and the counter sees few atomics. refill = 64 keeps whole
+// wave's pool: a share of its own, then chunks of LMGPU_RAY_CHUNK from the ray
+// counters with one atomic (Aila & Laine, HPG 2009, "persistent threads"), so
+// lanes do not sit idle behind a wave's slowest ray and the counters see few
+// atomics. refill = 64 keeps whole
 // waves of consecutive rays together (best for coherent rays), smaller
 // values keep lanes busy.
 // Each loop iteration advances the lanes of one kind of step: a wide node or
@@ -476,8 +490,8 @@ template <int W, bool ANY, bool COUNT, int LDS_DEPTH, int PRIV_DEPTH, int BLOCK,
 __device__ __forceinline__ void trace_persistent(const Node* __restrict__ nodes, const TriV* __restrict__ tris,
                                                  uint32_t n, unsigned long long* next, int (*lds)[BLOCK],
                                                  Fetch fetch, Emit emit, int32_t* status,
-                                                 unsigned long long* counters, int refill,
-                                                 uint32_t chunk_rays = LMGPU_RAY_CHUNK) {
+                                                 unsigned long long* counters, int refill) {
+    constexpr uint32_t chunk_rays = LMGPU_RAY_CHUNK;
     static_assert(LDS_DEPTH >= W, "one node's children must fit the LDS part of an empty stack");
     const int lane = threadIdx.x & 63;
     const int tid = threadIdx.x;
@@ -493,22 +507,25 @@ __device__ __forceinline__ void trace_persistent(const Node* __restrict__ nodes,
     int sp = 0;                  // stack entries
     lds[0][tid] = kDone;
     // Wave-uniform: ray ids of the wave not yet handed to a lane, and whether
-    // ids are left beyond them. Every wave starts with a share of its own, half
-    // of an even split in whole waves of rays (at least one), and `next` hands
-    // out what lies past all shares: atomics on one address from all XCDs take
-    // 12 ns each, so one per wave before any ray started took 74 us of every
-    // launch (16 spp of a small room at 256x256 6.40 -> 4.48 ms, one 360p
-    // preview pass 2.70 -> 1.74). Shares go to the waves of a block in a row, whose
-    // rays then meet in its L1; with fewer shares than waves they go to the
-    // blocks in turn, over all CUs.
+    // ids are left beyond them. Every wave starts with a share of its own
+    // (ray_share) and takes chunks of what lies past all shares from the ray
+    // counters. Atomics on one address from all XCDs take 12 ns each, so one per
+    // wave before any ray started took 74 us of every launch, and a last,
+    // empty-handed one per wave as much of its end. Group g of the blocks takes
+    // chunks g, g + 8, ... from a counter of its own: an eighth of the
+    // updates wait for each other, and all groups work on all parts of the
+    // rays. Shares go to the waves of a block in a row, whose rays then meet in
+    // its L1; with fewer shares than waves they go to the blocks in turn, over
+    // all CUs.
     const uint32_t nblk = gridDim.x, nwaves = nblk * (BLOCK / 64);
-    const uint32_t share = max(64u, n / nwaves / 2u & ~63u);
+    const uint32_t share = ray_share(n, nwaves);
     const uint32_t in_blk = threadIdx.x >> 6;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(n < nwaves * 64u ? in_blk * nblk + blockIdx.x
                                                                          : blockIdx.x * (BLOCK / 64) + in_blk);
     const uint32_t shared_from = nwaves * share;   // < n + 64 nwaves
+    const uint32_t groups = min(kRayCounters, nblk), group = blockIdx.x % groups;
     uint32_t pool_next = min(n, wave * share), pool_end = min(n, wave * share + share);
-    bool more = shared_from < n;                   // ids beyond the pool may be left
+    bool more = shared_from < n;                   // ids of the group beyond the pool may be left
     bool exhausted = pool_next == pool_end && !more;
     unsigned long long nv = 0, nt = 0;
     // component kx (shift 0), ky (3) or kz (6) of v: tests of single bits
@@ -565,11 +582,12 @@ __device__ __forceinline__ void trace_persistent(const Node* __restrict__ nodes,
                 uint32_t chunk = n, chunk_end = n;
                 if (avail < nidle && more) {
                     uint32_t b = 0;
-                    if (lane == 0) b = uint32_t(atomicAdd(next, (unsigned long long)chunk_rays));
+                    if (lane == 0) b = uint32_t(atomicAdd(next + group * kRayCounterStride, 1ull));
                     // wave-uniform from here on: scalar registers for the pool
-                    chunk = min(n, shared_from + __builtin_amdgcn_readfirstlane(b));
+                    const uint32_t at = (__builtin_amdgcn_readfirstlane(b) * groups + group) * chunk_rays;
+                    chunk = min(n, shared_from + at);
                     chunk_end = min(n, chunk + chunk_rays);
-                    more = chunk_end < n;
+                    more = chunk + groups * chunk_rays < n;
                 }
                 if (idle) {
                     const uint32_t rank = __popcll(idle_mask & ((1ull << lane) - 1ull));

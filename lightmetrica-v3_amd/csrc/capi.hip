@@ -151,8 +151,9 @@ int lmgpu_accel_status(const lmgpu_accel* accel, void* stream) {
 // a file-scope device array (one copy per GPU, held until the process ends):
 //   [0, 32*M)          rays  (lmgpu_ray, M = LMGPU_NOALLOC_MAX_RAYS)
 //   [32*M, 48*M)       hits  (lmgpu_hit)
-//   [48*M, 48*M + 8)   ray counter of the persistent traversal (zeroed by its launch)
+//   [48*M, 48*M + 8)   unused
 //   [48*M + 8, +4)     traversal overflow word (cleared before each call)
+//   [48*M + 256, ...)  ray counters of the persistent traversal (zeroed by its launch when it uses them)
 // In host code `scratch` names a host-side stand-in, not device memory: its
 // device address is looked up once per device (hipGetSymbolAddress, with that
 // device current) and only that address is used from then on.
@@ -163,7 +164,8 @@ constexpr size_t kNoallocHitBytes = size_t(LMGPU_NOALLOC_MAX_RAYS) * sizeof(lmgp
 static_assert(kNoallocRayBytes + kNoallocHitBytes + 256 == size_t(LMGPU_NOALLOC_SCRATCH_BYTES),
               "scratch layout and LMGPU_NOALLOC_SCRATCH_BYTES disagree");
 
-static __device__ __align__(256) unsigned char scratch[LMGPU_NOALLOC_SCRATCH_BYTES];
+static __device__ __align__(256) unsigned char
+    scratch[LMGPU_NOALLOC_SCRATCH_BYTES + kRayCounterWords * sizeof(unsigned long long)];
 
 constexpr int kNoallocMaxDevices = 64;
 static std::mutex g_noalloc_mu[kNoallocMaxDevices];
@@ -203,8 +205,8 @@ extern "C" int lmgpu_accel_intersect_host_noalloc(const lmgpu_accel* accel, cons
     LMGPU_TRY(noalloc_scratch(dev, &base));
     auto* drays = reinterpret_cast<lmgpu_ray*>(base);
     auto* dhits = reinterpret_cast<lmgpu_hit*>(base + kNoallocRayBytes);
-    auto* next = reinterpret_cast<unsigned long long*>(base + kNoallocRayBytes + kNoallocHitBytes);
-    auto* status = reinterpret_cast<int32_t*>(next + 1);
+    auto* status = reinterpret_cast<int32_t*>(base + kNoallocRayBytes + kNoallocHitBytes + 8);
+    auto* next = reinterpret_cast<unsigned long long*>(base + LMGPU_NOALLOC_SCRATCH_BYTES);
     hipStream_t s = nullptr;
     LMGPU_HIP(hipMemsetAsync(status, 0, sizeof(int32_t), s));
     LMGPU_HIP(hipMemcpyAsync(drays, rays, sizeof(lmgpu_ray) * size_t(n), hipMemcpyHostToDevice, s));

@@ -118,16 +118,16 @@ struct Accel {
         }
         return status.p;
     }
-    // Ray counter for one persistent launch: a ring of slots so launches that
+    // Ray counters for one persistent launch: a ring of slots so launches that
     // overlap on different streams use different counters (up to kRing in
     // flight at once).
     static constexpr int kRing = 256;
     unsigned long long* next_counter() const {
         if (!ring.p) {
             auto* self = const_cast<Accel*>(this);
-            if (self->ring.alloc(kRing) != LMGPU_OK) return nullptr;
+            if (self->ring.alloc(kRing * kRayCounterWords) != LMGPU_OK) return nullptr;
         }
-        return ring.p + (ring_pos.fetch_add(1) % kRing);
+        return ring.p + (ring_pos.fetch_add(1) % kRing) * kRayCounterWords;
     }
     // Stack entries needed in the worst case: (W-1) pushes per level.
     int stack_bound() const { return (width - 1) * depth; }

@@ -113,7 +113,7 @@ __global__ __launch_bounds__(BLOCK) void k_lt_regen(SceneDev sc, LTConsts c, int
     __shared__ int s_qbase, s_emit, s_idle;
     __shared__ unsigned int s_fin;
     if (threadIdx.x == 0)
-        s_idle = __hip_atomic_load(&ctl->remaining, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0;
+        s_idle = ctl->remaining == 0;
     __syncthreads();
     if (s_idle) return;
     if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&ctl->iterations, 1ull);
@@ -144,7 +144,7 @@ __global__ __launch_bounds__(BLOCK) void k_lt_regen(SceneDev sc, LTConsts c, int
         unsigned long long base = 0;
         int emit = 0, qb = 0;
         if (acc > 0) {
-            base = __hip_atomic_load(&ctl->work_next, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            base = ctl->work_next;
             if (base < (unsigned long long)total) base = atomicAdd(&ctl->work_next, (unsigned long long)acc);
             if (base < (unsigned long long)total) emit = int(min((unsigned long long)acc, (unsigned long long)total - base));
             if (emit > 0) qb = atomicAdd(q.counts + ext_count(in_q), emit);
@@ -319,7 +319,7 @@ __global__ __launch_bounds__(kBlock) void k_lt_shade(SceneDev sc, PathState ps, 
 
 template <int W>
 __global__ __launch_bounds__(kBlock, 6) void k_lt_connect(SceneDev sc, Queues q, int out_q, unsigned long long* next, int refill,
-                                                       double* __restrict__ film, int chunk_rays) {
+                                                       double* __restrict__ film) {
     __shared__ int lds[kLds + 1][kBlock];
     const int n = q.counts[shadow_count(out_q)];
     if (n == 0) return;   // no connections (whole grid)
@@ -342,13 +342,13 @@ __global__ __launch_bounds__(kBlock, 6) void k_lt_connect(SceneDev sc, Queues q,
         }
     };
     trace_persistent<W, true, false, kLds, kPriv, kBlock>(nodes_of<W>(sc), sc.tris, n, next, lds, fetch, emit,
-                                                          q.counts + 5, nullptr, refill, chunk_rays);
+                                                          q.counts + 5, nullptr, refill);
     if (blockIdx.x == 0 && threadIdx.x == 0)
         atomicAdd(reinterpret_cast<unsigned long long*>(q.counts + 12), (unsigned long long)n);
 }
 
 __global__ void k_lt_begin(unsigned long long* next, int32_t* counts, int out_q) {
-    if (threadIdx.x < 2) next[threadIdx.x] = 0ull;
+    if (threadIdx.x < 2 * kRayCounters) next[threadIdx.x * kRayCounterStride] = 0ull;
     if (threadIdx.x == 0) {
         counts[ext_count(out_q)] = 0;
         counts[shadow_count(out_q)] = 0;
@@ -387,12 +387,11 @@ void lt_regen_iteration(Scene& S, Wavefront& wf, const LTConsts& c, int64_t tota
     hipLaunchKernelGGL(k_lt_regen<kRegenBlock>, dim3(rg), dim3(kRegenBlock), 0, s, S.dev, c, total, npix, pass0,
                        wf.ppix.p, ppass, wf.pstate.p, wf.thr0.p, info, q, in_q, cap, wf.ctl.p);
     hipLaunchKernelGGL(k_lt_begin, dim3(1), dim3(64), 0, s, wf.next.p, wf.counts.p, in_q ^ 1);
-    hipLaunchKernelGGL(k_extend<W>, dim3(extend_grid<W>()), dim3(kBlock), 0, s, S.dev, q, in_q, wf.next.p, refill,
-                       LMGPU_REGEN_RAY_CHUNK);
+    hipLaunchKernelGGL(k_extend<W>, dim3(extend_grid<W>()), dim3(kBlock), 0, s, S.dev, q, in_q, wf.next.p, refill);
     hipLaunchKernelGGL(k_lt_shade, dim3(sg), dim3(kBlock), 0, s, S.dev, ps, q, c, in_q, wf.ppix.p, ppass,
                        wf.pstate.p);
-    hipLaunchKernelGGL(k_lt_connect<W>, dim3(lt_connect_grid<W>()), dim3(kBlock), 0, s, S.dev, q, in_q ^ 1, wf.next.p + 1, refill,
-                       film, LMGPU_REGEN_RAY_CHUNK);
+    hipLaunchKernelGGL(k_lt_connect<W>, dim3(lt_connect_grid<W>()), dim3(kBlock), 0, s, S.dev, q, in_q ^ 1, wf.next.p + kRayCounterWords, refill,
+                       film);
 }
 
 // ---------------------------------------------------------------------------
@@ -952,24 +951,21 @@ void bd_pass(Scene& S, const BDConsts& c, double* film, int refill, LVert* lv, h
     const int cg = lt_connect_grid<W>();
     hipLaunchKernelGGL(k_lt_begin, dim3(1), dim3(64), 0, s, S.next.p, S.counts.p, 1);
     hipLaunchKernelGGL(k_bd_lgen, dim3(gb), dim3(kBlock), 0, s, S.dev, ps, q, c, lv, S.blcount.p);
-    hipLaunchKernelGGL(k_lt_connect<W>, dim3(cg), dim3(kBlock), 0, s, S.dev, q, 1, S.next.p + 1, refill, film,
-                           LMGPU_RAY_CHUNK);
+    hipLaunchKernelGGL(k_lt_connect<W>, dim3(cg), dim3(kBlock), 0, s, S.dev, q, 1, S.next.p + kRayCounterWords, refill, film);
     for (int b = 0; b < c.max_verts - 2; b++) {   // y_1 .. y_{max_verts - 2}
         const int in_q = b & 1;
         hipLaunchKernelGGL(k_lt_begin, dim3(1), dim3(64), 0, s, S.next.p, S.counts.p, in_q ^ 1);
-        hipLaunchKernelGGL(k_extend<W>, dim3(tg), dim3(kBlock), 0, s, S.dev, q, in_q, S.next.p, refill, LMGPU_RAY_CHUNK);
+        hipLaunchKernelGGL(k_extend<W>, dim3(tg), dim3(kBlock), 0, s, S.dev, q, in_q, S.next.p, refill);
         hipLaunchKernelGGL(k_bd_lshade, dim3(sg), dim3(kBlock), 0, s, S.dev, ps, q, c, in_q, lv, S.blcount.p);
-        hipLaunchKernelGGL(k_lt_connect<W>, dim3(cg), dim3(kBlock), 0, s, S.dev, q, in_q ^ 1, S.next.p + 1, refill, film,
-                           LMGPU_RAY_CHUNK);
+        hipLaunchKernelGGL(k_lt_connect<W>, dim3(cg), dim3(kBlock), 0, s, S.dev, q, in_q ^ 1, S.next.p + kRayCounterWords, refill, film);
     }
     hipLaunchKernelGGL(k_bd_egen, dim3(gb), dim3(kBlock), 0, s, S.dev, ps, q, c);
     for (int b = 0; b < c.max_verts - 1; b++) {   // z_1 .. z_{max_verts - 1}
         const int in_q = b & 1;
         hipLaunchKernelGGL(k_lt_begin, dim3(1), dim3(64), 0, s, S.next.p, S.counts.p, in_q ^ 1);
-        hipLaunchKernelGGL(k_extend<W>, dim3(tg), dim3(kBlock), 0, s, S.dev, q, in_q, S.next.p, refill, LMGPU_RAY_CHUNK);
+        hipLaunchKernelGGL(k_extend<W>, dim3(tg), dim3(kBlock), 0, s, S.dev, q, in_q, S.next.p, refill);
         hipLaunchKernelGGL(k_bd_eshade, dim3(sg), dim3(kBlock), 0, s, S.dev, ps, q, c, in_q, lv, S.blcount.p, film);
-        hipLaunchKernelGGL(k_lt_connect<W>, dim3(cg), dim3(kBlock), 0, s, S.dev, q, in_q ^ 1, S.next.p + 1, refill, film,
-                           LMGPU_RAY_CHUNK);
+        hipLaunchKernelGGL(k_lt_connect<W>, dim3(cg), dim3(kBlock), 0, s, S.dev, q, in_q ^ 1, S.next.p + kRayCounterWords, refill, film);
     }
 }
 

@@ -141,14 +141,6 @@ __global__ __launch_bounds__(kBlock) void k_camera_nee(SceneDev sc, Queues q, PT
     }
 }
 
-__global__ void k_reset_counts(int32_t* counts, int out_q) {
-    if (threadIdx.x == 0) {
-        counts[ext_count(out_q)] = 0;
-        counts[shadow_count(out_q)] = 0;
-    }
-}
-
-
 // Unoccluded shadow rays add their contribution to the path radiance and,
 // when the vertex records guide training data, to the record's radiance
 // baseline (the NEE of a vertex is not part of its sampled direction's
@@ -204,8 +196,14 @@ __global__ __launch_bounds__(kBlock, 6) void k_connect(SceneDev sc, PathState ps
         atomicAdd(reinterpret_cast<unsigned long long*>(q.counts + 12), (unsigned long long)n);
 }
 
-__global__ void k_bounce_begin(unsigned long long* next) {
-    if (threadIdx.x < 2) next[threadIdx.x] = 0ull;
+// Clears what a bounce that fills queue out_q counts in: the ray counters of
+// its two traversals and the counts of that queue and its shadow queue.
+__global__ void k_bounce_begin(unsigned long long* next, int32_t* counts, int out_q) {
+    if (threadIdx.x < 2 * kRayCounters) next[threadIdx.x * kRayCounterStride] = 0ull;
+    if (threadIdx.x == 0) {
+        counts[ext_count(out_q)] = 0;
+        counts[shadow_count(out_q)] = 0;
+    }
 }
 
 
@@ -365,8 +363,8 @@ __global__ __launch_bounds__(kBlock, 6) void k_raycast(SceneDev sc, unsigned lon
                                                            nullptr, refill);
 }
 
-__global__ void k_zero_u64(unsigned long long* p) {
-    if (threadIdx.x == 0) *p = 0ull;
+__global__ void k_zero_ray_counters(unsigned long long* p) {
+    if (threadIdx.x < kRayCounters) p[threadIdx.x * kRayCounterStride] = 0ull;
 }
 
 __global__ void k_zero_i32(int32_t* p, int n) {
@@ -631,7 +629,7 @@ int Scene::ensure_workspace(int npix) {
     LMGPU_TRY(hit.alloc(npix));
     LMGPU_TRY(path0.alloc(npix)); LMGPU_TRY(path1.alloc(npix));
     LMGPU_TRY(counts.alloc(16));
-    LMGPU_TRY(next.alloc(2));
+    LMGPU_TRY(next.alloc(2 * kRayCounterWords));
     LMGPU_HIP(hipMemset(counts.p, 0, 16 * sizeof(int32_t)));
     ws_npix = npix;
     if (graph) { (void)hipGraphExecDestroy(graph); graph = nullptr; }
@@ -716,10 +714,10 @@ int Scene::enqueue_pass(const PTConsts& c, double* sum, double* sumsq, const Gui
     const int tg = accel.width == 4 ? pt_trace_grid<4>() : (accel.width == 8 ? pt_trace_grid<8>() : pt_trace_grid<2>());
     if (c.image && c.mode != LMGPU_SAMPLING_NAIVE) {
         // the camera vertex's light samples, traced before the first bounce
+        hipLaunchKernelGGL(k_bounce_begin, dim3(1), dim3(64), 0, s, next.p, counts.p, 1);
         hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(64), 0, s, counts.p + shadow_count(0), 1);
         hipLaunchKernelGGL(k_camera_nee, dim3(gb), dim3(kBlock), 0, s, dev, q, c);
-        hipLaunchKernelGGL(k_bounce_begin, dim3(1), dim3(64), 0, s, next.p);
-        unsigned long long* nx = next.p + 1;
+        unsigned long long* nx = next.p + kRayCounterWords;
         if (accel.width == 4)
             hipLaunchKernelGGL(k_connect<4>, dim3(tg), dim3(kBlock), 0, s, dev, ps, q, nx, 0, refill_primary, nullptr,
                                nullptr, sum);
@@ -734,18 +732,17 @@ int Scene::enqueue_pass(const PTConsts& c, double* sum, double* sumsq, const Gui
         const int in_q = b & 1;
         // camera rays are coherent: keep 64 consecutive rays per wave
         const int pm = b == 0 ? refill_primary : refill_secondary;
-        hipLaunchKernelGGL(k_bounce_begin, dim3(1), dim3(64), 0, s, next.p);
-        if (accel.width == 4) hipLaunchKernelGGL(k_extend<4>, dim3(tg), dim3(kBlock), 0, s, dev, q, in_q, next.p, pm, LMGPU_RAY_CHUNK);
-        else if (accel.width == 8) hipLaunchKernelGGL(k_extend<8>, dim3(tg), dim3(kBlock), 0, s, dev, q, in_q, next.p, pm, LMGPU_RAY_CHUNK);
-        else hipLaunchKernelGGL(k_extend<2>, dim3(tg), dim3(kBlock), 0, s, dev, q, in_q, next.p, pm, LMGPU_RAY_CHUNK);
+        hipLaunchKernelGGL(k_bounce_begin, dim3(1), dim3(64), 0, s, next.p, counts.p, in_q ^ 1);
+        if (accel.width == 4) hipLaunchKernelGGL(k_extend<4>, dim3(tg), dim3(kBlock), 0, s, dev, q, in_q, next.p, pm);
+        else if (accel.width == 8) hipLaunchKernelGGL(k_extend<8>, dim3(tg), dim3(kBlock), 0, s, dev, q, in_q, next.p, pm);
+        else hipLaunchKernelGGL(k_extend<2>, dim3(tg), dim3(kBlock), 0, s, dev, q, in_q, next.p, pm);
         if (gp)
             hipLaunchKernelGGL(k_pt_guide_infer<Queues>, dim3(std::max(1, std::min((npix + 127) / 128, 512))), dim3(256), 0, s,
                                dev, q, in_q, gp->g->Wbf.p, gp->g->P.p, box, gmix.p);
-        hipLaunchKernelGGL(k_reset_counts, dim3(1), dim3(64), 0, s, counts.p, in_q ^ 1);
         if (gp) hipLaunchKernelGGL(k_shade<true>, dim3(sg), dim3(kBlock), 0, s, dev, ps, q, c, in_q, gd);
         else hipLaunchKernelGGL(k_shade<false>, dim3(sg), dim3(kBlock), 0, s, dev, ps, q, c, in_q, gd);
         if (c.mode != LMGPU_SAMPLING_NAIVE) {
-            unsigned long long* nx = next.p + 1;
+            unsigned long long* nx = next.p + kRayCounterWords;
             if (accel.width == 4)
                 hipLaunchKernelGGL(k_connect<4>, dim3(tg), dim3(kBlock), 0, s, dev, ps, q, nx, in_q ^ 1, pm, crec, cshrec, sum);
             else if (accel.width == 8)
@@ -978,7 +975,7 @@ int Scene::raycast(const lmgpu_raycast_params* p, double* film_in, bool on_devic
     unsigned long long* next = accel.next_counter();
     int32_t* status = accel.status_dev();
     if (!next || !status) return fail(LMGPU_ERR_OUT_OF_MEMORY, "traversal counters");
-    hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, s, next);
+    hipLaunchKernelGGL(k_zero_ray_counters, dim3(1), dim3(64), 0, s, next);
     // camera rays are coherent: keep 64 consecutive pixels per wave
     const int refill = 64;
     if (accel.width == 4)

@@ -23,9 +23,6 @@
 #ifndef LMGPU_REGEN_MAX_SLOTS
 #define LMGPU_REGEN_MAX_SLOTS (1 << 24)
 #endif
-// Rays a wave takes per atomic on the traversal's ray counter in the
-// regenerating loops, whose queues stay long (the one-sample passes use
-// LMGPU_RAY_CHUNK: their late bounces queue few rays).
 // Path pool of a guided render, whose slots also hold training records
 // (record_depth x 96 B each): 4 slots per pixel, at most 2^23. With fewer
 // paths in flight an iteration finishes about half a sample per pixel's
@@ -35,9 +32,6 @@
 #endif
 #ifndef LMGPU_REGEN_GUIDED_MAX_SLOTS
 #define LMGPU_REGEN_GUIDED_MAX_SLOTS (1 << 23)
-#endif
-#ifndef LMGPU_REGEN_RAY_CHUNK
-#define LMGPU_REGEN_RAY_CHUNK 128
 #endif
 
 namespace lmgpu {
