@@ -8,14 +8,15 @@
 //   3. stable radix sort of (code, index) pairs (sort.hip), checked ordered,
 //   4. binary LBVH topology (Karras, HPG 2012), ties broken by index, or
 //      PLOC (ploc.hip),
-//   5. bottom-up bounds refit, level-synchronous over a frontier, which also
-//      fills the SAH cost tables of the collapse (sah_tables),
+//   5. triangles copied into traversal order (48 B each) and bottom-up bounds
+//      refit, one block per kRefitSpan leaves and one block for the nodes
+//      above, which also fills the SAH cost tables of the collapse
+//      (sah_tables),
 //   6. collapse into a W-wide tree (W = 2, 4, 8) of least SAH cost: the
 //      dynamic program decides which binary subtrees become wide nodes and
 //      which become leaves of at most `leaf_size` triangles (a contiguous
 //      range of the sorted triangle array); the greedy alternative opens the
-//      largest-area child until a node has W children,
-//   7. triangles copied into traversal order (48 B each).
+//      largest-area child until a node has W children.
 // and Accel_SAHBVH::intersect (:269-299) with the ordered wide traversal of
 // bvh.h.
 
@@ -40,12 +41,40 @@ namespace lmgpu {
 // triangle mesh, with the same hits).
 constexpr int kDefaultLeafSize = 2;
 constexpr float kDefaultSahTriCost = 0.5f;
-// Refit levels launched between two reads of the frontier size.
-constexpr int kRefitLevelsPerSync = 6;
+// Leaves per refit block: four for each thread, so a 1.3M triangle mesh still
+// gives every CU five blocks and only some 2600 nodes span blocks.
+constexpr int kRefitSpan = 1024;
+// Collapse levels launched between two reads of the level sizes; a level past
+// the last one is a launch of blocks that find no item (4 us), a read back is
+// a wait of some 40 us.
+constexpr int kCollapseLevelsPerSync = 16;
+constexpr int kCollapseMaxLevels = 4096;
+constexpr unsigned kCollapseMaxBlocks = 2048;
+
+// What the build kernels count, on the device; cleared when a build starts.
+struct BuildHead {
+    float4 root_lo, root_hi;   // bounds of the root
+    double sah;                // summed half areas of the collapse (unnormalised SAH cost)
+    int32_t leaves;            // wide-tree leaves
+    int32_t unsorted;          // the sort's result was not in order
+    int32_t frontier;          // nodes left to k_refit_top
+    int32_t pad;
+    // wide nodes of each level, and the slot of the first: level l holds the
+    // slots [first[l], first[l] + count[l])
+    int32_t count[kCollapseMaxLevels + kCollapseLevelsPerSync + 1];
+    int32_t first[kCollapseMaxLevels + kCollapseLevelsPerSync + 1];
+};
 
 // ---------------------------------------------------------------------------
 // build kernels
 // ---------------------------------------------------------------------------
+
+__device__ __forceinline__ void tri_bounds(const float* v, float4& lo, float4& hi) {
+    lo = make_float4(fminf(v[0], fminf(v[3], v[6])), fminf(v[1], fminf(v[4], v[7])), fminf(v[2], fminf(v[5], v[8])),
+                     0.f);
+    hi = make_float4(fmaxf(v[0], fmaxf(v[3], v[6])), fmaxf(v[1], fmaxf(v[4], v[7])), fmaxf(v[2], fmaxf(v[5], v[8])),
+                     0.f);
+}
 
 // Per-triangle AABB (float4 lo, hi); per-block centroid bounds into
 // `partial` (6 floats per block), reduced by k_reduce_bounds.
@@ -55,17 +84,13 @@ __global__ __launch_bounds__(256) void k_prep(const float* __restrict__ verts, i
     const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     float cmin[3] = {3e38f, 3e38f, 3e38f}, cmax[3] = {-3e38f, -3e38f, -3e38f};
     if (i < n) {
-        const float* v = verts + 9 * i;
-        float lo[3], hi[3];
-        for (int a = 0; a < 3; a++) {
-            lo[a] = fminf(v[a], fminf(v[3 + a], v[6 + a]));
-            hi[a] = fmaxf(v[a], fmaxf(v[3 + a], v[6 + a]));
-            const float c = (lo[a] + hi[a]) * 0.5f;
-            cmin[a] = c;
-            cmax[a] = c;
-        }
-        tlo[i] = make_float4(lo[0], lo[1], lo[2], 0.f);
-        thi[i] = make_float4(hi[0], hi[1], hi[2], 0.f);
+        float4 lo, hi;
+        tri_bounds(verts + 9 * i, lo, hi);
+        cmin[0] = cmax[0] = (lo.x + hi.x) * 0.5f;
+        cmin[1] = cmax[1] = (lo.y + hi.y) * 0.5f;
+        cmin[2] = cmax[2] = (lo.z + hi.z) * 0.5f;
+        tlo[i] = lo;
+        thi[i] = hi;
     }
     const int w = threadIdx.x >> 6;
     for (int a = 0; a < 3; a++) {
@@ -199,53 +224,6 @@ __global__ __launch_bounds__(256) void k_lbvh(const uint64_t* __restrict__ k, in
     bn[i] = node;
 }
 
-// One atomic per wave: a lane with `want` gets a slot of *counter (-1
-// otherwise). Every lane of the wave must call it.
-__device__ __forceinline__ int32_t wave_alloc(int32_t* counter, bool want, int32_t count = 1) {
-    const unsigned long long mask = __ballot(want);
-    if (mask == 0) return -1;
-    const int lane = threadIdx.x & 63;
-    const int leader = __ffsll(mask) - 1;
-    // inclusive prefix of the counts of the wanting lanes, in lane order
-    int32_t c = want ? count : 0, inc = c;
-    for (int off = 1; off < 64; off <<= 1) {
-        const int32_t y = __shfl_up(inc, off);
-        if (lane >= off) inc += y;
-    }
-    const int32_t total = __shfl(inc, 63);
-    int32_t base = 0;
-    if (lane == leader) base = atomicAdd(counter, total);
-    base = __shfl(base, leader);
-    return want ? base + inc - c : -1;
-}
-
-// Bottom-up refit without device-scope fences (which write back the
-// per-XCD L2s): level-synchronous over a frontier. A node enters the
-// frontier of launch k+1 when its second child finished in launch k (atomic
-// arrival counter), so both children's bounds were written by earlier
-// launches and are visible at kernel boundaries.
-__global__ __launch_bounds__(256) void k_refit_leaves(int64_t n, const int32_t* __restrict__ order,
-                                                      const float4* __restrict__ tlo, const float4* __restrict__ thi,
-                                                      const int32_t* __restrict__ parent_leaf,
-                                                      float4* __restrict__ leaf_lo, float4* __restrict__ leaf_hi,
-                                                      int32_t* __restrict__ flags, int32_t* __restrict__ frontier,
-                                                      int32_t* __restrict__ fcount) {
-    const int64_t j = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    bool push = false;
-    int32_t p = -1;
-    if (j < n) {
-        const int32_t ti = order[j];
-        leaf_lo[j] = tlo[ti];
-        leaf_hi[j] = thi[ti];
-        if (n > 1) {
-            p = parent_leaf[j];
-            push = atomicAdd(&flags[p], 1) == 1;
-        }
-    }
-    const int32_t k = wave_alloc(fcount, push);
-    if (push) frontier[k] = p;
-}
-
 __device__ __forceinline__ float half_area(float4 lo, float4 hi) {
     const float dx = hi.x - lo.x, dy = hi.y - lo.y, dz = hi.z - lo.z;
     return dx * dy + dy * dz + dz * dx;
@@ -276,25 +254,34 @@ __global__ __launch_bounds__(256) void k_parents(const BNode* __restrict__ bn, i
 struct SahDP {
     float* cost;
     uint8_t* choice;
-    int W;
     int pmax;
     float ctri;
 };
 
-__device__ __forceinline__ void sah_tables(const SahDP& dp, int32_t p, const BNode& nd, float area,
-                                           const float4& l0, const float4& h0, const float4& l1, const float4& h1) {
-    const int W = dp.W;
-    float cl[8], cr[8];
+template <int W>
+__device__ __forceinline__ void sah_tables(const SahDP& dp, int32_t p, int32_t left, int32_t right, int cnt,
+                                           float area, const float4& l0, const float4& h0, const float4& l1,
+                                           const float4& h1) {
+    float cl[W], cr[W];
     const float al = half_area(l0, h0) * dp.ctri, ar = half_area(l1, h1) * dp.ctri;
+    // loaded for leaves too (from node 0's place), so that the loads need no branch
+    const float* tl = dp.cost + int64_t(max(left, 0)) * W;
+    const float* tr = dp.cost + int64_t(max(right, 0)) * W;
     for (int i = 0; i < W; i++) {
-        cl[i] = nd.left < 0 ? al : dp.cost[int64_t(nd.left) * W + i];
-        cr[i] = nd.right < 0 ? ar : dp.cost[int64_t(nd.right) * W + i];
+        cl[i] = tl[i];
+        cr[i] = tr[i];
     }
-    float dist[8];
-    int arg[8];
+    for (int i = 0; i < W; i++) {
+        cl[i] = left < 0 ? al : cl[i];
+        cr[i] = right < 0 ? ar : cr[i];
+    }
+    float dist[W];
+    int arg[W];
+#pragma unroll
     for (int j = 2; j <= W; j++) {
         float best = __builtin_inff();
         int bk = 1;
+#pragma unroll
         for (int k = 1; k < j; k++) {
             const float c = cl[k - 1] + cr[j - k - 1];
             if (c < best) { best = c; bk = k; }
@@ -302,7 +289,6 @@ __device__ __forceinline__ void sah_tables(const SahDP& dp, int32_t p, const BNo
         dist[j - 1] = best;
         arg[j - 1] = bk;
     }
-    const int cnt = nd.last - nd.first + 1;
     const float cint = area + dist[W - 1];
     const float cprim = cnt <= dp.pmax ? area * float(cnt) * dp.ctri : __builtin_inff();
     float c = fminf(cprim, cint);
@@ -310,6 +296,7 @@ __device__ __forceinline__ void sah_tables(const SahDP& dp, int32_t p, const BNo
     uint8_t* ch = dp.choice + int64_t(p) * W;
     out[0] = c;
     ch[0] = cprim <= cint ? uint8_t(0xFF) : uint8_t(arg[W - 1]);
+#pragma unroll
     for (int i = 2; i <= W; i++) {
         if (c <= dist[i - 1]) {
             ch[i - 1] = 0;
@@ -321,153 +308,313 @@ __device__ __forceinline__ void sah_tables(const SahDP& dp, int32_t p, const BNo
     }
 }
 
-__global__ __launch_bounds__(256) void k_refit_nodes(const int32_t* __restrict__ fin, const int32_t* __restrict__ fin_count,
-                                                     const BNode* __restrict__ bn, int32_t root,
-                                                     const int32_t* __restrict__ parent_int,
-                                                     const float4* __restrict__ leaf_lo,
-                                                     const float4* __restrict__ leaf_hi, float4* __restrict__ node_lo,
-                                                     float4* __restrict__ node_hi, int32_t* __restrict__ flags,
-                                                     int32_t* __restrict__ fout, int32_t* __restrict__ fout_count,
-                                                     SahDP dp) {
-    const int cnt = *fin_count;
-    const int stride = gridDim.x * blockDim.x;
-    // whole waves run the same number of iterations (wave-level appends)
-    const int rounds = (cnt + stride - 1) / stride;
-    for (int r = 0; r < rounds; r++) {
-        const int idx = r * stride + blockIdx.x * blockDim.x + threadIdx.x;
-        bool push = false;
-        int32_t q = -1;
-        if (idx < cnt) {
-            const int32_t p = fin[idx];
-            const BNode nd = bn[p];
-            const float4 l0 = nd.left < 0 ? leaf_lo[~nd.left] : node_lo[nd.left];
-            const float4 h0 = nd.left < 0 ? leaf_hi[~nd.left] : node_hi[nd.left];
-            const float4 l1 = nd.right < 0 ? leaf_lo[~nd.right] : node_lo[nd.right];
-            const float4 h1 = nd.right < 0 ? leaf_hi[~nd.right] : node_hi[nd.right];
-            const float4 lo = make_float4(fminf(l0.x, l1.x), fminf(l0.y, l1.y), fminf(l0.z, l1.z), 0.f);
-            const float4 hi = make_float4(fmaxf(h0.x, h1.x), fmaxf(h0.y, h1.y), fmaxf(h0.z, h1.z), 0.f);
-            node_lo[p] = lo;
-            node_hi[p] = hi;
-            if (dp.cost) sah_tables(dp, p, nd, half_area(lo, hi), l0, h0, l1, h1);
-            if (p != root) {
-                q = parent_int[p];
-                push = atomicAdd(&flags[q], 1) == 1;
-            }
-        }
-        const int32_t k = wave_alloc(fout_count, push);
-        if (push) fout[k] = q;
+// Bottom-up refit. A node is done by the thread that counts its second child
+// as done, in the round after: rounds are separated by a barrier of the one
+// block whose threads wrote both children, so no device-scope fence (a write
+// back of the per-XCD L2s) is needed and no launch per level either.
+//
+// A round is bound by latency, and a mesh of 1.3M triangles takes 22 rounds
+// in the blocks and 28 above them: the list holds what a node's loads need, so
+// its children and its parent's links are read side by side. That mesh takes
+// 183 us in the blocks (with the 42 us of the triangles' gather) and 293 us
+// above them; a launch per level over a global list with an atomic per wave
+// took 890 us, and the gather was a pass of its own.
+struct Refit {
+    const BNode* bn;
+    const int32_t* parent_int;
+    const int32_t* parent_leaf;
+    float4* leaf_lo;
+    float4* leaf_hi;
+    float4* node_lo;
+    float4* node_hi;
+    int32_t* flags;      // children done, of the nodes that span blocks
+    int32_t root;
+    SahDP dp;
+    BuildHead* head;
+};
+
+// A node whose children are done.
+struct RefitItem {
+    int32_t node, parent, left, right;
+    int32_t first, last;
+};
+
+__device__ __forceinline__ RefitItem refit_item(const Refit& r, int32_t q) {
+    const BNode nd = r.bn[q];
+    return RefitItem{q, r.parent_int[q], nd.left, nd.right, nd.first, nd.last};
+}
+
+// Bounds and cost tables of a listed node.
+template <int W>
+__device__ __forceinline__ void refit_node(const Refit& r, const RefitItem it) {
+    const float4 l0 = *(it.left < 0 ? r.leaf_lo + ~it.left : r.node_lo + it.left);
+    const float4 h0 = *(it.left < 0 ? r.leaf_hi + ~it.left : r.node_hi + it.left);
+    const float4 l1 = *(it.right < 0 ? r.leaf_lo + ~it.right : r.node_lo + it.right);
+    const float4 h1 = *(it.right < 0 ? r.leaf_hi + ~it.right : r.node_hi + it.right);
+    const float4 lo = make_float4(fminf(l0.x, l1.x), fminf(l0.y, l1.y), fminf(l0.z, l1.z), 0.f);
+    const float4 hi = make_float4(fmaxf(h0.x, h1.x), fmaxf(h0.y, h1.y), fmaxf(h0.z, h1.z), 0.f);
+    if (r.dp.cost)
+        sah_tables<W>(r.dp, it.node, it.left, it.right, it.last - it.first + 1, half_area(lo, hi), l0, h0, l1, h1);
+    r.node_lo[it.node] = lo;
+    r.node_hi[it.node] = hi;
+    if (it.node == r.root) {
+        r.head->root_lo = lo;
+        r.head->root_hi = hi;
     }
 }
 
-__global__ __launch_bounds__(256) void k_reorder(int64_t n, const int32_t* __restrict__ order,
-                                                 const float* __restrict__ verts, TriV* __restrict__ tris) {
-    const int64_t j = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (j >= n) return;
-    const int32_t ti = order[j];
-    const float* v = verts + 9 * int64_t(ti);
-    TriV t;
-    t.v0 = make_float4(v[0], v[1], v[2], __int_as_float(ti));
-    t.v1 = make_float4(v[3], v[4], v[5], 0.f);
-    t.v2 = make_float4(v[6], v[7], v[8], 0.f);
-    tris[j] = t;
+// The leaves [kRefitSpan * block, + kRefitSpan): their triangles in traversal
+// order and bounds, and every node above whose range of leaves lies within
+// them, in rounds over a list of ready nodes in LDS (at most half the leaves,
+// and never longer than the one before it: each parent enters by exactly one
+// child). Children done are counted in LDS too, by the last leaf of the node's
+// left child, which no other node shares. A ready node that spans blocks is
+// counted in memory and goes to `frontier`: such nodes have disjoint ranges,
+// so there are fewer than blocks.
+template <int W>
+__global__ __launch_bounds__(256, 6) void k_refit_blocks(int64_t n, const int32_t* __restrict__ order,
+                                                         const float* __restrict__ verts, TriV* __restrict__ tris,
+                                                         Refit r, RefitItem* __restrict__ frontier) {
+    constexpr int kHalf = kRefitSpan / 2;
+    __shared__ int4 links[2 * kHalf];        // RefitItem: node, parent, left, right
+    __shared__ uint32_t range[2 * kHalf];    // its first and last leaf, in 16 bits each from the block's first
+    __shared__ uint32_t done[kRefitSpan / 4];
+    __shared__ int32_t size[2];
+    constexpr int kPer = kRefitSpan / 256;
+    const int32_t lead = int32_t(blockIdx.x) * kRefitSpan;
+    const int32_t tail = int32_t(std::min<int64_t>(n, int64_t(lead) + kRefitSpan) - 1);
+    if (threadIdx.x < 2) size[threadIdx.x] = 0;
+    static_assert(kRefitSpan / 4 <= 256 && kRefitSpan <= 65536, "one word of `done` per thread, 16-bit ranges");
+    if (threadIdx.x < kRefitSpan / 4) done[threadIdx.x] = 0;
+    __syncthreads();
+    // the child [first, last] of q's node is done
+    auto arrive = [&](const RefitItem q, int32_t first, int32_t last, int to) {
+        if (q.first >= lead && q.last <= tail) {
+            const uint32_t g = uint32_t((q.first == first ? last : first - 1) - lead);
+            const uint32_t sh = 8 * (g & 3);
+            if ((atomicAdd(&done[g >> 2], 1u << sh) >> sh & 0xffu) != 1u) return;
+            const int k = to * kHalf + atomicAdd(&size[to], 1);
+            links[k] = make_int4(q.node, q.parent, q.left, q.right);
+            range[k] = uint32_t(q.first - lead) | uint32_t(q.last - lead) << 16;
+        } else if (atomicAdd(&r.flags[q.node], 1) == 1) {
+            frontier[atomicAdd(&r.head->frontier, 1)] = q;
+        }
+    };
+    int32_t ti[kPer], up[kPer];
+#pragma unroll
+    for (int k = 0; k < kPer; k++) {
+        const int32_t j = min(lead + int32_t(threadIdx.x) + 256 * k, tail);
+        ti[k] = order[j];
+        up[k] = n > 1 ? r.parent_leaf[j] : 0;
+    }
+#pragma unroll
+    for (int k = 0; k < kPer; k++) {
+        const int32_t j = lead + int32_t(threadIdx.x) + 256 * k;
+        if (j > tail) break;
+        float v[9];
+#pragma unroll
+        for (int c = 0; c < 9; c++) v[c] = verts[9 * int64_t(ti[k]) + c];
+        RefitItem q{};
+        if (n > 1) q = refit_item(r, up[k]);
+        TriV t;
+        t.v0 = make_float4(v[0], v[1], v[2], __int_as_float(ti[k]));
+        t.v1 = make_float4(v[3], v[4], v[5], 0.f);
+        t.v2 = make_float4(v[6], v[7], v[8], 0.f);
+        tris[j] = t;
+        float4 lo, hi;
+        tri_bounds(v, lo, hi);
+        r.leaf_lo[j] = lo;
+        r.leaf_hi[j] = hi;
+        if (n > 1) {
+            arrive(q, j, j, 0);
+        } else {
+            r.head->root_lo = lo;
+            r.head->root_hi = hi;
+        }
+    }
+    int cur = 0;
+    while (true) {
+        __syncthreads();
+        const int m = size[cur];
+        if (m == 0) break;
+        for (int i = threadIdx.x; i < m; i += 256) {
+            const int4 l = links[cur * kHalf + i];
+            const uint32_t f = range[cur * kHalf + i];
+            const RefitItem it{l.x, l.y, l.z, l.w, lead + int32_t(f & 0xffffu), lead + int32_t(f >> 16)};
+            const RefitItem q = refit_item(r, max(it.parent, 0));
+            refit_node<W>(r, it);
+            if (it.node != r.root) arrive(q, it.first, it.last, cur ^ 1);
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) size[cur] = 0;
+        cur ^= 1;
+    }
 }
 
-struct CollapseItem {
-    int32_t bref;   // binary ref (internal index or ~leaf)
-    int32_t wnode;  // wide node slot
+// The nodes above the blocks: one block, rounds as above over lists in global
+// memory (list0 holds head->frontier items). They are some 1% of the nodes, so
+// one block's rate costs less than a launch per level.
+template <int W>
+__global__ __launch_bounds__(1024) void k_refit_top(Refit r, RefitItem* __restrict__ list0,
+                                                    RefitItem* __restrict__ list1) {
+    __shared__ int32_t size[2];
+    if (threadIdx.x == 0) {
+        size[0] = r.head->frontier;
+        size[1] = 0;
+    }
+    const RefitItem* in = list0;
+    RefitItem* out = list1;
+    int cur = 0;
+    while (true) {
+        __syncthreads();
+        const int m = size[cur];
+        if (m == 0) break;
+        for (int i = threadIdx.x; i < m; i += 1024) {
+            const RefitItem it = in[i];
+            const int32_t up = max(it.parent, 0);
+            const int32_t before = it.node != r.root ? atomicAdd(&r.flags[up], 1) : 0;
+            const RefitItem q = refit_item(r, up);
+            refit_node<W>(r, it);
+            if (before == 1) out[atomicAdd(&size[cur ^ 1], 1)] = q;
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) size[cur] = 0;
+        cur ^= 1;
+        RefitItem* t = const_cast<RefitItem*>(in);
+        in = out;
+        out = t;
+    }
+}
+
+// One level of the collapse into W-wide nodes: item i of the level is the
+// binary ref of the wide node in slot first[level] + i, and the nodes' inner
+// children are the next level's items.
+struct CollapseArgs {
+    const int32_t* in;
+    int32_t* out;
+    int level;
+    const BNode* bn;
+    const float4* node_lo;
+    const float4* node_hi;
+    const float4* leaf_lo;
+    const float4* leaf_hi;
+    const uint8_t* choice;   // SAH collapse: sah_tables
+    int leaf_size;           // greedy collapse
+    void* wnodes;
+    BuildHead* head;
 };
 
-// Writes wide node `it.wnode` from its nc <= W binary refs (each a leaf when
-// is_leaf(ref), else a wide child). The wide children of one node take
-// consecutive slots, so siblings share cache lines; they become next-level
-// items. Every lane of the wave calls it (`active` false for lanes without an
-// item): slots and queue positions are taken with one atomic per wave and
-// the SAH and leaf statistics are summed over the wave first.
-template <int W, class IsLeaf>
-__device__ __forceinline__ void emit_wide_node(bool active, const CollapseItem& it, const int32_t (&ref)[W], int nc,
-                                               IsLeaf is_leaf, const BNode* __restrict__ bn,
-                                               const float4* __restrict__ node_lo, const float4* __restrict__ node_hi,
-                                               const float4* __restrict__ leaf_lo, const float4* __restrict__ leaf_hi,
-                                               CollapseItem* __restrict__ out, int32_t* __restrict__ n_out,
-                                               int32_t* __restrict__ node_counter, WNode<W>* __restrict__ wnodes,
-                                               double* sah_acc, int32_t* leaf_counter) {
-    int nint = 0;
-    if (active)
-        for (int c = 0; c < nc; c++) nint += is_leaf(ref[c]) ? 0 : 1;
-    int32_t slot = wave_alloc(node_counter, nint > 0, nint);
-    int32_t q = wave_alloc(n_out, nint > 0, nint);
+// Runs a level: `expand(bref, ref, nc)` finds the nc <= W refs a wide node of
+// `bref` has as children, `is_leaf(ref)` tells which of them are leaves. The
+// wide children of one node take consecutive slots, so siblings share cache
+// lines. Whole blocks take their nodes' slots with one atomic, and the SAH
+// sum and leaf count of all a block's items are added once: same-address
+// atomics cost 12 ns each on the card, and with four per wave they were most
+// of the collapse's time (1.3M triangles, W = 4, 17 levels: 445 us, now
+// 245 us, at 10 to 33 us a level mostly the latency of the unfolding).
+template <int W, class Expand, class IsLeaf>
+__device__ __forceinline__ void collapse_level(const CollapseArgs& a, Expand expand, IsLeaf is_leaf) {
+    __shared__ int32_t wave_sum[4];
+    __shared__ int32_t block_base;
+    __shared__ double block_sah[4];
+    __shared__ int32_t block_leaves[4];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int32_t count = a.head->count[a.level], first = a.head->first[a.level];
+    const int32_t next = first + count;   // slot of the next level's first node
+    if (blockIdx.x == 0 && threadIdx.x == 0) a.head->first[a.level + 1] = next;
+    WNode<W>* wnodes = static_cast<WNode<W>*>(a.wnodes);
     double sah = 0.0;
     int nleaf = 0;
-    if (active) {
-        WNode<W> node;
-        for (int c = 0; c < W; c++) {
-            if (c < nc) {
-                const int32_t r = ref[c];
-                const float4 lo = r < 0 ? leaf_lo[~r] : node_lo[r];
-                const float4 hi = r < 0 ? leaf_hi[~r] : node_hi[r];
-                node.lox[c] = lo.x; node.loy[c] = lo.y; node.loz[c] = lo.z;
-                node.hix[c] = hi.x; node.hiy[c] = hi.y; node.hiz[c] = hi.z;
-                const int cnt = r < 0 ? 1 : bn[r].last - bn[r].first + 1;
-                const double a = double(half_area(lo, hi));
-                if (is_leaf(r)) {
-                    node.child[c] = r < 0 ? ~r : bn[r].first;
-                    node.count[c] = cnt;
-                    sah += a * cnt;
-                    nleaf++;
-                } else {
-                    node.child[c] = slot;
-                    node.count[c] = 0;
-                    sah += a;
-                    out[q++] = CollapseItem{r, slot++};
-                }
-            } else {
-                node.lox[c] = node.loy[c] = node.loz[c] = 1e30f;
-                node.hix[c] = node.hiy[c] = node.hiz[c] = -1e30f;
-                node.child[c] = 0;
-                node.count[c] = -1;
-            }
+    for (int64_t base = int64_t(blockIdx.x) * 256; base < count; base += int64_t(gridDim.x) * 256) {
+        const int64_t idx = base + threadIdx.x;
+        int32_t ref[W];
+        int nc = 0, nint = 0;
+        uint32_t inner = 0;
+        if (idx < count) {
+            expand(a.in[idx], ref, nc);
+            for (int c = 0; c < nc; c++)
+                if (!is_leaf(ref[c])) inner |= 1u << c;
+            nint = __popc(inner);
         }
-        wnodes[it.wnode] = node;
+        int inc = nint;
+        for (int off = 1; off < 64; off <<= 1) {
+            const int y = __shfl_up(inc, off);
+            if (lane >= off) inc += y;
+        }
+        if (lane == 63) wave_sum[w] = inc;
+        __syncthreads();
+        int before = 0, total = 0;
+        for (int k = 0; k < 4; k++) {
+            before += k < w ? wave_sum[k] : 0;
+            total += wave_sum[k];
+        }
+        if (threadIdx.x == 0) block_base = total ? atomicAdd(&a.head->count[a.level + 1], total) : 0;
+        __syncthreads();
+        int32_t q = block_base + before + inc - nint;
+        if (idx < count) {
+            WNode<W> node;
+            for (int c = 0; c < W; c++) {
+                if (c < nc) {
+                    const int32_t r = ref[c];
+                    const float4 lo = r < 0 ? a.leaf_lo[~r] : a.node_lo[r];
+                    const float4 hi = r < 0 ? a.leaf_hi[~r] : a.node_hi[r];
+                    node.lox[c] = lo.x; node.loy[c] = lo.y; node.loz[c] = lo.z;
+                    node.hix[c] = hi.x; node.hiy[c] = hi.y; node.hiz[c] = hi.z;
+                    const double area = double(half_area(lo, hi));
+                    if (inner >> c & 1u) {
+                        node.child[c] = next + q;
+                        node.count[c] = 0;
+                        sah += area;
+                        a.out[q++] = r;
+                    } else {
+                        const int cnt = r < 0 ? 1 : a.bn[r].last - a.bn[r].first + 1;
+                        node.child[c] = r < 0 ? ~r : a.bn[r].first;
+                        node.count[c] = cnt;
+                        sah += area * cnt;
+                        nleaf++;
+                    }
+                } else {
+                    node.lox[c] = node.loy[c] = node.loz[c] = 1e30f;
+                    node.hix[c] = node.hiy[c] = node.hiz[c] = -1e30f;
+                    node.child[c] = 0;
+                    node.count[c] = -1;
+                }
+            }
+            wnodes[first + idx] = node;
+        }
     }
     for (int off = 32; off > 0; off >>= 1) {
         sah += __shfl_xor(sah, off);
         nleaf += __shfl_xor(nleaf, off);
     }
-    if ((threadIdx.x & 63) == 0) {
-        atomicAdd(sah_acc, sah);
-        atomicAdd(leaf_counter, nleaf);
+    if (lane == 0) {
+        block_sah[w] = sah;
+        block_leaves[w] = nleaf;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0 && int64_t(blockIdx.x) * 256 < count) {
+        atomicAdd(&a.head->sah, block_sah[0] + block_sah[1] + block_sah[2] + block_sah[3]);
+        atomicAdd(&a.head->leaves, block_leaves[0] + block_leaves[1] + block_leaves[2] + block_leaves[3]);
     }
 }
 
-// SAH collapse: one work item per wide node; its children are the roots the
-// cost tables chose for D(p, W) (sah_tables), found by unfolding the choices
-// with a stack of (ref, slots) pairs whose slots sum to at most W.
+// SAH collapse: a wide node's children are the roots the cost tables chose
+// for D(p, W) (sah_tables), found by unfolding the choices with a stack of
+// (ref, slots) pairs whose slots sum to at most W.
 template <int W>
-__global__ __launch_bounds__(256) void k_collapse_sah(const CollapseItem* __restrict__ in,
-                                                      const int32_t* __restrict__ n_in, CollapseItem* __restrict__ out,
-                                                      int32_t* __restrict__ n_out, int32_t* __restrict__ node_counter,
-                                                      const BNode* __restrict__ bn, const float4* __restrict__ node_lo,
-                                                      const float4* __restrict__ node_hi,
-                                                      const float4* __restrict__ leaf_lo,
-                                                      const float4* __restrict__ leaf_hi,
-                                                      const uint8_t* __restrict__ choice, WNode<W>* __restrict__ wnodes,
-                                                      double* sah_acc, int32_t* leaf_counter) {
-    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool active = idx < *n_in;
-    const CollapseItem it = active ? in[idx] : CollapseItem{~0, 0};
+__global__ __launch_bounds__(256) void k_collapse_sah(CollapseArgs a) {
+    const uint8_t* choice = a.choice;
     auto is_leaf = [&](int32_t r) { return r < 0 || choice[int64_t(r) * W] == 0xFF; };
-    int32_t ref[W];
-    int nc = 0;
-    if (!active) {
-        // no item: only takes part in the wave's allocations
-    } else if (is_leaf(it.bref)) {
-        ref[nc++] = it.bref;   // the whole tree is one leaf (tiny scenes)
-    } else {
+    auto expand = [&](int32_t bref, int32_t (&ref)[W], int& nc) {
+        if (is_leaf(bref)) {
+            ref[nc++] = bref;   // the whole tree is one leaf (tiny scenes)
+            return;
+        }
         int32_t sr[W];
         int sj[W];
         int sp = 0;
-        const BNode b = bn[it.bref];
-        const int k = choice[int64_t(it.bref) * W];
+        const BNode b = a.bn[bref];
+        const int k = choice[int64_t(bref) * W];
         sr[sp] = b.right; sj[sp++] = W - k;
         sr[sp] = b.left; sj[sp++] = k;
         while (sp > 0) {
@@ -481,59 +628,50 @@ __global__ __launch_bounds__(256) void k_collapse_sah(const CollapseItem* __rest
                 continue;
             }
             const int c = choice[int64_t(m) * W + j - 1];
-            const BNode bm = bn[m];
+            const BNode bm = a.bn[m];
             sr[sp] = bm.right; sj[sp++] = j - c;
             sr[sp] = bm.left; sj[sp++] = c;
         }
-    }
-    emit_wide_node<W>(active, it, ref, nc, is_leaf, bn, node_lo, node_hi, leaf_lo, leaf_hi, out, n_out, node_counter,
-                      wnodes, sah_acc, leaf_counter);
+    };
+    collapse_level<W>(a, expand, is_leaf);
 }
 
-// Greedy collapse: one work item per wide node; open the largest-area child
-// until W, then write the node and emit the internal children as next-level
-// items.
+// Greedy collapse: open the largest-area child until there are W.
 template <int W>
-__global__ __launch_bounds__(256) void k_collapse(const CollapseItem* __restrict__ in, const int32_t* __restrict__ n_in,
-                                                  CollapseItem* __restrict__ out, int32_t* __restrict__ n_out,
-                                                  int32_t* __restrict__ node_counter, const BNode* __restrict__ bn,
-                                                  const float4* __restrict__ node_lo, const float4* __restrict__ node_hi,
-                                                  const float4* __restrict__ leaf_lo, const float4* __restrict__ leaf_hi,
-                                                  WNode<W>* __restrict__ wnodes, int leaf_size, double* sah_acc,
-                                                  int32_t* leaf_counter) {
-    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool active = idx < *n_in;
-    const CollapseItem it = active ? in[idx] : CollapseItem{~0, 0};
-    int32_t ref[W];
-    int nc = 0;
-    auto cnt_of = [&](int32_t r) -> int { return r < 0 ? 1 : bn[r].last - bn[r].first + 1; };
-    auto lo_of = [&](int32_t r) { return r < 0 ? leaf_lo[~r] : node_lo[r]; };
-    auto hi_of = [&](int32_t r) { return r < 0 ? leaf_hi[~r] : node_hi[r]; };
-    if (!active) {
-        // no item: only takes part in the wave's allocations
-    } else if (it.bref < 0 || cnt_of(it.bref) <= leaf_size) {
-        ref[nc++] = it.bref;   // whole range is one leaf (tiny scenes)
-    } else {
-        ref[nc++] = bn[it.bref].left;
-        ref[nc++] = bn[it.bref].right;
+__global__ __launch_bounds__(256) void k_collapse(CollapseArgs a) {
+    auto cnt_of = [&](int32_t r) -> int { return r < 0 ? 1 : a.bn[r].last - a.bn[r].first + 1; };
+    auto lo_of = [&](int32_t r) { return r < 0 ? a.leaf_lo[~r] : a.node_lo[r]; };
+    auto hi_of = [&](int32_t r) { return r < 0 ? a.leaf_hi[~r] : a.node_hi[r]; };
+    auto is_leaf = [&](int32_t r) { return r < 0 || cnt_of(r) <= a.leaf_size; };
+    auto expand = [&](int32_t bref, int32_t (&ref)[W], int& nc) {
+        if (is_leaf(bref)) {
+            ref[nc++] = bref;   // whole range is one leaf (tiny scenes)
+            return;
+        }
+        ref[nc++] = a.bn[bref].left;
+        ref[nc++] = a.bn[bref].right;
         while (nc < W) {
             int best = -1;
             float best_a = -1.f;
             for (int c = 0; c < nc; c++) {
-                if (ref[c] >= 0 && cnt_of(ref[c]) > leaf_size) {
-                    const float a = half_area(lo_of(ref[c]), hi_of(ref[c]));
-                    if (a > best_a) { best_a = a; best = c; }
+                if (!is_leaf(ref[c])) {
+                    const float area = half_area(lo_of(ref[c]), hi_of(ref[c]));
+                    if (area > best_a) { best_a = area; best = c; }
                 }
             }
             if (best < 0) break;
-            const BNode b = bn[ref[best]];
+            const BNode b = a.bn[ref[best]];
             ref[best] = b.left;
             ref[nc++] = b.right;
         }
-    }
-    auto is_leaf = [&](int32_t r) { return r < 0 || cnt_of(r) <= leaf_size; };
-    emit_wide_node<W>(active, it, ref, nc, is_leaf, bn, node_lo, node_hi, leaf_lo, leaf_hi, out, n_out, node_counter,
-                      wnodes, sah_acc, leaf_counter);
+    };
+    collapse_level<W>(a, expand, is_leaf);
+}
+
+__global__ void k_collapse_init(BuildHead* head, int32_t* items, int32_t root_ref) {
+    head->count[0] = 1;
+    head->first[0] = 0;
+    items[0] = root_ref;
 }
 
 // ---------------------------------------------------------------------------
@@ -577,16 +715,47 @@ __global__ __launch_bounds__(kTraceBlock, 6) void k_trace(const Node* __restrict
                                                                          status, counters, refill);
 }
 
-// Quantised copy of a built W-wide node array (bvh.h, quantise_node).
+// Quantised copy of a built W-wide node array (bvh.h, quantise_node), four
+// lanes per node: one for each axis's planes, one for the child entries. A
+// wave reads and writes 16 whole nodes side by side; a thread per node kept 64
+// lines in flight for each of its loads and refetched them (454K nodes, W = 4:
+// 171 us, now 31 us).
 template <int W>
 __global__ __launch_bounds__(256) void k_quantise(const WNode<W>* __restrict__ in, QNode<W>* __restrict__ out,
                                                   int64_t n) {
-    const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
-    if (i < n) out[i] = quantise_node<W>(in[i]);
-}
-
-__global__ void k_zero_i32_1(int32_t* c) {
-    if (threadIdx.x == 0) *c = 0;
+    const int64_t i = int64_t(blockIdx.x) * 64 + (threadIdx.x >> 2);
+    const int a = threadIdx.x & 3;
+    if (i >= n) return;   // whole quads
+    const WNode<W>& node = in[i];
+    QNode<W>& q = out[i];
+    const float* planes = reinterpret_cast<const float*>(&node);
+    float lo[W], hi[W];   // lane 3: the words of child and count
+    for (int c = 0; c < W; c++) {
+        lo[c] = planes[(a < 3 ? a : 6) * W + c];
+        hi[c] = planes[(a < 3 ? 3 + a : 7) * W + c];
+    }
+    uint32_t present = 0;
+    for (int c = 0; c < W; c++) present |= __float_as_int(hi[c]) >= 0 ? 1u << c : 0u;
+    present = __shfl(present, 3, 4);
+    QAxis<W> x{};
+    if (a < 3) x = quantise_axis<W>(lo, hi, present);
+    uint32_t e = uint32_t(x.e + 127) << (8 * a), es = uint32_t(x.e & 0xff) << (8 * a);
+    if (a == 3) e = es = 0;
+    for (int off = 1; off < 4; off <<= 1) {
+        e |= __shfl_xor(e, off, 4);
+        es |= __shfl_xor(es, off, 4);
+    }
+    if (a < 3) {
+        (a == 0 ? q.ox : a == 1 ? q.oy : q.oz) = x.org;
+        for (int k = 0; k < W / 4; k++) {
+            q.qlo[a][k] = x.ql[k];
+            q.qhi[a][k] = x.qh[k];
+        }
+    } else {
+        q.e = e;
+        q.es = es;
+        for (int c = 0; c < W; c++) q.ent[c] = quantised_entry(__float_as_int(lo[c]), __float_as_int(hi[c]));
+    }
 }
 
 __global__ void k_zero_counter(unsigned long long* c) {
@@ -599,20 +768,19 @@ __global__ void k_zero_counter(unsigned long long* c) {
 
 static inline unsigned nblocks(int64_t n, int b) { return unsigned((n + b - 1) / b); }
 
+// Leaves, triangles in traversal order, and every node's bounds (and tables).
 template <int W>
-static void launch_collapse(bool sah_collapse, const CollapseItem* in, const int32_t* n_in, CollapseItem* out,
-                            int32_t* n_out, int32_t* node_counter, const BNode* bn, const float4* node_lo,
-                            const float4* node_hi, const float4* leaf_lo, const float4* leaf_hi,
-                            const uint8_t* choice, void* wnodes, int leaf_size, double* sah, int32_t* leaves,
-                            int64_t count, hipStream_t s) {
-    if (sah_collapse)
-        hipLaunchKernelGGL(k_collapse_sah<W>, dim3(nblocks(count, 256)), dim3(256), 0, s, in, n_in, out, n_out,
-                           node_counter, bn, node_lo, node_hi, leaf_lo, leaf_hi, choice,
-                           static_cast<WNode<W>*>(wnodes), sah, leaves);
-    else
-        hipLaunchKernelGGL(k_collapse<W>, dim3(nblocks(count, 256)), dim3(256), 0, s, in, n_in, out, n_out,
-                           node_counter, bn, node_lo, node_hi, leaf_lo, leaf_hi, static_cast<WNode<W>*>(wnodes),
-                           leaf_size, sah, leaves);
+static void launch_refit(int64_t n, const int32_t* order, const float* verts, TriV* tris, const Refit& r,
+                         RefitItem* list0, RefitItem* list1, hipStream_t s) {
+    hipLaunchKernelGGL(k_refit_blocks<W>, dim3(nblocks(n, kRefitSpan)), dim3(256), 0, s, n, order, verts, tris, r,
+                       list0);
+    if (n > kRefitSpan) hipLaunchKernelGGL(k_refit_top<W>, dim3(1), dim3(1024), 0, s, r, list0, list1);
+}
+
+template <int W>
+static void launch_collapse(bool by_sah, const CollapseArgs& a, unsigned grid, hipStream_t s) {
+    if (by_sah) hipLaunchKernelGGL(k_collapse_sah<W>, dim3(grid), dim3(256), 0, s, a);
+    else hipLaunchKernelGGL(k_collapse<W>, dim3(grid), dim3(256), 0, s, a);
 }
 
 int Accel::build(const float* verts_in, int64_t n, bool on_device, const lmgpu_build_opts* opts, hipStream_t s) {
@@ -656,10 +824,9 @@ int Accel::build(const float* verts_in, int64_t n, bool on_device, const lmgpu_b
     DevBuf<float> cb, partial, dp_cost;
     DevBuf<uint8_t> dp_choice;
     DevBuf<uint64_t> keys, keys2;
-    DevBuf<int32_t> vals, vals2, parent_int, parent_leaf, flags, counters;
+    DevBuf<int32_t> vals, vals2, parent_int, parent_leaf, flags, q0, q1;
     DevBuf<BNode> bn;
-    DevBuf<CollapseItem> q0, q1;
-    DevBuf<double> sah;
+    DevBuf<BuildHead> head;
     LMGPU_TRY(tlo.alloc(n)); LMGPU_TRY(thi.alloc(n));
     LMGPU_TRY(leaf_lo.alloc(n)); LMGPU_TRY(leaf_hi.alloc(n));
     LMGPU_TRY(node_lo.alloc(m)); LMGPU_TRY(node_hi.alloc(m));
@@ -671,11 +838,10 @@ int Accel::build(const float* verts_in, int64_t n, bool on_device, const lmgpu_b
     LMGPU_TRY(parent_int.alloc(m));
     LMGPU_TRY(parent_leaf.alloc(n));
     LMGPU_TRY(flags.alloc(m));
-    LMGPU_TRY(counters.alloc(8));
+    LMGPU_TRY(head.alloc(1));
     LMGPU_TRY(bn.alloc(m));
     LMGPU_TRY(q0.alloc(n)); LMGPU_TRY(q1.alloc(n));
-    LMGPU_TRY(sah.alloc(1));
-    SahDP dp{nullptr, nullptr, W, leaf, ctri};
+    SahDP dp{nullptr, nullptr, leaf, ctri};
     if (collapse == LMGPU_COLLAPSE_SAH) {
         LMGPU_TRY(dp_cost.alloc(size_t(m) * W));
         LMGPU_TRY(dp_choice.alloc(size_t(m) * W));
@@ -683,6 +849,7 @@ int Accel::build(const float* verts_in, int64_t n, bool on_device, const lmgpu_b
         dp.choice = dp_choice.p;
     }
 
+    LMGPU_HIP(hipMemsetAsync(head.p, 0, sizeof(BuildHead), s));
     hipLaunchKernelGGL(k_prep, dim3(nb_prep), dim3(256), 0, s, verts, n, tlo.p, thi.p, partial.p);
     hipLaunchKernelGGL(k_reduce_bounds, dim3(1), dim3(256), 0, s, partial.p, int(nb_prep), cb.p);
     hipLaunchKernelGGL(k_morton, dim3(nblocks(n, 256)), dim3(256), 0, s, tlo.p, thi.p, n, cb.p, keys.p, vals.p);
@@ -692,10 +859,9 @@ int Accel::build(const float* verts_in, int64_t n, bool on_device, const lmgpu_b
     const int32_t* svals = in_alt ? vals2.p : vals.p;
     if (n > 1) {
         // the sort's result must be ordered before the tree is built on it
-        LMGPU_HIP(hipMemsetAsync(counters.p, 0, sizeof(int32_t), s));
-        hipLaunchKernelGGL(k_check_sorted, dim3(nblocks(n - 1, 256)), dim3(256), 0, s, skeys, n, counters.p);
+        hipLaunchKernelGGL(k_check_sorted, dim3(nblocks(n - 1, 256)), dim3(256), 0, s, skeys, n, &head.p->unsorted);
         int32_t unsorted = 0;
-        LMGPU_HIP(hipMemcpyAsync(&unsorted, counters.p, sizeof(int32_t), hipMemcpyDeviceToHost, s));
+        LMGPU_HIP(hipMemcpyAsync(&unsorted, &head.p->unsorted, sizeof(int32_t), hipMemcpyDeviceToHost, s));
         LMGPU_HIP(hipStreamSynchronize(s));
         if (unsorted) return fail(LMGPU_ERR_DEVICE, "Morton sort produced an unordered key array");
     }
@@ -717,101 +883,68 @@ int Accel::build(const float* verts_in, int64_t n, bool on_device, const lmgpu_b
         hipLaunchKernelGGL(k_lbvh, dim3(nblocks(n - 1, 256)), dim3(256), 0, s, skeys, n, bn.p, parent_int.p,
                            parent_leaf.p);
     }
-    {
-        // frontier refit (bounds, and the SAH cost tables when collapsing by
-        // SAH): q0/q1 (reinterpreted as int32 lists) hold the frontiers
-        if (n > 1) LMGPU_HIP(hipMemsetAsync(flags.p, 0, sizeof(int32_t) * (n - 1), s));
-        int32_t* fr[2] = {reinterpret_cast<int32_t*>(q0.p), reinterpret_cast<int32_t*>(q1.p)};
-        LMGPU_HIP(hipMemsetAsync(counters.p, 0, 2 * sizeof(int32_t), s));
-        hipLaunchKernelGGL(k_refit_leaves, dim3(nblocks(n, 256)), dim3(256), 0, s, n, order, tlo.p, thi.p,
-                           parent_leaf.p, leaf_lo.p, leaf_hi.p, flags.p, fr[0], counters.p);
-        // A frontier is never larger than the one before it (each parent
-        // enters from exactly one child of the previous frontier), so the
-        // grid sized for the last count read back serves the next
-        // kRefitLevelsPerSync levels, each launch reading its own count.
-        int cur = 0;
-        int levels_refit = 0;
-        while (n > 1) {
-            int32_t cnt = 0;
-            LMGPU_HIP(hipMemcpyAsync(&cnt, counters.p + cur, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-            LMGPU_HIP(hipStreamSynchronize(s));
-            if (cnt == 0) break;
-            for (int l = 0; l < kRefitLevelsPerSync; l++) {
-                hipLaunchKernelGGL(k_zero_i32_1, dim3(1), dim3(64), 0, s, counters.p + (cur ^ 1));
-                hipLaunchKernelGGL(k_refit_nodes, dim3(std::min(nblocks(cnt, 256), 2048u)), dim3(256), 0, s, fr[cur],
-                                   counters.p + cur, bn.p, root_ref, parent_int.p, leaf_lo.p, leaf_hi.p, node_lo.p,
-                                   node_hi.p, flags.p, fr[cur ^ 1], counters.p + (cur ^ 1), dp);
-                cur ^= 1;
-            }
-            levels_refit += kRefitLevelsPerSync;
-            if (levels_refit > 4096) return fail(LMGPU_ERR_DEVICE, "BVH refit did not terminate");
-        }
-    }
+    // refit (bounds, and the SAH cost tables when collapsing by SAH); q0 and
+    // q1 hold the nodes left to its second kernel
+    if (n > 1) LMGPU_HIP(hipMemsetAsync(flags.p, 0, sizeof(int32_t) * (n - 1), s));
+    const Refit refit{bn.p, parent_int.p, parent_leaf.p, leaf_lo.p, leaf_hi.p, node_lo.p, node_hi.p, flags.p, root_ref,
+                      dp, head.p};
     LMGPU_TRY(tris.alloc(n));
-    hipLaunchKernelGGL(k_reorder, dim3(nblocks(n, 256)), dim3(256), 0, s, n, order, verts, tris.p);
+    auto* list0 = reinterpret_cast<RefitItem*>(q0.p);
+    auto* list1 = reinterpret_cast<RefitItem*>(q1.p);
+    if (W == 2) launch_refit<2>(n, order, verts, tris.p, refit, list0, list1, s);
+    else if (W == 4) launch_refit<4>(n, order, verts, tris.p, refit, list0, list1, s);
+    else launch_refit<8>(n, order, verts, tris.p, refit, list0, list1, s);
 
     // collapse, level by level
     const size_t node_bytes = size_t(32) * W;
     const int64_t max_nodes = std::max<int64_t>(n, 1);
     LMGPU_TRY(nodes.alloc(size_t(max_nodes) * node_bytes / sizeof(float4)));
-    const CollapseItem root{root_ref, 0};
-    LMGPU_HIP(hipMemcpyAsync(q0.p, &root, sizeof(root), hipMemcpyHostToDevice, s));
-    int32_t init[4] = {1, 0, 1, 0};   // n_in, n_out, node_counter, leaves
-    LMGPU_HIP(hipMemcpyAsync(counters.p, init, sizeof(init), hipMemcpyHostToDevice, s));
-    LMGPU_HIP(hipMemsetAsync(sah.p, 0, sizeof(double), s));
-    int64_t count = 1;
+    hipLaunchKernelGGL(k_collapse_init, dim3(1), dim3(1), 0, s, head.p, q0.p, root_ref);
+    CollapseArgs ca{q0.p, q1.p, 0, bn.p, node_lo.p, node_hi.p, leaf_lo.p, leaf_hi.p, dp.choice, leaf, nodes.p, head.p};
+    // Levels are launched kCollapseLevelsPerSync at a time, each reading its
+    // own size; their grids cover what the last size read can have become.
+    int64_t bound = 1;
     int levels = 0;
-    CollapseItem* qin = q0.p;
-    CollapseItem* qout = q1.p;
-    while (count > 0) {
-        levels++;
-        LMGPU_HIP(hipMemsetAsync(counters.p + 1, 0, sizeof(int32_t), s));
-        const bool by_sah = collapse == LMGPU_COLLAPSE_SAH;
-        if (W == 2)
-            launch_collapse<2>(by_sah, qin, counters.p, qout, counters.p + 1, counters.p + 2, bn.p, node_lo.p,
-                               node_hi.p, leaf_lo.p, leaf_hi.p, dp.choice, nodes.p, leaf, sah.p, counters.p + 3, count,
-                               s);
-        else if (W == 4)
-            launch_collapse<4>(by_sah, qin, counters.p, qout, counters.p + 1, counters.p + 2, bn.p, node_lo.p,
-                               node_hi.p, leaf_lo.p, leaf_hi.p, dp.choice, nodes.p, leaf, sah.p, counters.p + 3, count,
-                               s);
-        else
-            launch_collapse<8>(by_sah, qin, counters.p, qout, counters.p + 1, counters.p + 2, bn.p, node_lo.p,
-                               node_hi.p, leaf_lo.p, leaf_hi.p, dp.choice, nodes.p, leaf, sah.p, counters.p + 3, count,
-                               s);
-        int32_t nout = 0;
-        LMGPU_HIP(hipMemcpyAsync(&nout, counters.p + 1, sizeof(int32_t), hipMemcpyDeviceToHost, s));
+    num_nodes = 0;
+    while (levels == ca.level) {
+        if (ca.level >= kCollapseMaxLevels) return fail(LMGPU_ERR_DEVICE, "BVH collapse did not terminate");
+        const int at = ca.level;
+        for (int l = 0; l < kCollapseLevelsPerSync; l++) {
+            const unsigned grid = std::min(nblocks(bound, 256), kCollapseMaxBlocks);
+            const bool by_sah = collapse == LMGPU_COLLAPSE_SAH;
+            if (W == 2) launch_collapse<2>(by_sah, ca, grid, s);
+            else if (W == 4) launch_collapse<4>(by_sah, ca, grid, s);
+            else launch_collapse<8>(by_sah, ca, grid, s);
+            bound = std::min<int64_t>(bound * W, n);
+            ca.level++;
+            ca.out = const_cast<int32_t*>(ca.in);
+            ca.in = ca.in == q0.p ? q1.p : q0.p;
+        }
+        int32_t sizes[kCollapseLevelsPerSync + 1];
+        LMGPU_HIP(hipMemcpyAsync(sizes, head.p->count + at, sizeof(sizes), hipMemcpyDeviceToHost, s));
         LMGPU_HIP(hipStreamSynchronize(s));
-        LMGPU_HIP(hipMemcpyAsync(counters.p, counters.p + 1, sizeof(int32_t), hipMemcpyDeviceToDevice, s));
-        count = nout;
-        std::swap(qin, qout);
-        if (levels > 4096) return fail(LMGPU_ERR_DEVICE, "BVH collapse did not terminate");
+        for (int l = 0; l < kCollapseLevelsPerSync && sizes[l] > 0; l++) {
+            num_nodes += sizes[l];
+            levels++;
+        }
+        bound = sizes[kCollapseLevelsPerSync];
+        if (bound == 0) break;
     }
     LMGPU_HIP(hipEventRecord(e1, s));
-    int32_t fin[4];
-    double sah_sum = 0;
-    LMGPU_HIP(hipMemcpyAsync(fin, counters.p, sizeof(fin), hipMemcpyDeviceToHost, s));
-    LMGPU_HIP(hipMemcpyAsync(&sah_sum, sah.p, sizeof(double), hipMemcpyDeviceToHost, s));
+    BuildHead h;   // its counters; the level sizes are known
+    LMGPU_HIP(hipMemcpyAsync(&h, head.p, offsetof(BuildHead, count), hipMemcpyDeviceToHost, s));
     LMGPU_HIP(hipStreamSynchronize(s));
     float ms = 0;
     LMGPU_HIP(hipEventElapsedTime(&ms, e0, e1));
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     // root half-area for the SAH normalisation
-    float4 rlo, rhi;
-    if (root_ref >= 0) {
-        LMGPU_HIP(hipMemcpy(&rlo, node_lo.p + root_ref, sizeof(float4), hipMemcpyDeviceToHost));
-        LMGPU_HIP(hipMemcpy(&rhi, node_hi.p + root_ref, sizeof(float4), hipMemcpyDeviceToHost));
-    } else {
-        LMGPU_HIP(hipMemcpy(&rlo, leaf_lo.p, sizeof(float4), hipMemcpyDeviceToHost));
-        LMGPU_HIP(hipMemcpy(&rhi, leaf_hi.p, sizeof(float4), hipMemcpyDeviceToHost));
-    }
+    const float4 rlo = h.root_lo, rhi = h.root_hi;
     const double ra = double(rhi.x - rlo.x) * (rhi.y - rlo.y) + double(rhi.y - rlo.y) * (rhi.z - rlo.z) +
                       double(rhi.z - rlo.z) * (rhi.x - rlo.x);
-    num_nodes = fin[2];
-    num_leaves = fin[3];
+    num_leaves = h.leaves;
     depth = levels;
-    sah_cost = ra > 0 ? 1.0 + sah_sum / ra : 1.0;
+    sah_cost = ra > 0 ? 1.0 + h.sah / ra : 1.0;
     build_ms = ms;
     root_lo[0] = rlo.x; root_lo[1] = rlo.y; root_lo[2] = rlo.z;
     root_hi[0] = rhi.x; root_hi[1] = rhi.y; root_hi[2] = rhi.z;
@@ -829,10 +962,10 @@ bool quantised_width(int width) {
 int quantise_nodes(int width, const float4* wnodes, float4* qnodes, int64_t n, hipStream_t s) {
     if (n <= 0) return LMGPU_OK;
     if (width == 4)
-        hipLaunchKernelGGL(k_quantise<4>, dim3(nblocks(n, 256)), dim3(256), 0, s,
+        hipLaunchKernelGGL(k_quantise<4>, dim3(nblocks(n, 64)), dim3(256), 0, s,
                            reinterpret_cast<const WNode<4>*>(wnodes), reinterpret_cast<QNode<4>*>(qnodes), n);
     else if (width == 8)
-        hipLaunchKernelGGL(k_quantise<8>, dim3(nblocks(n, 256)), dim3(256), 0, s,
+        hipLaunchKernelGGL(k_quantise<8>, dim3(nblocks(n, 64)), dim3(256), 0, s,
                            reinterpret_cast<const WNode<8>*>(wnodes), reinterpret_cast<QNode<8>*>(qnodes), n);
     else
         return fail(LMGPU_ERR_INVALID_ARGUMENT, "quantised nodes are 4- or 8-wide");

@@ -304,68 +304,88 @@ LMGPU_HD void child_keys(const QNode<W>& nd, const RayPre& r, float tmin, float 
     }
 }
 
-// Quantises a built W-wide node: per axis the grid starts at the smallest
-// child plane, with the smallest power-of-two step that spans the node in
-// 255 steps; each plane is rounded outward in the exact FP32 expression the
-// traversal decodes (qplane), so every decoded box contains the original.
+// One axis of a quantised node: grid origin, exponent of the step, and the
+// children's lower and upper planes (bytes).
+template <int W>
+struct QAxis {
+    float org;
+    int e;
+    uint32_t ql[W / 4], qh[W / 4];
+};
+
+// Quantises the children's bounds on one axis (bit c of `present`: slot c holds
+// a child): the grid starts at the smallest child plane, with the smallest
+// power-of-two step that spans the node in 255 steps; each plane is rounded
+// outward in the exact FP32 expression the traversal decodes (qplane), so every
+// decoded box contains the original.
+template <int W>
+LMGPU_HD QAxis<W> quantise_axis(const float (&lo)[W], const float (&hi)[W], uint32_t present) {
+    QAxis<W> q{};
+    float mn = __builtin_inff(), mx = -__builtin_inff();
+    for (int c = 0; c < W; c++)
+        if (present >> c & 1u) {
+            mn = std::min(mn, lo[c]);
+            mx = std::max(mx, hi[c]);
+        }
+    if (!(mn <= mx)) mn = mx = 0.f;   // no child (not produced by the builder)
+    q.org = mn;
+    // smallest e with fma(255, 2^e, mn) >= mx; steps of at least 2^-126.
+    // Start from ceil(log2(span / 255)), read off the binary exponent:
+    // x = m 2^k with m in [0.5, 1) gives ceil(log2 x) = k, or k - 1 when
+    // m = 0.5 exactly.
+    int e = -126;
+    const double span = double(mx) - double(mn);
+    if (span > 0.0) {
+        int k = 0;
+        const double m = std::frexp(span / 255.0, &k);
+        e = std::max(-126, m == 0.5 ? k - 1 : k);
+    }
+    while (e < 127 && std::fma(255.f, std::ldexp(1.f, e), mn) < mx) e++;
+    q.e = e;
+    const float step = std::ldexp(1.f, e);
+    for (int c = 0; c < W; c++) {
+        int l = 255, h = 0;   // an empty slot: no ray lies above plane 255 and below plane 0
+        if (present >> c & 1u) {
+            // division by the power-of-two step is an exact scaling
+            l = int(std::floor(std::ldexp(double(lo[c]) - double(mn), -e)));
+            l = std::min(std::max(l, 0), 255);
+            while (l > 0 && std::fma(float(l), step, mn) > lo[c]) l--;
+            h = int(std::ceil(std::ldexp(double(hi[c]) - double(mn), -e)));
+            h = std::min(std::max(h, 0), 255);
+            while (h < 255 && std::fma(float(h), step, mn) < hi[c]) h++;
+        }
+        q.ql[c >> 2] |= uint32_t(l) << (8 * (c & 3));
+        q.qh[c >> 2] |= uint32_t(h) << (8 * (c & 3));
+    }
+    return q;
+}
+
+// Stack entry of a wide node's child (WNode::child, WNode::count).
+LMGPU_HD int32_t quantised_entry(int32_t child, int32_t count) {
+    return count < 0 ? kQEmpty : (count == 0 ? child : encode_leaf(child, count));
+}
+
+// A whole quantised node.
 template <int W>
 LMGPU_HD QNode<W> quantise_node(const WNode<W>& n) {
     QNode<W> q;
-    const float* lo[3] = {n.lox, n.loy, n.loz};
-    const float* hi[3] = {n.hix, n.hiy, n.hiz};
-    float org[3];
-    uint32_t ebits = 0, esigned = 0;
+    uint32_t present = 0;
+    for (int c = 0; c < W; c++) present |= n.count[c] >= 0 ? 1u << c : 0u;
+    const QAxis<W> x[3] = {quantise_axis<W>(n.lox, n.hix, present), quantise_axis<W>(n.loy, n.hiy, present),
+                           quantise_axis<W>(n.loz, n.hiz, present)};
+    q.ox = x[0].org;
+    q.oy = x[1].org;
+    q.oz = x[2].org;
+    q.e = q.es = 0;
     for (int a = 0; a < 3; a++) {
-        float mn = __builtin_inff(), mx = -__builtin_inff();
-        for (int c = 0; c < W; c++)
-            if (n.count[c] >= 0) {
-                mn = std::min(mn, lo[a][c]);
-                mx = std::max(mx, hi[a][c]);
-            }
-        if (!(mn <= mx)) mn = mx = 0.f;   // no child (not produced by the builder)
-        org[a] = mn;
-        // smallest e with fma(255, 2^e, mn) >= mx; steps of at least 2^-126.
-        // Start from ceil(log2(span / 255)), read off the binary exponent:
-        // x = m 2^k with m in [0.5, 1) gives ceil(log2 x) = k, or k - 1 when
-        // m = 0.5 exactly.
-        int e = -126;
-        const double span = double(mx) - double(mn);
-        if (span > 0.0) {
-            int k = 0;
-            const double m = std::frexp(span / 255.0, &k);
-            e = std::max(-126, m == 0.5 ? k - 1 : k);
-        }
-        while (e < 127 && std::fma(255.f, std::ldexp(1.f, e), mn) < mx) e++;
-        ebits |= uint32_t(e + 127) << (8 * a);
-        esigned |= uint32_t(e & 0xff) << (8 * a);
-        uint32_t ql[W / 4] = {}, qh[W / 4] = {};
-        const float step = std::ldexp(1.f, e);
-        for (int c = 0; c < W; c++) {
-            int l = 255, h = 0;   // an empty slot: no ray lies above plane 255 and below plane 0
-            if (n.count[c] >= 0) {
-                // division by the power-of-two step is an exact scaling
-                l = int(std::floor(std::ldexp(double(lo[a][c]) - double(mn), -e)));
-                l = std::min(std::max(l, 0), 255);
-                while (l > 0 && std::fma(float(l), step, mn) > lo[a][c]) l--;
-                h = int(std::ceil(std::ldexp(double(hi[a][c]) - double(mn), -e)));
-                h = std::min(std::max(h, 0), 255);
-                while (h < 255 && std::fma(float(h), step, mn) < hi[a][c]) h++;
-            }
-            ql[c >> 2] |= uint32_t(l) << (8 * (c & 3));
-            qh[c >> 2] |= uint32_t(h) << (8 * (c & 3));
-        }
+        q.e |= uint32_t(x[a].e + 127) << (8 * a);
+        q.es |= uint32_t(x[a].e & 0xff) << (8 * a);
         for (int k = 0; k < W / 4; k++) {
-            q.qlo[a][k] = ql[k];
-            q.qhi[a][k] = qh[k];
+            q.qlo[a][k] = x[a].ql[k];
+            q.qhi[a][k] = x[a].qh[k];
         }
     }
-    q.ox = org[0];
-    q.oy = org[1];
-    q.oz = org[2];
-    q.e = ebits;
-    q.es = esigned;
-    for (int c = 0; c < W; c++)
-        q.ent[c] = n.count[c] < 0 ? kQEmpty : (n.count[c] == 0 ? n.child[c] : encode_leaf(n.child[c], n.count[c]));
+    for (int c = 0; c < W; c++) q.ent[c] = quantised_entry(n.child[c], n.count[c]);
     return q;
 }
 

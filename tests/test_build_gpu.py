@@ -1,0 +1,83 @@
+"""Device BVH build: the refit's blocks, the collapse's levels and the
+quantised copy at the edges of their tiles (csrc/accel.hip)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+SPAN = 1024   # leaves per refit block (kRefitSpan)
+
+
+def _mesh(n, kind):
+    rng = np.random.default_rng(n)
+    c = rng.random((n, 1, 3)) * 10
+    v = (c + (rng.random((n, 3, 3)) - 0.5) * (10 / n ** (1 / 3))).astype(np.float32).reshape(n, 9)
+    if kind == 'equal':      # one Morton code for half of them: long chains of ties
+        v[: n // 2] = v[0]
+    elif kind == 'line':     # deep, uneven trees
+        v = np.float32(v * 0.01 + np.exp2(-30 * rng.random((n, 1))))
+    return np.ascontiguousarray(v, np.float32)
+
+
+def _arrays(blob, width):
+    b = np.frombuffer(blob, np.uint8)
+    nt, nn, leaves = np.frombuffer(b[24:48].tobytes(), np.int64)
+    nodes = b[128:128 + nn * 32 * width].view(np.float32).reshape(nn, 8, width)
+    tris = b[128 + nn * 32 * width:].view(np.float32).reshape(nt, 3, 4)
+    return nodes, tris, int(leaves)
+
+
+@pytest.mark.parametrize('n,kind', [(1, ''), (2, ''), (SPAN - 1, ''), (SPAN, ''), (SPAN + 1, ''), (SPAN + 2, 'equal'),
+                                    (2 * SPAN + 1, 'line'), (5 * SPAN, 'equal'), (40 * SPAN + 3, ''),
+                                    (70 * SPAN + 511, 'line')])
+@pytest.mark.parametrize('width,collapse,builder', [(2, 0, 1), (4, 0, 1), (8, 0, 1), (4, 1, 1), (8, 0, 0)])
+def test_built_bounds_and_counts(n, kind, width, collapse, builder):
+    """Every child box is the exact FP32 bound of the triangles below it (a
+    minimum and a maximum round nothing: no tolerance), every triangle is in
+    one leaf, and the counts and the depth are those of the tree."""
+    from lm_amd.accel import Accel
+    verts = _mesh(n, kind)
+    acc = Accel(width, collapse=collapse, builder=builder)
+    acc.build(verts)
+    info = acc.info()
+    nodes, tris, leaves = _arrays(acc.serialize(), width)
+    child = nodes[:, 6].view(np.int32)
+    count = nodes[:, 7].view(np.int32)
+    order = tris[:, 0, 3].copy().view(np.int32)
+    assert np.array_equal(np.sort(order), np.arange(n))
+    assert np.array_equal(tris[:, :, :3].reshape(n, 9), verts[order])
+    assert len(nodes) == info['num_nodes'] and leaves == info['num_leaves'] == int((count > 0).sum())
+    lo, hi = tris[:, :, :3].min(1), tris[:, :, :3].max(1)
+    seen = np.zeros(n, np.int32)
+    box = np.empty((len(nodes), 2, 3), np.float32)
+    levels = [np.zeros(1, np.int64)]
+    while True:
+        below = child[levels[-1]][count[levels[-1]] == 0].astype(np.int64)
+        if len(below) == 0:
+            break
+        levels.append(below)
+    assert len(levels) == info['depth']
+    assert np.array_equal(np.sort(np.concatenate(levels)), np.arange(len(nodes)))
+    for level in reversed(levels):
+        for i in level:
+            for c in range(width):
+                if count[i, c] < 0:
+                    continue
+                if count[i, c] > 0:
+                    s = slice(child[i, c], child[i, c] + count[i, c])
+                    seen[s] += 1
+                    want = np.stack([lo[s].min(0), hi[s].max(0)])
+                else:
+                    want = box[child[i, c]]
+                got = np.stack([nodes[i, :3, c], nodes[i, 3:6, c]])
+                assert np.array_equal(got, want), (i, c)
+            used = count[i] >= 0
+            box[i] = np.stack([nodes[i, :3][:, used].min(1), nodes[i, 3:6][:, used].max(1)])
+    assert (seen == 1).all()
+    # the same triangles again, and half of them, into the same object
+    acc.build(verts)
+    assert acc.info()['num_nodes'] == len(nodes)
+    half = max(1, n // 2)
+    acc.build(verts[:half])
+    assert acc.info()['num_tris'] == half
+    assert np.array_equal(np.sort(_arrays(acc.serialize(), width)[1][:, 0, 3].copy().view(np.int32)), np.arange(half))
