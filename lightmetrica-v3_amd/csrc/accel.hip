@@ -783,6 +783,20 @@ static void launch_collapse(bool by_sah, const CollapseArgs& a, unsigned grid, h
     else hipLaunchKernelGGL(k_collapse<W>, dim3(grid), dim3(256), 0, s, a);
 }
 
+// A buffer kept from the last build serves one of a similar size (it may be up
+// to twice what is needed), so that a mesh rebuilt every frame allocates
+// nothing: hipMalloc and hipFree of the arrays of 1.3M triangles took 5.5 of a
+// rebuild's 7.5 ms.
+template <class T>
+static bool fits(const DevBuf<T>& b, size_t count) {
+    return b.p && b.n >= count && b.n / 2 <= count;
+}
+
+template <class T>
+static int reserve(DevBuf<T>& b, size_t count) {
+    return fits(b, count) ? LMGPU_OK : b.alloc(count);
+}
+
 int Accel::build(const float* verts_in, int64_t n, bool on_device, const lmgpu_build_opts* opts, hipStream_t s) {
     int W = opts && opts->width ? opts->width : 4;
     int leaf = opts && opts->leaf_size ? opts->leaf_size : kDefaultLeafSize;
@@ -802,66 +816,90 @@ int Accel::build(const float* verts_in, int64_t n, bool on_device, const lmgpu_b
     if (n <= 0) return fail(LMGPU_ERR_INVALID_ARGUMENT, "accel build needs at least one triangle");
     if (n >= (int64_t(1) << 27)) return fail(LMGPU_ERR_INVALID_ARGUMENT, "too many triangles (max 2^27)");
     if (!verts_in) return fail(LMGPU_ERR_INVALID_ARGUMENT, "verts is NULL");
-    release();
+    // A rebuild writes over the tree (and the workspace) of the last one:
+    // queries still in flight, on whichever stream, come first.
+    const bool rebuild = built;
+    if (nodes.p) LMGPU_HIP(hipDeviceSynchronize());
+    built = false;
+    if (!fits(tris, n)) tris.reset();
+    if (!fits(nodes, size_t(n) * 2 * W)) nodes.reset();
     width = W;
     leaf_size = leaf;
     refill = rf;
     num_tris = n;
-    DevBuf<float> dverts;
+    struct GiveBack {
+        DevBuf<char>& w;
+        bool keep;
+        ~GiveBack() {
+            if (!keep) w.reset();
+        }
+    } give_back{work, false};   // also when the build fails
+    // temporary arrays: one allocation, laid out by the first pass over take()
+    const int64_t m = std::max<int64_t>(n - 1, 1);   // binary internal nodes
+    const unsigned nb_prep = nblocks(n, 256);
+    const size_t sort_bytes = radix_sort_temp_bytes(n);
+    const bool sah = collapse == LMGPU_COLLAPSE_SAH;
+    float4 *tlo, *thi, *leaf_lo, *leaf_hi, *node_lo, *node_hi;
+    float *cb, *partial, *dverts;
+    uint64_t *keys, *keys2;
+    int32_t *vals, *vals2, *parent_int, *parent_leaf, *flags, *q0, *q1, *perm;
+    BNode* bn;
+    BuildHead* head;
+    char* sort_temp;
+    SahDP dp{nullptr, nullptr, leaf, ctri};
+    for (int pass = 0; pass < 2; pass++) {
+        size_t used = 0;
+        auto take = [&](auto*& ptr, size_t count) {
+            ptr = pass ? reinterpret_cast<std::remove_reference_t<decltype(ptr)>>(work.p + used) : nullptr;
+            used += (count * sizeof(*ptr) + 255) & ~size_t(255);
+        };
+        take(tlo, n); take(thi, n);
+        take(leaf_lo, n); take(leaf_hi, n);
+        take(node_lo, m); take(node_hi, m);
+        take(cb, 6);
+        take(partial, size_t(nb_prep) * 6);
+        take(keys, n); take(keys2, n);
+        take(vals, n); take(vals2, n);
+        take(parent_int, m);
+        take(parent_leaf, n);
+        take(flags, m);
+        take(head, 1);
+        take(bn, m);
+        take(q0, n); take(q1, n);
+        take(sort_temp, sort_bytes);
+        take(perm, builder == LMGPU_BUILDER_PLOC ? n : 0);
+        take(dverts, on_device ? 0 : size_t(n) * 9);
+        take(dp.cost, sah ? size_t(m) * W : 0);
+        take(dp.choice, sah ? size_t(m) * W : 0);
+        if (pass == 0) LMGPU_TRY(reserve(work, used));
+    }
+    if (!sah) {
+        dp.cost = nullptr;
+        dp.choice = nullptr;
+    }
     const float* verts = verts_in;
     if (!on_device) {
-        LMGPU_TRY(dverts.alloc(size_t(n) * 9));
-        LMGPU_HIP(hipMemcpyAsync(dverts.p, verts_in, sizeof(float) * 9 * n, hipMemcpyHostToDevice, s));
-        verts = dverts.p;
+        LMGPU_HIP(hipMemcpyAsync(dverts, verts_in, sizeof(float) * 9 * n, hipMemcpyHostToDevice, s));
+        verts = dverts;
     }
     hipEvent_t e0, e1;
     LMGPU_HIP(hipEventCreate(&e0));
     LMGPU_HIP(hipEventCreate(&e1));
     LMGPU_HIP(hipEventRecord(e0, s));
 
-    const int64_t m = std::max<int64_t>(n - 1, 1);   // binary internal nodes
-    DevBuf<float4> tlo, thi, leaf_lo, leaf_hi, node_lo, node_hi;
-    DevBuf<float> cb, partial, dp_cost;
-    DevBuf<uint8_t> dp_choice;
-    DevBuf<uint64_t> keys, keys2;
-    DevBuf<int32_t> vals, vals2, parent_int, parent_leaf, flags, q0, q1;
-    DevBuf<BNode> bn;
-    DevBuf<BuildHead> head;
-    LMGPU_TRY(tlo.alloc(n)); LMGPU_TRY(thi.alloc(n));
-    LMGPU_TRY(leaf_lo.alloc(n)); LMGPU_TRY(leaf_hi.alloc(n));
-    LMGPU_TRY(node_lo.alloc(m)); LMGPU_TRY(node_hi.alloc(m));
-    LMGPU_TRY(cb.alloc(6));
-    const unsigned nb_prep = nblocks(n, 256);
-    LMGPU_TRY(partial.alloc(size_t(nb_prep) * 6));
-    LMGPU_TRY(keys.alloc(n)); LMGPU_TRY(keys2.alloc(n));
-    LMGPU_TRY(vals.alloc(n)); LMGPU_TRY(vals2.alloc(n));
-    LMGPU_TRY(parent_int.alloc(m));
-    LMGPU_TRY(parent_leaf.alloc(n));
-    LMGPU_TRY(flags.alloc(m));
-    LMGPU_TRY(head.alloc(1));
-    LMGPU_TRY(bn.alloc(m));
-    LMGPU_TRY(q0.alloc(n)); LMGPU_TRY(q1.alloc(n));
-    SahDP dp{nullptr, nullptr, leaf, ctri};
-    if (collapse == LMGPU_COLLAPSE_SAH) {
-        LMGPU_TRY(dp_cost.alloc(size_t(m) * W));
-        LMGPU_TRY(dp_choice.alloc(size_t(m) * W));
-        dp.cost = dp_cost.p;
-        dp.choice = dp_choice.p;
-    }
-
-    LMGPU_HIP(hipMemsetAsync(head.p, 0, sizeof(BuildHead), s));
-    hipLaunchKernelGGL(k_prep, dim3(nb_prep), dim3(256), 0, s, verts, n, tlo.p, thi.p, partial.p);
-    hipLaunchKernelGGL(k_reduce_bounds, dim3(1), dim3(256), 0, s, partial.p, int(nb_prep), cb.p);
-    hipLaunchKernelGGL(k_morton, dim3(nblocks(n, 256)), dim3(256), 0, s, tlo.p, thi.p, n, cb.p, keys.p, vals.p);
+    LMGPU_HIP(hipMemsetAsync(head, 0, sizeof(BuildHead), s));
+    hipLaunchKernelGGL(k_prep, dim3(nb_prep), dim3(256), 0, s, verts, n, tlo, thi, partial);
+    hipLaunchKernelGGL(k_reduce_bounds, dim3(1), dim3(256), 0, s, partial, int(nb_prep), cb);
+    hipLaunchKernelGGL(k_morton, dim3(nblocks(n, 256)), dim3(256), 0, s, tlo, thi, n, cb, keys, vals);
     bool in_alt = false;
-    LMGPU_TRY(radix_sort_pairs_u64(keys.p, vals.p, keys2.p, vals2.p, n, 63, &in_alt, s));
-    const uint64_t* skeys = in_alt ? keys2.p : keys.p;
-    const int32_t* svals = in_alt ? vals2.p : vals.p;
+    LMGPU_TRY(radix_sort_pairs_u64(keys, vals, keys2, vals2, n, 63, &in_alt, sort_temp, s));
+    const uint64_t* skeys = in_alt ? keys2 : keys;
+    const int32_t* svals = in_alt ? vals2 : vals;
     if (n > 1) {
         // the sort's result must be ordered before the tree is built on it
-        hipLaunchKernelGGL(k_check_sorted, dim3(nblocks(n - 1, 256)), dim3(256), 0, s, skeys, n, &head.p->unsorted);
+        hipLaunchKernelGGL(k_check_sorted, dim3(nblocks(n - 1, 256)), dim3(256), 0, s, skeys, n, &head->unsorted);
         int32_t unsorted = 0;
-        LMGPU_HIP(hipMemcpyAsync(&unsorted, &head.p->unsorted, sizeof(int32_t), hipMemcpyDeviceToHost, s));
+        LMGPU_HIP(hipMemcpyAsync(&unsorted, &head->unsorted, sizeof(int32_t), hipMemcpyDeviceToHost, s));
         LMGPU_HIP(hipStreamSynchronize(s));
         if (unsorted) return fail(LMGPU_ERR_DEVICE, "Morton sort produced an unordered key array");
     }
@@ -869,28 +907,26 @@ int Accel::build(const float* verts_in, int64_t n, bool on_device, const lmgpu_b
     // (traversal position -> triangle)
     int32_t root_ref = n > 1 ? 0 : ~0;
     const int32_t* order = svals;
-    DevBuf<int32_t> perm;
-    if (n > 1) LMGPU_HIP(hipMemsetAsync(parent_int.p, 0xff, sizeof(int32_t) * (n - 1), s));
+    if (n > 1) LMGPU_HIP(hipMemsetAsync(parent_int, 0xff, sizeof(int32_t) * (n - 1), s));
     if (builder == LMGPU_BUILDER_PLOC) {
-        LMGPU_TRY(perm.alloc(n));
-        LMGPU_TRY(build_ploc(n, svals, tlo.p, thi.p, radius, bn.p, node_lo.p, node_hi.p, leaf_lo.p, leaf_hi.p,
-                             perm.p, &root_ref, s));
-        order = perm.p;
+        LMGPU_TRY(build_ploc(n, svals, tlo, thi, radius, bn, node_lo, node_hi, leaf_lo, leaf_hi,
+                             perm, &root_ref, s));
+        order = perm;
         if (n > 1)
-            hipLaunchKernelGGL(k_parents, dim3(nblocks(n - 1, 256)), dim3(256), 0, s, bn.p, n - 1, parent_int.p,
-                               parent_leaf.p);
+            hipLaunchKernelGGL(k_parents, dim3(nblocks(n - 1, 256)), dim3(256), 0, s, bn, n - 1, parent_int,
+                               parent_leaf);
     } else if (n > 1) {
-        hipLaunchKernelGGL(k_lbvh, dim3(nblocks(n - 1, 256)), dim3(256), 0, s, skeys, n, bn.p, parent_int.p,
-                           parent_leaf.p);
+        hipLaunchKernelGGL(k_lbvh, dim3(nblocks(n - 1, 256)), dim3(256), 0, s, skeys, n, bn, parent_int,
+                           parent_leaf);
     }
     // refit (bounds, and the SAH cost tables when collapsing by SAH); q0 and
     // q1 hold the nodes left to its second kernel
-    if (n > 1) LMGPU_HIP(hipMemsetAsync(flags.p, 0, sizeof(int32_t) * (n - 1), s));
-    const Refit refit{bn.p, parent_int.p, parent_leaf.p, leaf_lo.p, leaf_hi.p, node_lo.p, node_hi.p, flags.p, root_ref,
-                      dp, head.p};
-    LMGPU_TRY(tris.alloc(n));
-    auto* list0 = reinterpret_cast<RefitItem*>(q0.p);
-    auto* list1 = reinterpret_cast<RefitItem*>(q1.p);
+    if (n > 1) LMGPU_HIP(hipMemsetAsync(flags, 0, sizeof(int32_t) * (n - 1), s));
+    const Refit refit{bn, parent_int, parent_leaf, leaf_lo, leaf_hi, node_lo, node_hi, flags, root_ref,
+                      dp, head};
+    LMGPU_TRY(reserve(tris, n));
+    auto* list0 = reinterpret_cast<RefitItem*>(q0);
+    auto* list1 = reinterpret_cast<RefitItem*>(q1);
     if (W == 2) launch_refit<2>(n, order, verts, tris.p, refit, list0, list1, s);
     else if (W == 4) launch_refit<4>(n, order, verts, tris.p, refit, list0, list1, s);
     else launch_refit<8>(n, order, verts, tris.p, refit, list0, list1, s);
@@ -898,9 +934,9 @@ int Accel::build(const float* verts_in, int64_t n, bool on_device, const lmgpu_b
     // collapse, level by level
     const size_t node_bytes = size_t(32) * W;
     const int64_t max_nodes = std::max<int64_t>(n, 1);
-    LMGPU_TRY(nodes.alloc(size_t(max_nodes) * node_bytes / sizeof(float4)));
-    hipLaunchKernelGGL(k_collapse_init, dim3(1), dim3(1), 0, s, head.p, q0.p, root_ref);
-    CollapseArgs ca{q0.p, q1.p, 0, bn.p, node_lo.p, node_hi.p, leaf_lo.p, leaf_hi.p, dp.choice, leaf, nodes.p, head.p};
+    LMGPU_TRY(reserve(nodes, size_t(max_nodes) * node_bytes / sizeof(float4)));
+    hipLaunchKernelGGL(k_collapse_init, dim3(1), dim3(1), 0, s, head, q0, root_ref);
+    CollapseArgs ca{q0, q1, 0, bn, node_lo, node_hi, leaf_lo, leaf_hi, dp.choice, leaf, nodes.p, head};
     // Levels are launched kCollapseLevelsPerSync at a time, each reading its
     // own size; their grids cover what the last size read can have become.
     int64_t bound = 1;
@@ -911,17 +947,16 @@ int Accel::build(const float* verts_in, int64_t n, bool on_device, const lmgpu_b
         const int at = ca.level;
         for (int l = 0; l < kCollapseLevelsPerSync; l++) {
             const unsigned grid = std::min(nblocks(bound, 256), kCollapseMaxBlocks);
-            const bool by_sah = collapse == LMGPU_COLLAPSE_SAH;
-            if (W == 2) launch_collapse<2>(by_sah, ca, grid, s);
-            else if (W == 4) launch_collapse<4>(by_sah, ca, grid, s);
-            else launch_collapse<8>(by_sah, ca, grid, s);
+            if (W == 2) launch_collapse<2>(sah, ca, grid, s);
+            else if (W == 4) launch_collapse<4>(sah, ca, grid, s);
+            else launch_collapse<8>(sah, ca, grid, s);
             bound = std::min<int64_t>(bound * W, n);
             ca.level++;
             ca.out = const_cast<int32_t*>(ca.in);
-            ca.in = ca.in == q0.p ? q1.p : q0.p;
+            ca.in = ca.in == q0 ? q1 : q0;
         }
         int32_t sizes[kCollapseLevelsPerSync + 1];
-        LMGPU_HIP(hipMemcpyAsync(sizes, head.p->count + at, sizeof(sizes), hipMemcpyDeviceToHost, s));
+        LMGPU_HIP(hipMemcpyAsync(sizes, head->count + at, sizeof(sizes), hipMemcpyDeviceToHost, s));
         LMGPU_HIP(hipStreamSynchronize(s));
         for (int l = 0; l < kCollapseLevelsPerSync && sizes[l] > 0; l++) {
             num_nodes += sizes[l];
@@ -932,7 +967,7 @@ int Accel::build(const float* verts_in, int64_t n, bool on_device, const lmgpu_b
     }
     LMGPU_HIP(hipEventRecord(e1, s));
     BuildHead h;   // its counters; the level sizes are known
-    LMGPU_HIP(hipMemcpyAsync(&h, head.p, offsetof(BuildHead, count), hipMemcpyDeviceToHost, s));
+    LMGPU_HIP(hipMemcpyAsync(&h, head, offsetof(BuildHead, count), hipMemcpyDeviceToHost, s));
     LMGPU_HIP(hipStreamSynchronize(s));
     float ms = 0;
     LMGPU_HIP(hipEventElapsedTime(&ms, e0, e1));
@@ -950,6 +985,7 @@ int Accel::build(const float* verts_in, int64_t n, bool on_device, const lmgpu_b
     root_hi[0] = rhi.x; root_hi[1] = rhi.y; root_hi[2] = rhi.z;
     LMGPU_TRY(make_trav_nodes(s));
     LMGPU_HIP(hipGetLastError());
+    give_back.keep = rebuild;
     built = true;
     return LMGPU_OK;
 }
@@ -974,9 +1010,11 @@ int quantise_nodes(int width, const float4* wnodes, float4* qnodes, int64_t n, h
 }
 
 int Accel::make_trav_nodes(hipStream_t s) {
-    qnodes.reset();
-    if (!quantised_width(width)) return LMGPU_OK;
-    LMGPU_TRY(qnodes.alloc(size_t(num_nodes) * (size_t(width) * 16 / sizeof(float4))));
+    if (!quantised_width(width)) {
+        qnodes.reset();
+        return LMGPU_OK;
+    }
+    LMGPU_TRY(reserve(qnodes, size_t(num_nodes) * width));
     LMGPU_TRY(quantise_nodes(width, nodes.p, qnodes.p, num_nodes, s));
     LMGPU_HIP(hipStreamSynchronize(s));
     return LMGPU_OK;

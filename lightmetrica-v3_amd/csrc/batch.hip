@@ -637,7 +637,7 @@ int Batch::build_arena(int width, int leaf, hipStream_t s) {
             cleanup();
             return fail(rc, "job " + std::to_string(j) + ": " + lmgpu_last_error());
         }
-        Part p{{sc->accel.num_nodes, int64_t(sc->accel.tris.n), int64_t(sc->stri.n), int64_t(sc->mats.n),
+        Part p{{sc->accel.num_nodes, sc->accel.num_tris, int64_t(sc->stri.n), int64_t(sc->mats.n),
                 int64_t(sc->lights.n), int64_t(sc->light_cdf.n), int64_t(sc->light_tri.n), int64_t(sc->uvs.n),
                 int64_t(sc->texels.n), int64_t(sc->tex_info.n)}};
         parts.push_back(p);

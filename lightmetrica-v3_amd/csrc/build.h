@@ -17,9 +17,11 @@ struct BNode {
 // Stable LSD radix sort of n (key, value) pairs by the low `key_bits` bits
 // of the keys (8-bit digits), ping-ponging between (keys, vals) and
 // (keys_alt, vals_alt); *in_alt tells which pair holds the result.
-// Synchronizes s before returning (its temporary buffers are freed).
+// Enqueued on s, with a caller-owned temporary buffer of
+// radix_sort_temp_bytes(n).
+size_t radix_sort_temp_bytes(int64_t n);
 int radix_sort_pairs_u64(uint64_t* keys, int32_t* vals, uint64_t* keys_alt, int32_t* vals_alt, int64_t n,
-                         int key_bits, bool* in_alt, hipStream_t s);
+                         int key_bits, bool* in_alt, void* temp, hipStream_t s);
 
 // Exclusive prefix sum of n uint64 values (in == out allowed), enqueued on s,
 // with a caller-owned temporary buffer of exclusive_scan_u64_temp_bytes(n).

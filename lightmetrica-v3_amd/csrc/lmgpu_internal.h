@@ -81,9 +81,14 @@ bool quantised_width(int width);
 int quantise_nodes(int width, const float4* wnodes, float4* qnodes, int64_t n, hipStream_t s);
 
 struct Accel {
+    // The arrays may be longer than what they hold (num_nodes, num_tris).
     DevBuf<float4> nodes;   // W-wide nodes, 32*W bytes each
     DevBuf<float4> qnodes;  // quantised copy of the nodes (QNode<width>), when quantised_width(width)
     DevBuf<TriV> tris;      // triangles in traversal order
+    // Temporary arrays of the build. Given back when the first build of an
+    // object ends; an object that is built again is taken to be rebuilt every
+    // frame and keeps them (some 200 B a triangle) until it is released.
+    DevBuf<char> work;
     DevBuf<int32_t> status; // bit 0: traversal stack overflow
     DevBuf<unsigned long long> ring;  // per-launch ray counters of the persistent kernel
     mutable std::atomic<uint32_t> ring_pos{0};
@@ -108,6 +113,7 @@ struct Accel {
         nodes.reset();
         qnodes.reset();
         tris.reset();
+        work.reset();
         built = false;
     }
     int32_t* status_dev() const {

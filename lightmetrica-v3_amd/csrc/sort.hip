@@ -254,30 +254,29 @@ int exclusive_scan_u64(const uint64_t* in, uint64_t* out, int64_t n, void* temp,
     return LMGPU_OK;
 }
 
+size_t radix_sort_temp_bytes(int64_t n) { return (size_t(tiles(n)) + 1) * kRadix * sizeof(uint32_t); }
+
 int radix_sort_pairs_u64(uint64_t* keys, int32_t* vals, uint64_t* keys_alt, int32_t* vals_alt, int64_t n,
-                         int key_bits, bool* in_alt, hipStream_t s) {
+                         int key_bits, bool* in_alt, void* temp, hipStream_t s) {
     *in_alt = false;
     if (n <= 1) return LMGPU_OK;
     if (int64_t(tiles(n)) * kRadix >= (int64_t(1) << 31) || n >= (int64_t(1) << 32))
         return fail(LMGPU_ERR_INVALID_ARGUMENT, "radix sort: too many keys");
     const unsigned nt = tiles(n);
-    DevBuf<uint32_t> hist, totals;
-    LMGPU_TRY(hist.alloc(size_t(nt) * kRadix));
-    LMGPU_TRY(totals.alloc(kRadix));
+    uint32_t* hist = static_cast<uint32_t*>(temp);
+    uint32_t* totals = hist + size_t(nt) * kRadix;
     uint64_t* kbuf[2] = {keys, keys_alt};
     int32_t* vbuf[2] = {vals, vals_alt};
     int cur = 0;
     for (int shift = 0; shift < key_bits; shift += 8) {
-        hipLaunchKernelGGL(k_sort_upsweep, dim3(nt), dim3(kT), 0, s, kbuf[cur], n, shift, hist.p, nt);
-        hipLaunchKernelGGL(k_sort_scan, dim3(kRadix), dim3(kT), 0, s, hist.p, nt, totals.p);
+        hipLaunchKernelGGL(k_sort_upsweep, dim3(nt), dim3(kT), 0, s, kbuf[cur], n, shift, hist, nt);
+        hipLaunchKernelGGL(k_sort_scan, dim3(kRadix), dim3(kT), 0, s, hist, nt, totals);
         hipLaunchKernelGGL(k_sort_downsweep, dim3(nt), dim3(kT), 0, s, kbuf[cur], vbuf[cur], kbuf[cur ^ 1],
-                           vbuf[cur ^ 1], n, shift, hist.p, totals.p, nt);
+                           vbuf[cur ^ 1], n, shift, hist, totals, nt);
         cur ^= 1;
     }
     LMGPU_HIP(hipGetLastError());
     *in_alt = cur == 1;
-    // hist and totals are freed on return: wait for the passes that read them
-    LMGPU_HIP(hipStreamSynchronize(s));
     return LMGPU_OK;
 }
 
