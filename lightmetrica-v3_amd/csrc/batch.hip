@@ -62,6 +62,10 @@ constexpr int kRegenJobSlots = 64;
 // the run's counters at the end of the block. SINGLE: the run has one job
 // (kernels of a single scene's render read its fields as scalars, with no
 // job index per path), whose work items are its samples' pixels in order.
+// With `samples`, a finished sample is stored under its work item for
+// k_b_resolve instead of added to the film: 3 FP64 atomics a sample, 6 with
+// the squares, run at 26 G/s on the card, which at 16 spp of 1080p was most
+// of the kernel's 7.7 ms (now 4.0, and k_b_resolve 0.24).
 // The kernel also clears the counters of the iteration it opens: the ray
 // counters `next` and the counts of the other extension queue and the shadow
 // queue, which nothing reads until the traversal and shading that follow.
@@ -70,7 +74,8 @@ __global__ __launch_bounds__(BLOCK) void k_b_regen(const JobDev* __restrict__ jo
                                                    int nsegs, int64_t total, PoolDev P, BatchQ q, int in_q, int cap,
                                                    BatchCtl* ctl, unsigned long long* next,
                                                    unsigned long long* job_done, unsigned long long* job_time,
-                                                   double* film_sum, double* film_sq) {
+                                                   double* film_sum, double* film_sq,
+                                                   float4* __restrict__ samples) {
     constexpr int kWaves = BLOCK / 64;
     __shared__ int s_want[kRegenStrides][kWaves];   // slots taking work, then their exclusive prefix
     __shared__ unsigned long long s_base;           // first work item of the block
@@ -160,14 +165,19 @@ __global__ __launch_bounds__(BLOCK) void k_b_regen(const JobDev* __restrict__ jo
                 const int fj = SINGLE ? 0 : P.job[s];
                 const JobDev& J = jobs[fj];
                 const float4 L = P.L[s];
-                const int64_t f = J.film_off + 3 * int64_t(P.pixel[s]);
-                atomicAdd(film_sum + f + 0, double(L.x));
-                atomicAdd(film_sum + f + 1, double(L.y));
-                atomicAdd(film_sum + f + 2, double(L.z));
-                if (film_sq) {
-                    atomicAdd(film_sq + f + 0, double(L.x) * double(L.x));
-                    atomicAdd(film_sq + f + 1, double(L.y) * double(L.y));
-                    atomicAdd(film_sq + f + 2, double(L.z) * double(L.z));
+                if (SINGLE && samples) {
+                    const int64_t sample = int64_t(__float_as_int(L.w)) - segs[0].sample;
+                    samples[sample * J.npix + P.pixel[s]] = L;
+                } else {
+                    const int64_t f = J.film_off + 3 * int64_t(P.pixel[s]);
+                    atomicAdd(film_sum + f + 0, double(L.x));
+                    atomicAdd(film_sum + f + 1, double(L.y));
+                    atomicAdd(film_sum + f + 2, double(L.z));
+                    if (film_sq) {
+                        atomicAdd(film_sq + f + 0, double(L.x) * double(L.x));
+                        atomicAdd(film_sq + f + 1, double(L.y) * double(L.y));
+                        atomicAdd(film_sq + f + 2, double(L.z) * double(L.z));
+                    }
                 }
                 // count the finished sample in the block's job table, or
                 // straight into the job's counter when its entry is taken
@@ -238,6 +248,27 @@ __global__ __launch_bounds__(BLOCK) void k_b_regen(const JobDev* __restrict__ jo
             const unsigned long long c = s_cnt[k];
             if (atomicAdd(job_done + j, c) + c == need) job_time[j] = wall_clock64();
         }
+    }
+}
+
+// The samples of a run, spp records per pixel in sample order, go to the film
+// (one set of atomics a pixel: other renders may add to the same film).
+__global__ __launch_bounds__(256) void k_b_resolve(const float4* __restrict__ samples, int npix, int spp,
+                                                   double* film_sum, double* film_sq) {
+    const int p = blockIdx.x * 256 + threadIdx.x;
+    if (p >= npix) return;
+    double a[3] = {}, b[3] = {};
+    for (int k = 0; k < spp; k++) {
+        const float4 L = samples[int64_t(k) * npix + p];
+        const double v[3] = {double(L.x), double(L.y), double(L.z)};
+        for (int c = 0; c < 3; c++) {
+            a[c] += v[c];
+            b[c] += v[c] * v[c];
+        }
+    }
+    for (int c = 0; c < 3; c++) {
+        atomicAdd(film_sum + 3 * int64_t(p) + c, a[c]);
+        if (film_sq) atomicAdd(film_sq + 3 * int64_t(p) + c, b[c]);
     }
 }
 
@@ -781,7 +812,7 @@ int Wavefront::ensure_guided(int rec_depth, int64_t train_cap) {
 
 int Wavefront::run(const void* trav_nodes, const TriV* tris, int width, int block, bool single, int64_t total, int max_verts,
                    double* film_sum, double* fsq, double* elapsed, int64_t* iters, hipStream_t s,
-                   const RegenGuide* G) {
+                   const RegenGuide* G, bool resolve) {
     const int nsegs = int(dsegs.n);
     PoolDev P{pjob.p, ppix.p, pstate.p, pL.p};
     BatchQ q{{ext0.p, ext1.p}, {thr0.p, thr1.p}, {prev0.p, prev1.p}, hit.p, sh.p, shc.p, counts.p};
@@ -815,7 +846,8 @@ int Wavefront::run(const void* trav_nodes, const TriV* tris, int width, int bloc
         const unsigned rg = regen_grid(cap, block);
         auto regen = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, dim3(rg), dim3(unsigned(block)), 0, cs, djobs.p, dsegs.p, nsegs, total, P, q, in_q,
-                               cap, ctl.p, next.p, job_done.p, job_time.p, film_sum, fsq);
+                               cap, ctl.p, next.p, job_done.p, job_time.p, film_sum, fsq,
+                               resolve ? psample.p : nullptr);
         };
         auto extend = [&](auto kernel, auto* nd) {
             if (!extend_grid) extend_grid = occupancy_grid(kernel, kBlock);
@@ -1040,9 +1072,28 @@ int Scene::render_regen(const PTConsts& c, int spp, int sample_offset, double* s
     J.seed_lo = c.seed_lo;
     J.seed_hi = c.seed_hi;
     J.film_off = 0;
-    const int64_t total = int64_t(c.npix) * spp;
+    // Finished samples are kept until the run ends and then resolved into the
+    // film. A render of more samples than the buffer holds is split into runs
+    // of about equal numbers of samples per pixel (each ends with the few
+    // iterations in which the pool drains), but not while a guide trains,
+    // which goes on from run to run: its samples are added to the film as
+    // they finish.
+    const bool train = gp && gp->steps > 0;
+    const int64_t hold = std::max<int64_t>(1, LMGPU_REGEN_SAMPLES / c.npix);
+    bool resolve = !train || spp <= hold;
+    const int64_t runs = resolve ? (spp + hold - 1) / hold : 1;
+    int per_run = int((spp + runs - 1) / runs);
+    int64_t total = int64_t(c.npix) * per_run;
+    if (resolve && wf->psample.n < size_t(total) && wf->psample.alloc(size_t(total)) != LMGPU_OK) {
+        // no memory for it: one run that adds to the film
+        (void)hipGetLastError();
+        clear_error();
+        resolve = false;
+        per_run = spp;
+        total = int64_t(c.npix) * spp;
+    }
     // one job: items are its samples' pixels in order from the first sample
-    const std::vector<WorkSeg> segs{WorkSeg{0, 0, sample_offset}};
+    std::vector<WorkSeg> segs{WorkSeg{0, 0, sample_offset}};
     // pool: LMGPU_REGEN_SLOTS_PER_PIXEL paths per pixel (the slots of a
     // sample's short paths take the next sample's pixels)
     const int cap = gp ? Wavefront::pool_size(total, c.npix, LMGPU_REGEN_GUIDED_SLOTS_PER_PIXEL,
@@ -1068,19 +1119,31 @@ int Scene::render_regen(const PTConsts& c, int spp, int sample_offset, double* s
         LMGPU_TRY(wf->ensure_guided(G.rec_depth, int64_t(G.batch) * G.steps));
     }
     const std::vector<JobDev> jobs{J};
-    LMGPU_TRY(wf->set_work(jobs, segs, s));
     const void* tn = accel.width == 4 ? static_cast<const void*>(dev.nodes4)
                      : accel.width == 8 ? static_cast<const void*>(dev.nodes8) : static_cast<const void*>(dev.nodes2);
-    double sec = 0;
-    int64_t iters = 0;
-    LMGPU_TRY(wf->run(tn, accel.tris.p, accel.width, kSingleBlock, true, total, c.max_verts, sum, sumsq, &sec, &iters, s,
-                      gp ? &G : nullptr));
-    *ext_rays = int64_t(wf->last.ctl.ext_rays);
-    *shadow_rays = int64_t(wf->last.ctl.shadow_rays);
-    if (guide_records) {
-        unsigned long long r = 0;
-        if (gp) LMGPU_HIP(hipMemcpy(&r, wf->grecorded.p, sizeof(r), hipMemcpyDeviceToHost));
-        *guide_records = int64_t(r);
+    *ext_rays = *shadow_rays = 0;
+    if (guide_records) *guide_records = 0;
+    for (int done = 0; done < spp; done += per_run) {
+        const int n = std::min(per_run, spp - done);
+        total = int64_t(c.npix) * n;
+        segs[0].sample = sample_offset + done;
+        LMGPU_TRY(wf->set_work(jobs, segs, s));
+        double sec = 0;
+        int64_t iters = 0;
+        LMGPU_TRY(wf->run(tn, accel.tris.p, accel.width, kSingleBlock, true, total, c.max_verts, sum, sumsq, &sec,
+                          &iters, s, gp ? &G : nullptr, resolve));
+        if (resolve) {
+            hipLaunchKernelGGL(k_b_resolve, dim3(nblk(c.npix, 256)), dim3(256), 0, s, wf->psample.p, c.npix, n, sum,
+                               sumsq);
+            LMGPU_HIP(hipGetLastError());
+        }
+        *ext_rays += int64_t(wf->last.ctl.ext_rays);
+        *shadow_rays += int64_t(wf->last.ctl.shadow_rays);
+        if (guide_records && gp) {
+            unsigned long long r = 0;
+            LMGPU_HIP(hipMemcpy(&r, wf->grecorded.p, sizeof(r), hipMemcpyDeviceToHost));
+            *guide_records += int64_t(r);
+        }
     }
     return LMGPU_OK;
 }

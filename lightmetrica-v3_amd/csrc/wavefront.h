@@ -23,6 +23,11 @@
 #ifndef LMGPU_REGEN_MAX_SLOTS
 #define LMGPU_REGEN_MAX_SLOTS (1 << 24)
 #endif
+// Samples a render keeps before they go to the film together: 16 B each, 2 GB
+// at most (64 per pixel at 1080p).
+#ifndef LMGPU_REGEN_SAMPLES
+#define LMGPU_REGEN_SAMPLES (1 << 27)
+#endif
 // Path pool of a guided render, whose slots also hold training records
 // (record_depth x 96 B each): 4 slots per pixel, at most 2^23. With fewer
 // paths in flight an iteration finishes about half a sample per pixel's
@@ -128,6 +133,7 @@ struct Wavefront {
     DevBuf<lmgpu_ray> ext0, ext1, sh;
     DevBuf<lmgpu_hit> hit;
     DevBuf<float4> shc;
+    DevBuf<float4> psample;   // finished samples of a single scene's run, by work item
     DevBuf<BatchCtl> ctl;
     // pinned host copies of the control block and the queue counts, one per
     // parity of the pairs of iterations, with the pairs' events
@@ -169,10 +175,11 @@ struct Wavefront {
     // the one-sample mixture of guide and BSDF, and the guide trains online
     // on the records of finished paths.
     // single: one job, whose work segment 0 starts at its first sample
-    // (kernels specialised for it, at their own block size).
+    // (kernels specialised for it, at their own block size). resolve: its
+    // samples are left in psample, which holds `total`, not added to the film.
     int run(const void* trav_nodes, const TriV* tris, int width, int block, bool single, int64_t total, int max_verts,
             double* film_sum, double* film_sq, double* elapsed, int64_t* iters, hipStream_t s,
-            const RegenGuide* guide = nullptr);
+            const RegenGuide* guide = nullptr, bool resolve = false);
     // The loop itself: frees the pool, sets the run's counters for `total`
     // items and enqueues pairs of iteration(stream, 0) and iteration(stream, 1)
     // (the kernels of one iteration on queue parity 0 / 1), captured as one
