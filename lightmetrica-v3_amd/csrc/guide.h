@@ -290,31 +290,35 @@ __device__ __forceinline__ void dense64(const uint16_t* __restrict__ in, int pin
 // inputs are in lx ([32][kPitchX] bf16), with the weights staged in LDS by
 // stage_weights (wl). Raw outputs land in ly ([32][kPitchY] f32, columns
 // 0..39). `save(layer, e, t, bf16)` sees every hidden activation
-// (layer 1..3) for training. Every wave of the block calls this the same
+// (layer 1..3) for training, and `saved(layer, tile, pitch)` the wave's whole
+// tile of them in LDS. Every wave of the block calls this the same
 // number of times (block barriers between the layers); callers put a block
 // barrier after staging the weights and writing lx, and after this call
 // before reading ly.
-template <class Save>
+template <class Save, class Saved>
 __device__ __forceinline__ void mlp_tile_forward(const uint16_t* wl, const float* __restrict__ P, uint16_t* lx,
-                                                 uint16_t* lh, float* ly, int lane, Save save) {
+                                                 uint16_t* lh, float* ly, int lane, Save save, Saved saved) {
     dense64<kIn, kPW1, kIn / 16>(lx, kPitchX, wl, P + kOffB1, lane, [&](int row, int col, float v, int e, int t) {
         const uint16_t b = f2bf(fmaxf(v, 0.f));
         lh[row * kPitchH + col] = b;
         save(1, e, t, b);
     });
     __syncthreads();
+    saved(1, lh, kPitchH);
     dense64<kHid, kPWh, kHid / 16>(lh, kPitchH, wl + kWOff2, P + kOffB2, lane, [&](int row, int col, float v, int e, int t) {
         const uint16_t b = f2bf(fmaxf(v, 0.f));
         lx[row * kPitchX + col] = b;
         save(2, e, t, b);
     });
     __syncthreads();
+    saved(2, lx, kPitchX);
     dense64<kHid, kPWh, kHid / 16>(lx, kPitchX, wl + kWOff2 + kWOffH, P + kOffB3, lane, [&](int row, int col, float v, int e, int t) {
         const uint16_t b = f2bf(fmaxf(v, 0.f));
         lh[row * kPitchH + col] = b;
         save(3, e, t, b);
     });
     __syncthreads();
+    saved(3, lh, kPitchH);
     dense64<kHid, kPWh, kHid / 16>(lh, kPitchH, wl + kWOff2 + 2 * kWOffH, P + kOffB4, lane,
                            [&](int row, int col, float v, int, int) { ly[row * kPitchY + col] = v; });
 }

@@ -609,7 +609,8 @@ __global__ __launch_bounds__(256) void k_pt_guide_infer(SceneDev sc, Q q, int in
             }
         }
         __syncthreads();
-        mlp_tile_forward(wl, P, lx, lh, ly, lane, [](int, int, int, uint16_t) {});
+        mlp_tile_forward(wl, P, lx, lh, ly, lane, [](int, int, int, uint16_t) {},
+                         [](int, const uint16_t*, int) {});
         __syncthreads();
         {
             const int i = i0 + r;
