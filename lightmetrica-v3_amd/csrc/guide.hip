@@ -35,6 +35,7 @@ namespace {
 #ifndef LMGPU_DW_SLICE
 #define LMGPU_DW_SLICE 1024
 #endif
+static_assert(LMGPU_DW_SLICE % 64 == 0, "k_guide_dw takes 64 rows at a time");
 
 constexpr int kGB = 256;                  // 4 waves x 32 rows per block tile
 constexpr int kRowsPerBlock = 128;
@@ -121,7 +122,7 @@ __global__ __launch_bounds__(256) void k_guide_weights(int64_t n_max, const int3
 // (i / 32) * 32 F + 32 f + i % 32, F features. A wave writes its tile as one
 // run of 64 F bytes and k_guide_dw reads whole lines of it; with whole
 // columns (f B + i) each store put 2 bytes into 64 lines (65536 records:
-// k_guide_train_rows 99 us, now 37; k_guide_dw 27 us, now 23).
+// k_guide_train_rows 99 us, now 37; k_guide_dw 27 us, then 23).
 // Copies features [0, F) of a wave's LDS tile: a lane takes four rows of two
 // features at a time.
 template <int F>
@@ -332,16 +333,25 @@ __global__ __launch_bounds__(64) void k_guide_dw(int64_t n_max, const int32_t* n
     const bool bias = job.kt == 0;
     f32x16 acc = {};
     float bsum = 0.f;
-    for (int64_t i = i_beg; i < i_end; i += 16) {
-        // i is a multiple of 16: the upper or lower half of a tile's 32 rows
-        const int64_t tile = i & ~int64_t(31);
-        const int at = int(i & 31) + 8 * h;
-        const bf16x8 a = *reinterpret_cast<const bf16x8*>(A + tile * kHid + at);
-        const bf16x8 b = *reinterpret_cast<const bf16x8*>(Bm + tile * K + at);
-        acc = mfma_bf16(a, b, acc);
-        if (bias) {
+    // two tiles of 32 rows at a time (the rows are whole 128s): eight 16-byte
+    // loads in flight a lane, in a kernel that waits for memory (65536
+    // records: 23 us with two in flight, 15 with eight)
+    for (int64_t i = i_beg; i < i_end; i += 64) {
+        bf16x8 a[4], b[4];
 #pragma unroll
-            for (int e = 0; e < 8; e++) bsum += float(a[e]);
+        for (int k = 0; k < 4; k++) {
+            const int64_t tile = i + 32 * (k >> 1);
+            const int at = 16 * (k & 1) + 8 * h;
+            a[k] = *reinterpret_cast<const bf16x8*>(A + tile * kHid + at);
+            b[k] = *reinterpret_cast<const bf16x8*>(Bm + tile * K + at);
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            acc = mfma_bf16(a[k], b[k], acc);
+            if (bias) {
+#pragma unroll
+                for (int e = 0; e < 8; e++) bsum += float(a[k][e]);
+            }
         }
     }
     const int poff = job.layer == 1 ? kOffW1 : (job.layer == 2 ? kOffW2 : (job.layer == 3 ? kOffW3 : kOffW4));
