@@ -9,7 +9,7 @@
 //   4. binary LBVH topology (Karras, HPG 2012), ties broken by index, or
 //      PLOC (ploc.hip),
 //   5. triangles copied into traversal order (48 B each) and bottom-up bounds
-//      refit, one block per kRefitSpan leaves and one block for the nodes
+//      refit, one block per 1024 or 4096 leaves and one block for the nodes
 //      above, which also fills the SAH cost tables of the collapse
 //      (sah_tables),
 //   6. collapse into a W-wide tree (W = 2, 4, 8) of least SAH cost: the
@@ -41,9 +41,14 @@ namespace lmgpu {
 // triangle mesh, with the same hits).
 constexpr int kDefaultLeafSize = 2;
 constexpr float kDefaultSahTriCost = 0.5f;
-// Leaves per refit block: four for each thread, so a 1.3M triangle mesh still
-// gives every CU five blocks and only some 2600 nodes span blocks.
-constexpr int kRefitSpan = 1024;
+// Leaves per refit block, four for each thread. A large block leaves fewer
+// nodes that span blocks to the single block that does those (1.3M triangles:
+// 15560 for 1024 leaves, 4809 for 4096), a small one spreads a small mesh over
+// more CUs. Build times, 1024 / 2048 / 4096 leaves: 50K triangles 513, 519,
+// 531 us; 200K 566, 571, 583; 600K 750, 714, 695; 1.3M 1093, 997, 960; 4M 2847,
+// 2362, 2100.
+constexpr int kRefitSmall = 1024, kRefitLarge = 4096;
+constexpr int64_t kRefitLargeFrom = 400000;
 // Collapse levels launched between two reads of the level sizes; a level past
 // the last one is a launch of blocks that find no item (4 us), a read back is
 // a wait of some 40 us.
@@ -316,7 +321,7 @@ __device__ __forceinline__ void sah_tables(const SahDP& dp, int32_t p, int32_t l
 // A round is bound by latency, and a mesh of 1.3M triangles takes 22 rounds
 // in the blocks and 28 above them: the list holds what a node's loads need, so
 // its children and its parent's links are read side by side. That mesh takes
-// 183 us in the blocks (with the 42 us of the triangles' gather) and 293 us
+// 214 us in the blocks (with the 42 us of the triangles' gather) and 96 us
 // above them; a launch per level over a global list with an atomic per wave
 // took 890 us, and the gather was a pass of its own.
 struct Refit {
@@ -363,7 +368,7 @@ __device__ __forceinline__ void refit_node(const Refit& r, const RefitItem it) {
     }
 }
 
-// The leaves [kRefitSpan * block, + kRefitSpan): their triangles in traversal
+// The leaves [SPAN * block, + SPAN): their triangles in traversal
 // order and bounds, and every node above whose range of leaves lies within
 // them, in rounds over a list of ready nodes in LDS (at most half the leaves,
 // and never longer than the one before it: each parent enters by exactly one
@@ -371,21 +376,22 @@ __device__ __forceinline__ void refit_node(const Refit& r, const RefitItem it) {
 // left child, which no other node shares. A ready node that spans blocks is
 // counted in memory and goes to `frontier`: such nodes have disjoint ranges,
 // so there are fewer than blocks.
-template <int W>
-__global__ __launch_bounds__(256, 6) void k_refit_blocks(int64_t n, const int32_t* __restrict__ order,
+template <int W, int SPAN>
+__global__ __launch_bounds__(SPAN / 4) void k_refit_blocks(int64_t n, const int32_t* __restrict__ order,
                                                          const float* __restrict__ verts, TriV* __restrict__ tris,
                                                          Refit r, RefitItem* __restrict__ frontier) {
-    constexpr int kHalf = kRefitSpan / 2;
+    constexpr int kBlock = SPAN / 4;
+    constexpr int kHalf = SPAN / 2;
     __shared__ int4 links[2 * kHalf];        // RefitItem: node, parent, left, right
     __shared__ uint32_t range[2 * kHalf];    // its first and last leaf, in 16 bits each from the block's first
-    __shared__ uint32_t done[kRefitSpan / 4];
+    __shared__ uint32_t done[SPAN / 4];
     __shared__ int32_t size[2];
-    constexpr int kPer = kRefitSpan / 256;
-    const int32_t lead = int32_t(blockIdx.x) * kRefitSpan;
-    const int32_t tail = int32_t(std::min<int64_t>(n, int64_t(lead) + kRefitSpan) - 1);
+    constexpr int kPer = SPAN / kBlock;
+    const int32_t lead = int32_t(blockIdx.x) * SPAN;
+    const int32_t tail = int32_t(std::min<int64_t>(n, int64_t(lead) + SPAN) - 1);
     if (threadIdx.x < 2) size[threadIdx.x] = 0;
-    static_assert(kRefitSpan / 4 <= 256 && kRefitSpan <= 65536, "one word of `done` per thread, 16-bit ranges");
-    if (threadIdx.x < kRefitSpan / 4) done[threadIdx.x] = 0;
+    static_assert(SPAN / 4 <= kBlock && SPAN <= 65536, "one word of `done` per thread, 16-bit ranges");
+    if (threadIdx.x < SPAN / 4) done[threadIdx.x] = 0;
     __syncthreads();
     // the child [first, last] of q's node is done
     auto arrive = [&](const RefitItem q, int32_t first, int32_t last, int to) {
@@ -403,13 +409,13 @@ __global__ __launch_bounds__(256, 6) void k_refit_blocks(int64_t n, const int32_
     int32_t ti[kPer], up[kPer];
 #pragma unroll
     for (int k = 0; k < kPer; k++) {
-        const int32_t j = min(lead + int32_t(threadIdx.x) + 256 * k, tail);
+        const int32_t j = min(lead + int32_t(threadIdx.x) + kBlock * k, tail);
         ti[k] = order[j];
         up[k] = n > 1 ? r.parent_leaf[j] : 0;
     }
 #pragma unroll
     for (int k = 0; k < kPer; k++) {
-        const int32_t j = lead + int32_t(threadIdx.x) + 256 * k;
+        const int32_t j = lead + int32_t(threadIdx.x) + kBlock * k;
         if (j > tail) break;
         float v[9];
 #pragma unroll
@@ -437,7 +443,7 @@ __global__ __launch_bounds__(256, 6) void k_refit_blocks(int64_t n, const int32_
         __syncthreads();
         const int m = size[cur];
         if (m == 0) break;
-        for (int i = threadIdx.x; i < m; i += 256) {
+        for (int i = threadIdx.x; i < m; i += kBlock) {
             const int4 l = links[cur * kHalf + i];
             const uint32_t f = range[cur * kHalf + i];
             const RefitItem it{l.x, l.y, l.z, l.w, lead + int32_t(f & 0xffffu), lead + int32_t(f >> 16)};
@@ -772,9 +778,14 @@ static inline unsigned nblocks(int64_t n, int b) { return unsigned((n + b - 1) /
 template <int W>
 static void launch_refit(int64_t n, const int32_t* order, const float* verts, TriV* tris, const Refit& r,
                          RefitItem* list0, RefitItem* list1, hipStream_t s) {
-    hipLaunchKernelGGL(k_refit_blocks<W>, dim3(nblocks(n, kRefitSpan)), dim3(256), 0, s, n, order, verts, tris, r,
-                       list0);
-    if (n > kRefitSpan) hipLaunchKernelGGL(k_refit_top<W>, dim3(1), dim3(1024), 0, s, r, list0, list1);
+    auto blocks = [&](auto span) {
+        constexpr int SPAN = decltype(span)::value;
+        hipLaunchKernelGGL((k_refit_blocks<W, SPAN>), dim3(nblocks(n, SPAN)), dim3(SPAN / 4), 0, s, n, order, verts,
+                           tris, r, list0);
+        if (n > SPAN) hipLaunchKernelGGL(k_refit_top<W>, dim3(1), dim3(1024), 0, s, r, list0, list1);
+    };
+    if (n < kRefitLargeFrom) blocks(std::integral_constant<int, kRefitSmall>{});
+    else blocks(std::integral_constant<int, kRefitLarge>{});
 }
 
 template <int W>

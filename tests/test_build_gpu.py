@@ -5,7 +5,8 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
-SPAN = 1024   # leaves per refit block (kRefitSpan)
+SPAN = 1024   # leaves per refit block (kRefitSmall)
+LARGE = 400000   # from here on, blocks of 4096 leaves (kRefitLargeFrom)
 
 
 def _mesh(n, kind):
@@ -29,7 +30,8 @@ def _arrays(blob, width):
 
 @pytest.mark.parametrize('n,kind', [(1, ''), (2, ''), (SPAN - 1, ''), (SPAN, ''), (SPAN + 1, ''), (SPAN + 2, 'equal'),
                                     (2 * SPAN + 1, 'line'), (5 * SPAN, 'equal'), (40 * SPAN + 3, ''),
-                                    (70 * SPAN + 511, 'line')])
+                                    (70 * SPAN + 511, 'line'), (LARGE - 1, 'line'), (LARGE, 'equal'),
+                                    (LARGE + 4096 - LARGE % 4096 + 1, '')])
 @pytest.mark.parametrize('width,collapse,builder', [(2, 0, 1), (4, 0, 1), (8, 0, 1), (4, 1, 1), (8, 0, 0)])
 def test_built_bounds_and_counts(n, kind, width, collapse, builder):
     """Every child box is the exact FP32 bound of the triangles below it (a
@@ -59,20 +61,21 @@ def test_built_bounds_and_counts(n, kind, width, collapse, builder):
     assert len(levels) == info['depth']
     assert np.array_equal(np.sort(np.concatenate(levels)), np.arange(len(nodes)))
     for level in reversed(levels):
-        for i in level:
-            for c in range(width):
-                if count[i, c] < 0:
-                    continue
-                if count[i, c] > 0:
-                    s = slice(child[i, c], child[i, c] + count[i, c])
-                    seen[s] += 1
-                    want = np.stack([lo[s].min(0), hi[s].max(0)])
-                else:
-                    want = box[child[i, c]]
-                got = np.stack([nodes[i, :3, c], nodes[i, 3:6, c]])
-                assert np.array_equal(got, want), (i, c)
-            used = count[i] >= 0
-            box[i] = np.stack([nodes[i, :3][:, used].min(1), nodes[i, 3:6][:, used].max(1)])
+        got_lo, got_hi = nodes[level, :3].transpose(0, 2, 1), nodes[level, 3:6].transpose(0, 2, 1)   # [node, child, axis]
+        ch, ct = child[level], count[level]
+        want = np.empty((2,) + got_lo.shape, np.float32)
+        want[0], want[1] = np.inf, -np.inf
+        inner = ct == 0
+        want[0][inner], want[1][inner] = box[ch[inner], 0], box[ch[inner], 1]
+        for k in range(ct.max()):
+            m = ct > k
+            at = ch[m] + k
+            want[0][m] = np.minimum(want[0][m], lo[at])
+            want[1][m] = np.maximum(want[1][m], hi[at])
+            np.add.at(seen, at, 1)
+        used = ct >= 0
+        assert np.array_equal(got_lo[used], want[0][used]) and np.array_equal(got_hi[used], want[1][used])
+        box[level, 0], box[level, 1] = want[0].min(1), want[1].max(1)
     assert (seen == 1).all()
     # the same triangles again, and half of them, into the same object
     acc.build(verts)
