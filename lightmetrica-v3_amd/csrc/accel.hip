@@ -511,15 +511,15 @@ struct CollapseArgs {
 };
 
 // Runs a level: `expand(bref, ref, nc)` finds the nc <= W refs a wide node of
-// `bref` has as children, `is_leaf(ref)` tells which of them are leaves. The
+// `bref` has as children and returns the mask of those that are not leaves. The
 // wide children of one node take consecutive slots, so siblings share cache
 // lines. Whole blocks take their nodes' slots with one atomic, and the SAH
 // sum and leaf count of all a block's items are added once: same-address
 // atomics cost 12 ns each on the card, and with four per wave they were most
 // of the collapse's time (1.3M triangles, W = 4, 17 levels: 445 us, now
-// 245 us, at 10 to 33 us a level mostly the latency of the unfolding).
-template <int W, class Expand, class IsLeaf>
-__device__ __forceinline__ void collapse_level(const CollapseArgs& a, Expand expand, IsLeaf is_leaf) {
+// 220 us, at 10 to 33 us a level mostly the latency of the unfolding).
+template <int W, class Expand>
+__device__ __forceinline__ void collapse_level(const CollapseArgs& a, Expand expand) {
     __shared__ int32_t wave_sum[4];
     __shared__ int32_t block_base;
     __shared__ double block_sah[4];
@@ -537,9 +537,7 @@ __device__ __forceinline__ void collapse_level(const CollapseArgs& a, Expand exp
         int nc = 0, nint = 0;
         uint32_t inner = 0;
         if (idx < count) {
-            expand(a.in[idx], ref, nc);
-            for (int c = 0; c < nc; c++)
-                if (!is_leaf(ref[c])) inner |= 1u << c;
+            inner = expand(a.in[idx], ref, nc);
             nint = __popc(inner);
         }
         int inc = nint;
@@ -609,37 +607,45 @@ __device__ __forceinline__ void collapse_level(const CollapseArgs& a, Expand exp
 // (ref, slots) pairs whose slots sum to at most W.
 template <int W>
 __global__ __launch_bounds__(256) void k_collapse_sah(CollapseArgs a) {
-    const uint8_t* choice = a.choice;
-    auto is_leaf = [&](int32_t r) { return r < 0 || choice[int64_t(r) * W] == 0xFF; };
-    auto expand = [&](int32_t bref, int32_t (&ref)[W], int& nc) {
-        if (is_leaf(bref)) {
+    // a node's W choices as one word, read together with the node itself: a
+    // step of the unfolding waits once for memory (17 levels 245 -> 220 us)
+    using Row = std::conditional_t<W == 2, uint16_t, std::conditional_t<W == 4, uint32_t, uint64_t>>;
+    auto row_of = [&](int32_t r) { return reinterpret_cast<const Row*>(a.choice)[r]; };
+    auto choice = [](Row row, int i) { return int(row >> (8 * i)) & 0xff; };
+    auto expand = [&](int32_t bref, int32_t (&ref)[W], int& nc) -> uint32_t {
+        const Row first = row_of(max(bref, 0));
+        const BNode b = a.bn[max(bref, 0)];
+        if (bref < 0 || choice(first, 0) == 0xFF) {
             ref[nc++] = bref;   // the whole tree is one leaf (tiny scenes)
-            return;
+            return 0;
         }
+        uint32_t inner = 0;
         int32_t sr[W];
         int sj[W];
         int sp = 0;
-        const BNode b = a.bn[bref];
-        const int k = choice[int64_t(bref) * W];
+        const int k = choice(first, 0);
         sr[sp] = b.right; sj[sp++] = W - k;
         sr[sp] = b.left; sj[sp++] = k;
         while (sp > 0) {
             --sp;
             const int32_t m = sr[sp];
             int j = sj[sp];
+            const Row row = row_of(max(m, 0));
+            const BNode bm = a.bn[max(m, 0)];
             if (m >= 0)
-                while (j > 1 && choice[int64_t(m) * W + j - 1] == 0) j--;
+                while (j > 1 && choice(row, j - 1) == 0) j--;
             if (m < 0 || j == 1) {
+                if (m >= 0 && choice(row, 0) != 0xFF) inner |= 1u << nc;
                 ref[nc++] = m;
                 continue;
             }
-            const int c = choice[int64_t(m) * W + j - 1];
-            const BNode bm = a.bn[m];
+            const int c = choice(row, j - 1);
             sr[sp] = bm.right; sj[sp++] = j - c;
             sr[sp] = bm.left; sj[sp++] = c;
         }
+        return inner;
     };
-    collapse_level<W>(a, expand, is_leaf);
+    collapse_level<W>(a, expand);
 }
 
 // Greedy collapse: open the largest-area child until there are W.
@@ -649,10 +655,10 @@ __global__ __launch_bounds__(256) void k_collapse(CollapseArgs a) {
     auto lo_of = [&](int32_t r) { return r < 0 ? a.leaf_lo[~r] : a.node_lo[r]; };
     auto hi_of = [&](int32_t r) { return r < 0 ? a.leaf_hi[~r] : a.node_hi[r]; };
     auto is_leaf = [&](int32_t r) { return r < 0 || cnt_of(r) <= a.leaf_size; };
-    auto expand = [&](int32_t bref, int32_t (&ref)[W], int& nc) {
+    auto expand = [&](int32_t bref, int32_t (&ref)[W], int& nc) -> uint32_t {
         if (is_leaf(bref)) {
             ref[nc++] = bref;   // whole range is one leaf (tiny scenes)
-            return;
+            return 0;
         }
         ref[nc++] = a.bn[bref].left;
         ref[nc++] = a.bn[bref].right;
@@ -670,8 +676,12 @@ __global__ __launch_bounds__(256) void k_collapse(CollapseArgs a) {
             ref[best] = b.left;
             ref[nc++] = b.right;
         }
+        uint32_t inner = 0;
+        for (int c = 0; c < nc; c++)
+            if (!is_leaf(ref[c])) inner |= 1u << c;
+        return inner;
     };
-    collapse_level<W>(a, expand, is_leaf);
+    collapse_level<W>(a, expand);
 }
 
 __global__ void k_collapse_init(BuildHead* head, int32_t* items, int32_t root_ref) {
