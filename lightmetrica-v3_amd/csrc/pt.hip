@@ -15,7 +15,7 @@
 //              contributions added to the path radiance
 //   accumulate per-pixel FP64 sum and sum of squares (Film_Bitmap is FP64,
 //   src/film/film_bitmap.cpp:19-55)
-// Queues are SoA arrays appended with one atomic per wave (ballot + popcount);
+// Queues are SoA arrays, both appended with one 64-bit atomic per block;
 // counts live in device memory so the whole pass is captured once as a
 // hipGraph and replayed per sample.
 //

@@ -14,9 +14,9 @@
 #include "lmgpu_internal.h"
 #include "pt_device.h"
 
-// Path pool of a fixed-spp render: slots per pixel and at most (1080p
-// config 2: 2 per pixel 431, 4: 503, 8: 547, 16: 558 M samples/s; 2^24 slots
-// take 3.6 GB).
+// Path pool of a fixed-spp render: slots per pixel and at most (1080p, 1.32M
+// triangles, 16 spp: 1 per pixel 69.7 ms, 2: 56.6, 4: 51.2, 8: 47.6, before
+// samples were resolved at the end of a run; 2^24 slots take 3.6 GB).
 #ifndef LMGPU_REGEN_SLOTS_PER_PIXEL
 #define LMGPU_REGEN_SLOTS_PER_PIXEL 8
 #endif
@@ -124,7 +124,7 @@ struct RegenGuide {
 };
 
 // Path pool, work queue and the loop that drains it (regenerate -> extend ->
-// shade -> connect, two iterations per graph replay), shared by the batch
+// shade -> connect, pairs of iterations one ahead of the device), shared by the batch
 // and by lmgpu_pt_render's regenerating path.
 struct Wavefront {
     int cap = 0;
@@ -170,7 +170,7 @@ struct Wavefront {
     // vectors live until the run has ended.
     int set_work(const std::vector<JobDev>& jobs, const std::vector<WorkSeg>& segs, hipStream_t s);
     // Renders every work item of the tables set last into film_sum / film_sq
-    // (FP64 atomics; film_sq may be null) and waits for the end.
+    // (film_sq may be null) and waits for the end.
     // With a guide, the directions at diffuse and glossy vertices come from
     // the one-sample mixture of guide and BSDF, and the guide trains online
     // on the records of finished paths.
