@@ -64,8 +64,7 @@ static_assert(sizeof(WNode<4>) == 128, "BVH4 node must be one 128-B line");
 // lower / upper plane on axis a is byte c % 4 of qlo[a][c / 4] / qhi[a][c / 4];
 // ent[c] is its stack entry (inner node index >= 0, or
 // encode_leaf(first, count) < 0), kQEmpty, a leaf of no triangles, for an
-// empty slot (whose planes are stored inverted, so that a ray meets it only
-// within the slack of a flat node).
+// empty slot.
 template <int W>
 struct alignas(W * 16) QNode {
     float ox, oy, oz;
@@ -299,8 +298,10 @@ LMGPU_HD void child_keys(const QNode<W>& nd, const RayPre& r, float tmin, float 
         }
         const float n = fmaxf(fmaxf(tn[0], tn[1]), fmaxf(tn[2], tmin));
         const float f = fminf(fminf(tf[0], tf[1]), fminf(tf[2], tmax));
-        key[c] = n <= f * 1.00000036f ? n : __builtin_inff();
-        ent[c] = nd.ent[c];
+        const int e = nd.ent[c];
+        const bool hit = n <= f * 1.00000036f && (c < 2 || e != kQEmpty);
+        key[c] = hit ? n : __builtin_inff();
+        ent[c] = e;
     }
 }
 
@@ -344,16 +345,14 @@ LMGPU_HD QAxis<W> quantise_axis(const float (&lo)[W], const float (&hi)[W], uint
     q.e = e;
     const float step = std::ldexp(1.f, e);
     for (int c = 0; c < W; c++) {
-        int l = 255, h = 0;   // an empty slot: no ray lies above plane 255 and below plane 0
-        if (present >> c & 1u) {
-            // division by the power-of-two step is an exact scaling
-            l = int(std::floor(std::ldexp(double(lo[c]) - double(mn), -e)));
-            l = std::min(std::max(l, 0), 255);
-            while (l > 0 && std::fma(float(l), step, mn) > lo[c]) l--;
-            h = int(std::ceil(std::ldexp(double(hi[c]) - double(mn), -e)));
-            h = std::min(std::max(h, 0), 255);
-            while (h < 255 && std::fma(float(h), step, mn) < hi[c]) h++;
-        }
+        if (!(present >> c & 1u)) continue;
+        // division by the power-of-two step is an exact scaling
+        int l = int(std::floor(std::ldexp(double(lo[c]) - double(mn), -e)));
+        l = std::min(std::max(l, 0), 255);
+        while (l > 0 && std::fma(float(l), step, mn) > lo[c]) l--;
+        int h = int(std::ceil(std::ldexp(double(hi[c]) - double(mn), -e)));
+        h = std::min(std::max(h, 0), 255);
+        while (h < 255 && std::fma(float(h), step, mn) < hi[c]) h++;
         q.ql[c >> 2] |= uint32_t(l) << (8 * (c & 3));
         q.qh[c >> 2] |= uint32_t(h) << (8 * (c & 3));
     }

@@ -8,7 +8,9 @@
 // grazing its faces, edges and corners, starting on its faces or running
 // parallel to them, every child whose exact box the ray meets in
 // [tmin, tmax] (decided in exact arithmetic: __float128 products of the FP32
-// inputs) is hit. Prints "ok <nodes> <rays>" or the first failure and exits
+// inputs) is hit. Last, no ray meets an empty slot: near, far beyond the
+// node's extent, parallel to its planes, or with an origin or a direction that
+// is infinite or NaN. Prints "ok <nodes> <rays>" or the first failure and exits
 // non-zero.
 #include <cstdio>
 #include <random>
@@ -175,6 +177,54 @@ int check_slab(std::mt19937_64& rng, int n_nodes, int rays_per_node, long long& 
     return 0;
 }
 
+// Rays against nodes with empty slots (two children or more, as every node but
+// the root of a single leaf): their keys stay infinite, whatever the
+// ray, so that they neither take part in the order of the children nor go on
+// the stack.
+template <int W>
+int check_empty(std::mt19937_64& rng, int n_nodes, int rays_per_node) {
+    std::uniform_real_distribution<double> U(0.0, 1.0);
+    const float odd[4] = {std::nanf(""), __builtin_inff(), -__builtin_inff(), 0.f};
+    for (int it = 0; it < n_nodes; it++) {
+        WNode<W> n;
+        const double extent = std::pow(10.0, U(rng) * 10 - 7);
+        const int nvalid = 2 + int(U(rng) * (W - 2));
+        for (int c = 0; c < W; c++) {
+            float* lo[3] = {&n.lox[c], &n.loy[c], &n.loz[c]};
+            float* hi[3] = {&n.hix[c], &n.hiy[c], &n.hiz[c]};
+            for (int a = 0; a < 3; a++) {
+                *lo[a] = c < nvalid ? float(U(rng) * extent) : 1e30f;
+                *hi[a] = c < nvalid ? *lo[a] + float(U(rng) * extent) : -1e30f;
+            }
+            n.count[c] = c < nvalid ? c % 3 : -1;
+            n.child[c] = c < nvalid ? 1 + c : 0;
+        }
+        const QNode<W> q = lmgpu::quantise_node<W>(n);
+        for (int k = 0; k < rays_per_node; k++) {
+            const double dist = extent * std::pow(10.0, U(rng) * 12 - 1);
+            float o[3], d[3];
+            for (int a = 0; a < 3; a++) {
+                o[a] = float((U(rng) - 0.5) * 2 * dist);
+                d[a] = float(U(rng) * extent - o[a]);
+            }
+            if (k % 4 == 1) d[int(U(rng) * 3) % 3] = 0.f;
+            if (k % 4 == 2) o[int(U(rng) * 3) % 3] = odd[int(U(rng) * 4) % 4];
+            if (k % 4 == 3) d[int(U(rng) * 3) % 3] = odd[int(U(rng) * 4) % 4];
+            const lmgpu::RayPre r = lmgpu::ray_prepare(lmgpu::mk(o[0], o[1], o[2]), lmgpu::mk(d[0], d[1], d[2]));
+            float key[W];
+            int ent[W];
+            lmgpu::child_keys<W>(q, r, 0.f, __builtin_inff(), key, ent);
+            for (int c = nvalid; c < W; c++)
+                if (key[c] != __builtin_inff()) {
+                    std::printf("W%d node %d: ray o (%.9g, %.9g, %.9g) d (%.9g, %.9g, %.9g) meets empty slot %d at %g\n",
+                                W, it, o[0], o[1], o[2], d[0], d[1], d[2], c, key[c]);
+                    return 1;
+                }
+        }
+    }
+    return 0;
+}
+
 int main() {
     std::mt19937_64 rng(12345);
     const int kNodes = 200000;
@@ -183,6 +233,7 @@ int main() {
     if (check_slab<4>(rng, 100000, 16, n_rays, n_exact, n_extra) ||
         check_slab<8>(rng, 50000, 16, n_rays, n_exact, n_extra))
         return 1;
+    if (check_empty<4>(rng, 20000, 32) || check_empty<8>(rng, 20000, 32)) return 1;
     std::printf("ok %d %lld (exact hits %lld, accepted beyond the exact boxes %lld)\n", 2 * kNodes, n_rays, n_exact,
                 n_extra);
     return 0;

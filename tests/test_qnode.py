@@ -8,8 +8,8 @@ fma per plane from the exact grid, the near and far plane picked by the
 direction's sign, offsets widened by a rounding bound) never misses a child
 whose exact box the ray meets: 2.3 million rays aimed at faces, edges and
 corners, starting on the box's planes or parallel to them, decided in exact
-arithmetic (with the widening removed, the first node already fails). GPU
-hit parity with the quantised traversal is covered by the accel tests."""
+arithmetic (with the widening removed, the first node already fails). No ray,
+near, far, parallel, infinite or NaN, meets an empty slot. GPU hit parity with the quantised traversal is covered by the accel tests."""
 import os
 import shutil
 import subprocess
