@@ -755,12 +755,8 @@ __global__ __launch_bounds__(256) void k_quantise(const WNode<W>* __restrict__ i
     present = __shfl(present, 3, 4);
     QAxis<W> x{};
     if (a < 3) x = quantise_axis<W>(lo, hi, present);
-    uint32_t e = uint32_t(x.e + 127) << (8 * a), es = uint32_t(x.e & 0xff) << (8 * a);
-    if (a == 3) e = es = 0;
-    for (int off = 1; off < 4; off <<= 1) {
-        e |= __shfl_xor(e, off, 4);
-        es |= __shfl_xor(es, off, 4);
-    }
+    uint32_t e = a < 3 ? uint32_t(x.e & 0xff) << (8 * a) : 0u;
+    for (int off = 1; off < 4; off <<= 1) e |= __shfl_xor(e, off, 4);
     if (a < 3) {
         (a == 0 ? q.ox : a == 1 ? q.oy : q.oz) = x.org;
         for (int k = 0; k < W / 4; k++) {
@@ -769,7 +765,6 @@ __global__ __launch_bounds__(256) void k_quantise(const WNode<W>* __restrict__ i
         }
     } else {
         q.e = e;
-        q.es = es;
         for (int c = 0; c < W; c++) q.ent[c] = quantised_entry(__float_as_int(lo[c]), __float_as_int(hi[c]));
     }
 }

@@ -68,11 +68,10 @@ static_assert(sizeof(WNode<4>) == 128, "BVH4 node must be one 128-B line");
 template <int W>
 struct alignas(W * 16) QNode {
     float ox, oy, oz;
-    uint32_t e;        // biased FP32 exponents of the x, y, z grid steps in bytes 0, 1, 2
+    uint32_t e;        // exponents of the x, y, z grid steps: signed bytes 0, 1, 2 (read with the origin)
     uint32_t qlo[3][W / 4];
     uint32_t qhi[3][W / 4];
     int32_t ent[W];
-    uint32_t es;       // the grid exponents again, unbiased: signed bytes 0, 1, 2
 };
 using QNode4 = QNode<4>;
 static_assert(sizeof(QNode<4>) == 64, "quantised BVH4 node must be 64 B");
@@ -275,7 +274,7 @@ LMGPU_HD void child_keys(const QNode<W>& nd, const RayPre& r, float tmin, float 
         }
 #pragma unroll
     for (int k = 0; k < 3; k++) {
-        a[k] = ldexpf(inv[k], int32_t(nd.es << (24 - 8 * k)) >> 24);
+        a[k] = ldexpf(inv[k], int32_t(nd.e << (24 - 8 * k)) >> 24);
         const float b = (org[k] - o[k]) * inv[k];
         const float x = fabsf(b) + fmaf(fabsf(org[k]), fabsf(inv[k]), 255.f * fabsf(a[k]));
         bn[k] = fmaf(x, -0x1p-20f, b);   // Ex = 2^-20 x
@@ -375,10 +374,9 @@ LMGPU_HD QNode<W> quantise_node(const WNode<W>& n) {
     q.ox = x[0].org;
     q.oy = x[1].org;
     q.oz = x[2].org;
-    q.e = q.es = 0;
+    q.e = 0;
     for (int a = 0; a < 3; a++) {
-        q.e |= uint32_t(x[a].e + 127) << (8 * a);
-        q.es |= uint32_t(x[a].e & 0xff) << (8 * a);
+        q.e |= uint32_t(x[a].e & 0xff) << (8 * a);
         for (int k = 0; k < W / 4; k++) {
             q.qlo[a][k] = x[a].ql[k];
             q.qhi[a][k] = x[a].qh[k];

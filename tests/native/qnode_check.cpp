@@ -12,6 +12,7 @@
 // node's extent, parallel to its planes, or with an origin or a direction that
 // is infinite or NaN. Prints "ok <nodes> <rays>" or the first failure and exits
 // non-zero.
+#include <cstddef>
 #include <cstdio>
 #include <random>
 
@@ -19,6 +20,9 @@
 
 using lmgpu::QNode;
 using lmgpu::WNode;
+
+// the exponents the traversal reads come with the grid origin's 16 bytes
+static_assert(offsetof(QNode<4>, e) == 12 && offsetof(QNode<8>, e) == 12, "grid exponents beside the origin");
 
 template <int W>
 int check(std::mt19937_64& rng, int n_nodes) {
@@ -56,7 +60,7 @@ int check(std::mt19937_64& rng, int n_nodes) {
             if (n.count[c] < 0) continue;
             const float lo[3] = {n.lox[c], n.loy[c], n.loz[c]}, hi[3] = {n.hix[c], n.hiy[c], n.hiz[c]};
             for (int a = 0; a < 3; a++) {
-                const float step = std::ldexp(1.f, int((q.e >> (8 * a)) & 0xffu) - 127);
+                const float step = std::ldexp(1.f, int8_t(q.e >> (8 * a)));
                 const float dl = lmgpu::qplane(q.qlo[a][c / 4], c % 4, step, org[a]);
                 const float dh = lmgpu::qplane(q.qhi[a][c / 4], c % 4, step, org[a]);
                 if (!(dl <= lo[a] && dh >= hi[a])) {

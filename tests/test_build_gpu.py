@@ -1,5 +1,7 @@
 """Device BVH build: the refit's blocks, the collapse's levels and the
 quantised copy at the edges of their tiles (csrc/accel.hip)."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -84,3 +86,77 @@ def test_built_bounds_and_counts(n, kind, width, collapse, builder):
     acc.build(verts[:half])
     assert acc.info()['num_tris'] == half
     assert np.array_equal(np.sort(_arrays(acc.serialize(), width)[1][:, 0, 3].copy().view(np.int32)), np.arange(half))
+
+
+def _quantised(nodes, width):
+    """QNode<width> words of WNode<width> arrays ([n, 8, width] float32; csrc/bvh.h, quantise_node). Sums of a plane
+    number times a power of two and an FP32 origin are exact in FP64, so their FP32 rounding is the fma's."""
+    n = len(nodes)
+    count, child = nodes[:, 7].view(np.int32).astype(np.int64), nodes[:, 6].view(np.int32).astype(np.int64)
+    present = count >= 0
+    out = np.zeros((n, 4 * width), np.uint32)
+    for a in range(3):
+        lo, hi = nodes[:, a].astype(np.float64), nodes[:, 3 + a].astype(np.float64)
+        mn = np.where(present, lo, np.inf).min(1)
+        mx = np.where(present, hi, -np.inf).max(1)
+        m, k = np.frexp((mx - mn) / 255.0)
+        e = np.where(mx > mn, np.maximum(np.where(m == 0.5, k - 1, k), -126), -126)
+        plane = lambda q, e: (q * np.exp2(e.astype(np.float64)) + mn).astype(np.float32)   # noqa: E731
+        while True:
+            grow = (plane(255.0, e) < mx) & (e < 127)
+            if not grow.any():
+                break
+            e = e + grow
+        out[:, a] = mn.astype(np.float32).view(np.uint32)
+        out[:, 3] |= (e & 0xff).astype(np.uint32) << np.uint32(8 * a)
+        for c in range(width):
+            step = np.exp2(e.astype(np.float64))
+            ql = np.clip(np.floor((lo[:, c] - mn) / step), 0, 255)
+            qh = np.clip(np.ceil((hi[:, c] - mn) / step), 0, 255)
+            while True:
+                down = (plane(ql, e) > lo[:, c]) & (ql > 0) & present[:, c]
+                up = (plane(qh, e) < hi[:, c]) & (qh < 255) & present[:, c]
+                if not (down.any() or up.any()):
+                    break
+                ql, qh = ql - down, qh + up
+            at, sh = 4 + a * (width // 4) + c // 4, np.uint32(8 * (c % 4))
+            out[:, at] |= np.where(present[:, c], ql, 0).astype(np.uint32) << sh
+            out[:, at + 3 * (width // 4)] |= np.where(present[:, c], qh, 0).astype(np.uint32) << sh
+    leaf = -((child << 4) | count) - 1
+    ent = np.where(count < 0, -1, np.where(count == 0, child, leaf))
+    first = 4 + 6 * (width // 4)
+    out[:, first:first + width] = ent.astype(np.int32).view(np.uint32)
+    return out, first + width
+
+
+@pytest.mark.parametrize('width', [4, 8])
+@pytest.mark.parametrize('n', [1, 15, 16, 17, 63, 64, 65, 1000])
+def test_quantised_copy(device, width, n):
+    """k_quantise, word for word, at node counts around its waves (16 nodes)
+    and blocks (64): partly empty nodes, flat boxes, several scales."""
+    import torch
+    from lm_amd import _lib
+    rng = np.random.default_rng([n, width])
+    nodes = np.empty((n, 8, width), np.float32)
+    extent = 10.0 ** rng.uniform(-5, 3, (n, 1, 1))
+    lo = (rng.uniform(-1, 1, (n, 3, 1)) * 10 + rng.random((n, 3, width)) * extent).astype(np.float32)
+    flat = rng.random((n, 3, width)) < 0.1
+    hi = np.maximum(lo, (lo + rng.random((n, 3, width)) * extent * ~flat).astype(np.float32))
+    used = np.arange(width) < rng.integers(1, width + 1, (n, 1))
+    nodes[:, :3] = np.where(used[:, None], lo, np.float32(1e30))
+    nodes[:, 3:6] = np.where(used[:, None], hi, np.float32(-1e30))
+    nodes[:, 6] = np.where(used, rng.integers(0, 1 << 20, (n, width)), 0).astype(np.int32).view(np.float32)
+    nodes[:, 7] = np.where(used, rng.integers(0, 16, (n, width)), -1).astype(np.int32).view(np.float32)
+    words, held = _quantised(nodes, width)
+    src = torch.from_numpy(nodes.view(np.int32).copy()).to(device)
+    dst = torch.full((n + 1, 4 * width), 77, dtype=torch.int32, device=device)
+    # lmgpu::quantise_nodes(int, const float4*, float4*, int64_t, hipStream_t)
+    fn = getattr(_lib.lib(), '_ZN5lmgpu14quantise_nodesEiPK15HIP_vector_typeIfLj4EEPS1_lP12ihipStream_t')
+    fn.argtypes = [ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p]
+    fn.restype = ctypes.c_int
+    torch.cuda.synchronize()
+    assert fn(width, src.data_ptr(), dst.data_ptr(), n, None) == 0
+    torch.cuda.synchronize()
+    got = dst.cpu().numpy().view(np.uint32)
+    assert np.array_equal(got[:n, :held], words[:, :held])
+    assert (got[n] == 77).all()
