@@ -783,10 +783,8 @@ int Wavefront::set_work(const std::vector<JobDev>& jobs, const std::vector<WorkS
     const int nj = int(jobs.size());
     if (djobs.n != size_t(nj)) LMGPU_TRY(djobs.alloc(nj));
     if (dsegs.n != segs.size()) LMGPU_TRY(dsegs.alloc(segs.size()));
-    if (job_done.n != size_t(nj)) {
-        LMGPU_TRY(job_done.alloc(nj));
-        LMGPU_TRY(job_time.alloc(nj));
-    }
+    if (job_done.n != size_t(nj)) LMGPU_TRY(job_done.alloc(nj));
+    if (job_time.n != size_t(nj)) LMGPU_TRY(job_time.alloc(nj));
     LMGPU_HIP(hipMemcpyAsync(djobs.p, jobs.data(), sizeof(JobDev) * nj, hipMemcpyHostToDevice, s));
     LMGPU_HIP(hipMemcpyAsync(dsegs.p, segs.data(), sizeof(WorkSeg) * segs.size(), hipMemcpyHostToDevice, s));
     hipLaunchKernelGGL(k_b_fill_u64, dim3(nblk(nj, 256)), dim3(256), 0, s, job_done.p, int64_t(nj));
@@ -1055,6 +1053,13 @@ int Batch::run_once(int width, int block, int spp_cap, bool keep_results, bool w
 
 void wavefront_destroy(Wavefront* w) { delete w; }
 
+bool wavefront_give_back(Wavefront* w, int64_t keep) {
+    if (!w || !w->psample.p) return false;
+    if (keep > 0 && w->psample.n <= size_t(std::max<int64_t>(2 * keep, 16 * int64_t(w->cap)))) return false;
+    w->psample.reset();
+    return true;
+}
+
 int Scene::render_regen(const PTConsts& c, int spp, int sample_offset, double* sum, double* sumsq, int64_t* ext_rays,
                         int64_t* shadow_rays, hipStream_t s, const GuidedPass* gp, int64_t* guide_records) {
     if (!wf) {
@@ -1084,22 +1089,15 @@ int Scene::render_regen(const PTConsts& c, int spp, int sample_offset, double* s
     const int64_t runs = resolve ? (spp + hold - 1) / hold : 1;
     int per_run = int((spp + runs - 1) / runs);
     int64_t total = int64_t(c.npix) * per_run;
-    if (resolve && wf->psample.n < size_t(total) && wf->psample.alloc(size_t(total)) != LMGPU_OK) {
-        // no memory for it: one run that adds to the film
-        (void)hipGetLastError();
-        clear_error();
-        resolve = false;
-        per_run = spp;
-        total = int64_t(c.npix) * spp;
-    }
     // one job: items are its samples' pixels in order from the first sample
+    const std::vector<JobDev> jobs{J};
     std::vector<WorkSeg> segs{WorkSeg{0, 0, sample_offset}};
     // pool: LMGPU_REGEN_SLOTS_PER_PIXEL paths per pixel (the slots of a
-    // sample's short paths take the next sample's pixels)
+    // sample's short paths take the next sample's pixels); a run of the whole
+    // render would have the same
     const int cap = gp ? Wavefront::pool_size(total, c.npix, LMGPU_REGEN_GUIDED_SLOTS_PER_PIXEL,
                                               LMGPU_REGEN_GUIDED_MAX_SLOTS)
                        : Wavefront::pool_size(total, c.npix);
-    LMGPU_TRY(wf->ensure_pool(cap));
     RegenGuide G;
     if (gp) {
         G.g = gp->g;
@@ -1115,10 +1113,25 @@ int Scene::render_regen(const PTConsts& c, int spp, int sample_offset, double* s
         G.steps = gp->steps;
         G.rec_depth = gp->rec_depth;
         G.npix = c.npix;
-        if (G.steps > 0) LMGPU_TRY(gp->g->ensure_train(G.batch));
-        LMGPU_TRY(wf->ensure_guided(G.rec_depth, int64_t(G.batch) * G.steps));
     }
-    const std::vector<JobDev> jobs{J};
+    // What the render cannot do without comes first, the kept samples from
+    // what is left: without them it is one run that adds to the film.
+    LMGPU_TRY(with_memory([&]() -> int {
+        LMGPU_TRY(wf->ensure_pool(cap));
+        if (gp) {
+            if (G.steps > 0) LMGPU_TRY(gp->g->ensure_train(G.batch));
+            LMGPU_TRY(wf->ensure_guided(G.rec_depth, int64_t(G.batch) * G.steps));
+        }
+        LMGPU_TRY(wf->ensure_host());
+        return wf->set_work(jobs, segs, s);
+    }));
+    if (resolve && wf->psample.n < size_t(total) && wf->psample.alloc(size_t(total)) != LMGPU_OK) {
+        (void)hipGetLastError();
+        clear_error();
+        resolve = false;
+        per_run = spp;
+        total = int64_t(c.npix) * spp;
+    }
     const void* tn = accel.width == 4 ? static_cast<const void*>(dev.nodes4)
                      : accel.width == 8 ? static_cast<const void*>(dev.nodes8) : static_cast<const void*>(dev.nodes2);
     *ext_rays = *shadow_rays = 0;
@@ -1126,8 +1139,10 @@ int Scene::render_regen(const PTConsts& c, int spp, int sample_offset, double* s
     for (int done = 0; done < spp; done += per_run) {
         const int n = std::min(per_run, spp - done);
         total = int64_t(c.npix) * n;
-        segs[0].sample = sample_offset + done;
-        LMGPU_TRY(wf->set_work(jobs, segs, s));
+        if (done > 0) {
+            segs[0].sample = sample_offset + done;
+            LMGPU_TRY(wf->set_work(jobs, segs, s));
+        }
         double sec = 0;
         int64_t iters = 0;
         LMGPU_TRY(wf->run(tn, accel.tris.p, accel.width, kSingleBlock, true, total, c.max_verts, sum, sumsq, &sec,

@@ -540,6 +540,7 @@ int Guide::ensure_train(int64_t B) {
     if (B % 128) return fail(LMGPU_ERR_INVALID_ARGUMENT, "training capacity must be a multiple of 128");
     if (B > (int64_t(1) << 22)) return fail(LMGPU_ERR_INVALID_ARGUMENT, "training batch above 2^22 records");
     if (B <= train_cap) return LMGPU_OK;
+    train_cap = 0;   // until all of it is there
     LMGPU_TRY(xT.alloc(size_t(kIn) * B));
     LMGPU_TRY(hT.alloc(size_t(3) * kHid * B));
     LMGPU_TRY(dT.alloc(size_t(4) * kHid * B));

@@ -985,7 +985,7 @@ int Scene::lt_render(const lmgpu_lt_params* p, double* film_in, bool on_device, 
     // the per-pixel buffers of the one-sample passes are not needed
     double* film = film_in;
     if (!on_device) {
-        if (fsum.n != size_t(npix) * 3) LMGPU_TRY(fsum.alloc(size_t(npix) * 3));
+        LMGPU_TRY(with_memory([&]() { return fsum.n != size_t(npix) * 3 ? fsum.alloc(size_t(npix) * 3) : LMGPU_OK; }));
         film = fsum.p;
         LMGPU_HIP(hipMemsetAsync(film, 0, sizeof(double) * 3 * size_t(npix), s));
     }
@@ -1011,7 +1011,7 @@ int Scene::lt_render(const lmgpu_lt_params* p, double* film_in, bool on_device, 
     const int W = accel.width;
     int64_t ext = 0, shd = 0;
     auto run_loop = [&](int64_t total, uint32_t pass0) -> int {
-        LMGPU_TRY(wf->ensure_pool(Wavefront::pool_size(total, npix)));
+        LMGPU_TRY(with_memory([&]() { return wf->ensure_pool(Wavefront::pool_size(total, npix)); }));
         auto iteration = [&](hipStream_t cs, int in_q) {
             if (W == 4) lt_regen_iteration<4>(*this, *wf, c, total, npix, pass0, film, in_q, cs);
             else if (W == 8) lt_regen_iteration<8>(*this, *wf, c, total, npix, pass0, film, in_q, cs);
@@ -1072,22 +1072,23 @@ int Scene::bdpt_render(const lmgpu_lt_params* p, double* film_in, bool on_device
     if (dev.num_lights == 0) return fail(LMGPU_ERR_INVALID_ARGUMENT, "bidirectional path tracing needs a light");
     const auto t0 = std::chrono::steady_clock::now();
     const int npix = w * h;
-    LMGPU_TRY(ensure_workspace(npix));
     // samples per pass: the largest power of two in [2^18, 2^21] whose stored
     // light vertices (P (max_verts - 1) LVerts of 96 B) fit in 2 GiB, at most
     // w*h; the connection queue has as many entries
     const int lstride = p->max_verts - 1;
     const int P = int(std::min<int64_t>(npix, bdpt_pass_size(lstride)));
     const size_t nv = size_t(P) * lstride;
-    if (blverts.n < nv * sizeof(LVert) / sizeof(float4)) LMGPU_TRY(blverts.alloc(nv * sizeof(LVert) / sizeof(float4)));
-    if (bsh.n < nv) {
-        LMGPU_TRY(bsh.alloc(nv));
-        LMGPU_TRY(bshc.alloc(nv));
-    }
-    if (blcount.n < size_t(P)) LMGPU_TRY(blcount.alloc(P));
+    LMGPU_TRY(with_memory([&]() -> int {
+        LMGPU_TRY(ensure_workspace(npix));
+        if (blverts.n < nv * sizeof(LVert) / sizeof(float4)) LMGPU_TRY(blverts.alloc(nv * sizeof(LVert) / sizeof(float4)));
+        if (bsh.n < nv) LMGPU_TRY(bsh.alloc(nv));
+        if (bshc.n < nv) LMGPU_TRY(bshc.alloc(nv));
+        if (blcount.n < size_t(P)) LMGPU_TRY(blcount.alloc(P));
+        return LMGPU_OK;
+    }));
     double* film = film_in;
     if (!on_device) {
-        if (fsum.n != size_t(npix) * 3) LMGPU_TRY(fsum.alloc(size_t(npix) * 3));
+        LMGPU_TRY(with_memory([&]() { return fsum.n != size_t(npix) * 3 ? fsum.alloc(size_t(npix) * 3) : LMGPU_OK; }));
         film = fsum.p;
         LMGPU_HIP(hipMemsetAsync(film, 0, sizeof(double) * 3 * size_t(npix), s));
     }

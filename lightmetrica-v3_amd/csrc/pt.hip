@@ -641,7 +641,7 @@ int Scene::ensure_guided(int npix, const GuidedPass& gp) {
     auto drop_graph = [&]() {
         if (graph) { (void)hipGraphExecDestroy(graph); graph = nullptr; }
     };
-    if (gmix.n != size_t(npix) * kOut) {
+    if (gmix.n != size_t(npix) * kOut || gshrec.n != size_t(npix)) {
         drop_graph();
         LMGPU_TRY(gmix.alloc(size_t(npix) * kOut));
         LMGPU_TRY(gshrec.alloc(npix));
@@ -649,6 +649,7 @@ int Scene::ensure_guided(int npix, const GuidedPass& gp) {
     const int64_t slots = int64_t(gp.rec_depth) * npix;
     if (slots > grec_slots) {
         drop_graph();
+        grec_slots = 0;
         LMGPU_TRY(grec.alloc(slots));
         LMGPU_TRY(grec_list.alloc(slots));
         grec_slots = int(slots);
@@ -794,10 +795,13 @@ int Scene::render(const lmgpu_pt_params* p, double* sum_in, double* sumsq_in, bo
     // samples per pixel, guided or not; 1-spp calls and the image mode replay
     // the one-sample pass graph
     const bool regen = !image && (p->render_time > 0 || p->spp >= 2);
-    if (!regen) LMGPU_TRY(ensure_workspace(npix));
+    // kept samples far beyond this render's are given back (not between the
+    // chunks of a time-scheduled render, whose sizes vary)
+    if (regen && p->render_time <= 0) (void)wavefront_give_back(wf, int64_t(npix) * p->spp);
+    if (!regen) LMGPU_TRY(with_memory([&]() { return ensure_workspace(npix); }));
     GuidedPass gpv;
     if (gp && !regen) {
-        LMGPU_TRY(ensure_guided(npix, *gp));
+        LMGPU_TRY(with_memory([&]() { return ensure_guided(npix, *gp); }));
         // buffers as they are after ensure_guided (it may grow the guide's training workspace)
         gpv = *gp;
         gpv.uid = gp->g->uid;
@@ -807,12 +811,13 @@ int Scene::render(const lmgpu_pt_params* p, double* sum_in, double* sumsq_in, bo
     double* sum = sum_in;
     double* sumsq = sumsq_in;
     if (!on_device) {
-        if (fsum.n != size_t(npix) * 3) LMGPU_TRY(fsum.alloc(size_t(npix) * 3));
+        LMGPU_TRY(with_memory([&]() -> int {
+            if (fsum.n != size_t(npix) * 3) LMGPU_TRY(fsum.alloc(size_t(npix) * 3));
+            if (sumsq_in && fsq.n != size_t(npix) * 3) LMGPU_TRY(fsq.alloc(size_t(npix) * 3));
+            return LMGPU_OK;
+        }));
         sum = fsum.p;
-        if (sumsq_in) {
-            if (fsq.n != size_t(npix) * 3) LMGPU_TRY(fsq.alloc(size_t(npix) * 3));
-            sumsq = fsq.p;
-        }
+        if (sumsq_in) sumsq = fsq.p;
         const unsigned zb = unsigned((int64_t(npix) * 3 + 255) / 256);
         hipLaunchKernelGGL(k_zero_f64, dim3(zb), dim3(256), 0, s, sum, int64_t(npix) * 3);
         if (sumsq) hipLaunchKernelGGL(k_zero_f64, dim3(zb), dim3(256), 0, s, sumsq, int64_t(npix) * 3);
@@ -963,7 +968,7 @@ int Scene::raycast(const lmgpu_raycast_params* p, double* film_in, bool on_devic
     const int npix = w * h;
     double* film = film_in;
     if (!on_device) {
-        if (fsum.n != size_t(npix) * 3) LMGPU_TRY(fsum.alloc(size_t(npix) * 3));
+        LMGPU_TRY(with_memory([&]() { return fsum.n != size_t(npix) * 3 ? fsum.alloc(size_t(npix) * 3) : LMGPU_OK; }));
         film = fsum.p;
     }
     RaycastConsts rc;

@@ -26,6 +26,10 @@ struct GuidedPass {
 // Path pool and work-queue loop of the regenerating wavefront (batch.hip).
 struct Wavefront;
 void wavefront_destroy(Wavefront* w);
+// Frees the buffer of kept samples: keep = 0 whatever its size, keep > 0 (the
+// samples of the next render) if it is more than twice that and more than the
+// path slots beside it take (16 samples a slot). True if it freed one.
+bool wavefront_give_back(Wavefront* w, int64_t keep);
 
 struct Scene {
     Accel accel;
@@ -73,6 +77,19 @@ struct Scene {
     int create(const lmgpu_scene_desc* d, const lmgpu_build_opts* opts);
     int ensure_workspace(int npix);
     int ensure_guided(int npix, const GuidedPass& gp);
+    // Runs `allocate` (which can be called again after it failed); when it is
+    // out of memory the samples kept by an earlier render, up to 2 GB, are
+    // given back and it runs once more.
+    template <class F>
+    int with_memory(F allocate) {
+        int rc = allocate();
+        if (rc == LMGPU_ERR_OUT_OF_MEMORY && wavefront_give_back(wf, 0)) {
+            (void)hipGetLastError();
+            clear_error();
+            rc = allocate();
+        }
+        return rc;
+    }
     int enqueue_pass(const PTConsts& c, double* sum, double* sumsq, const GuidedPass* gp, hipStream_t s);
     int render(const lmgpu_pt_params* p, double* sum, double* sumsq, bool on_device, const GuidedPass* gp,
                lmgpu_pt_stats* st, hipStream_t s);

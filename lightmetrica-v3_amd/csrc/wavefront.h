@@ -24,7 +24,10 @@
 #define LMGPU_REGEN_MAX_SLOTS (1 << 24)
 #endif
 // Samples a render keeps before they go to the film together: 16 B each, 2 GB
-// at most (64 per pixel at 1080p).
+// at most (64 per pixel at 1080p). The buffer is allocated last, from what memory
+// is left, outlives the render, and is given back when a later call of the
+// scene has no memory for buffers of its own or renders far fewer samples
+// (wavefront_give_back).
 #ifndef LMGPU_REGEN_SAMPLES
 #define LMGPU_REGEN_SAMPLES (1 << 27)
 #endif
