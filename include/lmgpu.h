@@ -120,7 +120,12 @@ int lmgpu_accel_destroy(lmgpu_accel* accel);
  * (p1, p2, p3 world-space positions, FP32), replacing
  * Accel_SAHBVH::build (src/accel/accel_sahbvh.cpp:127-267).
  * `verts_on_device` != 0: `verts` is a device pointer, else host memory.
- * `stream` is a hipStream_t (NULL = default stream). Synchronous on return. */
+ * `stream` is a hipStream_t (NULL = default stream). Synchronous on return.
+ * The build's temporary arrays (some 200 B a triangle) are freed when the first
+ * build of an object ends. An object built again keeps them for its next build
+ * if they are of 2 GiB at most, together with tree arrays of up to twice the
+ * size needed, until lmgpu_accel_destroy or lmgpu_accel_deserialize; a build
+ * that finds no memory beside them frees them first. */
 int lmgpu_accel_build(lmgpu_accel* accel, const float* verts, int64_t num_tris, int verts_on_device,
                       const lmgpu_build_opts* opts, void* stream);
 

@@ -813,7 +813,22 @@ static int reserve(DevBuf<T>& b, size_t count) {
     return fits(b, count) ? LMGPU_OK : b.alloc(count);
 }
 
-int Accel::build(const float* verts_in, int64_t n, bool on_device, const lmgpu_build_opts* opts, hipStream_t s) {
+// With what an object keeps from its last tree a build can find less memory
+// than a first one would: it then starts again as a first one.
+int Accel::build(const float* verts, int64_t n, bool on_device, const lmgpu_build_opts* opts, hipStream_t s) {
+    const bool kept = nodes.p != nullptr;
+    int rc = build_once(verts, n, on_device, opts, s);
+    if (rc == LMGPU_ERR_OUT_OF_MEMORY && kept) {
+        release();
+        (void)hipGetLastError();
+        clear_error();
+        rc = build_once(verts, n, on_device, opts, s);
+    }
+    if (rc != LMGPU_OK && !built) release();
+    return rc;
+}
+
+int Accel::build_once(const float* verts_in, int64_t n, bool on_device, const lmgpu_build_opts* opts, hipStream_t s) {
     int W = opts && opts->width ? opts->width : 4;
     int leaf = opts && opts->leaf_size ? opts->leaf_size : kDefaultLeafSize;
     const int rf = opts && opts->refill ? opts->refill : kDefaultRefill;
@@ -834,11 +849,14 @@ int Accel::build(const float* verts_in, int64_t n, bool on_device, const lmgpu_b
     if (!verts_in) return fail(LMGPU_ERR_INVALID_ARGUMENT, "verts is NULL");
     // A rebuild writes over the tree (and the workspace) of the last one:
     // queries still in flight, on whichever stream, come first.
-    const bool rebuild = built;
+    const bool rebuild = built_here;
     if (nodes.p) LMGPU_HIP(hipDeviceSynchronize());
-    built = false;
+    built = built_here = false;
     if (!fits(tris, n)) tris.reset();
-    if (!fits(nodes, size_t(n) * 2 * W)) nodes.reset();
+    if (!fits(nodes, size_t(n) * 2 * W)) {
+        nodes.reset();
+        qnodes.reset();
+    }
     width = W;
     leaf_size = leaf;
     refill = rf;
@@ -898,10 +916,16 @@ int Accel::build(const float* verts_in, int64_t n, bool on_device, const lmgpu_b
         LMGPU_HIP(hipMemcpyAsync(dverts, verts_in, sizeof(float) * 9 * n, hipMemcpyHostToDevice, s));
         verts = dverts;
     }
-    hipEvent_t e0, e1;
-    LMGPU_HIP(hipEventCreate(&e0));
-    LMGPU_HIP(hipEventCreate(&e1));
-    LMGPU_HIP(hipEventRecord(e0, s));
+    struct Events {
+        hipEvent_t from = nullptr, to = nullptr;
+        ~Events() {
+            if (from) (void)hipEventDestroy(from);
+            if (to) (void)hipEventDestroy(to);
+        }
+    } ev;
+    LMGPU_HIP(hipEventCreate(&ev.from));
+    LMGPU_HIP(hipEventCreate(&ev.to));
+    LMGPU_HIP(hipEventRecord(ev.from, s));
 
     LMGPU_HIP(hipMemsetAsync(head, 0, sizeof(BuildHead), s));
     hipLaunchKernelGGL(k_prep, dim3(nb_prep), dim3(256), 0, s, verts, n, tlo, thi, partial);
@@ -981,14 +1005,12 @@ int Accel::build(const float* verts_in, int64_t n, bool on_device, const lmgpu_b
         bound = sizes[kCollapseLevelsPerSync];
         if (bound == 0) break;
     }
-    LMGPU_HIP(hipEventRecord(e1, s));
+    LMGPU_HIP(hipEventRecord(ev.to, s));
     BuildHead h;   // its counters; the level sizes are known
     LMGPU_HIP(hipMemcpyAsync(&h, head, offsetof(BuildHead, count), hipMemcpyDeviceToHost, s));
     LMGPU_HIP(hipStreamSynchronize(s));
     float ms = 0;
-    LMGPU_HIP(hipEventElapsedTime(&ms, e0, e1));
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
+    LMGPU_HIP(hipEventElapsedTime(&ms, ev.from, ev.to));
     // root half-area for the SAH normalisation
     const float4 rlo = h.root_lo, rhi = h.root_hi;
     const double ra = double(rhi.x - rlo.x) * (rhi.y - rlo.y) + double(rhi.y - rlo.y) * (rhi.z - rlo.z) +
@@ -1001,8 +1023,8 @@ int Accel::build(const float* verts_in, int64_t n, bool on_device, const lmgpu_b
     root_hi[0] = rhi.x; root_hi[1] = rhi.y; root_hi[2] = rhi.z;
     LMGPU_TRY(make_trav_nodes(s));
     LMGPU_HIP(hipGetLastError());
-    give_back.keep = rebuild;
-    built = true;
+    give_back.keep = rebuild && work.n <= kKeptWorkBytes;
+    built = built_here = true;
     return LMGPU_OK;
 }
 

@@ -85,10 +85,13 @@ struct Accel {
     DevBuf<float4> nodes;   // W-wide nodes, 32*W bytes each
     DevBuf<float4> qnodes;  // quantised copy of the nodes (QNode<width>), when quantised_width(width)
     DevBuf<TriV> tris;      // triangles in traversal order
-    // Temporary arrays of the build. Given back when the first build of an
-    // object ends; an object that is built again is taken to be rebuilt every
-    // frame and keeps them (some 200 B a triangle) until it is released.
+    // Temporary arrays of the build, some 200 B a triangle. Given back when the
+    // first build of an object ends; an object that is built again is taken to
+    // be rebuilt every frame and keeps them until it is released, if they are
+    // of kKeptWorkBytes at most.
     DevBuf<char> work;
+    static constexpr size_t kKeptWorkBytes = size_t(1) << 31;
+    bool built_here = false;   // by build() rather than from a serialized form
     DevBuf<int32_t> status; // bit 0: traversal stack overflow
     DevBuf<unsigned long long> ring;  // per-launch ray counters of the persistent kernel
     mutable std::atomic<uint32_t> ring_pos{0};
@@ -114,7 +117,7 @@ struct Accel {
         qnodes.reset();
         tris.reset();
         work.reset();
-        built = false;
+        built = built_here = false;
     }
     int32_t* status_dev() const {
         if (!status.p) {
@@ -139,6 +142,7 @@ struct Accel {
     int stack_bound() const { return (width - 1) * depth; }
 
     int build(const float* verts, int64_t n, bool on_device, const lmgpu_build_opts* opts, hipStream_t s);
+    int build_once(const float* verts, int64_t n, bool on_device, const lmgpu_build_opts* opts, hipStream_t s);
     int trace(const lmgpu_ray* rays, lmgpu_hit* hits, uint8_t* occl, int64_t n, bool any,
               unsigned long long* counters, hipStream_t s) const;
     // As trace, with the caller's ray counter (zeroed by the launch itself)
