@@ -20,7 +20,10 @@ traversal, k_trace): algorithmic bytes per launch = rays x B_ray, with
 B_ray = 32 + 16 + N_node * 32 + N_tri * 36 from the reference SAH BVH's
 mean node visits / triangle tests on the same rays
 (tests/golden/c1_traversal_stats.json), divided by the mean kernel time
-measured with HIP events on the launch stream. `cpu_baseline` times the FP64
+measured with HIP events on the launch stream. That is a model of another
+algorithm's bytes, most of which caches serve here, so its fraction can exceed
+1; what this kernel moved and what bounds it by its counters is in
+`roofline.counted`. `cpu_baseline` times the FP64
 oracle restatement of accel::sahbvh on the host cores.
 """
 from __future__ import annotations
@@ -51,19 +54,21 @@ def log(*a):
     print(*a, file=sys.stderr, flush=True)
 
 
-def traffic_from_profiles():
-    """HBM bytes per launch of the traversal kernel from the committed
-    rocprofv3 --pmc summary (FETCH_SIZE + WRITE_SIZE, scaled by the copy
-    kernel calibration); None if absent."""
+def counters_from_profiles():
+    """Counters of the traversal kernel from the committed rocprofv3 --pmc
+    summary: HBM bytes per launch (FETCH_SIZE + WRITE_SIZE, scaled by the copy
+    kernel calibration) and the busy shares of the units that bound it; {}
+    if absent."""
     p = os.path.join(ROOT, 'profiles', 'trace_c1_incoherent_pmc.json')
     if not os.path.exists(p):
-        return None
+        return {}
     try:
         with open(p) as f:
             d = json.load(f)
-        return float(d['hbm_bytes_per_launch'])
+        keys = ('hbm_bytes_per_launch', 'valu_issue_busy', 'data_return_busy', 'address_unit_busy', 'valu_active_lanes')
+        return {k: float(d[k]) for k in keys}
     except Exception:
-        return None
+        return {}
 
 
 def host_cores():
@@ -251,7 +256,8 @@ def main():
         ref_stats = json.load(f)
     b_ray = ref_stats['incoherent']['bytes_per_ray']
     achieved = n_inc * b_ray / (kern_ms / 1e3) / 1e9
-    traffic = traffic_from_profiles()
+    counted = counters_from_profiles()
+    traffic = counted.pop('hbm_bytes_per_launch', None)
     # the same bytes priced on this build's own tree: its node visits and
     # triangle tests on these rays, at its node size (quantised nodes for
     # widths 4 and 8) and 48-B triangles
@@ -272,6 +278,10 @@ def main():
                              'tri_tests_per_ray': round(own_nt / n_inc, 2), 'node_bytes': node_b,
                              'bytes_per_ray': round(own_b_ray, 1), 'achieved': round(own_achieved, 1),
                              'frac': round(own_achieved / HBM_PEAK_GBS, 4)}}
+    if traffic:
+        gbs = traffic / (kern_ms / 1e3) / 1e9
+        roofline['counted'] = {'achieved': round(gbs, 1), 'frac': round(gbs / HBM_PEAK_GBS, 4),
+                               **{k: round(v, 3) for k, v in counted.items()}}
 
     extra = {'coherent_mrays_s': round(coherent, 1), 'bvh_build_ms': round(info['build_ms'], 2),
              'bvh': {k: info[k] for k in ('width', 'leaf_size', 'num_nodes', 'depth', 'sah_cost')}}

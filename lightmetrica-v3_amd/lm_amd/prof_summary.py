@@ -11,7 +11,11 @@ Counter summary of one kernel (JSON) from the --pmc passes of
 lm_amd/profile_trace.py (FETCH_SIZE, WRITE_SIZE, TCC_HIT/MISS, SQ_*):
 
     python3 lightmetrica-v3_amd/lm_amd/prof_summary.py --pmc 'k_trace<4' --fetch F.csv --write W.csv \
-        [--tcc T.csv] [--sq S.csv] [--trace KT.csv]
+        [--tcc T.csv] [--sq S.csv] [--ta A.csv] [--trace KT.csv]
+
+--ta is a pass of TA_TA_BUSY_sum, TD_TD_BUSY_sum and GRBM_GUI_ACTIVE (summed
+over the 8 XCDs): busy shares of the vector memory path's address and
+data-return units and, with --sq, of the vector ALUs' issue.
 """
 import argparse
 import csv
@@ -19,6 +23,9 @@ import re
 import sqlite3
 import sys
 from collections import defaultdict
+
+
+XCDS, CUS = 8, 256   # of the MI355X
 
 
 def load(path):
@@ -51,13 +58,14 @@ def main(argv=None):
     ap.add_argument('--write')
     ap.add_argument('--tcc')
     ap.add_argument('--sq')
+    ap.add_argument('--ta')
     ap.add_argument('--trace')
     ap.add_argument('--units', type=int, default=0)
     a = ap.parse_args(argv)
     if a.pmc:
         import json
         print(json.dumps(pmc_summary(a.pmc, a.fetch, a.write, a.tcc, a.sq, a.trace or a.path,
-                                     units_per_launch=a.units or None), indent=1))
+                                     units_per_launch=a.units or None, ta_csv=a.ta), indent=1))
         return 0
     stats = defaultdict(list)
     for name, dur in load(a.path):
@@ -74,7 +82,7 @@ def main(argv=None):
 
 
 def pmc_summary(kernel_substr, fetch_csv, write_csv, tcc_csv=None, sq_csv=None, trace_csv=None, copy_bytes=512 << 20,
-                units_per_launch=None):
+                units_per_launch=None, ta_csv=None):
     """HBM traffic and efficiency counters of one kernel from rocprofv3
     --pmc runs of lm_amd/profile_trace.py. FETCH_SIZE / WRITE_SIZE (KiB per
     dispatch) are scaled by what they read for the profile driver's device
@@ -125,6 +133,15 @@ def pmc_summary(kernel_substr, fetch_csv, write_csv, tcc_csv=None, sq_csv=None, 
         if 'SQ_THREAD_CYCLES_VALU' in out['SQ'] and 'SQ_ACTIVE_INST_VALU' in out['SQ']:
             # average active lanes per VALU instruction (of 64)
             out['valu_active_lanes'] = out['SQ']['SQ_THREAD_CYCLES_VALU'] / out['SQ']['SQ_ACTIVE_INST_VALU']
+    if ta_csv:
+        ta = per_dispatch(ta_csv, kern)
+        cycles = mean(ta, 'GRBM_GUI_ACTIVE') / XCDS
+        out['cycles'] = cycles
+        out['address_unit_busy'] = mean(ta, 'TA_TA_BUSY_sum') / (cycles * CUS)
+        out['data_return_busy'] = mean(ta, 'TD_TD_BUSY_sum') / (cycles * CUS)
+        if 'SQ' in out:
+            # SQ_ACTIVE_INST_VALU counts in units of 4 cycles, over 4 SIMDs a CU
+            out['valu_issue_busy'] = 4.0 * out['SQ']['SQ_ACTIVE_INST_VALU'] / (cycles * 4 * CUS)
     return out
 
 
