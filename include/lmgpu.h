@@ -290,7 +290,10 @@ typedef struct lmgpu_pt_stats {
  * `film_sum` / `film_sumsq` (either may be NULL... sum is required).
  * `film_on_device` != 0: device pointers, else host pointers (copied back on
  * return). The film value of renderer::pt is film_sum / spp
- * (renderer_pt.cpp:307-308). Synchronous. */
+ * (renderer_pt.cpp:307-308). Synchronous. A scene keeps its path pool and, when
+ * memory allows, up to 2 GB of finished samples between renders; the samples'
+ * buffer is freed by a render of far fewer samples or when a call of the scene
+ * needs the memory, both by lmgpu_scene_destroy. */
 int lmgpu_pt_render(lmgpu_scene* scene, const lmgpu_pt_params* params, double* film_sum, double* film_sumsq,
                     int film_on_device, lmgpu_pt_stats* stats, void* stream);
 

@@ -488,8 +488,9 @@ __device__ __host__ inline uint32_t ray_share(uint32_t n, uint32_t nwaves) {
 // multi-BVH arena);
 // `emit(id, res)` consumes its result.
 //
-// The loop is bound by the instructions it issues (26 of 64 lanes active),
-// so a node step has no branch in the common case: lds[0][lane] holds kDone
+// The loop is bound by the instructions it issues (29 of 64 lanes active; vector
+// issue busy 78% on incoherent rays) and by the return of its divergent 16-B
+// node loads (data return busy 77%, address unit 68%), so a node step has no branch in the common case: lds[0][lane] holds kDone
 // and entry i of the lane's stack lds[1 + i][lane]; each child is written at
 // the top of the stack and the stack grows by one only if the child was hit,
 // so what lies above the top is garbage that the next push overwrites; and
@@ -500,9 +501,8 @@ __device__ __host__ inline uint32_t ray_share(uint32_t n, uint32_t nwaves) {
 // only when lanes are refilled: done as each ray ends, the FP64
 // re-evaluation ran in most iterations for a lane or two.
 // Measured on the 1.32M-triangle mesh together with the waves' own shares
-// (below): 2.07M primary rays 723 -> 492 us, 2M incoherent rays 952 -> 890
-// (bound by the 16-B accesses of its divergent node loads: the address unit is
-// busy 75% of the time), 500K any-hit rays on the 8-wide tree 515 -> 382.
+// (below), timed in turn: 2.07M primary rays 719 -> 459 us, 2M incoherent rays
+// 1018 -> 904, 500K any-hit rays on the 8-wide tree 516 -> 353.
 template <int W, bool ANY, bool COUNT, int LDS_DEPTH, int PRIV_DEPTH, int BLOCK, class Node, class Fetch, class Emit>
 __device__ __forceinline__ void trace_persistent(const Node* __restrict__ nodes, const TriV* __restrict__ tris,
                                                  uint32_t n, unsigned long long* next, int (*lds)[BLOCK],

@@ -95,8 +95,8 @@ struct Scene {
                lmgpu_pt_stats* st, hipStream_t s);
     int raycast(const lmgpu_raycast_params* p, double* film, bool on_device, hipStream_t s);
     // A fixed-spp pixel-mode render through the regenerating wavefront: a pool of
-    // path slots that take the render's (sample, pixel) items in order and add a
-    // finished sample to the film at once (FP64 atomics), so paths of later samples
+    // path slots that take the render's (sample, pixel) items in order and keep
+    // finished samples until they go to the film together, so paths of later samples
     // fill the slots that short paths free instead of each bounce waiting for a
     // pass's longest paths. Same Philox streams and per-vertex code as the passes.
     // With a guide (gp), directions at diffuse and glossy vertices come from
